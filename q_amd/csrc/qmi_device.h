@@ -55,6 +55,7 @@ struct WinDev {
   int g_off, ngrp, ngrp_solute;     // charge groups
   int wc_off, nwc, sc_off, nsc, qc_off, nqc;
   int sh_off, nshell;               // water polarisation shells
+  long long wp_off;                 // first entry of the window's shell rows in Dev::wtheta
   int nsteps, nbcycle, iene, iout;
   int use_lrf, wpol, separate_scaling, iac_ow;   // iac_ow: 0-based type of water O
   int ndegf, ndegfree, ndegf_solute, ndegfree_solute, ndegf_solvent, ndegfree_solvent;
@@ -128,6 +129,8 @@ constexpr int kTempParts = 8;      // blocks per window of the kinetic-energy su
 // part order; fixed, so the expansions do not depend on launch shapes
 constexpr int kLrfParts = 8;
 constexpr int kIntBlock = 256;     // atoms per block of the integrator
+constexpr int kWpolMaxShell = 8;
+constexpr int kWpolLds = 4096;     // waters of one polarisation shell held (and ordered) in LDS
 constexpr int kGatherAtoms = 256;  // atoms per block of the bonded gather
 constexpr int kGatherSlots = 2048; // slots staged in LDS per gather block
 constexpr int kBondTileTerms = 512; // bonded terms per tile
@@ -323,11 +326,7 @@ struct Dev {
   const int4* iu; const int* iu_atom; const int4* ib;
   // water shells
   ShellDev* shells;
-  double* wtheta;        // per water (global water index), theta
-  int* wshell;           // shell index (-1 if none)
-  int* wrank;            // place in its shell's order (theta, water index), from 0
-  const int* w_off;      // per window: first global water index
-  const int* wat_win;    // per global water: its window
+  double* wtheta;        // windows of more than kWpolLds waters: theta per shell and water, at WinDev::wp_off
   int nwat_total;
   // energy snapshots for output: [ring slot][window][E_NSLOT] + temperature
   long long* e_ring;

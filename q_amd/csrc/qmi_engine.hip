@@ -231,7 +231,7 @@ static int build_device(qmi_engine* e) {
   std::vector<float2> sc_w;
   // shells
   std::vector<ShellDev> shells;
-  std::vector<int> w_off(NW), wat_win;
+  long long wp_rows = 0;
   // static Q tiles (host-built), per type: per i-cluster lists
   struct HT { std::vector<std::vector<std::pair<int, uint2>>> l; std::vector<std::vector<uint2>> m14; };
   HT qt[4];  // T_QP, T_PQ, T_QW, T_WQ
@@ -751,14 +751,15 @@ static int build_device(qmi_engine* e) {
     // --- water shells
     D.sh_off = (int)shells.size();
     D.nshell = (int)W.wshell.size();
-    if (D.nshell > 8) return set_err(-10, "more than 8 water polarisation shells");
+    if (D.nshell > kWpolMaxShell) return set_err(-10, "more than 8 water polarisation shells");
+    D.wp_off = wp_rows;
+    if (W.nwat > kWpolLds) wp_rows += (long long)D.nshell * W.nwat;
     for (auto& sh : W.wshell) {
       ShellDev s{};
       s.rout = sh.rout; s.dr = sh.dr; s.cstb = sh.cstb; s.theta_corr = sh.theta_corr;
       s.avtheta = 0.f; s.avn_insh = 0.f; s.n_insh = 0;
       shells.push_back(s);
     }
-    w_off[wi] = woff;
     // --- state
     WinState& st = wst[wi];
     std::memset(&st, 0, sizeof(st));
@@ -769,7 +770,6 @@ static int build_device(qmi_engine* e) {
     st.tscale_solvent = 0.0;
     ao += N;
     goff += (int)t.cgp.size();
-    for (int iw = 0; iw < W.nwat; ++iw) wat_win.push_back(wi);
     woff += W.nwat;
     qoff += fp.nqat;
     toff += t.natyps;
@@ -1183,11 +1183,7 @@ static int build_device(qmi_engine* e) {
   UP(f2, sc_w); d.sc_w = f2;
   ShellDev* sd;
   UP(sd, shells); d.shells = sd;
-  if ((rc = dev_alloc(e, &d.wtheta, (size_t)e->nwat_total)) != 0) return rc;
-  if ((rc = dev_alloc(e, &d.wshell, (size_t)e->nwat_total)) != 0) return rc;
-  if ((rc = dev_alloc(e, &d.wrank, (size_t)e->nwat_total)) != 0) return rc;
-  UP(ip, w_off); d.w_off = ip;
-  UP(ip, wat_win); d.wat_win = ip;
+  if ((rc = dev_alloc(e, &d.wtheta, (size_t)wp_rows)) != 0) return rc;
   d.nwat_total = e->nwat_total;
   // two chunks of kChunk steps: one drains while the next runs
   d.ring_n = 2 * kChunk;

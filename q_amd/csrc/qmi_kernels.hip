@@ -2199,67 +2199,96 @@ __global__ void __launch_bounds__(64) k_prestr(Dev d) {
   }
 }
 
-// water polarisation restraint (watpol, md.f90:15122-15288) in two passes.
-// Pass 1, one thread per water: the angle theta between the dipole and the
-// radial vector, and the shell the oxygen lies in.
-__global__ void __launch_bounds__(256) k_watpol_theta(Dev d) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= d.nwat_total) return;
-  const int w = d.wat_win[g];
-  const WinDev& W = d.win[w];
-  d.wshell[g] = -1;
-  if (!d.ws[w].active || !W.wpol || W.nshell == 0) return;
-  const ShellDev* sh = d.shells + W.sh_off;
-  const int nsh = W.nshell;
-  const int iw = g - d.w_off[w];
-  const int i = W.ao + W.nat_solute + 3 * iw;
-  d.wtheta[g] = 0.0;
-  if (d.aflag[i] & 1) return;
-  const double* x = d.x;
-  double rmu[3], rcu[3];
+// water polarisation restraint (watpol, md.f90:15122-15288), one block per
+// (window, shell): the waters whose oxygen lies in the shell are collected in
+// LDS with the angle theta between their dipole and the radial vector, each
+// one's place in the order of the reference's first-minimum selection sort
+// (theta ascending, ties by water index) is found by counting the members
+// before it, and the place gives its target angle theta0, energy and forces.
+// The block also advances the shell's theta averages.
+//
+// Bound by latency: a shell has a few hundred waters, so counting is
+// n^2 LDS reads over one block.  A member's count is split over as many
+// threads as the block has for it (2 at 400 members), and compares one FP64
+// value per step; ties, which need the indices, are recounted.  As three
+// kernels (angles per water, ranking with a quarter of the threads, forces
+// per water) with the places passed through memory the chain took 30 us alone
+// for one 1109-water window and 65 us for a 1693-water one and was the step's
+// critical path there: a step of one window took 116 and 166 us, now 96 and
+// 124 us.
+__device__ __forceinline__ void water_dipole(const double* x, int i, const double cent[3], double rmu[3], double rcu[3],
+                                             double* rm, double* rc) {
   for (int c = 0; c < 3; ++c) rmu[c] = x[3 * (i + 1) + c] + x[3 * (i + 2) + c] - 2. * x[3 * i + c];
-  const double rm = sqrt(rmu[0] * rmu[0] + rmu[1] * rmu[1] + rmu[2] * rmu[2]);
-  for (int c = 0; c < 3; ++c) rmu[c] /= rm;
-  for (int c = 0; c < 3; ++c) rcu[c] = x[3 * i + c] - W.xwcent[c];
-  const double rc = sqrt(rcu[0] * rcu[0] + rcu[1] * rcu[1] + rcu[2] * rcu[2]);
-  for (int c = 0; c < 3; ++c) rcu[c] /= rc;
-  double scp = rmu[0] * rcu[0] + rmu[1] * rcu[1] + rmu[2] * rcu[2];
-  scp = fmin(1.0, fmax(-1.0, scp));
-  d.wtheta[g] = acos(scp);
-  // shell bounds are real(4): rout - dr is a single-precision difference
-  if (rc > (double)(sh[nsh - 1].rout - sh[nsh - 1].dr)) {
-    int is = nsh - 1;
-    for (; is >= 1; --is)
-      if (rc <= (double)sh[is].rout) break;
-    d.wshell[g] = is;
+  *rm = sqrt(rmu[0] * rmu[0] + rmu[1] * rmu[1] + rmu[2] * rmu[2]);
+  for (int c = 0; c < 3; ++c) rmu[c] /= *rm;
+  for (int c = 0; c < 3; ++c) rcu[c] = x[3 * i + c] - cent[c];
+  *rc = sqrt(rcu[0] * rcu[0] + rcu[1] * rcu[1] + rcu[2] * rcu[2]);
+  for (int c = 0; c < 3; ++c) rcu[c] /= *rc;
+}
+// cosine of the angle between the unit vectors, clipped to [-1, 1]
+__device__ __forceinline__ double dipole_cos(const double rmu[3], const double rcu[3]) {
+  const double scp = rmu[0] * rcu[0] + rmu[1] * rcu[1] + rmu[2] * rcu[2];
+  return fmin(1.0, fmax(-1.0, scp));
+}
+// energy and forces of water atom group i (its oxygen) at place `rank` of the
+// n members of its shell
+__device__ __forceinline__ double watpol_force(const Dev& d, const WinDev& W, float cstb_f, float corr_f, int n, int i,
+                                               int rank, double th) {
+  const double pi = (double)(4.0f * atanf(1.0f));
+  const double cstb = (double)cstb_f, tc = (double)corr_f;
+  const int il = rank + 1;
+  const float argf = 1.0f + (1.0f - 2.0f * (float)il) / (float)n;
+  double th0 = acos((double)argf);
+  th0 = th0 - 3. * sin(th0) * cstb / 2.;
+  th0 = fmin(fmax(th0, 0.0), pi);
+  const double dth = th - th0 + tc;
+  const double dv = W.fkwpol * dth;
+  double rmu[3], rcu[3], rm, rc;
+  water_dipole(d.x, i, W.xwcent, rmu, rcu, &rm, &rc);
+  const double scp = dipole_cos(rmu, rcu);
+  double f0 = sin(acos(scp));
+  if (fabs(f0) < 1.e-12) f0 = 1.e-12;
+  f0 = dv * (-1.0 / f0);
+  double f1[3], f2[3];
+  for (int c = 0; c < 3; ++c) {
+    f1[c] = (rcu[c] - rmu[c] * scp) / rm;
+    f2[c] = (rmu[c] - rcu[c] * scp) / rc;
   }
+  add_grad(d.f, i, f0 * (-2. * f1[0] + f2[0]), f0 * (-2. * f1[1] + f2[1]), f0 * (-2. * f1[2] + f2[2]));
+  add_grad(d.f, i + 1, f0 * f1[0], f0 * f1[1], f0 * f1[2]);
+  add_grad(d.f, i + 2, f0 * f1[0], f0 * f1[1], f0 * f1[2]);
+  return 0.5 * W.fkwpol * dth * dth;
 }
 
-// Pass 2, one block per (window, shell): the shell's waters are gathered in
-// LDS with their theta and sorted (theta ascending, ties by water index: the
-// order of the reference's first-minimum selection sort); a water's place in
-// that order, stored per water, gives its target angle theta0 in pass 3.  The
-// block also advances the shell's theta averages.
-constexpr int kWpolMaxShell = 8;
-constexpr int kWpolLds = 4096;       // waters of one shell held (and sorted) in LDS
-constexpr int kWpolRank = 1024;      // shells up to this size are ordered by counting
-constexpr int kWpolBlock = 256;      // threads per (window, shell) block
-__global__ void __launch_bounds__(kWpolBlock) k_watpol_shell(Dev d) {
+// up to this many windows per engine a block has 1024 threads, beyond it 256:
+// a wide block shortens the chain (a step of one 1693-water window 153 -> 124
+// us, of 4 177 -> 147, of 16 259 -> 254), but its 16 waves start only on a CU
+// with that many free slots, and among many windows the ranking is not what
+// the step waits for (32 small windows 185 -> 187 us, 64 mixed 583 -> 598).
+// The results do not depend on the block size
+constexpr int kWpolWide = 24;
+constexpr int kWpolSum = 256;        // threads of the theta sum (its order is part of the result)
+template <int kWpolBlock>            // threads per (window, shell) block
+__global__ void __launch_bounds__(kWpolBlock) k_watpol(Dev d) {
+  constexpr int kWpolHeld = kWpolLds / kWpolBlock;   // members per thread of a shell held in LDS
   const int w = blockIdx.x / kWpolMaxShell, is = blockIdx.x % kWpolMaxShell;
   if (w >= d.nwin) return;
   const WinState& st = d.ws[w];
   const WinDev& W = d.win[w];
-  if (!st.active || !W.wpol || W.nwat == 0 || is >= W.nshell) return;
+  const int nsh = W.nshell;
+  if (!st.active || !W.wpol || W.nwat == 0 || is >= nsh) return;
+  const ShellDev* shells = d.shells + W.sh_off;
   ShellDev& sh = d.shells[W.sh_off + is];
-  const int wo = d.w_off[w];
   __shared__ double s_th[kWpolLds];
-  __shared__ int s_iw[kWpolLds];
+  __shared__ int s_iw[kWpolLds], s_rank[kWpolBlock];
   __shared__ int s_n;
-  __shared__ double s_red[4][2];
+  __shared__ float s_corr;
+  __shared__ double s_red[kWpolSum / 64];
+  const int t = threadIdx.x;
   // theta_corr follows the shell's mean theta every 100 steps; only the
   // pot_energy calls of the run (MD steps and the final evaluation) advance
   // the shell averages, so extra evaluations (tuning, queries) leave them
-  if (threadIdx.x == 0) {
+  if (t == 0) {
     if (st.wpol_acc && st.istep != 0 && st.istep % 100 == 0) {
       sh.avtheta = sh.avtheta / 100.0f;
       sh.avn_insh = sh.avn_insh / 100.0f;
@@ -2267,160 +2296,120 @@ __global__ void __launch_bounds__(kWpolBlock) k_watpol_shell(Dev d) {
       sh.avtheta = 0.0f;
       sh.avn_insh = 0.0f;
     }
+    s_corr = sh.theta_corr;
     s_n = 0;
   }
+  s_rank[t] = 0;
   __syncthreads();
-  for (int iw = threadIdx.x; iw < W.nwat; iw += blockDim.x) {
-    if (d.wshell[wo + iw] != is) continue;
+  // the shell's bounds: waters beyond the innermost radius (a single-precision
+  // difference, as the bounds are real(4)) lie in the innermost shell whose
+  // outer radius holds them, the rest in shell 0
+  const double r_in = (double)(shells[nsh - 1].rout - shells[nsh - 1].dr);
+  const double r_out = is > 0 ? (double)sh.rout : 1e300;
+  const double r_next = is < nsh - 1 ? (double)shells[is + 1].rout : r_in;
+  const int o0 = W.ao + W.nat_solute;
+  // a window whose shells could outgrow LDS has a row of its waters' angles
+  // per shell in memory (-1: not in the shell)
+  double* row = W.nwat > kWpolLds ? d.wtheta + W.wp_off + (size_t)is * W.nwat : nullptr;
+  for (int iw = t; iw < W.nwat; iw += kWpolBlock) {
+    const int i = o0 + 3 * iw;
+    if (row) row[iw] = -1.0;
+    if (d.aflag[i] & 1) continue;
+    double c[3];
+    for (int k = 0; k < 3; ++k) c[k] = d.x[3 * i + k] - W.xwcent[k];
+    const double rc = sqrt(c[0] * c[0] + c[1] * c[1] + c[2] * c[2]);
+    if (!(rc > r_in && rc > r_next && rc <= r_out)) continue;
+    double rmu[3], rcu[3], rm, rd;
+    water_dipole(d.x, i, W.xwcent, rmu, rcu, &rm, &rd);
+    const double th = acos(dipole_cos(rmu, rcu));
+    if (row) row[iw] = th;
     const int k = atomicAdd(&s_n, 1);
-    if (k < kWpolLds) { s_th[k] = d.wtheta[wo + iw]; s_iw[k] = iw; }
+    if (k < kWpolLds) { s_th[k] = th; s_iw[k] = iw; }
   }
   __syncthreads();
   const int n = s_n;
   const bool in_lds = n <= kWpolLds;
-  if (n <= kWpolRank) {
-    // place of each member by counting the members before it in the order
-    // (theta, water index), then a scatter to that place: the sorted order
-    // the bitonic network gives, in n^2/blockDim compares instead of its
-    // log^2 barrier stages
-    double th[kWpolRank / kWpolBlock];
-    int iw[kWpolRank / kWpolBlock], rank[kWpolRank / kWpolBlock];
+  double th[kWpolHeld];
+  int iw[kWpolHeld], rank[kWpolHeld];
+  if (in_lds) {
+    // threads per member: 8, 4, 2 or 1; a part's j are uniform over a wave
+    int span = 128;
+    while (span < n && span < kWpolBlock) span <<= 1;
+    const int parts = kWpolBlock / span, part = t / span, j0 = part * n / parts, j1 = (part + 1) * n / parts;
 #pragma unroll
-    for (int m = 0; m < kWpolRank / kWpolBlock; ++m) {
-      const int k = threadIdx.x + kWpolBlock * m;
+    for (int m = 0; m < kWpolHeld; ++m) {
+      const int k = t % span + kWpolBlock * m;
       rank[m] = -1;
       if (k >= n) continue;
       th[m] = s_th[k];
       iw[m] = s_iw[k];
-      int r = 0;
-      for (int j = 0; j < n; ++j) {
+      int r = 0, eq = 0;
+      for (int j = j0; j < j1; ++j) {
         const double tj = s_th[j];
-        r += (tj < th[m] || (tj == th[m] && s_iw[j] < iw[m])) ? 1 : 0;
+        r += tj < th[m] ? 1 : 0;
+        eq += tj == th[m] ? 1 : 0;
       }
+      if (eq > (k >= j0 && k < j1 ? 1 : 0))   // other members at the same angle
+        for (int j = j0; j < j1; ++j) r += (s_th[j] == th[m] && s_iw[j] < iw[m]) ? 1 : 0;
       rank[m] = r;
+      if (parts > 1) atomicAdd(&s_rank[k], r);
     }
     __syncthreads();
+    // the members in order
 #pragma unroll
-    for (int m = 0; m < kWpolRank / kWpolBlock; ++m)
-      if (rank[m] >= 0) { s_th[rank[m]] = th[m]; s_iw[rank[m]] = iw[m]; }
-    __syncthreads();
-  } else if (in_lds) {
-    // bitonic sort of (theta, water index) ascending; padding keys sort last
-    int np = 1;
-    while (np < n) np <<= 1;
-    for (int k = n + threadIdx.x; k < np; k += blockDim.x) { s_th[k] = 1e300; s_iw[k] = 0x7fffffff; }
-    __syncthreads();
-    for (int size = 2; size <= np; size <<= 1) {
-      for (int stride = size >> 1; stride > 0; stride >>= 1) {
-        for (int k = threadIdx.x; k < np; k += blockDim.x) {
-          const int l = k ^ stride;
-          if (l > k) {
-            const bool up = (k & size) == 0;
-            const double tk = s_th[k], tl = s_th[l];
-            const int ik = s_iw[k], il = s_iw[l];
-            const bool k_after_l = tk > tl || (tk == tl && ik > il);
-            if (k_after_l == up) { s_th[k] = tl; s_th[l] = tk; s_iw[k] = il; s_iw[l] = ik; }
-          }
-        }
-        __syncthreads();
-      }
+    for (int m = 0; m < kWpolHeld; ++m) {
+      if (rank[m] < 0 || part != 0) continue;
+      const int r = parts > 1 ? s_rank[t] : rank[m];
+      s_th[r] = th[m];
+      s_iw[r] = iw[m];
     }
+    __syncthreads();
   }
-  // each member's place in the order, for the per-water pass, and the
-  // shell's theta sum in a fixed order: members sorted in LDS (place =
-  // index), or (shell larger than LDS) straight from the window's waters with
-  // their place counted
-  double tsum = 0.0;
-  const int nloop = in_lds ? n : W.nwat;
-  for (int k = threadIdx.x; k < nloop; k += blockDim.x) {
-    int iw, rank = 0;
-    double th;
+  // the shell's theta sum in a fixed order: members in their order (or, from
+  // memory, in water order), over kWpolSum threads, the waves, the wave sums
+  if (t < kWpolSum) {
+    double tsum = 0.0;
     if (in_lds) {
-      iw = s_iw[k];
-      th = s_th[k];
-      rank = k;
+      for (int k = t; k < n; k += kWpolSum) tsum += s_th[k];
     } else {
-      iw = k;
-      if (d.wshell[wo + iw] != is) continue;
-      th = d.wtheta[wo + iw];
-      for (int jw = 0; jw < W.nwat; ++jw) {
-        if (d.wshell[wo + jw] != is) continue;
-        const double tj = d.wtheta[wo + jw];
-        rank += (tj < th || (tj == th && jw < iw)) ? 1 : 0;
-      }
+      for (int k = t; k < W.nwat; k += kWpolSum) tsum += row[k] >= 0.0 ? row[k] : 0.0;
     }
-    d.wrank[wo + iw] = rank;
-    tsum += th;
+    tsum = wave_sum(tsum);
+    if ((t & 63) == 0) s_red[t >> 6] = tsum;
   }
-  // block sum in a fixed order (waves, then the 4 wave results)
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const double t_w = wave_sum(tsum);
-  if (lane == 0) s_red[wv][0] = t_w;
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (t == 0) {
     if (n > 0 && st.wpol_acc) {
-      const double avtdum = (s_red[0][0] + s_red[1][0]) + (s_red[2][0] + s_red[3][0]);
+      const double avtdum = (s_red[0] + s_red[1]) + (s_red[2] + s_red[3]);
       // real(4) + real(8) quotient, rounded once (md.f90:15285)
       sh.avtheta = (float)((double)sh.avtheta + avtdum / (double)(float)n);
       sh.avn_insh = sh.avn_insh + (float)n;
     }
     sh.n_insh = n;
   }
-}
-
-// Pass 3, one thread per water in a shell: the target angle theta0 from the
-// water's place in its shell's order, then the restraint's energy and the
-// forces on its three atoms (the loop over il of watpol)
-__global__ void __launch_bounds__(256) k_watpol_force(Dev d) {
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  int w = 0;
-  bool on = false;
-  double e = 0.0;
-  if (g < d.nwat_total) {
-    w = d.wat_win[g];
-    const WinState& st = d.ws[w];
-    const WinDev& W = d.win[w];
-    const int is = d.wshell[g];   // -1 unless in a shell of an active window with polarisation
-    if (is >= 0) {
-      const ShellDev& sh = d.shells[W.sh_off + is];
-      const double pi = (double)(4.0f * atanf(1.0f));
-      const double cstb = (double)sh.cstb, tc = (double)sh.theta_corr;
-      const int n = sh.n_insh;
-      const int il = d.wrank[g] + 1;
-      const double th = d.wtheta[g];
-      const float argf = 1.0f + (1.0f - 2.0f * (float)il) / (float)n;
-      double th0 = acos((double)argf);
-      th0 = th0 - 3. * sin(th0) * cstb / 2.;
-      th0 = fmin(fmax(th0, 0.0), pi);
-      const double dth = th - th0 + tc;
-      e = 0.5 * W.fkwpol * dth * dth;
-      on = st.energy_now;
-      const double dv = W.fkwpol * dth;
-      const int i = W.ao + W.nat_solute + 3 * (g - d.w_off[w]);
-      const double* x = d.x;
-      double rmu[3], rcu[3];
-      for (int c = 0; c < 3; ++c) rmu[c] = x[3 * (i + 1) + c] + x[3 * (i + 2) + c] - 2. * x[3 * i + c];
-      const double rm = sqrt(rmu[0] * rmu[0] + rmu[1] * rmu[1] + rmu[2] * rmu[2]);
-      for (int c = 0; c < 3; ++c) rmu[c] /= rm;
-      for (int c = 0; c < 3; ++c) rcu[c] = x[3 * i + c] - W.xwcent[c];
-      const double rc = sqrt(rcu[0] * rcu[0] + rcu[1] * rcu[1] + rcu[2] * rcu[2]);
-      for (int c = 0; c < 3; ++c) rcu[c] /= rc;
-      double scp = rmu[0] * rcu[0] + rmu[1] * rcu[1] + rmu[2] * rcu[2];
-      scp = fmin(1.0, fmax(-1.0, scp));
-      double f0 = sin(acos(scp));
-      if (fabs(f0) < 1.e-12) f0 = 1.e-12;
-      f0 = dv * (-1.0 / f0);
-      double f1[3], f2[3];
-      for (int c = 0; c < 3; ++c) {
-        f1[c] = (rcu[c] - rmu[c] * scp) / rm;
-        f2[c] = (rmu[c] - rcu[c] * scp) / rc;
+  // forces, every lane to the energy sum
+  const int nloop = in_lds ? n : W.nwat;
+  const bool en = st.energy_now;
+  for (int k0 = 0; k0 < nloop; k0 += kWpolBlock) {
+    const int k = k0 + t;
+    double e = 0.0;
+    bool on = k < nloop;
+    if (on && in_lds) {
+      e = watpol_force(d, W, sh.cstb, s_corr, n, o0 + 3 * s_iw[k], k, s_th[k]);
+    } else if (on) {
+      const double tk = row[k];
+      on = tk >= 0.0;
+      if (on) {
+        int r = 0;
+        for (int j = 0; j < W.nwat; ++j) {
+          const double tj = row[j];
+          r += tj >= 0.0 && (tj < tk || (tj == tk && j < k)) ? 1 : 0;
+        }
+        e = watpol_force(d, W, sh.cstb, s_corr, n, o0 + 3 * k, r, tk);
       }
-      add_grad(d.f, i, f0 * (-2. * f1[0] + f2[0]), f0 * (-2. * f1[1] + f2[1]), f0 * (-2. * f1[2] + f2[2]));
-      add_grad(d.f, i + 1, f0 * f1[0], f0 * f1[1], f0 * f1[2]);
-      add_grad(d.f, i + 2, f0 * f1[0], f0 * f1[1], f0 * f1[2]);
     }
+    wave_energy(d.ws, w, E_WPOL, e, on && en);
   }
-  wave_energy(d.ws, w, E_WPOL, e, on);
 }
 
 // the FP32 coordinates of atom i from its FP64 ones, into x32 and, for a
@@ -2957,9 +2946,8 @@ hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, hipSt
 // large pair kernels of the other streams instead of after them
 void launch_other_forces(const Dev& d, hipStream_t s, bool atom_terms) {
   if (d.nwat_total) {
-    k_watpol_theta<<<blocks(d.nwat_total, 256), 256, 0, s>>>(d);
-    k_watpol_shell<<<d.nwin * kWpolMaxShell, kWpolBlock, 0, s>>>(d);
-    k_watpol_force<<<blocks(d.nwat_total, 256), 256, 0, s>>>(d);
+    if (d.nwin <= kWpolWide) k_watpol<1024><<<d.nwin * kWpolMaxShell, 1024, 0, s>>>(d);
+    else k_watpol<256><<<d.nwin * kWpolMaxShell, 256, 0, s>>>(d);
   }
   if (atom_terms) k_atom_terms<false><<<blocks(d.ntot, 256), 256, 0, s>>>(d);
   int nb = d.nbond + d.nang + d.ntor + d.nimp + d.nqb + d.nqa + d.nqt + d.nqi;
