@@ -122,7 +122,7 @@ int qmi_window_info(qmi_engine* e, int w, int32_t* info, int cap);
 int qmi_write_restart(qmi_engine* e, int w, const char* path);
 
 /* The autotuner (on by default) times candidate launch shapes of the Q-tile,
- * pair-row, LRF-build and bonded kernels on the engine's own windows during
+ * pair-row and bonded kernels on the engine's own windows during
  * qmi_prepare and keeps the fastest; the candidates do not change results.
  * Call before qmi_prepare.  No reference counterpart. */
 int qmi_set_autotune(qmi_engine* e, int on);
@@ -130,8 +130,8 @@ int qmi_set_autotune(qmi_engine* e, int on);
 /* Choices of the autotuner: Q tiles per wave, threads per block of the row,
  * LRF-build and bonded kernels, whether blocks are grouped by XCD (0/1),
  * the bonded mode (0: per-term slots and a per-atom gather, 1: atomics, 2:
- * LDS sums per tile of terms), the number of source parts
- * of the LRF build, then the measured microseconds of the first six chosen
+ * LDS sums per tile of terms), the number of source shares
+ * of the LRF build (its shapes are fixed), then the measured microseconds of the first six chosen
  * configurations (13 values).  Returns the number written. */
 int qmi_tuning(qmi_engine* e, double* out, int cap);
 

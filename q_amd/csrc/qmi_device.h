@@ -125,9 +125,11 @@ struct TileList {
 // T_free solute, T_free solvent
 constexpr int kTRing = 6;
 constexpr int kTempParts = 8;      // blocks per window of the kinetic-energy sum
-// the LRF build splits a window's source groups in this many parts, summed in
-// part order; fixed, so the expansions do not depend on launch shapes
-constexpr int kLrfParts = 8;
+// the LRF build splits a window's source groups in kLrfParts parts (blocks) of
+// kLrfWaves shares (waves), summed in a fixed order; constants, so the
+// expansions do not depend on launch shapes
+constexpr int kLrfParts = 4;
+constexpr int kLrfWaves = 8;
 constexpr int kIntBlock = 256;     // atoms per block of the integrator
 constexpr int kWpolMaxShell = 8;
 constexpr int kWpolLds = 4096;     // waters of one polarisation shell held (and ordered) in LDS
@@ -193,9 +195,9 @@ struct Dev {
   double* g_cent;       // 3 per group
   double* g_lrf;        // 20 per group: phi0, phi1(3), phi2(6: xx xy xz yy yz zz), phi3(10)
   int ngrp_all;         // groups of all windows
-  int nlrfw;            // LRF build blocks: (window, first target group, count, source part)
+  int nlrfw;            // LRF build blocks: (window, first target group, count <= 64, source part)
   const int4* lrf_work;
-  double* g_lrf_part;    // [part][group][20] partial sums over the kLrfParts source parts
+  double* g_lrf_part;    // [part][group][20] sums over the kLrfParts source parts (lrf_add)
   // LRF sources, packed at every build: switching atom of each group
   // (x, y, z, excluded) and the group's non-q atoms (x, y, z, charge)
   double4* ls_sw;
@@ -251,7 +253,7 @@ struct Dev {
   RowList rl[4];
   // launch shapes chosen by the autotuner (threads per block); none of
   // them changes the arithmetic of a wave or thread
-  int bs_rows, bs_lrf, bs_bonded;
+  int bs_rows, bs_bonded;
   // 1: blocks on one XCD take consecutive work (block_id in the kernels)
   int xcd;
   // bonded mode.  0: bonded terms and q-q pairs write per-term slots that

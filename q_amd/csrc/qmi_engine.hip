@@ -94,13 +94,10 @@ struct qmi_engine {
   // autotuner: work-item variants of the static Q lists and the choices made
   int4* qwork[T_NTYPES][4] = {};
   int nqwork[T_NTYPES][4] = {};
-  // LRF build blocks for 64, 128, 256 threads, each over kLrfParts source parts
-  int4* lrfwork[3] = {};
-  int nlrfwork[3] = {};
   bool autotune = true;
   // Q chunk index, row / LRF / bonded block sizes, XCD map, atomic bonded
   // gradients, LRF source parts
-  int tuned[7] = {2, 256, 256, 256, 0, 0, 1};
+  int tuned[7] = {2, 256, 64 * kLrfWaves, 256, 0, 0, kLrfParts * kLrfWaves};
   double tune_us[6] = {0, 0, 0, 0, 0, 0};   // time of the chosen configuration per group
   // the launch sequence of one MD step, captured once and replayed: index
   // bit 0 with the pair-list and LRF kernels (some window updates its lists),
@@ -791,7 +788,7 @@ static int build_device(qmi_engine* e) {
 
   Dev& d = e->d;
   d.nwin = NW;
-  d.bs_rows = d.bs_lrf = d.bs_bonded = 256;
+  d.bs_rows = d.bs_bonded = 256;
   d.xcd = 0;
   d.bond_atomic = 2;   // bonded tiles until the autotuner picks
   d.ntot = ao;
@@ -822,22 +819,17 @@ static int build_device(qmi_engine* e) {
   if ((rc = dev_alloc(e, &d.g_lrf, 20 * (size_t)goff)) != 0) return rc;
   d.ngrp_all = goff;
   {
-    // LRF build: one block per (window, block-size consecutive targets,
-    // part of the sources), a variant per block size of the autotuner
-    for (int vi = 0; vi < 3; ++vi) {
-      const int bsz = 64 << vi, parts = kLrfParts;
-      std::vector<int4> lw;
-      for (int wi = 0; wi < NW; ++wi)
-        for (int g0 = 0; g0 < wd[wi].ngrp; g0 += bsz)
-          for (int p = 0; p < parts; ++p)
-            lw.push_back(make_int4(wi, wd[wi].g_off + g0, std::min(bsz, wd[wi].ngrp - g0), p));
-      int4* lwp;
-      UP(lwp, lw);
-      e->lrfwork[vi] = lwp;
-      e->nlrfwork[vi] = (int)lw.size();
-    }
-    d.lrf_work = e->lrfwork[2];
-    d.nlrfw = e->nlrfwork[2];
+    // LRF build: one block per (window, 64 consecutive targets, part of the
+    // sources)
+    std::vector<int4> lw;
+    for (int wi = 0; wi < NW; ++wi)
+      for (int g0 = 0; g0 < wd[wi].ngrp; g0 += 64)
+        for (int p = 0; p < kLrfParts; ++p)
+          lw.push_back(make_int4(wi, wd[wi].g_off + g0, std::min(64, wd[wi].ngrp - g0), p));
+    int4* lwp;
+    UP(lwp, lw);
+    d.lrf_work = lwp;
+    d.nlrfw = (int)lw.size();
     if ((rc = dev_alloc(e, &d.g_lrf_part, kLrfParts * 20 * (size_t)std::max(goff, 1))) != 0) return rc;
     // packed sources: non-q atoms of every group, in group order
     std::vector<int> ls_first(goff), ls_n(goff), ls_atom;
@@ -1611,26 +1603,10 @@ static int autotune(qmi_engine* e) {
     e->tuned[1 + g] = bb;
     e->tune_us[1 + g] = bt;
   }
-  // 2, 6: threads per block of the LRF build (its source parts are fixed:
-  // they set the order of its sums)
-  {
-    int bv = 2;
-    double bt = 1e30;
-    auto set_lrf = [&](int vi) {
-      d.bs_lrf = 64 << vi;
-      d.lrf_work = e->lrfwork[vi];
-      d.nlrfw = e->nlrfwork[vi];
-    };
-    for (int vi = 2; vi >= 0; --vi) {
-      set_lrf(vi);
-      const double t = time_us([&] { launch_lrf_build(d, e->stream); });
-      if (faster(t, bt)) { bt = t; bv = vi; }
-    }
-    set_lrf(bv);
-    e->tuned[2] = d.bs_lrf;
-    e->tune_us[2] = bt;
-    e->tuned[6] = kLrfParts;
-  }
+  // 2, 6: the LRF build (fixed shapes: they set the order of its sums)
+  e->tuned[2] = 64 * kLrfWaves;
+  e->tune_us[2] = time_us([&] { launch_lrf_build(d, e->stream); });
+  e->tuned[6] = kLrfParts * kLrfWaves;
   // 4: XCD-grouped block order of the pair, Q-tile, LRF-build and gather kernels
   {
     double tx[2];

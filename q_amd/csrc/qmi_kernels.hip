@@ -1456,67 +1456,69 @@ __global__ void __launch_bounds__(256) k_lrf_pack(Dev d) {
   }
 }
 
-// Build: one thread per target group, one block per (window, blockDim
-// consecutive targets).  Source groups pass through LDS in chunks of
-// blockDim, so all threads read the same source at the same time; each
-// thread sums its own 20 terms in a fixed order (sources in index order).
 __device__ __forceinline__ double r2_pos(double ax, double ay, double az, double bx, double by, double bz) {
 #pragma clang fp contract(off)
   const double dx = __dsub_rn(ax, bx), dy = __dsub_rn(ay, by), dz = __dsub_rn(az, bz);
   return __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz));
 }
 
-
 // Taylor terms of one source charge q at d = x(source) - centre: potential,
 // field, field gradient and its derivative (the sums of nbpw/nbww lists with
-// LRF, md.f90:5589-5700), with the shared factors hoisted.  The terms of the
-// form u - f0 (diagonal of the gradient) and u - g d (derivative) are split:
-// acc takes the u parts and aux the sums of f0 and of g d_x, g d_y, g d_z,
-// which lrf_finish subtracts once (the sums are linear, so this is the same
-// sum with fewer instructions per source).
-__device__ __forceinline__ void lrf_add(double acc[20], double aux[4], double q, double dx, double dy, double dz) {
+// LRF, md.f90:5589-5700).  The derivatives of 1/r are traceless, so of the 20
+// terms only 16 are independent; with u = q/r, the sums kept are
+//   0      u              1..3   u/r^2 d_a          9       u/r^2
+//   4..8   u/r^4 d_a d_b  (xx xy xz yy yz)          10..12  u/r^4 d_a
+//   13..19 u/r^6 d_a d_b d_c  (xxx xxy xxz xyy xyz yyy yyz)
+// and the sums with a further z factor follow from r^2 = x^2 + y^2 + z^2
+// (k_lrf_reduce): 45 FP64 instructions per source, where forming all terms
+// took 58.
+constexpr int kLrfSums = 20;
+__device__ __forceinline__ void lrf_add(double s[kLrfSums], double q, double dx, double dy, double dz) {
   const double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
   const double ir = rsqrt_e(r2);
   const double ir2 = ir * ir;
-  const double qr = q * ir;            // q / r
-  const double f0 = qr * ir2;          // q / r^3
-  const double f1 = 3.0 * f0 * ir2;    // 3 q / r^5
-  const double f2 = -f1 * ir2;         // -3 q / r^7
-  acc[0] += qr;
-  acc[1] -= f0 * dx; acc[2] -= f0 * dy; acc[3] -= f0 * dz;
-  const double ax = f1 * dx, ay = f1 * dy;
-  acc[4] += ax * dx; acc[5] += ax * dy; acc[6] += ax * dz;
-  acc[7] += ay * dy; acc[8] += ay * dz; acc[9] += f1 * dz * dz;
-  aux[0] += f0;
-  // f2 (5 d_a d_b d_c - r2 (delta_ab d_c + delta_ac d_b + delta_bc d_a))
-  const double c5 = 5.0 * f2, g = f2 * r2;
-  const double px = c5 * dx, py = c5 * dy;
-  const double xx = px * dx, yy = py * dy, zz = c5 * dz * dz;
-  acc[10] += xx * dx; acc[11] += xx * dy; acc[12] += xx * dz;
-  acc[13] += yy * dx; acc[14] += px * dy * dz; acc[15] += zz * dx;
-  acc[16] += yy * dy; acc[17] += yy * dz; acc[18] += zz * dy;
-  acc[19] += zz * dz;
-  aux[1] += g * dx; aux[2] += g * dy; aux[3] += g * dz;
-}
-__device__ __forceinline__ void lrf_finish(double acc[20], const double aux[4]) {
-  acc[4] -= aux[0]; acc[7] -= aux[0]; acc[9] -= aux[0];
-  acc[10] -= 3.0 * aux[1]; acc[11] -= aux[2]; acc[12] -= aux[3];
-  acc[13] -= aux[1]; acc[15] -= aux[1];
-  acc[16] -= 3.0 * aux[2]; acc[17] -= aux[3]; acc[18] -= aux[2];
-  acc[19] -= 3.0 * aux[3];
+  const double u = q * ir, u3 = u * ir2, u5 = u3 * ir2, u7 = u5 * ir2;
+  s[0] += u;
+  s[1] = fma(u3, dx, s[1]); s[2] = fma(u3, dy, s[2]); s[3] = fma(u3, dz, s[3]);
+  s[9] += u3;
+  const double ax = u5 * dx, ay = u5 * dy;
+  s[4] = fma(ax, dx, s[4]); s[5] = fma(ax, dy, s[5]); s[6] = fma(ax, dz, s[6]);
+  s[7] = fma(ay, dy, s[7]); s[8] = fma(ay, dz, s[8]);
+  s[10] += ax; s[11] += ay; s[12] = fma(u5, dz, s[12]);
+  const double px = u7 * dx, py = u7 * dy;
+  const double xx = px * dx, xy = px * dy, yy = py * dy;
+  s[13] = fma(xx, dx, s[13]); s[14] = fma(xx, dy, s[14]); s[15] = fma(xx, dz, s[15]);
+  s[16] = fma(yy, dx, s[16]); s[17] = fma(xy, dz, s[17]);
+  s[18] = fma(yy, dy, s[18]); s[19] = fma(yy, dz, s[19]);
 }
 
-__global__ void __launch_bounds__(256) k_lrf_build(Dev d) {
+// Build: one lane per target group; a block takes 64 consecutive targets and
+// one of kLrfParts parts of the window's source groups, each of its kLrfWaves
+// waves a contiguous share of the part.  The sources are the same for all
+// lanes, so they are read into scalar registers.  Every wave sums its sources
+// in index order, the waves are added pairwise in LDS in a fixed order and the
+// parts in k_lrf_reduce, so the sums depend on neither batch nor scheduling.
+//
+// Bound by the FP64 rate for many windows (46 instructions a term at one per
+// 4 cycles, of 1.04 ms for the 64-window ladder's 820 M terms) and by latency
+// for one, which is why the sources are cut 32 ways (one 1109-water window:
+// 576 waves on 1024 SIMDs); the split stays within the block, so 4 partial
+// sums a group go through memory and not 32.  Loading the next group's record
+// and sources ahead costs 34 registers and with them three of seven waves a
+// SIMD: 1.54 ms for the ladder against 1.38 without.  With sources broadcast
+// through LDS and vector loads, all terms formed and 8 parts it was 2.07 ms,
+// and 131 us for the one window, now 40.
+typedef const double __attribute__((address_space(4))) * ConstD;   // read with scalar loads
+typedef const int __attribute__((address_space(4))) * ConstI;
+__global__ void __launch_bounds__(64 * kLrfWaves, 4) k_lrf_build(Dev d) {
   const int4 lw = d.lrf_work[block_id(d.xcd)];   // window, first target group, count, source part
-  const int w = lw.x;
-  const WinState& st = d.ws[w];
-  const WinDev& W = d.win[w];
+  const WinState& st = d.ws[lw.x];
+  const WinDev& W = d.win[lw.x];
   if (!st.active || !st.list_now || !W.use_lrf) return;   // uniform over the block
-  __shared__ double4 s_sw[256];
-  __shared__ int s_first[256], s_n[256];
-  const int t = threadIdx.x;
-  const int g = lw.y + t;
-  bool g_ok = t < lw.z;
+  __shared__ double s_sum[kLrfWaves / 2][kLrfSums][64];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int g = lw.y + lane;
+  bool g_ok = lane < lw.z;
   double4 sg = make_double4(0, 0, 0, 1);
   double cx = 0, cy = 0, cz = 0;
   bool gw = false;
@@ -1526,56 +1528,92 @@ __global__ void __launch_bounds__(256) k_lrf_build(Dev d) {
     gw = (g - W.g_off) >= W.ngrp_solute;
     cx = d.g_cent[3 * g]; cy = d.g_cent[3 * g + 1]; cz = d.g_cent[3 * g + 2];
   }
-  // cut-off against a water source group and against a solute source group
-  const double rc_hw = gw ? W.rcww2 : W.rcpw2, rc_hs = gw ? W.rcpw2 : W.rcpp2, rclrf2 = W.rclrf2;
-  const int h_sol = W.g_off + W.ngrp_solute;
-  double acc[20], aux[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int k = 0; k < 20; ++k) acc[k] = 0.0;
-  // this block's part of the window's source groups
-  constexpr int P = kLrfParts;
-  const int h_beg = W.g_off + (int)(((long long)lw.w * W.ngrp) / P);
-  const int h_end = W.g_off + (int)(((long long)(lw.w + 1) * W.ngrp) / P);
-  const double4* __restrict__ xq = d.ls_xq;
-  for (int h0 = h_beg; h0 < h_end; h0 += blockDim.x) {
-    const int hl = h0 + t;
-    if (hl < h_end) {
-      s_sw[t] = d.ls_sw[hl];
-      s_first[t] = d.ls_first[hl];
-      s_n[t] = d.ls_n[hl];
-    }
-    __syncthreads();
-    const int nh = min((int)blockDim.x, h_end - h0);
-    for (int j = 0; j < nh; ++j) {
-      const int h = h0 + j;
-      const double4 sh = s_sw[j];
-      if (!g_ok || h == g || sh.w != 0.0) continue;
-      const double rc2 = h >= h_sol ? rc_hw : rc_hs;
-      const double r2g = r2_pos(sg.x, sg.y, sg.z, sh.x, sh.y, sh.z);
-      if (r2g <= rc2 || r2g > rclrf2) continue;
-      const int f0 = s_first[j], n = s_n[j];
-      for (int k = 0; k < n; ++k) {
-        const double4 a = xq[f0 + k];
-        lrf_add(acc, aux, a.w, a.x - cx, a.y - cy, a.z - cz);
+  const double rclrf2 = W.rclrf2;
+  double acc[kLrfSums];
+  for (int k = 0; k < kLrfSums; ++k) acc[k] = 0.0;
+  constexpr int P = kLrfParts * kLrfWaves;
+  const int sub = lw.w * kLrfWaves + wv;
+  // (wave-uniform: kept in scalar registers, with what they index)
+  const int h_beg = __builtin_amdgcn_readfirstlane(W.g_off + (int)(((long long)sub * W.ngrp) / P));
+  const int h_end = __builtin_amdgcn_readfirstlane(W.g_off + (int)(((long long)(sub + 1) * W.ngrp) / P));
+  const int h_sol = __builtin_amdgcn_readfirstlane(min(max(W.g_off + W.ngrp_solute, h_beg), h_end));
+  const ConstD sw = (ConstD)(const double*)d.ls_sw, xq = (ConstD)(const double*)d.ls_xq;
+  const ConstI nn = (ConstI)d.ls_n;
+  // the groups' sources are consecutive
+  int f = __builtin_amdgcn_readfirstlane(h_beg < h_end ? d.ls_first[h_beg] : 0);
+  for (int seg = 0; seg < 2; ++seg) {
+    // cut-off against a solute, then against a water source group
+    const double rc2 = seg ? (gw ? W.rcww2 : W.rcpw2) : (gw ? W.rcpw2 : W.rcpp2);
+    const int h1 = seg ? h_end : h_sol;
+    for (int h = seg ? h_sol : h_beg; h < h1; ++h) {
+      const int n = nn[h];
+      const ConstD hs = sw + 4 * (size_t)h;
+      // (a target is within the cut-off of itself)
+      const double r2g = r2_pos(sg.x, sg.y, sg.z, hs[0], hs[1], hs[2]);
+      if (hs[3] == 0.0 && g_ok && !(r2g <= rc2) && !(r2g > rclrf2)) {
+        for (int k = 0; k < n; ++k) {
+          const ConstD a = xq + 4 * (size_t)(f + k);
+          lrf_add(acc, a[3], a[0] - cx, a[1] - cy, a[2] - cz);
+        }
       }
+      f += n;
     }
+  }
+  // waves s .. 2s-1 onto waves 0 .. s-1
+#pragma unroll
+  for (int s = kLrfWaves / 2; s > 0; s >>= 1) {
+    if (wv >= s && wv < 2 * s)
+      for (int k = 0; k < kLrfSums; ++k) s_sum[wv - s][k][lane] = acc[k];
+    __syncthreads();
+    if (wv < s)
+      for (int k = 0; k < kLrfSums; ++k) acc[k] += s_sum[wv][k][lane];
     __syncthreads();
   }
-  if (!g_ok) return;
-  lrf_finish(acc, aux);
-  double* out = P == 1 ? d.g_lrf + 20 * (size_t)g : d.g_lrf_part + 20 * ((size_t)lw.w * d.ngrp_all + g);
-  for (int k = 0; k < 20; ++k) out[k] = acc[k];
+  if (wv != 0 || !g_ok) return;
+  double* out = d.g_lrf_part + kLrfSums * ((size_t)lw.w * d.ngrp_all + g);
+  for (int k = 0; k < kLrfSums; ++k) out[k] = acc[k];
 }
 
-// sum of the source parts in part order, one thread per (group, term)
-__global__ void __launch_bounds__(256) k_lrf_reduce(Dev d) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= 20 * d.ngrp_all) return;
-  const int g = i / 20;
-  const int w = d.g_win[g];
-  if (!d.ws[w].active || !d.ws[w].list_now || !d.win[w].use_lrf || d.ls_sw[g].w != 0.0) return;
+// sum of the source parts in part order, one thread per (group, sum), then
+// the 20 Taylor terms of each group from its sums
+constexpr int kLrfReduceGroups = 12;
+__global__ void __launch_bounds__(kLrfReduceGroups * kLrfSums) k_lrf_reduce(Dev d) {
+  __shared__ double s_v[kLrfReduceGroups][kLrfSums];
+  const int lg = threadIdx.x / kLrfSums, k = threadIdx.x % kLrfSums, g = blockIdx.x * kLrfReduceGroups + lg;
+  bool on = g < d.ngrp_all;
+  if (on) {
+    const int w = d.g_win[g];
+    on = d.ws[w].active && d.ws[w].list_now && d.win[w].use_lrf && d.ls_sw[g].w == 0.0;
+  }
   double v = 0.0;
-  for (int p = 0; p < kLrfParts; ++p) v += d.g_lrf_part[(size_t)p * 20 * d.ngrp_all + i];
-  d.g_lrf[i] = v;
+  if (on)
+    for (int p = 0; p < kLrfParts; ++p) v += d.g_lrf_part[((size_t)p * d.ngrp_all + g) * kLrfSums + k];
+  s_v[lg][k] = v;
+  __syncthreads();
+  if (!on) return;
+  const double* s = s_v[lg];
+  double o;
+  switch (k) {
+    case 0: o = s[0]; break;
+    case 1: case 2: case 3: o = -s[k]; break;
+    case 4: o = 3.0 * s[4] - s[9]; break;                        // xx
+    case 5: o = 3.0 * s[5]; break;
+    case 6: o = 3.0 * s[6]; break;
+    case 7: o = 3.0 * s[7] - s[9]; break;                        // yy
+    case 8: o = 3.0 * s[8]; break;
+    case 9: o = 3.0 * (s[9] - s[4] - s[7]) - s[9]; break;        // zz
+    case 10: o = 9.0 * s[10] - 15.0 * s[13]; break;              // xxx
+    case 11: o = 3.0 * s[11] - 15.0 * s[14]; break;              // xxy
+    case 12: o = 3.0 * s[12] - 15.0 * s[15]; break;              // xxz
+    case 13: o = 3.0 * s[10] - 15.0 * s[16]; break;              // xyy
+    case 14: o = -15.0 * s[17]; break;                           // xyz
+    case 15: o = 3.0 * s[10] - 15.0 * (s[10] - s[13] - s[16]); break;   // xzz
+    case 16: o = 9.0 * s[11] - 15.0 * s[18]; break;              // yyy
+    case 17: o = 3.0 * s[12] - 15.0 * s[19]; break;              // yyz
+    case 18: o = 3.0 * s[11] - 15.0 * (s[11] - s[14] - s[18]); break;   // yzz
+    default: o = 9.0 * s[12] - 15.0 * (s[12] - s[15] - s[19]); break;   // zzz
+  }
+  d.g_lrf[20 * (size_t)g + k] = o;
 }
 
 // Evaluation per atom (lrf_taylor, md.f90:3646-3712), FP64.
@@ -2757,8 +2795,8 @@ void launch_begin(const Dev& d, hipStream_t s, int force_energy, int eval_only, 
 void launch_lrf_build(const Dev& d, hipStream_t s) {
   if (!d.nlrfw) return;
   k_lrf_pack<<<blocks(std::max(d.ngrp_all, d.nls), 256), 256, 0, s>>>(d);
-  k_lrf_build<<<d.nlrfw, d.bs_lrf, 0, s>>>(d);
-  k_lrf_reduce<<<blocks(20LL * d.ngrp_all, 256), 256, 0, s>>>(d);
+  k_lrf_build<<<d.nlrfw, 64 * kLrfWaves, 0, s>>>(d);
+  k_lrf_reduce<<<blocks(d.ngrp_all, kLrfReduceGroups), kLrfReduceGroups * kLrfSums, 0, s>>>(d);
 }
 
 void launch_bonded(const Dev& d, hipStream_t s) {
