@@ -65,7 +65,7 @@ int qmi_window_add(qmi_engine* e, const char* inp_path, long long seed_override,
  * qmi_prepare. */
 int qmi_window_set_log(qmi_engine* e, int w, const char* path);
 
-/* Upload all windows to the GPU, build the static Q-atom lists, pick tiles
+/* Upload all windows to the GPU, build the static Q-atom lists, pick launch shapes
  * and capture the step graph.  Replaces distribute_nonbonds
  * (md.f90:1044-1361) and the set-up half of md_run (md.f90:3917-4000). */
 int qmi_prepare(qmi_engine* e);
@@ -121,13 +121,13 @@ int qmi_window_info(qmi_engine* e, int w, int32_t* info, int cap);
 /* Write window w's restart file (write_xfin, md.f90:15452-15470). */
 int qmi_write_restart(qmi_engine* e, int w, const char* path);
 
-/* The autotuner (on by default) times candidate launch shapes of the Q-tile,
+/* The autotuner (on by default) times candidate launch shapes of the
  * pair-row and bonded kernels on the engine's own windows during
  * qmi_prepare and keeps the fastest; the candidates do not change results.
  * Call before qmi_prepare.  No reference counterpart. */
 int qmi_set_autotune(qmi_engine* e, int on);
 
-/* Choices of the autotuner: Q tiles per wave, threads per block of the row,
+/* Choices of the autotuner: q-atoms per chunk of the q kernels (fixed), threads per block of the row,
  * LRF-build and bonded kernels, whether blocks are grouped by XCD (0/1),
  * the bonded mode (0: per-term slots and a per-atom gather, 1: atomics, 2:
  * LDS sums per tile of terms), the number of source shares
@@ -152,7 +152,7 @@ int qmi_timings(qmi_engine* e, double* out, int cap);
  * `reps` launches in a row on the engine's stream between two HIP events (no
  * reference counterpart; for measurement).  which 0: the water-water force
  * kernel.  Call between qmi_run calls while the windows are still running:
- * the launches add to the gradient, so the engine then evaluates the
+ * the launches disturb the gradient, so the engine then evaluates the
  * gradient and energies again at the current coordinates, as qmi_evaluate
  * does without rebuilding lists. */
 int qmi_time_kernel(qmi_engine* e, int which, int reps, double* us);

@@ -54,6 +54,8 @@ struct WinDev {
   int qs_off, qsc_off;              // first entry of the [q][state] and [q][type][state] tables
   int g_off, ngrp, ngrp_solute;     // charge groups
   int wc_off, nwc, sc_off, nsc, qc_off, nqc;
+  int nqch;                         // chunks of kQItem q-atoms (2 per 4 q-clusters)
+  long long qp14_off;               // first entry of the window in Dev::qp14
   int sh_off, nshell;               // water polarisation shells
   long long wp_off;                 // first entry of the window's shell rows in Dev::wtheta
   int nsteps, nbcycle, iene, iout;
@@ -104,23 +106,9 @@ struct WinState {
 
 struct ShellDev { float rout, dr, cstb, theta_corr, avtheta, avn_insh; int n_insh; int pad; };
 
-// tile types (i-centric): WW, W<-P, P<-W, P<-P, Q<-P, P<-Q, Q<-W, W<-Q
-enum TileType { T_WW = 0, T_WP, T_PW, T_PP, T_QP, T_PQ, T_QW, T_WQ, T_NTYPES };
+// dynamic pair lists (i-centric): WW, W<-P, P<-W, P<-P
+enum RowType { T_WW = 0, T_WP, T_PW, T_PP, T_NTYPES };
 
-struct TileList {
-  int* start;      // per i-cluster: first entry (fixed-capacity layout)
-  int* count;      // per i-cluster: number of entries
-  int* jc;         // j-cluster (global index)
-  uint2* mask;     // 64-bit lane mask: bit (a*8 + b)
-  uint2* m14;      // 1-4 mask (P<-P, Q<-P, P<-Q)
-  int nicl;        // number of i-clusters (all windows)
-  int cap_total;
-  // static lists are cut into work items (a multiple of kQGroup tiles, the
-  // size picked by the autotuner), one wave each: (i-cluster, first entry,
-  // number of entries)
-  const int4* work;
-  int nwork;
-};
 // temperature ring record per window and step: T_tot, T_free, Ekin, step tag,
 // T_free solute, T_free solvent
 constexpr int kTRing = 6;
@@ -137,9 +125,7 @@ constexpr int kGatherAtoms = 256;  // atoms per block of the bonded gather
 constexpr int kGatherSlots = 2048; // slots staged in LDS per gather block
 constexpr int kBondTileTerms = 512; // bonded terms per tile
 constexpr int kBondSpan = 1024;     // atoms of a tile's LDS gradient sums
-constexpr int kQGroup = 4;        // Q-tile sums go to fixed point every 4 tiles of a list
-constexpr int kQChunkN = 4;
-constexpr int kQChunks[kQChunkN] = {4, 8, 16, 32};   // autotuner candidates, tiles per wave
+constexpr int kQItem = 16;          // q-atoms of a chunk of the q kernels: half the members of 4 q-clusters
 
 // Neighbour rows of the dynamic pair lists (WW, W<-P, P<-W, P<-P): row
 // ic*8 + a belongs to member a of i-cluster ic and holds the j entries of
@@ -174,6 +160,12 @@ struct Dev {
   const int* qmslot;
   float4* ljp;          // avdw1, bvdw1, avdw3, bvdw3
   long long* f;         // gradient, 3 per atom, fixed point 2^-32
+  // the row kernels' and the q kernels' sums, 3 per entry: entry 3 * slot +
+  // site for the waters' cluster slots (nwslot of them), then one per solute
+  // slot; rslot: an atom's entry, or -1 (q-atoms)
+  long long *grow, *gq;
+  int nwslot;
+  const int* rslot;
   long long* fterm;     // per-atom terms of the step's gradient (LRF evaluation, atom restraints), fixed point
   const float* winv;
   const double* mass;
@@ -212,7 +204,6 @@ struct Dev {
   // clusters
   const int* wc_o;      // 8 per water cluster: O atom or -1
   const int* sc_a;      // 8 per solute cluster: atom or -1
-  const int* qc_q;      // 8 per q cluster: window-local q index or -1
   // per q-cluster member (8 per cluster): its global atom (or -1), and per
   // state (kMaxS per member) the water-side factors of k_qw: A and B of the
   // pair with the water oxygen, the charge products with O and with H, and
@@ -224,14 +215,18 @@ struct Dev {
   // A, B, charge product and soft-core term ([(m * kMaxS + s) * 2 + k - 1])
   const float4* qcw_h;
   int any_wat3;          // some window has a 3-atom solvent
-  // q-atom share of the Q tiles, written per tile by the non-q side into
-  // slot ent_slot[entry] (8 members x 3 int64); a q-cluster's slots are
-  // contiguous, qg_start[c] .. qg_start[c+1]-1, so k_q_gather reads runs
-  long long* qslot;
-  int qslot_wq, nqc_all;  // qslot_wq: offset of the W<-Q entries in ent_slot
-  const int* qg_start;
-  const int* ent_slot;    // P<-Q entries, then W<-Q entries
-  const int* wc_win; const int* sc_win; const int* qc_win;
+  // the same in FP64 for the energy terms: A, B, soft-core term, charge
+  // product of member, state and water atom ([(m * kMaxS + s) * 3 + k])
+  const double4* qcw_e;
+  // static Q lists: whether the water (solute atom) of a cluster slot is in
+  // them, the 1-4 pairs of a solute slot with the q-atoms of a chunk (bit
+  // 4 member + cluster, [qp14_off + slot of the window * nqch + chunk]), and the
+  // work items: window, first slot, slots (at most 64)
+  const uint8_t* qw_on; const uint8_t* qp_on;
+  const uint16_t* qp14;
+  int nqw_work, nqp_work;
+  const int4* qw_work; const int4* qp_work;
+  const int* wc_win; const int* sc_win;
   double* wc_bs;        // bounding sphere per water cluster (x, y, z, r)
   double* sc_bs;        // bounding sphere of the switch atoms of the members
   // per cluster member, written at list steps: its switching atom's x, y, z
@@ -248,9 +243,7 @@ struct Dev {
   // topology LJ params in double per window type (energy path)
   const double* t_lj;    // [(t_off + t)*4]
   const double4* ljd;    // per atom: its type's row of t_lj
-  // tiles (static Q lists) and neighbour rows (dynamic lists, index T_WW..T_PP)
-  TileList tl[T_NTYPES];
-  RowList rl[4];
+  RowList rl[T_NTYPES];  // neighbour rows
   // launch shapes chosen by the autotuner (threads per block); none of
   // them changes the arithmetic of a wave or thread
   int bs_rows, bs_bonded;

@@ -87,17 +87,15 @@ struct qmi_engine {
   int ngrp = 0, nwc = 0, nsc = 0, nqc = 0, ntot = 0, nwat_total = 0;
   int shake_any = 0;
   // host-side tables for pair-list export
-  std::vector<int> h_wc_o, h_sc_a, h_qc_q, h_atom_win;
+  std::vector<int> h_wc_o, h_sc_a, h_atom_win;
   std::vector<double> timings;
   bool timing_on = false;
   hipEvent_t ev[8] = {};
-  // autotuner: work-item variants of the static Q lists and the choices made
-  int4* qwork[T_NTYPES][4] = {};
-  int nqwork[T_NTYPES][4] = {};
+  // the autotuner's choices
   bool autotune = true;
-  // Q chunk index, row / LRF / bonded block sizes, XCD map, atomic bonded
+  // q-atoms per work item, row / LRF / bonded block sizes, XCD map, atomic bonded
   // gradients, LRF source parts
-  int tuned[7] = {2, 256, 64 * kLrfWaves, 256, 0, 0, kLrfParts * kLrfWaves};
+  int tuned[7] = {kQItem, 256, 64 * kLrfWaves, 256, 0, 0, kLrfParts * kLrfWaves};
   double tune_us[6] = {0, 0, 0, 0, 0, 0};   // time of the chosen configuration per group
   // the launch sequence of one MD step, captured once and replayed: index
   // bit 0 with the pair-list and LRF kernels (some window updates its lists),
@@ -197,7 +195,7 @@ static int build_device(qmi_engine* e) {
   std::vector<int> sp_start, sp_j;
   std::vector<uint8_t> sp_t;
   // clusters
-  std::vector<int> wc_o, sc_a, qc_q, wc_win, sc_win, qc_win;
+  std::vector<int> wc_o, sc_a, qc_q, wc_win, sc_win;
   // q tables
   std::vector<int> q_atom;
   std::vector<float> q_crg, q_sc;
@@ -229,9 +227,10 @@ static int build_device(qmi_engine* e) {
   // shells
   std::vector<ShellDev> shells;
   long long wp_rows = 0;
-  // static Q tiles (host-built), per type: per i-cluster lists
-  struct HT { std::vector<std::vector<std::pair<int, uint2>>> l; std::vector<std::vector<uint2>> m14; };
-  HT qt[4];  // T_QP, T_PQ, T_QW, T_WQ
+  // static Q lists (Dev::qw_on .. qp_work)
+  std::vector<uint8_t> qw_on, qp_on;
+  std::vector<uint16_t> qp14;
+  std::vector<int4> qw_work, qp_work;
   int ao = 0, goff = 0, woff = 0, qoff = 0, toff = 0;
   e->shake_any = 0;
   for (int wi = 0; wi < NW; ++wi) {
@@ -431,12 +430,13 @@ static int build_device(qmi_engine* e) {
       }
     }
     D.nsc = (int)sc_win.size() - D.sc_off;
-    D.qc_off = (int)qc_win.size();
+    D.qc_off = (int)(qc_q.size() / kCl);
     for (int k = 0; k < fp.nqat; k += kCl) {
       for (int m = 0; m < kCl; ++m) qc_q.push_back(k + m < fp.nqat ? k + m : -1);
-      qc_win.push_back(wi);
     }
-    D.nqc = (int)qc_win.size() - D.qc_off;
+    D.nqc = (int)(qc_q.size() / kCl) - D.qc_off;
+    D.nqch = (D.nqc + 3) / 4 * 2;
+    D.qp14_off = (long long)qp14.size();
     // --- q tables
     for (int q = 0; q < fp.nqat; ++q) {
       q_atom.push_back(ao + fp.iqseq[q]);
@@ -558,71 +558,35 @@ static int build_device(qmi_engine* e) {
           }
         }
       }
-      // tiles: QW / WQ
-      auto setbit = [](uint2& m, int bit) { if (bit < 32) m.x |= 1u << bit; else m.y |= 1u << (bit - 32); };
-      for (int qcl = 0; qcl < D.nqc; ++qcl) {
-        std::vector<std::pair<int, uint2>> lqw, lqp;
-        std::vector<uint2> m14qp;
-        for (int wc = 0; wc < D.nwc; ++wc) {
-          uint2 m = {0, 0};
-          for (int a = 0; a < kCl; ++a) {
-            int q = qc_q[(D.qc_off + qcl) * kCl + a];
-            if (q < 0) continue;
-            for (int b = 0; b < kCl; ++b) {
-              int o = wc_o[(D.wc_off + wc) * kCl + b];
-              if (o < 0) continue;
-              int k = (o - ao - NS) / 3;
-              if (wlisted[k]) setbit(m, a * 8 + b);
-            }
-          }
-          if (m.x | m.y) lqw.push_back({D.wc_off + wc, m});
-        }
-        for (int sc = 0; sc < D.nsc; ++sc) {
-          uint2 m = {0, 0}, m14 = {0, 0};
-          for (int a = 0; a < kCl; ++a) {
-            int q = qc_q[(D.qc_off + qcl) * kCl + a];
-            if (q < 0) continue;
-            for (int b = 0; b < kCl; ++b) {
-              int at = sc_a[(D.sc_off + sc) * kCl + b];
-              if (at < 0) continue;
-              int li = at - ao;
-              if (!plisted[li]) continue;
-              setbit(m, a * 8 + b);
-              if (qc(0, li, q) == 4) setbit(m14, a * 8 + b);
-            }
-          }
-          if (m.x | m.y) { lqp.push_back({D.sc_off + sc, m}); m14qp.push_back(m14); }
-        }
-        qt[0].l.push_back(lqp); qt[0].m14.push_back(m14qp);   // T_QP
-        qt[2].l.push_back(lqw); qt[2].m14.push_back({});      // T_QW
+      for (size_t m = qw_on.size(); m < wc_o.size(); ++m) {
+        const int o = wc_o[m];
+        qw_on.push_back(o >= 0 && wlisted[(o - ao - NS) / 3]);
       }
-      // transposed lists (i = solute / water cluster, j = q cluster)
-      auto transpose = [](uint2 m) {
-        uint2 r = {0, 0};
-        for (int bit = 0; bit < 64; ++bit) {
-          bool on = bit < 32 ? (m.x >> bit) & 1 : (m.y >> (bit - 32)) & 1;
-          if (!on) continue;
-          int a = bit >> 3, b = bit & 7, nb = b * 8 + a;
-          if (nb < 32) r.x |= 1u << nb; else r.y |= 1u << (nb - 32);
+      for (size_t m = qp_on.size(); m < sc_a.size(); ++m) {
+        const int at = sc_a[m];
+        qp_on.push_back(at >= 0 && plisted[at - ao]);
+        for (int ch = 0; ch < D.nqch; ++ch) {
+          unsigned bits = 0;
+          for (int j = 0; j < kQItem && qp_on.back(); ++j) {
+            const int q = (ch >> 1) * 4 * kCl + (ch & 1) * 4 + kCl * (j & 3) + (j >> 2);
+            if (q < nq && qc(0, at - ao, q) == 4) bits |= 1u << j;
+          }
+          qp14.push_back((uint16_t)bits);
         }
-        return r;
+      }
+      auto items = [&](std::vector<int4>& work, const std::vector<uint8_t>& on, int first, int n) {
+        for (int s0 = first; s0 < first + n; s0 += 64) {
+          const int m = std::min(64, first + n - s0);
+          bool any = false;
+          for (int k = 0; k < m; ++k) any = any || on[s0 + k];
+          if (any) work.push_back(make_int4(wi, s0, m, 0));
+        }
       };
-      std::vector<std::vector<std::pair<int, uint2>>> pq(D.nsc), wq(D.nwc);
-      std::vector<std::vector<uint2>> pq14(D.nsc);
-      for (int qcl = 0; qcl < D.nqc; ++qcl) {
-        size_t base = qt[0].l.size() - D.nqc + qcl;
-        for (size_t k = 0; k < qt[0].l[base].size(); ++k) {
-          int sc = qt[0].l[base][k].first - D.sc_off;
-          pq[sc].push_back({D.qc_off + qcl, transpose(qt[0].l[base][k].second)});
-          pq14[sc].push_back(transpose(qt[0].m14[base][k]));
-        }
-        for (auto& pr : qt[2].l[base]) wq[pr.first - D.wc_off].push_back({D.qc_off + qcl, transpose(pr.second)});
-      }
-      for (int sc = 0; sc < D.nsc; ++sc) { qt[1].l.push_back(pq[sc]); qt[1].m14.push_back(pq14[sc]); }
-      for (int wc = 0; wc < D.nwc; ++wc) { qt[3].l.push_back(wq[wc]); qt[3].m14.push_back({}); }
+      items(qw_work, qw_on, D.wc_off * kCl, D.nwc * kCl);
+      items(qp_work, qp_on, D.sc_off * kCl, D.nsc * kCl);
     } else {
-      for (int sc = 0; sc < D.nsc; ++sc) { qt[1].l.push_back({}); qt[1].m14.push_back({}); }
-      for (int wc = 0; wc < D.nwc; ++wc) { qt[3].l.push_back({}); qt[3].m14.push_back({}); }
+      qw_on.resize(wc_o.size(), 0);
+      qp_on.resize(sc_a.size(), 0);
     }
     // --- restraints of the .inp (p_restrain); angles converted to radians
     {
@@ -780,11 +744,9 @@ static int build_device(qmi_engine* e) {
   e->ngrp = goff;
   e->nwc = (int)wc_win.size();
   e->nsc = (int)sc_win.size();
-  e->nqc = (int)qc_win.size();
   e->nwat_total = woff;
   e->h_wc_o = wc_o;
   e->h_sc_a = sc_a;
-  e->h_qc_q = qc_q;
 
   Dev& d = e->d;
   d.nwin = NW;
@@ -879,10 +841,21 @@ static int build_device(qmi_engine* e) {
     UP(ip, wslot); d.wslot = ip;
   }
   UP(ip, sc_a); d.sc_a = ip;
-  UP(ip, qc_q); d.qc_q = ip;
+  {
+    // entries of the row buffers
+    std::vector<int> rslot(x32.size(), -1);
+    d.nwslot = (int)wc_o.size();
+    for (size_t m = 0; m < wc_o.size(); ++m)
+      for (int k = 0; k < 3 && wc_o[m] >= 0; ++k) rslot[wc_o[m] + k] = 3 * (int)m + k;
+    for (size_t m = 0; m < sc_a.size(); ++m)
+      if (sc_a[m] >= 0) rslot[sc_a[m]] = 3 * d.nwslot + (int)m;
+    UP(ip, rslot); d.rslot = ip;
+    const size_t n = 3 * (3 * wc_o.size() + sc_a.size());
+    if ((rc = dev_alloc(e, &d.grow, n)) != 0) return rc;
+    if ((rc = dev_alloc(e, &d.gq, n)) != 0) return rc;
+  }
   UP(ip, wc_win); d.wc_win = ip;
   UP(ip, sc_win); d.sc_win = ip;
-  UP(ip, qc_win); d.qc_win = ip;
   if ((rc = dev_alloc(e, &d.wc_bs, 4 * (size_t)e->nwc)) != 0) return rc;
   if ((rc = dev_alloc(e, &d.sc_bs, 4 * (size_t)e->nsc)) != 0) return rc;
   if ((rc = dev_alloc(e, &d.wc_cm, (size_t)kCl * e->nwc)) != 0) return rc;
@@ -936,6 +909,38 @@ static int build_device(qmi_engine* e) {
     UP(pp, qcw_par); d.qcw_par = pp;
     float* fp;
     UP(fp, qcw_sc); d.qcw_sc = fp;
+    // the same per water atom in FP64, for the energies (real(4) charge
+    // products, as the reference forms them)
+    {
+      std::vector<double4> qcw_e(std::max<size_t>(1, qc_q.size() * kMaxS * 3), make_double4(0, 0, 0, 0));
+      for (int wi = 0; wi < NW; ++wi) {
+        const WinDev& D = wd[wi];
+        for (int m = D.qc_off * kCl; m < (D.qc_off + D.nqc) * kCl && D.nwat > 0; ++m) {
+          const int iq = qc_q[m];
+          if (iq < 0) continue;
+          for (int st = 0; st < D.S; ++st) {
+            const double* qd = &q_ljd[(size_t)(D.qs_off + iq * D.S + st) * 4];
+            const float qcv = q_crg[D.qs_off + iq * D.S + st];
+            for (int k = 0; k < 3; ++k) {
+              const double* hd = &t_lj[(size_t)(D.t_off + D.iac_w[k]) * 4];
+              double A, B;
+              lj_ab(qd[0], qd[1], hd[0], hd[1], D.arith != 0, &A, &B);
+              const double sc = D.qvdw ? q_scd[D.qsc_off + ((size_t)iq * D.natyps + D.iac_w[k]) * D.S + st] : 0.0;
+              qcw_e[((size_t)m * kMaxS + st) * 3 + k] = make_double4(A, B, sc, (double)(D.crg_w[k] * qcv));
+            }
+          }
+        }
+      }
+      double4* ep;
+      UP(ep, qcw_e); d.qcw_e = ep;
+    }
+    UP(up, qw_on); d.qw_on = up;
+    UP(up, qp_on); d.qp_on = up;
+    uint16_t* u16;
+    UP(u16, qp14); d.qp14 = u16;
+    int4* qwp;
+    UP(qwp, qw_work); d.qw_work = qwp; d.nqw_work = (int)qw_work.size();
+    UP(qwp, qp_work); d.qp_work = qwp; d.nqp_work = (int)qp_work.size();
     // 3-atom solvent: the hydrogens' factors, formed like the oxygen's
     bool any3 = false;
     for (int wi = 0; wi < NW; ++wi) any3 = any3 || wd[wi].wat3;
@@ -1217,7 +1222,7 @@ static int build_device(qmi_engine* e) {
   // candidate count at the start (switching atoms within the cut-off plus
   // 1 A), with room for density fluctuations; a row that overflows flags
   // its window
-  auto max_rows = [&](TileType tt) -> int {
+  auto max_rows = [&](RowType tt) -> int {
     int best = 0;
     for (int wi = 0; wi < NW; ++wi) {
       const Window& W = *e->wins[wi].w;
@@ -1270,7 +1275,7 @@ static int build_device(qmi_engine* e) {
     }
     return best;
   };
-  auto make_rows = [&](TileType tt, const std::vector<int>& iwin) -> int {
+  auto make_rows = [&](RowType tt, const std::vector<int>& iwin) -> int {
     RowList& L = d.rl[tt];
     L.nicl = (int)iwin.size();
     int maxj = 0;
@@ -1289,78 +1294,6 @@ static int build_device(qmi_engine* e) {
   if ((rc = make_rows(T_WP, wc_win)) != 0) return rc;
   if ((rc = make_rows(T_PW, sc_win)) != 0) return rc;
   if ((rc = make_rows(T_PP, sc_win)) != 0) return rc;
-  std::vector<int> jc_all[T_NTYPES];
-  auto make_static = [&](TileType tt, const HT& h) -> int {
-    TileList& L = d.tl[tt];
-    std::vector<int> start, count, jc;
-    std::vector<uint2> mask, m14;
-    for (size_t ic = 0; ic < h.l.size(); ++ic) {
-      start.push_back((int)jc.size());
-      count.push_back((int)h.l[ic].size());
-      for (size_t k = 0; k < h.l[ic].size(); ++k) {
-        jc.push_back(h.l[ic][k].first);
-        mask.push_back(h.l[ic][k].second);
-        m14.push_back(k < h.m14[ic].size() ? h.m14[ic][k] : make_uint2(0, 0));
-      }
-    }
-    L.nicl = (int)h.l.size();
-    L.cap_total = (int)jc.size();
-    // work items for every candidate size of the autotuner; the default
-    // until it runs is the 16-tile form
-    int r;
-    for (int ci = 0; ci < kQChunkN; ++ci) {
-      const int ch = kQChunks[ci];
-      std::vector<int4> work;
-      for (size_t ic = 0; ic < h.l.size(); ++ic)
-        for (int k = 0; k < count[ic]; k += ch)
-          work.push_back(make_int4((int)ic, start[ic] + k, std::min(ch, count[ic] - k), 0));
-      int4* wp = nullptr;
-      if ((r = dev_upload(e, &wp, work)) != 0) return r;
-      e->qwork[tt][ci] = wp;
-      e->nqwork[tt][ci] = (int)work.size();
-    }
-    // the q-side lists only carry the per-state energy pass (few rows, long
-    // lists): the smallest work items give it the most waves; the non-q
-    // side starts at 16 tiles until the autotuner picks
-    const int ci0 = (tt == T_QP || tt == T_QW) ? 0 : 2;
-    L.work = e->qwork[tt][ci0];
-    L.nwork = e->nqwork[tt][ci0];
-    if ((r = dev_upload(e, &L.start, start)) != 0) return r;
-    if ((r = dev_upload(e, &L.count, count)) != 0) return r;
-    if ((r = dev_upload(e, &L.jc, jc)) != 0) return r;
-    if ((r = dev_upload(e, &L.mask, mask)) != 0) return r;
-    if ((r = dev_upload(e, &L.m14, m14)) != 0) return r;
-    jc_all[tt] = jc;
-    return 0;
-  };
-  if ((rc = make_static(T_QP, qt[0])) != 0) return rc;
-  if ((rc = make_static(T_PQ, qt[1])) != 0) return rc;
-  if ((rc = make_static(T_QW, qt[2])) != 0) return rc;
-  if ((rc = make_static(T_WQ, qt[3])) != 0) return rc;
-  // q-atom gather: per q-cluster, the P<-Q and W<-Q entries that list it, in
-  // entry order, get consecutive slots
-  {
-    const int nqc = d.tl[T_QW].nicl;
-    const int npq = (int)jc_all[T_PQ].size(), nwq = (int)jc_all[T_WQ].size();
-    std::vector<std::vector<int>> by(nqc);
-    for (int k = 0; k < npq; ++k) by[jc_all[T_PQ][k]].push_back(k);
-    for (int k = 0; k < nwq; ++k) by[jc_all[T_WQ][k]].push_back(npq + k);
-    std::vector<int> qg_start(nqc + 1, 0), ent_slot(npq + nwq, 0);
-    int pos = 0;
-    for (int c = 0; c < nqc; ++c) {
-      for (int k : by[c]) ent_slot[k] = pos++;
-      qg_start[c + 1] = pos;
-    }
-    d.nqc_all = nqc;
-    d.qslot_wq = npq;
-    int r;
-    int* gp = nullptr;
-    if ((r = dev_upload(e, &gp, qg_start)) != 0) return r;
-    d.qg_start = gp;
-    if ((r = dev_upload(e, &gp, ent_slot)) != 0) return r;
-    d.ent_slot = gp;
-    if ((r = dev_alloc(e, &d.qslot, (size_t)std::max(1, npq + nwq) * kCl * 3)) != 0) return r;
-  }
   return 0;
 }
 
@@ -1575,19 +1508,9 @@ static int autotune(qmi_engine* e) {
   // timed alone, close candidates differ by noise, and in the step graph,
   // where the kernels share the GPU, the coarser groupings fare better.
   auto faster = [](double t, double best) { return t < 0.98 * best; };
-  // 0: Q-tile work-item size
-  {
-    int bi = kQChunkN - 1;
-    double bt = 1e30;
-    for (int ci = kQChunkN - 1; ci >= 0; --ci) {
-      for (int tt : {T_PQ, T_WQ}) { d.tl[tt].work = e->qwork[tt][ci]; d.tl[tt].nwork = e->nqwork[tt][ci]; }
-      const double t = time_us([&] { launch_q_tiles(d, e->stream); });
-      if (faster(t, bt)) { bt = t; bi = ci; }
-    }
-    for (int tt : {T_PQ, T_WQ}) { d.tl[tt].work = e->qwork[tt][bi]; d.tl[tt].nwork = e->nqwork[tt][bi]; }
-    e->tuned[0] = bi;
-    e->tune_us[0] = bt;
-  }
+  // 0: the q kernels (fixed work items)
+  e->tuned[0] = kQItem;
+  e->tune_us[0] = time_us([&] { launch_q(d, e->stream, false); });
   // 1, 3: threads per block of the row kernels and of the bonded terms
   int* field[3] = {&d.bs_rows, nullptr, &d.bs_bonded};
   for (int g : {0, 2}) {
@@ -1617,7 +1540,7 @@ static int autotune(qmi_engine* e) {
       // difference in its own run-to-run spread)
       tx[x] = time_us([&] {
         launch_nonbonded(d, e->stream, true, false);
-        launch_q_tiles(d, e->stream, false);
+        launch_q(d, e->stream, false);
       });
     }
     // ungrouped unless grouped is clearly faster (grouping keeps each XCD's
@@ -2378,7 +2301,7 @@ int qmi_get_pairlist(qmi_engine* e, int w, int kind, int32_t* pi, int32_t* pj, i
         if (in[p[1]]) out.push_back({p[0] + 1, p[1] + 1, p[2]});
     }
   } else {
-    TileType tt = kind == QMI_LIST_WW ? T_WW : kind == QMI_LIST_PW ? T_PW : kind == QMI_LIST_PP ? T_PP : T_NTYPES;
+    RowType tt = kind == QMI_LIST_WW ? T_WW : kind == QMI_LIST_PW ? T_PW : kind == QMI_LIST_PP ? T_PP : T_NTYPES;
     if (tt == T_NTYPES) return set_err(-3, "invalid list kind");
     const RowList& L = e->d.rl[tt];
     const size_t nrow = (size_t)kCl * L.nicl;
@@ -2445,7 +2368,7 @@ int qmi_set_autotune(qmi_engine* e, int on) {
 int qmi_tuning(qmi_engine* e, double* out, int cap) {
   if (!e || !out) return set_err(-1, "null argument");
   if (!e->prepared) return set_err(-2, "engine not prepared");
-  const double v[13] = {(double)kQChunks[e->tuned[0]], (double)e->tuned[1], (double)e->tuned[2],
+  const double v[13] = {(double)e->tuned[0], (double)e->tuned[1], (double)e->tuned[2],
                         (double)e->tuned[3], (double)e->tuned[4], (double)e->tuned[5], (double)e->tuned[6],
                         e->tune_us[0], e->tune_us[1], e->tune_us[2], e->tune_us[3], e->tune_us[4], e->tune_us[5]};
   const int n = std::min(cap, 13);
@@ -2482,8 +2405,8 @@ int qmi_time_kernel(qmi_engine* e, int which, int reps, double* us) {
     if (x) (void)hipEventDestroy(x);
   if (err != hipSuccess) return set_err(-5, std::string("HIP error: ") + hipGetErrorString(err));
   *us = 1000.0 * (double)ms / reps;
-  // the repeated launches added to the gradient: recompute it, and the
-  // energies, at the current coordinates
+  // the repeated launches overwrote the water rows' gradient: recompute it,
+  // and the energies, at the current coordinates
   return evaluate(e, 0, 1);
 }
 

@@ -1,15 +1,15 @@
 // HIP kernels of the MI355X qdyn step (gfx950, wave64).
 //
-// Nonbonded work is organised as 8x8 cluster tiles, one wave per i-cluster:
-// lane l handles the pair (i-member l/8, j-member l%8) of every tile of its
-// i-cluster and accumulates the gradient of its i-member only ("owner
-// computes": each unordered pair is evaluated from both sides), so no
-// per-pair atomics are needed; the 8 lanes sharing an i-member are reduced
-// with cross-lane shuffles and added once into the int64 fixed-point
-// gradient.  Tile masks are built with the reference's FP64 group cut-off
-// tests, so the set of interacting pairs equals the reference pair lists.
-// Pair arithmetic is FP32; Q-atom energies on energy steps use double-float
-// (two-FP32) arithmetic; LRF, bonded terms, restraints, leapfrog and SHAKE
+// Bulk nonbonded work runs over neighbour rows, one wave per cluster of 8
+// molecules or atoms: lane l takes every eighth entry of row l/8 and
+// accumulates the gradient of that row's member only ("owner computes": each
+// unordered pair is evaluated from both sides), so no per-pair atomics are
+// needed.  The q-atoms are taken one after the other by waves of 64 waters or
+// solute atoms.  Sums go to int64 fixed point, into buffers that a kernel
+// owns or the shared gradient, and the integrator adds them.  Rows are built
+// with the reference's FP64 group cut-off tests, so the set of interacting
+// pairs equals the reference pair lists.  Pair arithmetic is FP32; energy
+// terms on energy steps, LRF, bonded terms, restraints, leapfrog and SHAKE
 // run in FP64.
 #include <hip/hip_runtime.h>
 #include <algorithm>
@@ -68,19 +68,12 @@ __device__ __forceinline__ void add_grad(long long* f, int atom, double gx, doub
   atomicAdd((unsigned long long*)&f[3 * atom + 1], (unsigned long long)fix(gy, kFScale));
   atomicAdd((unsigned long long*)&f[3 * atom + 2], (unsigned long long)fix(gz, kFScale));
 }
-// the gradient of one atom from a per-atom pass: added to the gradient array
-// with atomics (LOCAL false), or summed in the lane's own fixed-point
-// registers (LOCAL true) for a kernel that owns the atom.  The integers are
-// the same either way.
-template <bool LOCAL>
-__device__ __forceinline__ void atom_grad(const Dev& d, long long* acc, int atom, double gx, double gy, double gz) {
-  if (LOCAL) {
-    acc[0] += fix(gx, kFScale);
-    acc[1] += fix(gy, kFScale);
-    acc[2] += fix(gz, kFScale);
-  } else {
-    add_grad(d.f, atom, gx, gy, gz);
-  }
+// the gradient of one atom from a per-atom pass, summed in the lane's own
+// fixed-point registers
+__device__ __forceinline__ void atom_grad(long long acc[3], double gx, double gy, double gz) {
+  acc[0] += fix(gx, kFScale);
+  acc[1] += fix(gy, kFScale);
+  acc[2] += fix(gz, kFScale);
 }
 
 // gradient of term atom k (in term order): into its own slot (fixed point, no
@@ -233,10 +226,6 @@ __device__ __forceinline__ void wave_energy(WinState* ws, int w, int slot, doubl
 
 __device__ __forceinline__ double row8_sum(double v) { return row8_sum_t(v); }
 __device__ __forceinline__ double col8_sum(double v) { return col8_sum_t(v); }
-
-__device__ __forceinline__ bool lane_bit(uint2 m, int lane) {
-  return lane < 32 ? ((m.x >> lane) & 1u) : ((m.y >> (lane - 32)) & 1u);
-}
 
 // squared distance in FP64 evaluated as the reference does, left to right
 // and without fused multiply-add: (dx*dx + dy*dy) + dz*dz
@@ -479,6 +468,41 @@ __device__ __forceinline__ int row_chunks(int n) {
   return (m + kCl - 1) / kCl;
 }
 
+// FP32 pair expressions with their rounding spelled out: which products of a
+// sum the compiler fuses differs from kernel to kernel and with what stands
+// beside them, and the gradient's last bits, and with them a trajectory,
+// should not change when a kernel is reorganised.
+// squared distance
+__device__ __forceinline__ float r2_f(float dx, float dy, float dz) {
+#pragma clang fp contract(off)
+  return __builtin_fmaf(dz, dz, __builtin_fmaf(dx, dx, dy * dy));
+}
+// dv = r2inv (-qq rinv - 12 va + 6 vb), the product with va or, CHARGE, with
+// the charges fused
+template <bool CHARGE>
+__device__ __forceinline__ float pair_dv(float r2inv, float rinv, float qq, float va, float vb) {
+#pragma clang fp contract(off)
+  const float t = CHARGE ? __builtin_fmaf(qq, -rinv, -(12.f * va)) : __builtin_fmaf(va, -12.f, -(qq * rinv));
+  return r2inv * __builtin_fmaf(6.f, vb, t);
+}
+
+// the gradient of a row's member: the sums over the row's 8 lanes, lane b
+// holding component b in fixed point (lo) and every lane component 8 (hi)
+struct RowGrad {
+  long long lo = 0, hi = 0;
+  template <int N>
+  __device__ __forceinline__ void add(const float* g, int b) {
+    double s[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) s[k] = row8_sum((double)g[k]);
+    double v = s[0];
+#pragma unroll
+    for (int k = 1; k < (N < 8 ? N : 8); ++k) v = b == k ? s[k] : v;
+    lo += fix(v, kFScale);
+    if constexpr (N == 9) hi += fix(s[8], kFScale);
+  }
+};
+
 // --------------------------------------------------- nonbonded rows --
 // Lane (a, b) of the wave for i-cluster ic evaluates entries b, b+8, ... of
 // row a and accumulates the gradient of its i-member only (each pair is
@@ -489,7 +513,7 @@ __device__ __forceinline__ int row_chunks(int n) {
 // The energy sums run only on energy steps: EN selects the form of the
 // loop for the wave's window (uniform over the wave).
 template <bool EN, bool W3>
-__device__ __forceinline__ void ww_impl(const Dev& d) {
+__device__ __forceinline__ void ww_impl(const Dev& d, RowGrad& rg) {
   const int wave = wave_id(d);
   const int lane = threadIdx.x & 63;
   const RowList L = d.rl[T_WW];
@@ -569,29 +593,25 @@ __device__ __forceinline__ void ww_impl(const Dev& d) {
     for (int p = 0; p < 3; ++p) {
       for (int q = 0; q < 3; ++q) {
         float dx = pj[q].x - pi[p].x, dy = pj[q].y - pi[p].y, dz = pj[q].z - pi[p].z;
-        float r2 = dx * dx + dy * dy + dz * dz;
+        // (the force-only loop sums the squares of an oxygen's distances from x)
+        const float r2 = !EN && q == 0 ? r2_f(dy, dx, dz) : r2_f(dx, dy, dz);
         float rinv = rsq_r2(r2);
         float r2inv = rinv * rinv;
-        float vel = qq[p][q] * rinv;
         float dv;
         if (W3 || (p == 0 && q == 0)) {
           float r6 = r2inv * r2inv * r2inv;
           const float a_ = W3 ? W.ww3_a[3 * p + q] : A, b_ = W3 ? W.ww3_b[3 * p + q] : B;
-          float va = a_ * r6 * r6, vb = b_ * r6;
-          dv = r2inv * (-vel - 12.f * va + 6.f * vb);
+          dv = pair_dv<W3>(r2inv, rinv, qq[p][q], a_ * r6 * r6, b_ * r6);
         } else {
-          dv = r2inv * (-vel);
+          dv = r2inv * (-(qq[p][q] * rinv));
         }
-        g[3 * p + 0] -= dv * dx;
-        g[3 * p + 1] -= dv * dy;
-        g[3 * p + 2] -= dv * dz;
+        g[3 * p + 0] = __builtin_fmaf(-dx, dv, g[3 * p + 0]);
+        g[3 * p + 1] = __builtin_fmaf(-dy, dv, g[3 * p + 1]);
+        g[3 * p + 2] = __builtin_fmaf(-dz, dv, g[3 * p + 2]);
       }
     }
   }
-  double gs[9];
-  for (int k = 0; k < 9; ++k) gs[k] = row8_sum((double)g[k]);
-  if (b == 0 && oa >= 0)
-    for (int p = 0; p < 3; ++p) add_grad(d.f, oa + p, gs[3 * p], gs[3 * p + 1], gs[3 * p + 2]);
+  rg.add<9>(g, b);
   if (en) {
     eel = wave_sum(eel);
     evdw = wave_sum(evdw);
@@ -599,27 +619,12 @@ __device__ __forceinline__ void ww_impl(const Dev& d) {
   }
 }
 
-// W3: the instance for windows with a 3-atom solvent (launched only when
-// there are any); each instance skips the other windows' rows
-// EK: the instance launched on steps where some window computes energies
-// (it also serves that step's other windows); the instance without energy
-// terms keeps the smaller register footprint of the force-only loop
-template <bool W3, bool EK>
-__global__ void __launch_bounds__(256) k_ww(Dev d) {
-  const int wave = wave_id(d);
-  if (wave >= d.rl[T_WW].nicl) return;
-  const int w = d.wc_win[wave];
-  if ((d.win[w].wat3 != 0) != W3) return;
-  if (EK && d.ws[w].energy_now) ww_impl<EK, W3>(d);
-  else ww_impl<false, W3>(d);
-}
-
 // solute atom - water: LJ on O (on all three sites for a 3-atom solvent),
 // Coulomb on all three sites (nonbond_pw, md.f90:10631-10682).  WATER_SIDE: rows are waters and entries solute atoms
 // (W<-P); otherwise rows are solute atoms and entries water slots (P<-W),
 // which also counts the energies.
 template <bool WATER_SIDE, bool EN, bool W3>
-__device__ __forceinline__ void pw_impl(const Dev& d) {
+__device__ __forceinline__ void pw_impl(const Dev& d, RowGrad& rg) {
   const int wave = wave_id(d);
   const int lane = threadIdx.x & 63;
   const RowList L = d.rl[WATER_SIDE ? T_WP : T_PW];
@@ -695,20 +700,18 @@ __device__ __forceinline__ void pw_impl(const Dev& d) {
       for (int k = 0; k < 3; ++k) {
         // dx = x(water atom) - x(solute atom), as nonbond_pw with i solute, j water
         float dx = pw[k].x - ps.x, dy = pw[k].y - ps.y, dz = pw[k].z - ps.z;
-        float r2 = dx * dx + dy * dy + dz * dz;
+        const float r2 = r2_f(dx, dy, dz);
         float rinv = rsq_r2(r2);
         float r2inv = rinv * rinv;
-        float vel = (ps.w * pw[k].w) * rinv;
-        float dv, ev = 0.f;
+        const float qq = ps.w * pw[k].w;
+        float dv;
         if (k == 0 || wat3) {
           float r6 = r2inv * r2inv * r2inv;
           float A, B;
           lj_ab(lj.x, lj.y, k == 0 ? W.aO1 : W.aw[k], k == 0 ? W.bO1 : W.bw[k], arith, &A, &B);
-          float va = A * r6 * r6, vb = B * r6;
-          dv = r2inv * (-vel - 12.f * va + 6.f * vb);
-          ev = va - vb;
+          dv = pair_dv<!W3 && !en>(r2inv, rinv, qq, A * r6 * r6, B * r6);
         } else {
-          dv = r2inv * (-vel);
+          dv = r2inv * (-(qq * rinv));
         }
         if (!v[u]) continue;
         if (en) {
@@ -721,20 +724,15 @@ __device__ __forceinline__ void pw_impl(const Dev& d) {
             evdw += Ad[k] * r6d * r6d - Bd[k] * r6d;
           }
         }
-        (void)ev;
-        if (WATER_SIDE) {
-          g[3 * k + 0] += dv * dx; g[3 * k + 1] += dv * dy; g[3 * k + 2] += dv * dz;
-        } else {
-          g[0] -= dv * dx; g[1] -= dv * dy; g[2] -= dv * dz;
-        }
+        const float sd = WATER_SIDE ? dv : -dv;
+        const int o = WATER_SIDE ? 3 * k : 0;
+        g[o] = __builtin_fmaf(sd, dx, g[o]);
+        g[o + 1] = __builtin_fmaf(sd, dy, g[o + 1]);
+        g[o + 2] = __builtin_fmaf(sd, dz, g[o + 2]);
       }
     }
   }
-  const int nat = WATER_SIDE ? 3 : 1;
-  double gs[9];
-  for (int k = 0; k < 3 * nat; ++k) gs[k] = row8_sum((double)g[k]);
-  if (b == 0 && ea >= 0)
-    for (int p = 0; p < nat; ++p) add_grad(d.f, ea + p, gs[3 * p], gs[3 * p + 1], gs[3 * p + 2]);
+  rg.add<WATER_SIDE ? 9 : 3>(g, b);
   if (en) {
     eel = wave_sum(eel);
     evdw = wave_sum(evdw);
@@ -742,20 +740,10 @@ __device__ __forceinline__ void pw_impl(const Dev& d) {
   }
 }
 
-template <bool WATER_SIDE, bool W3, bool EK>
-__global__ void __launch_bounds__(256) k_pw(Dev d) {
-  const int wave = wave_id(d);
-  if (wave >= d.rl[WATER_SIDE ? T_WP : T_PW].nicl) return;
-  const int w = WATER_SIDE ? d.wc_win[wave] : d.sc_win[wave];
-  if ((d.win[w].wat3 != 0) != W3) return;
-  if (EK && !WATER_SIDE && d.ws[w].energy_now) pw_impl<WATER_SIDE, EK, W3>(d);
-  else pw_impl<WATER_SIDE, false, W3>(d);
-}
-
 // solute-solute (nonbond_pp, md.f90:10387-10491): 1-4 pairs use the third
 // LJ column and the el14 scale
 template <bool EN>
-__device__ __forceinline__ void pp_impl(const Dev& d) {
+__device__ __forceinline__ void pp_impl(const Dev& d, RowGrad& rg) {
   const int wave = wave_id(d);
   const int lane = threadIdx.x & 63;
   const RowList L = d.rl[T_PP];
@@ -809,7 +797,7 @@ __device__ __forceinline__ void pp_impl(const Dev& d) {
       const bool is14 = (e[u] & kRow14) != 0;
       const int eb = e[u] & ~kRow14;
       float dx = pj[u].x - pi.x, dy = pj[u].y - pi.y, dz = pj[u].z - pi.z;
-      float r2 = dx * dx + dy * dy + dz * dz;
+      const float r2 = r2_f(dx, dy, dz);
       float rinv = rsq_r2(r2);
       float r2inv = rinv * rinv;
       float r6 = r2inv * r2inv * r2inv;
@@ -817,10 +805,10 @@ __device__ __forceinline__ void pp_impl(const Dev& d) {
       float aa, bb;
       if (is14) { vel *= W.el14; lj_ab(li.z, li.w, lj[u].z, lj[u].w, arith, &aa, &bb); }
       else lj_ab(li.x, li.y, lj[u].x, lj[u].y, arith, &aa, &bb);
-      float va = r6 * r6 * aa, vb = r6 * bb;
-      float dv = r2inv * (-vel - 12.f * va + 6.f * vb);
+      const float va = r6 * r6 * aa, vb = r6 * bb;
+      const float dv = r2inv * __builtin_fmaf(6.f, vb, __builtin_fmaf(va, -12.f, -vel));
       if (v[u]) {
-        g0 -= dv * dx; g1 -= dv * dy; g2 -= dv * dz;
+        g0 = __builtin_fmaf(-dx, dv, g0); g1 = __builtin_fmaf(-dy, dv, g1); g2 = __builtin_fmaf(-dz, dv, g2);
         if (en && ea < eb) {
           const double ddx = d.x[3 * eb] - xs[0], ddy = d.x[3 * eb + 1] - xs[1], ddz = d.x[3 * eb + 2] - xs[2];
           const double4 tlj = d.ljd[eb];   // the j atom's type row, without the type lookup
@@ -840,8 +828,8 @@ __device__ __forceinline__ void pp_impl(const Dev& d) {
       }
     }
   }
-  double s0x = row8_sum((double)g0), s0y = row8_sum((double)g1), s0z = row8_sum((double)g2);
-  if (b == 0 && ea >= 0) add_grad(d.f, ea, s0x, s0y, s0z);
+  const float g[3] = {g0, g1, g2};
+  rg.add<3>(g, b);
   if (en) {
     eel = wave_sum(eel);
     evdw = wave_sum(evdw);
@@ -849,477 +837,446 @@ __device__ __forceinline__ void pp_impl(const Dev& d) {
   }
 }
 
-template <bool EK>
-__global__ void __launch_bounds__(256) k_pp(Dev d) {
+// The rows of one i-cluster, a wave each: k_wrow the water-water and
+// water<-solute rows of a water cluster, k_srow the solute<-water and
+// solute<-solute rows of a solute cluster.  The gradient of the cluster's
+// members is stored in the row buffer (Dev::grow), which the integrator adds:
+// atomics on the shared gradient array go past the XCDs' L2s to memory, at
+// about 22 per ns for the whole GPU, and were most of what these kernels
+// spent.  64-window ladder, force-only: water rows 58 + 67 us as two kernels
+// with atomics, 89 as one with stores; solute rows 34 + 55, now 68.  What
+// bounds them now is VALU issue.
+// W3: the instance for windows with a 3-atom solvent (launched only when
+// there are any); each instance skips the other windows' rows.
+// EK: the instance launched on steps where some window computes energies
+// (it also serves that step's other windows); the instance without energy
+// terms keeps the smaller register footprint of the force-only loop.
+// PART (k_wrow): 1 water-water rows alone, 2 water<-solute rows alone, added
+// to what part 1 stored (for timing them), 3 both.
+template <bool W3, bool EK, int PART>
+__global__ void __launch_bounds__(256) k_wrow(Dev d) {
+  const int wave = wave_id(d);
+  if (wave >= d.rl[T_WW].nicl) return;
+  const int w = d.wc_win[wave];
+  if ((d.win[w].wat3 != 0) != W3 || !d.ws[w].active) return;
+  RowGrad rg;
+  if (PART & 1) {
+    if (EK && d.ws[w].energy_now) ww_impl<EK, W3>(d, rg);
+    else ww_impl<false, W3>(d, rg);
+  }
+  if (PART & 2) pw_impl<true, false, W3>(d, rg);
+  const int lane = threadIdx.x & 63, b = lane & 7, row = wave * kCl + (lane >> 3);
+  if (d.wc_o[row] < 0) return;
+  long long* o = d.grow + 9 * (size_t)row;
+  if (PART == 2) rg.lo += o[b];
+  o[b] = rg.lo;
+  if (b == 0) o[8] = PART == 2 ? o[8] + rg.hi : rg.hi;
+}
+
+template <bool W3, bool EK>
+__global__ void __launch_bounds__(256) k_srow(Dev d) {
   const int wave = wave_id(d);
   if (wave >= d.rl[T_PP].nicl) return;
-  if (EK && d.ws[d.sc_win[wave]].energy_now) pp_impl<EK>(d);
-  else pp_impl<false>(d);
+  const int w = d.sc_win[wave];
+  if ((d.win[w].wat3 != 0) != W3 || !d.ws[w].active) return;
+  RowGrad rg;
+  if (EK && d.ws[w].energy_now) {
+    pw_impl<false, EK, W3>(d, rg);
+    pp_impl<EK>(d, rg);
+  } else {
+    pw_impl<false, false, W3>(d, rg);
+    pp_impl<false>(d, rg);
+  }
+  const int lane = threadIdx.x & 63, b = lane & 7, row = wave * kCl + (lane >> 3);
+  if (b < 3 && d.sc_a[row] >= 0) d.grow[9 * (size_t)d.nwslot + 3 * row + b] = rg.lo;
 }
 
-// ---- Q-atom tiles: q-atom vs water (nonbond_qw_spc, md.f90:11302-11411) and
-// q-atom vs solute atom (nonbond_qp_qvdw / nonbond_qp, md.f90:11138-11204,
-// 10980-11045), all states; gradients are lambda-weighted over states.
-
-
-// Q-atom tiles: lane (a, b) of a work item takes member a of the i-cluster
-// and member b of each listed j-cluster.  Forces are computed once per pair,
-// on the non-q side (rows of water or solute clusters, entries q-clusters),
-// in FP32 with the hardware reciprocal.  The row member's gradient sums go
-// to fixed point every kQGroup tiles of its list, so they do not depend on
-// the work-item size; the q-atoms' share of each tile is summed over the
-// tile's rows and stored in the tile's own slots (q_reaction), which
-// k_q_gather adds up per q-atom in entry order.  On energy steps the q side
-// makes its own pass for the per-state energies in FP64.
+// ---- q-atoms against water (nonbond_qw_spc, md.f90:11302-11411; 3-atom
+// solvent nonbond_qw_3atom, 11545-11670) and against solute atoms
+// (nonbond_qp_qvdw / nonbond_qp, 11138-11204, 10980-11045), all states;
+// gradients are lambda-weighted over states.
+//
+// One block per 64 consecutive cluster slots (one water or solute atom per
+// lane): its waves take the window's q-atoms in chunks of up to 16, whose
+// coordinates and parameters are the same for every lane and come through
+// scalar loads.  The q-atoms of a chunk are members 4h .. 4h+3 (h its half) of
+// four consecutive q-clusters, taken member by member: FP32 sums run over the
+// four clusters, what is added up beyond that is FP64, in an order the window
+// alone sets, so the result does not depend on the batch.  The waves' sums
+// are added in LDS and stored in the q row buffer (Dev::gq), which the
+// integrator adds.  Reactions on a q-atom are summed over a cluster's 8 lanes
+// in FP32, over the clusters in FP64, and one atomic per chunk adds them.  On
+// energy steps the same pass adds the per-state energies in FP64.
+//
+// Bound by VALU issue (about 150 instructions per 64 pairs with water and
+// two states).  As 8 x 8 tiles with both sides gathered per lane, the q-atom
+// records cost a texture-address gather each (58 cycles a wave-load), the
+// reactions went through memory to a gather kernel, and the energies were two
+// more kernels.  Chunks of 16: four waves hold the 50 q-atoms of a ligand.
+// (With a wave per chunk and an atomic per component the kernel took 157 us
+// for the 64-window ladder, all of it atomics.)  64-window ladder, force-only:
+// water 86 + solute 39 + gather 9 us as tiles, now 29 + 26.
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
+// (12 va - 6 vb) ratio
+__device__ __forceinline__ float lj_f(float va, float vb, float ratio) {
+#pragma clang fp contract(off)
+  return __builtin_fmaf(12.f, va, -(6.f * vb)) * ratio;
+}
+// dv + r2inv (-q r - t) lam
+__device__ __forceinline__ float dv_f(float dv, float r2inv, float q, float r, float t, float lam) {
+#pragma clang fp contract(off)
+  return __builtin_fmaf(r2inv * __builtin_fmaf(-q, r, -t), lam, dv);
+}
+typedef const float __attribute__((address_space(4))) * ConstF;    // read with scalar loads
+typedef const double __attribute__((address_space(4))) * ConstD;
+typedef const int __attribute__((address_space(4))) * ConstI;
 
-// q-atom share of kQGroup tiles starting at entry e0 of a non-q-side list:
-// each lane's reaction r (gradient of its row member, summed over the
-// member's sites) is summed over the 8 rows in FP32 in a fixed order, and
-// the q-atom b of the tile takes -r in its slot (no atomics)
-__device__ __forceinline__ void q_reaction(const Dev& d, int slot0, int lane, int e0, int t0, int n, const float* rx,
-                                           const float* ry, const float* rz) {
+constexpr int kQWaves = 4;
+// the block's work item: window, first slot, slots (at most 64)
+__device__ __forceinline__ int4 q_item(const int4* work, int block) {
+  const ConstI k = (ConstI)(const int*)work + 4 * (size_t)block;
+  return make_int4(k[0], k[1], k[2], k[3]);
+}
+// the waves' sums of the N components of 64 slots (s[k][lane] of a wave) into
+// out[N * slot + k], for the item's slots
+template <int N>
+__device__ __forceinline__ void q_store(const double* acc, int slots, long long* out) {
+  __shared__ double s_acc[kQWaves][N][64];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
 #pragma unroll
-  for (int u = 0; u < kQGroup; ++u) {
-    const float x = col8_sum_t(rx[u]), y = col8_sum_t(ry[u]), z = col8_sum_t(rz[u]);
-    if (lane < kCl && t0 + u < n) {
-      long long* q = d.qslot + 3 * ((size_t)d.ent_slot[slot0 + e0 + u] * kCl + lane);
-      q[0] = fix(-(double)x, kFScale);
-      q[1] = fix(-(double)y, kFScale);
-      q[2] = fix(-(double)z, kFScale);
+  for (int k = 0; k < N; ++k) s_acc[wv][k][lane] = acc[k];
+  __syncthreads();
+  for (int i = threadIdx.x; i < N * slots; i += 64 * kQWaves) {
+    const int m = i / N, k = i % N;
+    out[i] = fix((s_acc[0][k][m] + s_acc[1][k][m]) + (s_acc[2][k][m] + s_acc[3][k][m]), kFScale);
+  }
+}
+
+// The q-atoms' gradients of a chunk: add() takes each lane's reaction on the
+// chunk's q-atom j (-r is its gradient), flush() adds them.  Every lane calls
+// both.
+struct QReaction {
+  double v[2] = {0.0, 0.0};   // lane (k, c): component c of q-atoms k and k + 8
+  __device__ __forceinline__ void add(int j, float x, float y, float z) {
+    x = row8_sum_t(x);
+    y = row8_sum_t(y);
+    z = row8_sum_t(z);
+    const int c = threadIdx.x & 7;
+    const double t = col8_sum_t((double)(c == 0 ? x : c == 1 ? y : z));
+    if ((int)((threadIdx.x >> 3) & 7) == (j & 7)) v[j >> 3] = t;
+  }
+  // slot0: q-cluster slot of the chunk's first q-atom (j = 4 member + cluster)
+  __device__ __forceinline__ void flush(const Dev& d, int slot0, int q_left) const {
+    const int c = threadIdx.x & 7, k = (threadIdx.x >> 3) & 7;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int j = k + 8 * h, m = kCl * (j & 3) + (j >> 2);
+      if (c < 3 && m < q_left)
+        atomicAdd((unsigned long long*)&d.f[3 * (size_t)d.qc_atom[slot0 + m] + c], (unsigned long long)fix(-v[h], kFScale));
     }
   }
-}
+};
 
-// q-atom gradients from the tile slots: kQGatherParts waves per q-cluster;
-// lane (b, k) of part p sums slots p*8+k, p*8+k + 8*kQGatherParts, ... of
-// the cluster's run for member b (coalesced) and the parts add with
-// atomics; integer sums, so the result does not depend on the order
-constexpr int kQGatherParts = 8;
-__global__ void __launch_bounds__(256) k_q_gather(Dev d) {
-  const int wv = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const int qc = wv / kQGatherParts, part = wv % kQGatherParts;
-  const int lane = threadIdx.x & 63;
-  if (qc >= d.nqc_all) return;
-  const int w = d.qc_win[qc];
-  if (!d.ws[w].active) return;
-  const int b = lane & 7, k = lane >> 3;
-  long long gx = 0, gy = 0, gz = 0;
-  for (int m = d.qg_start[qc] + part * kCl + k; m < d.qg_start[qc + 1]; m += kCl * kQGatherParts) {
-    const long long* q = d.qslot + 3 * ((size_t)m * kCl + b);
-    gx += q[0]; gy += q[1]; gz += q[2];
-  }
-  gx = col8_sum_t(gx);
-  gy = col8_sum_t(gy);
-  gz = col8_sum_t(gz);
-  const int iq = d.qc_q[qc * kCl + b];
-  if (k == 0 && iq >= 0) add_grad_fix(d.f, d.q_atom[d.win[w].q_off + iq], gx, gy, gz);
-}
-
-// q-atom vs water (nonbond_qw_spc, md.f90:11302-11411)
-template <bool Q_SIDE, bool W3>
-__global__ void __launch_bounds__(256) k_qw(Dev d) {
-  const int wave = wave_id(d);
-  const int lane = threadIdx.x & 63;
-  const TileList L = d.tl[Q_SIDE ? T_QW : T_WQ];
-  if (wave >= L.nwork) return;
-  const int4 wk = L.work[wave];
-  const int ic = wk.x;
-  const int w = Q_SIDE ? d.qc_win[ic] : d.wc_win[ic];
-  const WinState& st = d.ws[w];
-  if (!st.active) return;
-  const WinDev& W = d.win[w];
-  const int S = W.S;
+// NS: number of states, or 0 to read it from the window
+template <bool W3, bool EN, int NS>
+__device__ __forceinline__ void qw_impl(const Dev& d, const WinDev& W, const int4 wk, double acc[9]) {
+  const int lane = threadIdx.x & 63, w = wk.x;
+  const int S = NS ? NS : W.S;
   const bool qvdw = W.qvdw;
-  const int a = lane >> 3, b = lane & 7;
-  int iq_l = -1, qa = -1, ow = -1;
-  if (Q_SIDE) {
-    iq_l = d.qc_q[ic * kCl + a];
-    if (iq_l >= 0) qa = d.q_atom[W.q_off + iq_l];
-  } else {
-    ow = d.wc_o[ic * kCl + a];
-  }
-  const float aO = W.aO1, bO = W.bO1, qow = W.crg_ow, qhw = W.crg_hw;
-  // instances for 3-atom solvent windows (W3) and for SPC windows
-  constexpr bool wat3 = W3;
-  if ((W.wat3 != 0) != W3) return;
+  const int slot = wk.y + (lane < wk.z ? lane : 0);
+  const int ow = lane < wk.z ? d.wc_o[slot] : -1;
+  const bool on = ow >= 0 && d.qw_on[slot] && d.qin[ow];   // the lane's water is in the Q lists
+  float4 pw[3];
+  for (int k = 0; k < 3; ++k) pw[k] = d.xw[3 * (size_t)slot + k];
+  double pd[9];
+  if (EN)
+    for (int k = 0; k < 3; ++k) {
+      const double4 t = d.xwd[3 * (size_t)slot + k];
+      pd[3 * k] = t.x; pd[3 * k + 1] = t.y; pd[3 * k + 2] = t.z;
+    }
   float lam[kMaxS];
   for (int s = 0; s < kMaxS; ++s) lam[s] = s < S ? (float)W.lambda[s] : 0.f;
-  // per-state parameters of the lane's q-atom (fixed on the q side)
-  float h_qc[kMaxS] = {}, h_sc[kMaxS] = {};
-  float4 h_ql[kMaxS] = {};
-  if (Q_SIDE && iq_l >= 0) {
-    for (int s = 0; s < S; ++s) {
-      h_ql[s] = d.q_lj[W.qs_off + iq_l * S + s];
-      h_qc[s] = d.q_crg[W.qs_off + iq_l * S + s];
-      h_sc[s] = qvdw ? d.q_sc[W.qsc_off + ((size_t)iq_l * W.natyps + W.iac_ow) * S + s] : 0.f;
-    }
-  }
-  const float4 pq_fixed = (Q_SIDE && qa >= 0) ? d.x32[qa] : make_float4(0, 0, 0, 0);
-  float4 pw_fixed[3];
-  for (int k = 0; k < 3; ++k) pw_fixed[k] = (!Q_SIDE && ow >= 0) ? d.x32[ow + k] : make_float4(0, 0, 0, 0);
-  const bool w_in = Q_SIDE || (ow >= 0 && d.qin[ow]);   // the lane's water is in the Q lists
-  const int s0 = wk.y, n = wk.z, lst = L.start[ic];
-  float g[9];
-  for (int k = 0; k < 9; ++k) g[k] = 0.f;
-  long long gfix[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  // the q side only computes energies (on energy steps)
-  if (Q_SIDE && !st.energy_now) return;
-  // kQGroup tiles per pass (work items start on a kQGroup boundary of the
-  // list): the tile, index and coordinate loads of the pass are issued
-  // before its arithmetic; the sums run in tile order and go to fixed point
-  // after each pass
-  for (int t0 = 0; !Q_SIDE && t0 < n; t0 += kQGroup) {
-    bool on[kQGroup];
-    int jx[kQGroup];
-#pragma unroll
-    for (int u = 0; u < kQGroup; ++u) {
-      const int tt = s0 + min(t0 + u, n - 1);
-      const int jc = L.jc[tt];
-      on[u] = t0 + u < n && lane_bit(L.mask[tt], lane) && w_in;
-      // water O atom (q side), or the q-cluster member index (water side)
-      jx[u] = Q_SIDE ? d.wc_o[jc * kCl + b] : jc * kCl + b;
-    }
-    float4 pwv[kQGroup][3];
-    float4 pqv[kQGroup];
-    float rx[kQGroup] = {}, ry[kQGroup] = {}, rz[kQGroup] = {};   // water side: reaction per tile
-#pragma unroll
-    for (int u = 0; u < kQGroup; ++u) {
-      if (Q_SIDE) {
-        const int jj = on[u] ? jx[u] : 0;
-        for (int k = 0; k < 3; ++k) pwv[u][k] = d.x32[jj + k];
-      } else {
-        pqv[u] = d.xq[on[u] ? jx[u] : 0];   // the q-atom's coordinates from its q-cluster slot
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kQGroup; ++u) {
-      if (!on[u]) continue;
-      const float4 pq = Q_SIDE ? pq_fixed : pqv[u];
-      float dxv[3], dyv[3], dzv[3], r2v[3];
-      for (int k = 0; k < 3; ++k) {
-        const float4 pw = Q_SIDE ? pwv[u][k] : pw_fixed[k];
-        dxv[k] = pw.x - pq.x; dyv[k] = pw.y - pq.y; dzv[k] = pw.z - pq.z;
-        r2v[k] = dxv[k] * dxv[k] + dyv[k] * dyv[k] + dzv[k] * dzv[k];
-      }
-      const float rO = rsq_r2(r2v[0]), r2O = rO * rO;
-      const float rH1 = rsq_r2(r2v[1]), r2H1 = rH1 * rH1;
-      const float rH2 = rsq_r2(r2v[2]), r2H2 = rH2 * rH2;
-      const float r6hc = r2v[0] * r2v[0] * r2v[0];
-      float dvO = 0.f, dvH1 = 0.f, dvH2 = 0.f;
-      for (int s = 0; s < S; ++s) {
-        // A, B with the oxygen and the charge products (packed per member
-        // on the water side, formed from the lane's q-atom on the q side)
-        float4 P;
-        float sc;
-        if (Q_SIDE) {
-          float A, B;
-          lj_ab(h_ql[s].x, h_ql[s].y, aO, bO, W.arith != 0, &A, &B);
-          P = make_float4(A, B, qow * h_qc[s], qhw * h_qc[s]);
-          sc = h_sc[s];
-        } else {
-          P = d.qcw_par[(size_t)jx[u] * kMaxS + s];
-          sc = d.qcw_sc[(size_t)jx[u] * kMaxS + s];
-        }
-        float va, vb, ratio = 1.f;
-        if (qvdw) {
-          const float inv = rcp(r6hc + sc);
-          va = P.x * inv * inv;
-          vb = P.y * inv;
-          ratio = r6hc * inv;
-        } else {
-          const float r6 = r2O * r2O * r2O;
-          va = P.x * r6 * r6;
-          vb = P.y * r6;
-        }
-        const float velO = P.z * rO, velH1 = P.w * rH1, velH2 = P.w * rH2;
-        dvO += r2O * (-velO - (12.f * va - 6.f * vb) * ratio) * lam[s];
-        if (!Q_SIDE && wat3) {
-          // 3-atom solvent: LJ and soft-core on the hydrogens too, and their
-          // own charges (nonbond_qw_3atom, md.f90:11620-11640)
-          for (int k = 1; k < 3; ++k) {
-            const float4 H = d.qcw_h[((size_t)jx[u] * kMaxS + s) * 2 + k - 1];
-            const float r2k = r2v[k], r2ik = k == 1 ? r2H1 : r2H2, rk = k == 1 ? rH1 : rH2;
-            const float r6k = r2k * r2k * r2k;
-            float vak, vbk, ratk = 1.f;
-            if (qvdw) {
-              const float inv = rcp(r6k + H.w);
-              vak = H.x * inv * inv;
-              vbk = H.y * inv;
-              ratk = r6k * inv;
-            } else {
-              const float r6i = r2ik * r2ik * r2ik;
-              vak = H.x * r6i * r6i;
-              vbk = H.y * r6i;
-            }
-            const float dvk = r2ik * (-(H.z * rk) - (12.f * vak - 6.f * vbk) * ratk) * lam[s];
-            if (k == 1) dvH1 += dvk;
-            else dvH2 += dvk;
-          }
-        } else {
-          dvH1 -= r2H1 * velH1 * lam[s];
-          dvH2 -= r2H2 * velH2 * lam[s];
-        }
-      }
-      if (Q_SIDE) {
-        g[0] -= dvO * dxv[0] + dvH1 * dxv[1] + dvH2 * dxv[2];
-        g[1] -= dvO * dyv[0] + dvH1 * dyv[1] + dvH2 * dyv[2];
-        g[2] -= dvO * dzv[0] + dvH1 * dzv[1] + dvH2 * dzv[2];
-      } else {
-        g[0] += dvO * dxv[0]; g[1] += dvO * dyv[0]; g[2] += dvO * dzv[0];
-        g[3] += dvH1 * dxv[1]; g[4] += dvH1 * dyv[1]; g[5] += dvH1 * dzv[1];
-        g[6] += dvH2 * dxv[2]; g[7] += dvH2 * dyv[2]; g[8] += dvH2 * dzv[2];
-        rx[u] = dvO * dxv[0] + dvH1 * dxv[1] + dvH2 * dxv[2];
-        ry[u] = dvO * dyv[0] + dvH1 * dyv[1] + dvH2 * dyv[2];
-        rz[u] = dvO * dzv[0] + dvH1 * dzv[1] + dvH2 * dzv[2];
-      }
-    }
-    for (int k = 0; k < 9; ++k) { gfix[k] += fix((double)g[k], kFScale); g[k] = 0.f; }
-    if (!Q_SIDE) q_reaction(d, d.qslot_wq, lane, s0 + t0, t0, n, rx, ry, rz);
-  }
-  if (!Q_SIDE) {
-    long long gs[9];
-    for (int k = 0; k < 9; ++k) gs[k] = row8_sum_i(gfix[k]);
-    if (b == 0 && ow >= 0)
-      for (int p = 0; p < 3; ++p) add_grad_fix(d.f, ow + p, gs[3 * p], gs[3 * p + 1], gs[3 * p + 2]);
-    return;
-  }
-  // energy pass (FP64), q side only: the lane's q-atom is fixed, so its
-  // per-state charge products and, per LJ site of the water (the oxygen, or
-  // all three atoms of a 3-atom solvent, nonbond_qw_3atom), A, B and the
-  // soft-core term are formed once before the tile loop
+  const ConstF xq = (ConstF)(const float*)d.xq, par = (ConstF)(const float*)d.qcw_par, sct = (ConstF)d.qcw_sc;
+  const ConstF parh = (ConstF)(const float*)d.qcw_h;
+  const ConstD pare = (ConstD)(const double*)d.qcw_e, xd = (ConstD)d.x;
+  const ConstI qat = (ConstI)d.qc_atom;
   constexpr int NLJ = W3 ? 3 : 1;
-  float qqk[kMaxS][3];
-  double A[kMaxS][NLJ], B[kMaxS][NLJ], SC[kMaxS][NLJ];
-#pragma unroll
-  for (int s = 0; s < kMaxS; ++s) {
-    const int ss = s < S ? s : 0;
-    const int iqs = iq_l >= 0 ? iq_l : 0;
-    const float qc = d.q_crg[W.qs_off + iqs * S + ss];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) qqk[s][k] = W.crg_w[k] * qc;   // real(4) products as in the reference
-    const double* ql = &d.q_ljd[(size_t)(W.qs_off + iqs * S + ss) * 4];
-#pragma unroll
-    for (int k = 0; k < NLJ; ++k) {
-      const double* tl = &d.t_lj[(W.t_off + W.iac_w[k]) * 4];
-      lj_ab(ql[0], ql[1], tl[0], tl[1], W.arith != 0, &A[s][k], &B[s][k]);
-      SC[s][k] = W.qvdw ? d.q_scd[W.qsc_off + ((size_t)iqs * W.natyps + W.iac_w[k]) * S + ss] : 0.0;
-    }
-  }
-  long long efix[kMaxS][2] = {};
   double eel[kMaxS] = {}, evdw[kMaxS] = {};
-  const int qa0 = qa >= 0 ? qa : 0;
-  const double xq = d.x[3 * qa0], yq = d.x[3 * qa0 + 1], zq = d.x[3 * qa0 + 2];
-  for (int t = 0; t < n; ++t) {
-    const int jc = L.jc[s0 + t];
-    const uint2 m = L.mask[s0 + t];
-    const int o = d.wc_o[jc * kCl + b];
-    if (lane_bit(m, lane) && d.qin[o]) {
-      double rinv[3], r6[NLJ];
+  for (int ch = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); ch < W.nqch; ch += kQWaves) {
+    const int q0 = (ch >> 1) * 4 * kCl + (ch & 1) * 4;   // the chunk's first q-atom
+    const int slot0 = W.qc_off * kCl + q0;
+    QReaction react;
+#pragma unroll 1
+    for (int mb = 0; mb < 4; ++mb) {
+      if (q0 + mb >= W.nq) break;
+      float g[9] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+      for (int u = 0; u < 4; ++u) {
+        if (q0 + kCl * u + mb >= W.nq) break;
+        const int m = slot0 + kCl * u + mb;
+        const float qx = xq[4 * m], qy = xq[4 * m + 1], qz = xq[4 * m + 2];
+        float rx = 0.f, ry = 0.f, rz = 0.f;
+        if (on) {
+          float dxv[3], dyv[3], dzv[3], r2v[3];
+  #pragma unroll
+          for (int k = 0; k < 3; ++k) {
+            dxv[k] = pw[k].x - qx; dyv[k] = pw[k].y - qy; dzv[k] = pw[k].z - qz;
+            r2v[k] = r2_f(dxv[k], dyv[k], dzv[k]);
+          }
+          const float rO = rsq_r2(r2v[0]), r2O = rO * rO;
+          const float rH1 = rsq_r2(r2v[1]), r2H1 = rH1 * rH1;
+          const float rH2 = rsq_r2(r2v[2]), r2H2 = rH2 * rH2;
+          const float r6hc = r2v[0] * r2v[0] * r2v[0];
+          float dvO = 0.f, dvH1 = 0.f, dvH2 = 0.f;
+  #pragma unroll
+          for (int s = 0; s < (NS ? NS : kMaxS); ++s) {
+            if (!NS && s >= S) break;
+            // A, B with the oxygen, the charge products with oxygen and
+            // hydrogen, the soft-core term
+            const ConstF P = par + 4 * ((size_t)m * kMaxS + s);
+            const float pa = P[0], pb = P[1], po = P[2], ph = P[3];
+            float va, vb, ratio = 1.f;
+            if (qvdw) {
+              const float inv = rcp(r6hc + sct[(size_t)m * kMaxS + s]);
+              va = pa * inv * inv;
+              vb = pb * inv;
+              ratio = r6hc * inv;
+            } else {
+              const float r6 = r2O * r2O * r2O;
+              va = pa * r6 * r6;
+              vb = pb * r6;
+            }
+            dvO = dv_f(dvO, r2O, po, rO, lj_f(va, vb, ratio), lam[s]);
+            if (W3) {
+              // 3-atom solvent: LJ and soft-core on the hydrogens too, and their
+              // own charges (md.f90:11620-11640)
+  #pragma unroll
+              for (int k = 1; k < 3; ++k) {
+                const ConstF H = parh + 4 * (((size_t)m * kMaxS + s) * 2 + k - 1);
+                const float r2k = r2v[k], r2ik = k == 1 ? r2H1 : r2H2, rk = k == 1 ? rH1 : rH2;
+                const float r6k = r2k * r2k * r2k;
+                float vak, vbk, ratk = 1.f;
+                if (qvdw) {
+                  const float inv = rcp(r6k + H[3]);
+                  vak = H[0] * inv * inv;
+                  vbk = H[1] * inv;
+                  ratk = r6k * inv;
+                } else {
+                  const float r6i = r2ik * r2ik * r2ik;
+                  vak = H[0] * r6i * r6i;
+                  vbk = H[1] * r6i;
+                }
+                float& dvk = k == 1 ? dvH1 : dvH2;
+                dvk = dv_f(dvk, r2ik, H[2], rk, lj_f(vak, vbk, ratk), lam[s]);
+              }
+            } else {
+              dvH1 = __builtin_fmaf(-(r2H1 * (ph * rH1)), lam[s], dvH1);
+              dvH2 = __builtin_fmaf(-(r2H2 * (ph * rH2)), lam[s], dvH2);
+            }
+          }
+          const float dv[3] = {dvO, dvH1, dvH2};
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        // the water's FP64 coordinates from its cluster slot
-        const double4 pw = d.xwd[3 * (jc * kCl + b) + k];
-        const double dx = pw.x - xq;
-        const double dy = pw.y - yq;
-        const double dz = pw.z - zq;
-        const double r2 = dx * dx + dy * dy + dz * dz;
-        rinv[k] = rsqrt_e(r2);
-        if (k < NLJ) r6[k < NLJ ? k : 0] = r2 * r2 * r2;
-      }
-#pragma unroll
-      for (int s = 0; s < kMaxS; ++s) {
-        if (s >= S) break;
-        double e = 0.0;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) e += (double)qqk[s][k] * rinv[k];
-        eel[s] += e;
-        double ev = 0.0;
-#pragma unroll
-        for (int k = 0; k < NLJ; ++k) {
-          const double inv = rcp_e(r6[k] + SC[s][k]);
-          ev += A[s][k] * inv * inv - B[s][k] * inv;
+          for (int k = 0; k < 3; ++k) {
+            g[3 * k] = __builtin_fmaf(dv[k], dxv[k], g[3 * k]);
+            g[3 * k + 1] = __builtin_fmaf(dv[k], dyv[k], g[3 * k + 1]);
+            g[3 * k + 2] = __builtin_fmaf(dv[k], dzv[k], g[3 * k + 2]);
+          }
+          rx = __builtin_fmaf(dvH2, dxv[2], W3 ? __builtin_fmaf(dvH1, dxv[1], dvO * dxv[0])
+                                               : __builtin_fmaf(dvO, dxv[0], dvH1 * dxv[1]));
+          ry = __builtin_fmaf(dvH2, dyv[2], __builtin_fmaf(dvO, dyv[0], dvH1 * dyv[1]));
+          rz = __builtin_fmaf(dvH2, dzv[2], __builtin_fmaf(dvO, dzv[0], dvH1 * dzv[1]));
+          if (EN) {
+            const ConstD qd = xd + 3 * (size_t)qat[m];
+            double rinv[3], r6[NLJ];
+  #pragma unroll
+            for (int k = 0; k < 3; ++k) {
+              const double dx = pd[3 * k] - qd[0], dy = pd[3 * k + 1] - qd[1], dz = pd[3 * k + 2] - qd[2];
+              const double r2 = dx * dx + dy * dy + dz * dz;
+              rinv[k] = rsqrt_e(r2);
+              if (k < NLJ) r6[k < NLJ ? k : 0] = r2 * r2 * r2;
+            }
+  #pragma unroll
+            for (int s = 0; s < (NS ? NS : kMaxS); ++s) {
+              if (!NS && s >= S) break;
+  #pragma unroll
+              for (int k = 0; k < 3; ++k) {
+                const ConstD E = pare + 4 * (((size_t)m * kMaxS + s) * 3 + k);   // A, B, soft-core, charge product
+                eel[s] += E[3] * rinv[k];
+                if (k < NLJ) {
+                  const double inv = rcp_e(r6[k < NLJ ? k : 0] + E[2]);
+                  evdw[s] += E[0] * inv * inv - E[1] * inv;
+                }
+              }
+            }
+          }
         }
-        evdw[s] += ev;
+        react.add(4 * mb + u, rx, ry, rz);
+      }
+      for (int k = 0; k < 9; ++k) acc[k] += (double)g[k];
+    }
+    react.flush(d, slot0, W.nq - q0);
+  }
+  if (EN)
+#pragma unroll
+    for (int s = 0; s < (NS ? NS : kMaxS); ++s) {
+      if (!NS && s >= S) break;
+      const long long e1 = wave_sum_i(fix(eel[s], kEScale)), e2 = wave_sum_i(fix(evdw[s], kEScale));
+      if (lane == 0) {
+        add_energy_fix(d.ws, w, E_QW0 + 2 * s, e1);
+        add_energy_fix(d.ws, w, E_QW0 + 2 * s + 1, e2);
       }
     }
-    if (((s0 + t - lst) % kQGroup) == kQGroup - 1 || t == n - 1)
-      for (int s = 0; s < kMaxS; ++s) {
-        efix[s][0] += fix(eel[s], kEScale); efix[s][1] += fix(evdw[s], kEScale);
-        eel[s] = 0.0; evdw[s] = 0.0;
-      }
-  }
-  for (int s = 0; s < S; ++s) {
-    const long long e1 = wave_sum_i(efix[s][0]), e2 = wave_sum_i(efix[s][1]);
-    if (lane == 0) { add_energy_fix(d.ws, w, E_QW0 + 2 * s, e1); add_energy_fix(d.ws, w, E_QW0 + 2 * s + 1, e2); }
-  }
 }
 
-// q-atom vs solute atom (nonbond_qp_qvdw / nonbond_qp, md.f90:11138-11204,
-// 10980-11045)
-template <bool Q_SIDE>
-__global__ void __launch_bounds__(256) k_qp(Dev d) {
-  const int wave = wave_id(d);
-  const int lane = threadIdx.x & 63;
-  const TileList L = d.tl[Q_SIDE ? T_QP : T_PQ];
-  if (wave >= L.nwork) return;
-  const int4 wk = L.work[wave];
-  const int ic = wk.x;
-  const int w = Q_SIDE ? d.qc_win[ic] : d.sc_win[ic];
-  const WinState& st = d.ws[w];
-  if (!st.active) return;
-  const WinDev& W = d.win[w];
-  const int S = W.S;
+// W3: the instance for 3-atom solvent windows; EK: the instance of steps
+// where some window computes energies
+template <bool W3, bool EK>
+__global__ void __launch_bounds__(64 * kQWaves) k_qw(Dev d) {
+  const int4 wk = q_item(d.qw_work, block_id(d.xcd));
+  const WinDev& W = d.win[wk.x];
+  if (!d.ws[wk.x].active || (W.wat3 != 0) != W3) return;   // uniform over the block
+  const bool en = EK && d.ws[wk.x].energy_now;
+  double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  if (W.S == 2) {
+    if (en) qw_impl<W3, EK, 2>(d, W, wk, acc);
+    else qw_impl<W3, false, 2>(d, W, wk, acc);
+  } else {
+    if (en) qw_impl<W3, EK, 0>(d, W, wk, acc);
+    else qw_impl<W3, false, 0>(d, W, wk, acc);
+  }
+  q_store<9>(acc, wk.z, d.gq + 9 * (size_t)wk.y);
+}
+
+template <bool EN, int NS>
+__device__ __forceinline__ void qp_impl(const Dev& d, const WinDev& W, const int4 wk, double acc[3]) {
+  const int lane = threadIdx.x & 63, w = wk.x;
+  const int S = NS ? NS : W.S;
   const bool qvdw = W.qvdw, arith = W.arith;
   const float el14 = W.el14;
-  const int a = lane >> 3, b = lane & 7;
-  int iq_l = -1, qa = -1, pa = -1;
-  if (Q_SIDE) {
-    iq_l = d.qc_q[ic * kCl + a];
-    if (iq_l >= 0) qa = d.q_atom[W.q_off + iq_l];
-  } else {
-    pa = d.sc_a[ic * kCl + a];
+  const int slot = wk.y + (lane < wk.z ? lane : 0);
+  const int pa = lane < wk.z ? d.sc_a[slot] : -1;
+  const bool on = pa >= 0 && d.qp_on[slot] && d.qin[pa];   // the lane's solute atom is in the Q lists
+  const int ia = pa >= 0 ? pa : W.ao;
+  const float4 pj = d.x32[ia], lj = d.ljp[ia];
+  const int iacj = d.iac[ia];
+  double xj[3];
+  double4 tlj = make_double4(0, 0, 0, 0);
+  if (EN) {
+    for (int c = 0; c < 3; ++c) xj[c] = d.x[3 * (size_t)ia + c];
+    tlj = d.ljd[ia];
   }
   float lam[kMaxS];
   for (int s = 0; s < kMaxS; ++s) lam[s] = s < S ? (float)W.lambda[s] : 0.f;
-  float h_qc[kMaxS] = {};
-  float4 h_ql[kMaxS] = {};
-  if (Q_SIDE && iq_l >= 0) {
-    for (int s = 0; s < S; ++s) {
-      h_ql[s] = d.q_lj[W.qs_off + iq_l * S + s];
-      h_qc[s] = d.q_crg[W.qs_off + iq_l * S + s];
-    }
-  }
-  const float4 pq_fixed = (Q_SIDE && qa >= 0) ? d.x32[qa] : make_float4(0, 0, 0, 0);
-  const float4 pp_fixed = (!Q_SIDE && pa >= 0) ? d.x32[pa] : make_float4(0, 0, 0, 0);
-  const float4 lj_fixed = (!Q_SIDE && pa >= 0) ? d.ljp[pa] : make_float4(0, 0, 0, 0);
-  const int iac_fixed = (!Q_SIDE && pa >= 0) ? d.iac[pa] : 0;
-  const bool p_in = Q_SIDE || (pa >= 0 && d.qin[pa]);   // the lane's solute atom is in the Q lists
-  const int s0 = wk.y, n = wk.z, lst = L.start[ic];
-  float g0 = 0.f, g1 = 0.f, g2 = 0.f;
-  long long gx = 0, gy = 0, gz = 0;
-  if (Q_SIDE && !st.energy_now) return;   // the q side only computes energies
-  // kQGroup tiles per pass, loads first (as in k_qw)
-  for (int t0 = 0; !Q_SIDE && t0 < n; t0 += kQGroup) {
-    bool on[kQGroup], o14[kQGroup];
-    int jx[kQGroup], jm[kQGroup];
-#pragma unroll
-    for (int u = 0; u < kQGroup; ++u) {
-      const int tt = s0 + min(t0 + u, n - 1);
-      const int jc = L.jc[tt];
-      on[u] = t0 + u < n && lane_bit(L.mask[tt], lane) && p_in;
-      o14[u] = lane_bit(L.m14[tt], lane);
-      jm[u] = jc * kCl + b;   // the member's slot
-      jx[u] = Q_SIDE ? d.sc_a[jm[u]] : d.qc_q[jm[u]];
-    }
-    float4 pv[kQGroup], lv[kQGroup];
-    int iacv[kQGroup];
-    float rx[kQGroup] = {}, ry[kQGroup] = {}, rz[kQGroup] = {};   // solute side: reaction per tile
-#pragma unroll
-    for (int u = 0; u < kQGroup; ++u) {
-      const int jj = on[u] ? jx[u] : 0;
-      if (Q_SIDE) {
-        pv[u] = d.x32[jj];
-        lv[u] = d.ljp[jj];
-        iacv[u] = d.iac[jj];
-      } else {
-        // the q-atom's coordinates from its q-cluster slot
-        pv[u] = d.xq[on[u] ? jm[u] : 0];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kQGroup; ++u) {
-      if (!on[u]) continue;
-      const bool is14 = o14[u];
-      const int iq = Q_SIDE ? iq_l : jx[u];
-      const float4 pq = Q_SIDE ? pq_fixed : pv[u];
-      const float4 pj = Q_SIDE ? pv[u] : pp_fixed;
-      const float4 lj = Q_SIDE ? lv[u] : lj_fixed;
-      const int iacj = Q_SIDE ? iacv[u] : iac_fixed;
-      const float dx = pj.x - pq.x, dy = pj.y - pq.y, dz = pj.z - pq.z;
-      const float r2 = dx * dx + dy * dy + dz * dz;
-      const float rinv = rsq_r2(r2), r2inv = rinv * rinv;
-      const float r6hc = r2 * r2 * r2;
-      float dv = 0.f;
-      for (int s = 0; s < S; ++s) {
-        const float4 ql = Q_SIDE ? h_ql[s] : d.q_lj[W.qs_off + iq * S + s];
-        const float qc = Q_SIDE ? h_qc[s] : d.q_crg[W.qs_off + iq * S + s];
-        float aLJ, bLJ;
-        if (is14) lj_ab(ql.z, ql.w, lj.z, lj.w, arith, &aLJ, &bLJ);
-        else lj_ab(ql.x, ql.y, lj.x, lj.y, arith, &aLJ, &bLJ);
-        float vel = (qc * pj.w) * rinv;
-        if (is14) vel *= el14;
-        float va, vb, ratio = 1.f;
-        if (qvdw) {
-          const float inv = rcp(r6hc + d.q_sc[W.qsc_off + ((size_t)iq * W.natyps + iacj) * S + s]);
-          va = aLJ * inv * inv;
-          vb = bLJ * inv;
-          ratio = r6hc * inv;
-        } else {
-          const float r6 = r2inv * r2inv * r2inv;
-          va = aLJ * r6 * r6;
-          vb = bLJ * r6;
-        }
-        dv += r2inv * (-vel - (12.f * va - 6.f * vb) * ratio) * lam[s];
-      }
-      if (Q_SIDE) { g0 -= dv * dx; g1 -= dv * dy; g2 -= dv * dz; }
-      else {
-        g0 += dv * dx; g1 += dv * dy; g2 += dv * dz;
-        rx[u] = dv * dx; ry[u] = dv * dy; rz[u] = dv * dz;
-      }
-    }
-    gx += fix((double)g0, kFScale); gy += fix((double)g1, kFScale); gz += fix((double)g2, kFScale);
-    g0 = g1 = g2 = 0.f;
-    if (!Q_SIDE) q_reaction(d, 0, lane, s0 + t0, t0, n, rx, ry, rz);
-  }
-  if (!Q_SIDE) {
-    const long long sx = row8_sum_i(gx), sy = row8_sum_i(gy), sz = row8_sum_i(gz);
-    if (b == 0 && pa >= 0) add_grad_fix(d.f, pa, sx, sy, sz);
-    return;
-  }
-  // energy pass (FP64); the per-state parameters are loaded in the tile
-  // loop (holding them in registers costs more occupancy than it saves)
-  long long efix[kMaxS][2] = {};
+  const ConstF xq = (ConstF)(const float*)d.xq, qlj = (ConstF)(const float*)(d.q_lj + W.qs_off);
+  const ConstF qcr = (ConstF)(d.q_crg + W.qs_off);
+  const ConstD xd = (ConstD)d.x, qljd = (ConstD)(d.q_ljd + 4 * (size_t)W.qs_off);
+  const ConstI qat = (ConstI)d.qc_atom;
+  const float* sct = d.q_sc + W.qsc_off + (size_t)iacj * S;
+  const double* scd = d.q_scd + W.qsc_off + (size_t)iacj * S;
   double eel[kMaxS] = {}, evdw[kMaxS] = {};
-  const double* x = d.x;
-  for (int t = 0; t < n; ++t) {
-    const int jc = L.jc[s0 + t];
-    const uint2 m = L.mask[s0 + t];
-    const int j = d.sc_a[jc * kCl + b];
-    if (lane_bit(m, lane) && j >= 0 && d.qin[j]) {
-      const bool is14 = lane_bit(L.m14[s0 + t], lane);
-      // nonbond_qp_qvdw (md.f90:11138-11204): per state
-      const double dx = x[3 * j] - x[3 * qa], dy = x[3 * j + 1] - x[3 * qa + 1], dz = x[3 * j + 2] - x[3 * qa + 2];
-      const double r2 = dx * dx + dy * dy + dz * dz;
-      const double rinv = rsqrt_e(r2);
-      const double r6 = r2 * r2 * r2;
-      const float qj = d.x32[j].w;
-      const int iacj = d.iac[j];
-      const double* tl = &d.t_lj[(W.t_off + iacj) * 4];
-      const int k = is14 ? 2 : 0;
-      const double ta = tl[k], tb = tl[k + 1];
-      for (int s = 0; s < S; ++s) {
-        double vel = (double)(d.q_crg[W.qs_off + iq_l * S + s] * qj) * rinv;
-        if (is14) vel *= W.el14d;
-        eel[s] += vel;
-        const double* ql = &d.q_ljd[(size_t)(W.qs_off + iq_l * S + s) * 4];
-        double aLJ, bLJ;
-        lj_ab(ql[k], ql[k + 1], ta, tb, W.arith != 0, &aLJ, &bLJ);
-        const double sc = W.qvdw ? d.q_scd[W.qsc_off + ((size_t)iq_l * W.natyps + iacj) * S + s] : 0.0;
-        const double inv = rcp_e(r6 + sc);
-        evdw[s] += aLJ * inv * inv - bLJ * inv;
+  for (int ch = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); ch < W.nqch; ch += kQWaves) {
+    const int q0 = (ch >> 1) * 4 * kCl + (ch & 1) * 4;   // the chunk's first q-atom
+    const int slot0 = W.qc_off * kCl + q0;
+    // 1-4 pairs with the chunk's q-atoms, bit j for q-atom j
+    const unsigned m14 = d.qp14[W.qp14_off + (size_t)(slot - W.sc_off * kCl) * W.nqch + ch];
+    QReaction react;
+#pragma unroll 1
+    for (int mb = 0; mb < 4; ++mb) {
+      if (q0 + mb >= W.nq) break;
+      float g0 = 0.f, g1 = 0.f, g2 = 0.f;
+#pragma unroll 1
+      for (int u = 0; u < 4; ++u) {
+        const int iq = q0 + kCl * u + mb;
+        if (iq >= W.nq) break;
+        const int m = slot0 + kCl * u + mb, j = 4 * mb + u;
+        const float qx = xq[4 * m], qy = xq[4 * m + 1], qz = xq[4 * m + 2];
+        float rx = 0.f, ry = 0.f, rz = 0.f;
+        if (on) {
+          const bool is14 = (m14 >> j) & 1u;
+          const float dx = pj.x - qx, dy = pj.y - qy, dz = pj.z - qz;
+          const float r2 = r2_f(dx, dy, dz);
+          const float rinv = rsq_r2(r2), r2inv = rinv * rinv;
+          const float r6hc = r2 * r2 * r2;
+          float dv = 0.f;
+  #pragma unroll
+          for (int s = 0; s < (NS ? NS : kMaxS); ++s) {
+            if (!NS && s >= S) break;
+            const ConstF ql = qlj + 4 * (iq * S + s);
+            const float qc = qcr[iq * S + s];
+            float aLJ, bLJ;
+            if (is14) lj_ab((float)ql[2], (float)ql[3], lj.z, lj.w, arith, &aLJ, &bLJ);
+            else lj_ab((float)ql[0], (float)ql[1], lj.x, lj.y, arith, &aLJ, &bLJ);
+            float vel = (qc * pj.w) * rinv;
+            if (is14) vel *= el14;
+            float va, vb, ratio = 1.f;
+            if (qvdw) {
+              const float inv = rcp(r6hc + sct[(size_t)iq * W.natyps * S + s]);
+              va = aLJ * inv * inv;
+              vb = bLJ * inv;
+              ratio = r6hc * inv;
+            } else {
+              const float r6 = r2inv * r2inv * r2inv;
+              va = aLJ * r6 * r6;
+              vb = bLJ * r6;
+            }
+            // (the charge term's factors are rounded one by one: el14 comes between)
+            dv = __builtin_fmaf(r2inv * __builtin_fmaf(-ratio, lj_f(va, vb, 1.f), -vel), lam[s], dv);
+          }
+          g0 = __builtin_fmaf(dv, dx, g0); g1 = __builtin_fmaf(dv, dy, g1); g2 = __builtin_fmaf(dv, dz, g2);
+          rx = dv * dx; ry = dv * dy; rz = dv * dz;
+          if (EN) {
+            const ConstD qd = xd + 3 * (size_t)qat[m];
+            const double ex = xj[0] - qd[0], ey = xj[1] - qd[1], ez = xj[2] - qd[2];
+            const double rr = ex * ex + ey * ey + ez * ez;
+            const double ri = rsqrt_e(rr), r6 = rr * rr * rr;
+            const double ta = is14 ? tlj.z : tlj.x, tb = is14 ? tlj.w : tlj.y;
+  #pragma unroll
+            for (int s = 0; s < (NS ? NS : kMaxS); ++s) {
+              if (!NS && s >= S) break;
+              double vel = (double)(qcr[iq * S + s] * pj.w) * ri;
+              if (is14) vel *= W.el14d;
+              eel[s] += vel;
+              const ConstD ql = qljd + 4 * (iq * S + s);
+              double aLJ, bLJ;
+              lj_ab(is14 ? (double)ql[2] : (double)ql[0], is14 ? (double)ql[3] : (double)ql[1], ta, tb, arith, &aLJ, &bLJ);
+              const double inv = rcp_e(r6 + (qvdw ? scd[(size_t)iq * W.natyps * S + s] : 0.0));
+              evdw[s] += aLJ * inv * inv - bLJ * inv;
+            }
+          }
+        }
+        react.add(j, rx, ry, rz);
+      }
+      acc[0] += (double)g0; acc[1] += (double)g1; acc[2] += (double)g2;
+    }
+    react.flush(d, slot0, W.nq - q0);
+  }
+  if (EN)
+#pragma unroll
+    for (int s = 0; s < (NS ? NS : kMaxS); ++s) {
+      if (!NS && s >= S) break;
+      const long long e1 = wave_sum_i(fix(eel[s], kEScale)), e2 = wave_sum_i(fix(evdw[s], kEScale));
+      if (lane == 0) {
+        add_energy_fix(d.ws, w, E_Q0 + 8 * s + 6, e1);
+        add_energy_fix(d.ws, w, E_Q0 + 8 * s + 7, e2);
       }
     }
-    if (((s0 + t - lst) % kQGroup) == kQGroup - 1 || t == n - 1)
-      for (int s = 0; s < kMaxS; ++s) {
-        efix[s][0] += fix(eel[s], kEScale); efix[s][1] += fix(evdw[s], kEScale);
-        eel[s] = 0.0; evdw[s] = 0.0;
-      }
+}
+
+template <bool EK>
+__global__ void __launch_bounds__(64 * kQWaves) k_qp(Dev d) {
+  const int4 wk = q_item(d.qp_work, block_id(d.xcd));
+  const WinDev& W = d.win[wk.x];
+  if (!d.ws[wk.x].active) return;   // uniform over the block
+  const bool en = EK && d.ws[wk.x].energy_now;
+  double acc[3] = {0, 0, 0};
+  if (W.S == 2) {
+    if (en) qp_impl<EK, 2>(d, W, wk, acc);
+    else qp_impl<false, 2>(d, W, wk, acc);
+  } else {
+    if (en) qp_impl<EK, 0>(d, W, wk, acc);
+    else qp_impl<false, 0>(d, W, wk, acc);
   }
-  for (int s = 0; s < S; ++s) {
-    const long long e1 = wave_sum_i(efix[s][0]), e2 = wave_sum_i(efix[s][1]);
-    if (lane == 0) { add_energy_fix(d.ws, w, E_Q0 + 8 * s + 6, e1); add_energy_fix(d.ws, w, E_Q0 + 8 * s + 7, e2); }
-  }
+  q_store<3>(acc, wk.z, d.gq + 9 * (size_t)d.nwslot + 3 * (size_t)wk.y);
 }
 
 // q-q and q-(bonded neighbour) pairs (nonbond_qq, md.f90:10763-10868), one
@@ -1508,8 +1465,6 @@ __device__ __forceinline__ void lrf_add(double s[kLrfSums], double q, double dx,
 // SIMD: 1.54 ms for the ladder against 1.38 without.  With sources broadcast
 // through LDS and vector loads, all terms formed and 8 parts it was 2.07 ms,
 // and 131 us for the one window, now 40.
-typedef const double __attribute__((address_space(4))) * ConstD;   // read with scalar loads
-typedef const int __attribute__((address_space(4))) * ConstI;
 __global__ void __launch_bounds__(64 * kLrfWaves, 4) k_lrf_build(Dev d) {
   const int4 lw = d.lrf_work[block_id(d.xcd)];   // window, first target group, count, source part
   const WinState& st = d.ws[lw.x];
@@ -1617,7 +1572,6 @@ __global__ void __launch_bounds__(kLrfReduceGroups * kLrfSums) k_lrf_reduce(Dev 
 }
 
 // Evaluation per atom (lrf_taylor, md.f90:3646-3712), FP64.
-template <bool LOCAL>
 __device__ __forceinline__ void lrf_taylor_atom(const Dev& d, int i, long long* acc) {
   bool on = false;
   int w = 0;
@@ -1647,7 +1601,7 @@ __device__ __forceinline__ void lrf_taylor_atom(const Dev& d, int i, long long* 
                         0.5 * (t_xyz * r0 + t_yyz * r1 + t_yzz * r2) * r1 +
                         0.5 * (t_xzz * r0 + t_yzz * r1 + t_zzz * r2) * r2;
       const double q = (double)d.x32[i].w;
-      atom_grad<LOCAL>(d, acc, i, -q * f0, -q * f1, -q * f2);
+      atom_grad(acc, -q * f0, -q * f1, -q * f2);
       e = 0.5 * q * vij;
       on = st.energy_now;
     }
@@ -2030,7 +1984,6 @@ __global__ void __launch_bounds__(256) k_bonded_gather(Dev d) {
 
 // fixed/shell restraints (fix_shell, md.f90:1414-1450) and the radial
 // solvent restraint (restrain_solvent, 14910-14957), per atom
-template <bool LOCAL>
 __device__ __forceinline__ void restr_atom(const Dev& d, int i, long long* acc) {
   int w = 0;
   bool en = false, is_fix = false, is_shell = false, is_rad = false;
@@ -2046,7 +1999,7 @@ __device__ __forceinline__ void restr_atom(const Dev& d, int i, long long* acc) 
         const double fk = (fl & 1) ? 200.0 : W.fk_pshell;
         double dr[3];
         for (int c = 0; c < 3; ++c) dr[c] = d.x[3 * i + c] - d.xtop[3 * i + c];
-        atom_grad<LOCAL>(d, acc, i, fk * dr[0], fk * dr[1], fk * dr[2]);
+        atom_grad(acc, fk * dr[0], fk * dr[1], fk * dr[2]);
         e_fs = 0.5 * fk * (dr[0] * dr[0] + dr[1] * dr[1] + dr[2] * dr[2]);
         is_fix = fl & 1;
         is_shell = fl & 2;
@@ -2069,7 +2022,7 @@ __device__ __forceinline__ void restr_atom(const Dev& d, int i, long long* acc) 
         } else {
           dv = 0.0;
         }
-        atom_grad<LOCAL>(d, acc, i, dv * dr[0], dv * dr[1], dv * dr[2]);
+        atom_grad(acc, dv * dr[0], dv * dr[1], dv * dr[2]);
         is_rad = true;
       }
     }
@@ -2083,20 +2036,23 @@ __device__ __forceinline__ void restr_atom(const Dev& d, int i, long long* acc) 
 // fixed, shell and solvent restraints (one thread per atom; every lane
 // reaches the wave energy sums of both).  STORE: the atom's sum of them is
 // stored in fterm, which k_integrate adds to the gradient (an MD step, where
-// it runs beside the pair kernels); else it is added to the gradient with
-// atomics (an evaluation)
+// it runs beside the pair kernels); else it is added to the gradient with the
+// row kernels' and q kernels' sums, after every other kernel of an evaluation
 template <bool STORE>
 __global__ void __launch_bounds__(256) k_atom_terms(Dev d) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  long long g[3] = {0, 0, 0};
+  lrf_taylor_atom(d, i, g);
+  restr_atom(d, i, g);
+  if (i >= d.ntot) return;
   if (STORE) {
-    long long g[3] = {0, 0, 0};
-    lrf_taylor_atom<true>(d, i, g);
-    restr_atom<true>(d, i, g);
-    if (i < d.ntot)
-      for (int c = 0; c < 3; ++c) d.fterm[3 * i + c] = g[c];
-  } else {
-    lrf_taylor_atom<false>(d, i, nullptr);
-    restr_atom<false>(d, i, nullptr);
+    for (int c = 0; c < 3; ++c) d.fterm[3 * i + c] = g[c];
+  } else if (d.ws[d.wid[i]].active) {
+    const int r = d.rslot[i];
+    for (int c = 0; c < 3; ++c) {
+      if (r >= 0) g[c] += d.grow[3 * (size_t)r + c] + d.gq[3 * (size_t)r + c];
+      d.f[3 * i + c] += g[c];
+    }
   }
 }
 
@@ -2493,11 +2449,13 @@ __device__ __forceinline__ void leapfrog_vals(const Dev& d, const WinState& st, 
 
 // gradient of atom i for the integrator: the step's per-atom terms (LRF
 // evaluation, fixed/shell and radial solvent restraints, stored by
-// k_atom_terms<true>) and the other kernels' gradient, stored back, so the
-// gradient array ends complete without per-atom atomics
+// k_atom_terms<true>), the row kernels' and q kernels' sums, and the gradient
+// the other kernels added up, stored back, so the gradient array ends complete
 __device__ __forceinline__ void step_gradient(const Dev& d, int i, long long g[3]) {
+  const int r = d.rslot[i];
   for (int c = 0; c < 3; ++c) {
     g[c] = d.fterm[3 * i + c] + d.f[3 * i + c];
+    if (r >= 0) g[c] += d.grow[3 * (size_t)r + c] + d.gq[3 * (size_t)r + c];
     d.f[3 * i + c] = g[c];
   }
 }
@@ -2834,165 +2792,137 @@ void launch_lists(const Dev& d, hipStream_t s, int ngrp, int nwc, int nsc) {
   launch_lrf_build(d, s);
 }
 
-// q_energy false: the q-side energy passes are left out (a step where no
-// window computes energies)
-// the q-side energy passes (energy steps only): q-water, q-solute
-static void launch_q_energy_qw(const Dev& d, hipStream_t s) {
-  if (d.tl[T_QW].nwork) k_qw<true, false><<<blocks((long long)d.tl[T_QW].nwork * 64, 256), 256, 0, s>>>(d);
-  if (d.tl[T_QW].nwork && d.any_wat3)
-    k_qw<true, true><<<blocks((long long)d.tl[T_QW].nwork * 64, 256), 256, 0, s>>>(d);
+// the q-atoms against water and solute; `energy`: the instances that also
+// evaluate the energy terms of windows at an energy step
+static void launch_qw(const Dev& d, hipStream_t s, bool energy) {
+  if (!d.nqw_work) return;
+  if (energy) k_qw<false, true><<<d.nqw_work, 64 * kQWaves, 0, s>>>(d);
+  else k_qw<false, false><<<d.nqw_work, 64 * kQWaves, 0, s>>>(d);
+  if (!d.any_wat3) return;
+  if (energy) k_qw<true, true><<<d.nqw_work, 64 * kQWaves, 0, s>>>(d);
+  else k_qw<true, false><<<d.nqw_work, 64 * kQWaves, 0, s>>>(d);
 }
-static void launch_q_energy_qp(const Dev& d, hipStream_t s) {
-  if (d.tl[T_QP].nwork) k_qp<true><<<blocks((long long)d.tl[T_QP].nwork * 64, 256), 256, 0, s>>>(d);
+static void launch_qp(const Dev& d, hipStream_t s, bool energy) {
+  if (!d.nqp_work) return;
+  if (energy) k_qp<true><<<d.nqp_work, 64 * kQWaves, 0, s>>>(d);
+  else k_qp<false><<<d.nqp_work, 64 * kQWaves, 0, s>>>(d);
 }
-// the Q tiles' forces (non-q side) and the q-atom gather
-static void launch_q_forces(const Dev& d, hipStream_t s) {
-  if (d.tl[T_WQ].nwork) k_qw<false, false><<<blocks((long long)d.tl[T_WQ].nwork * 64, 256), 256, 0, s>>>(d);
-  if (d.tl[T_WQ].nwork && d.any_wat3)
-    k_qw<false, true><<<blocks((long long)d.tl[T_WQ].nwork * 64, 256), 256, 0, s>>>(d);
-  if (d.tl[T_PQ].nwork) k_qp<false><<<blocks((long long)d.tl[T_PQ].nwork * 64, 256), 256, 0, s>>>(d);
-  if (d.nqc_all) k_q_gather<<<blocks((long long)d.nqc_all * kQGatherParts * 64, 256), 256, 0, s>>>(d);
-}
-void launch_q_tiles(const Dev& d, hipStream_t s, bool q_energy) {
-  if (q_energy) launch_q_energy_qw(d, s);
-  if (q_energy) launch_q_energy_qp(d, s);
-  launch_q_forces(d, s);
+void launch_q(const Dev& d, hipStream_t s, bool energy) {
+  launch_qw(d, s, energy);
+  launch_qp(d, s, energy);
 }
 
-template <bool EK>
-static void launch_ww_k(const Dev& d, hipStream_t s) {
+// water rows; part: k_wrow's PART
+template <bool EK, int PART>
+static void launch_wrow_k(const Dev& d, hipStream_t s) {
   const int nb = blocks((long long)d.rl[T_WW].nicl * 64, d.bs_rows);
-  if (d.rl[T_WW].nicl) k_ww<false, EK><<<nb, d.bs_rows, 0, s>>>(d);
-  if (d.rl[T_WW].nicl && d.any_wat3) k_ww<true, EK><<<nb, d.bs_rows, 0, s>>>(d);
+  if (d.rl[T_WW].nicl) k_wrow<false, EK, PART><<<nb, d.bs_rows, 0, s>>>(d);
+  if (d.rl[T_WW].nicl && d.any_wat3) k_wrow<true, EK, PART><<<nb, d.bs_rows, 0, s>>>(d);
+}
+static void launch_wrow(const Dev& d, hipStream_t s, bool energy) {
+  if (energy) launch_wrow_k<true, 3>(d, s);
+  else launch_wrow_k<false, 3>(d, s);
 }
 void launch_ww(const Dev& d, hipStream_t s, bool energy) {
-  if (energy) launch_ww_k<true>(d, s);
-  else launch_ww_k<false>(d, s);
+  if (energy) launch_wrow_k<true, 1>(d, s);
+  else launch_wrow_k<false, 1>(d, s);
 }
-
-// water_side: the rows of water i-clusters (W<-P), else those of solute
-// i-clusters (P<-W)
+// solute rows
 template <bool EK>
-static void launch_pw_k(const Dev& d, hipStream_t s, bool water_side) {
-  const int nwp = blocks((long long)d.rl[T_WP].nicl * 64, d.bs_rows);
-  const int npw = blocks((long long)d.rl[T_PW].nicl * 64, d.bs_rows);
-  if (water_side) {
-    if (d.rl[T_WP].nicl) k_pw<true, false, EK><<<nwp, d.bs_rows, 0, s>>>(d);
-    if (d.rl[T_WP].nicl && d.any_wat3) k_pw<true, true, EK><<<nwp, d.bs_rows, 0, s>>>(d);
-  } else {
-    if (d.rl[T_PW].nicl) k_pw<false, false, EK><<<npw, d.bs_rows, 0, s>>>(d);
-    if (d.rl[T_PW].nicl && d.any_wat3) k_pw<false, true, EK><<<npw, d.bs_rows, 0, s>>>(d);
-  }
-}
-static void launch_pw_side(const Dev& d, hipStream_t s, bool energy, bool water_side) {
-  if (energy) launch_pw_k<true>(d, s, water_side);
-  else launch_pw_k<false>(d, s, water_side);
-}
-static void launch_pw(const Dev& d, hipStream_t s, bool energy) {
-  launch_pw_side(d, s, energy, true);
-  launch_pw_side(d, s, energy, false);
-}
-static void launch_pp(const Dev& d, hipStream_t s, bool energy) {
-  if (!d.rl[T_PP].nicl) return;
+static void launch_srow_k(const Dev& d, hipStream_t s) {
   const int nb = blocks((long long)d.rl[T_PP].nicl * 64, d.bs_rows);
-  if (energy) k_pp<true><<<nb, d.bs_rows, 0, s>>>(d);
-  else k_pp<false><<<nb, d.bs_rows, 0, s>>>(d);
+  if (d.rl[T_PP].nicl) k_srow<false, EK><<<nb, d.bs_rows, 0, s>>>(d);
+  if (d.rl[T_PP].nicl && d.any_wat3) k_srow<true, EK><<<nb, d.bs_rows, 0, s>>>(d);
+}
+static void launch_srow(const Dev& d, hipStream_t s, bool energy) {
+  if (energy) launch_srow_k<true>(d, s);
+  else launch_srow_k<false>(d, s);
 }
 
 void launch_nonbonded(const Dev& d, hipStream_t s, bool with_ww, bool q_energy) {
-  if (with_ww) launch_ww(d, s, q_energy);
-  launch_pw(d, s, q_energy);
-  launch_pp(d, s, q_energy);
-  launch_q_tiles(d, s, q_energy);
+  if (with_ww) launch_wrow(d, s, q_energy);
+  else launch_wrow_k<false, 2>(d, s);   // added to what launch_ww stored
+  launch_srow(d, s, q_energy);
+  launch_q(d, s, q_energy);
   launch_qq(d, s);
 }
 
+static void launch_watpol(const Dev& d, hipStream_t s) {
+  if (!d.nwat_total) return;
+  if (d.nwin <= kWpolWide) k_watpol<1024><<<d.nwin * kWpolMaxShell, 1024, 0, s>>>(d);
+  else k_watpol<256><<<d.nwin * kWpolMaxShell, 256, 0, s>>>(d);
+}
+// bonded terms with their gather, which also collects the q-q pair slots
+// written by k_qq, and sequence restraints
+static void launch_bonded_gather(const Dev& d, hipStream_t s) {
+  const int nb = d.nbond + d.nang + d.ntor + d.nimp + d.nqb + d.nqa + d.nqt + d.nqi;
+  launch_bonded(d, s);
+  if ((nb || d.nqq) && !d.bond_atomic && d.ngw) k_bonded_gather<<<d.ngw, 256, 0, s>>>(d);
+  if (d.nrst) k_prestr<<<d.nrst, 64, 0, s>>>(d);
+}
+void launch_other_forces(const Dev& d, hipStream_t s, bool atom_terms) {
+  launch_watpol(d, s);
+  launch_bonded_gather(d, s);
+  if (atom_terms && d.ntot) k_atom_terms<false><<<blocks(d.ntot, 256), 256, 0, s>>>(d);   // last: completes the gradient
+}
+
 // The lists and forces of an MD step on three streams (after k_begin on s):
-//   s3: on list steps the solute rows (solute<-water, solute-solute) once
-//       the group centres are there; the Q tiles' forces (static lists:
-//       they need only the step's coordinates); the solute-solute rows, and
-//       on energy steps the q-water energy pass;
-//   s2, after the group centres: the q-q pairs, water polarisation, the
-//       bonded terms with their slot gather (which also collects the q-q
-//       slots; in bonded mode 2 the q-q slots have a gather of their own)
-//       and sequence restraints, then on list steps, once every pair kernel
-//       of the step is done, the LRF expansions;
-//   s:  on list steps the group centres and the water rows, then the
-//       water-water and solute-water rows and on energy steps the q-solute
-//       energy pass; it then waits for s2 and s3.
-// The LRF build comes last because it fills every CU for about two
-// milliseconds of FP64 work: beside the row builds and pair kernels it
-// starves them (they wait for its long-running blocks), and cutting its
-// occupancy so that they fit slows it more than it frees them.  Only the
-// per-atom terms (k_atom_terms<true>) read the expansions.
-// All of them write the gradient and the energies only through integer
-// atomic adds, so the result does not depend on how they overlap.  The
-// per-atom terms (LRF evaluation, atom restraints) go to their own array,
-// which the integrator adds: after the pair kernels of the water stream, or
-// after the LRF build on list steps.
-hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, hipStream_t s3, const hipEvent_t ev[6],
+//   s:  on list steps the group centres and the water rows; then the water
+//       rows' forces, the per-atom terms, and the q-atoms against solute;
+//   s2: water polarisation (few latency-bound blocks, which start beside the
+//       large kernels of the other streams), q-q pairs, bonded terms and
+//       restraints; on list steps, once every other kernel of the step is
+//       done, the LRF expansions and then the per-atom terms;
+//   s3: on list steps the solute rows, after the group centres; then the
+//       q-atoms against water and the solute rows' forces.
+// s then waits for s2 and s3.  The kernels' times alone add up to about the
+// same on each stream, so none is left to run by itself at the end (64-window
+// ladder, us a step: 512; bonded terms behind the water rows on s 533; water
+// polarisation last on s2 549; q-atoms against water behind the bonded terms
+// 527).
+// The LRF build comes last because it fills every CU for more than a
+// millisecond of FP64 work: beside the row builds and pair kernels it starves
+// them (they wait for its long-running blocks), and cutting its occupancy so
+// that they fit slows it more than it frees them.
+// The kernels write the energies and the shared gradient only through integer
+// atomic adds, and everything else to buffers of their own, which the
+// integrator adds, so the result does not depend on how they overlap.
+hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, hipStream_t s3, const hipEvent_t ev[5],
                               bool lists, int ngrp, int nwc, int nsc, bool q_energy) {
   hipError_t err = hipEventRecord(ev[0], s);
-  if (err == hipSuccess) err = hipStreamWaitEvent(s3, ev[0], 0);
-  if (err != hipSuccess) return err;
-  if (lists) launch_list_prep(d, s, ngrp, nwc, nsc);
-  err = hipEventRecord(ev[2], s);
-  if (err == hipSuccess) err = hipStreamWaitEvent(s2, ev[2], 0);
-  if (err == hipSuccess && lists) err = hipStreamWaitEvent(s3, ev[2], 0);
+  if (err == hipSuccess) err = hipStreamWaitEvent(s2, ev[0], 0);
+  if (err == hipSuccess && !lists) err = hipStreamWaitEvent(s3, ev[0], 0);
   if (err != hipSuccess) return err;
   if (lists) {
-    launch_rows_solute(d, s3);
-    err = hipEventRecord(ev[5], s3);
+    launch_list_prep(d, s, ngrp, nwc, nsc);
+    err = hipEventRecord(ev[2], s);
+    if (err == hipSuccess) err = hipStreamWaitEvent(s3, ev[2], 0);
     if (err != hipSuccess) return err;
+    launch_rows_solute(d, s3);
+    launch_rows_water(d, s);
   }
-  launch_q_forces(d, s3);
+  launch_watpol(d, s2);
   launch_qq(d, s2);
-  launch_other_forces(d, s2, false);
-  if (lists) launch_rows_water(d, s);
-  launch_pp(d, s3, q_energy);
-  if (q_energy) launch_q_energy_qw(d, s3);
+  launch_bonded_gather(d, s2);
+  launch_wrow(d, s, q_energy);
+  launch_qw(d, s3, q_energy);
+  launch_srow(d, s3, q_energy);
   err = hipEventRecord(ev[1], s3);
   if (err != hipSuccess) return err;
-  launch_ww(d, s, q_energy);
-  launch_pw_side(d, s, q_energy, true);
+  if (!lists) launch_atom_terms(d, s);
+  launch_qp(d, s, q_energy);
   if (lists) {
-    err = hipStreamWaitEvent(s, ev[5], 0);
-    if (err != hipSuccess) return err;
-  }
-  launch_pw_side(d, s, q_energy, false);
-  if (q_energy) launch_q_energy_qp(d, s);
-  if (lists) {
-    // the LRF build once every pair kernel of the step is done, then the
-    // per-atom terms that evaluate its expansions
     err = hipEventRecord(ev[4], s);
     if (err == hipSuccess) err = hipStreamWaitEvent(s2, ev[4], 0);
     if (err == hipSuccess) err = hipStreamWaitEvent(s2, ev[1], 0);
     if (err != hipSuccess) return err;
     launch_lrf_build(d, s2);
     launch_atom_terms(d, s2);
-  } else {
-    // the stream of the water kernels finishes first
-    launch_atom_terms(d, s);
   }
   err = hipEventRecord(ev[3], s2);
   if (err == hipSuccess) err = hipStreamWaitEvent(s, ev[1], 0);
   if (err == hipSuccess) err = hipStreamWaitEvent(s, ev[3], 0);
   return err;
-}
-
-// water polarisation first: its few latency-bound blocks then run beside the
-// large pair kernels of the other streams instead of after them
-void launch_other_forces(const Dev& d, hipStream_t s, bool atom_terms) {
-  if (d.nwat_total) {
-    if (d.nwin <= kWpolWide) k_watpol<1024><<<d.nwin * kWpolMaxShell, 1024, 0, s>>>(d);
-    else k_watpol<256><<<d.nwin * kWpolMaxShell, 256, 0, s>>>(d);
-  }
-  if (atom_terms) k_atom_terms<false><<<blocks(d.ntot, 256), 256, 0, s>>>(d);
-  int nb = d.nbond + d.nang + d.ntor + d.nimp + d.nqb + d.nqa + d.nqt + d.nqi;
-  launch_bonded(d, s);
-  // the gather also collects the q-q pair slots written by k_qq
-  if ((nb || d.nqq) && !d.bond_atomic && d.ngw) k_bonded_gather<<<d.ngw, 256, 0, s>>>(d);
-  if (d.nrst) k_prestr<<<d.nrst, 64, 0, s>>>(d);
 }
 
 void launch_atom_terms(const Dev& d, hipStream_t s) {
