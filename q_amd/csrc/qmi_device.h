@@ -121,8 +121,6 @@ constexpr int kLrfWaves = 8;
 constexpr int kIntBlock = 256;     // atoms per block of the integrator
 constexpr int kWpolMaxShell = 8;
 constexpr int kWpolLds = 4096;     // waters of one polarisation shell held (and ordered) in LDS
-constexpr int kGatherAtoms = 256;  // atoms per block of the bonded gather
-constexpr int kGatherSlots = 2048; // slots staged in LDS per gather block
 constexpr int kBondTileTerms = 512; // bonded terms per tile
 constexpr int kBondSpan = 1024;     // atoms of a tile's LDS gradient sums
 constexpr int kQItem = 16;          // q-atoms of a chunk of the q kernels: half the members of 4 q-clusters
@@ -159,14 +157,14 @@ struct Dev {
   float4* xq;
   const int* qmslot;
   float4* ljp;          // avdw1, bvdw1, avdw3, bvdw3
-  long long* f;         // gradient, 3 per atom, fixed point 2^-32
+  long long* f;         // shared gradient, 3 per atom, fixed point 2^-32; zero between steps
   // the row kernels' and the q kernels' sums, 3 per entry: entry 3 * slot +
   // site for the waters' cluster slots (nwslot of them), then one per solute
   // slot; rslot: an atom's entry, or -1 (q-atoms)
   long long *grow, *gq;
   int nwslot;
   const int* rslot;
-  long long* fterm;     // per-atom terms of the step's gradient (LRF evaluation, atom restraints), fixed point
+  long long* fterm;     // per-atom terms of the step (LRF evaluation, atom restraints), then the complete gradient
   const float* winv;
   const double* mass;
   const int* wid;       // window of atom
@@ -178,6 +176,7 @@ struct Dev {
   // the last list update; always 1 where the lists are static
   uint8_t* qin;
   const int* qref;      // the atom whose distance decides qin, -1: never updated
+  int any_qdyn;         // some window's Q lists are rebuilt at list updates
   // charge groups
   const int* g_sw;      // switch atom (global); water groups: O
   const int* g_first;   // into g_atoms
@@ -246,26 +245,22 @@ struct Dev {
   RowList rl[T_NTYPES];  // neighbour rows
   // launch shapes chosen by the autotuner (threads per block); none of
   // them changes the arithmetic of a wave or thread
-  int bs_rows, bs_bonded;
+  int bs_rows;
   // 1: blocks on one XCD take consecutive work (block_id in the kernels)
   int xcd;
-  // bonded mode.  0: bonded terms and q-q pairs write per-term slots that
-  // k_bonded_gather sums per atom; 1: both add their gradients with atomics;
-  // 2: the bonded terms sum in LDS per tile (k_bonded_tiles) and the q-q
-  // pairs use atomics.  All give the same int64 sums.
-  int bond_atomic;
-  // bonded tiles: (first entry of btile_terms, terms, first atom, atoms
-  // spanned); btile_terms: term indices, grouped by kind within a tile
+  // bonded tiles, each of one window: (first entry of btile_terms, terms, first
+  // atom, atoms spanned); btile_terms: term indices, grouped by kind within a tile
   int nbtile;
   const int4* btile;
   const int* btile_terms;
-  // bonded mode 2: the q-q pair slots (slot k >= qq_slot0 at qq_map[k -
-  // qq_slot0] of qqslot), contiguous per atom: atoms qqg_atom, runs qqg_start
-  long long* qqslot;
-  const int* qq_map;
+  // q-q pairs per atom for the forces: atom qqg_atom[k] has the records
+  // qqg_start[k] .. qqg_start[k+1]-1 of two float4 each: charge product,
+  // el_scale, A, B; soft-core term, partner atom, state (| 8: LJ code 3,
+  // | 16: exponential repulsion), unused
   int nqqg;
   const int* qqg_atom;
   const int* qqg_start;
+  const float4* qqg_ent;
   // q-q pairs (static)
   int nqq;
   const int4* qq_ij;     // iq (window-local), j (global), jq (1-based q or 0), ljcod
@@ -289,19 +284,6 @@ struct Dev {
   const int4* qa_ijk; const double2* qa_par; const int2* qa_ws;
   const int4* qt_ijkl; const double4* qt_par; const int2* qt_ws; // fk, rmult, deltor
   const int4* qi_ijkl; const double2* qi_par; const int2* qi_ws; // fk, imp0
-  // per-term gradient slots of the bonded terms and q-q pairs (3 int64
-  // each), grouped by atom: atom bg_atom[k] owns slots bg_start[k] ..
-  // bg_start[k+1]-1
-  long long* bslot;
-  int qq_slot0;          // first slot of the q-q pairs (2 per pair, after the bonded terms)
-  int nbg;
-  const int* bg_atom; const int* bg_start;
-  // gather blocks: (first k, end k) with at most kGatherAtoms atoms and, for
-  // all but single-atom blocks, at most kGatherSlots slots
-  int ngw;
-  const int2* gather_work;
-  const int* slot_map;   // term atom (in term order) -> slot; an atom's slots are contiguous
-  const int* slot_atom;  // term atom (in term order) -> global atom
   // restraints: (kind, window, i, j) global atoms; (k, flag) with flag = ih
   // (sequence, wall) or ipsi (position, distance, angle); 8 parameters each
   int nrst;

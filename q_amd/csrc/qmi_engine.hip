@@ -750,9 +750,8 @@ static int build_device(qmi_engine* e) {
 
   Dev& d = e->d;
   d.nwin = NW;
-  d.bs_rows = d.bs_bonded = 256;
+  d.bs_rows = 256;
   d.xcd = 0;
-  d.bond_atomic = 2;   // bonded tiles until the autotuner picks
   d.ntot = ao;
   int rc = 0;
 #define UP(dst, src) if ((rc = dev_upload(e, &dst, src)) != 0) return rc
@@ -772,6 +771,7 @@ static int build_device(qmi_engine* e) {
   UP(up, aflag); d.aflag = up;
   UP(up, qin); d.qin = up;
   UP(ip, qref); d.qref = ip;
+  for (int wi = 0; wi < NW; ++wi) d.any_qdyn |= wd[wi].qlist_dynamic;
   UP(ip, g_sw); d.g_sw = ip;
   UP(ip, g_first); d.g_first = ip;
   UP(ip, g_n); d.g_n = ip;
@@ -1012,9 +1012,8 @@ static int build_device(qmi_engine* e) {
   UP(i4, qa_ijk); d.qa_ijk = i4; UP(d2, qa_par); d.qa_par = d2; UP(i2, qa_ws); d.qa_ws = i2;
   UP(i4, qt_ijkl); d.qt_ijkl = i4; UP(d4, qt_par); d.qt_par = d4; UP(i2, qt_ws); d.qt_ws = i2;
   UP(i4, qi_ijkl); d.qi_ijkl = i4; UP(d2, qi_par); d.qi_par = d2; UP(i2, qi_ws); d.qi_ws = i2;
-  // bonded gradient slots, in the order k_bonded writes them
   {
-    std::vector<int> slot_atom;
+    std::vector<int> slot_atom;   // atoms of the bonded terms, in term order
     for (auto& v : b_ij) { slot_atom.push_back(v.x); slot_atom.push_back(v.y); }
     for (auto& v : a_ijk) { slot_atom.push_back(v.x); slot_atom.push_back(v.y); slot_atom.push_back(v.z); }
     for (auto& v : t_ijkl) for (int a : {v.x, v.y, v.z, v.w}) slot_atom.push_back(a);
@@ -1023,48 +1022,9 @@ static int build_device(qmi_engine* e) {
     for (auto& v : qa_ijk) { slot_atom.push_back(v.x); slot_atom.push_back(v.y); slot_atom.push_back(v.z); }
     for (auto& v : qt_ijkl) for (int a : {v.x, v.y, v.z, v.w}) slot_atom.push_back(a);
     for (auto& v : qi_ijkl) for (int a : {v.x, v.y, v.z, v.w}) slot_atom.push_back(a);
-    // q-q pairs: q-atom i, partner j
-    d.qq_slot0 = (int)slot_atom.size();
-    for (size_t k = 0; k < qq_ij.size(); ++k) {
-      const int wq = qq_win[k];
-      slot_atom.push_back(q_atom[wd[wq].q_off + qq_ij[k].x]);
-      slot_atom.push_back(qq_ij[k].y);
-    }
-    std::vector<int> per_atom(ao, 0);
-    for (int a : slot_atom) per_atom[a]++;
-    std::vector<int> bg_atom, bg_start, pos(ao, -1);
-    for (int a = 0; a < ao; ++a)
-      if (per_atom[a]) { pos[a] = (int)bg_atom.size(); bg_atom.push_back(a); }
-    bg_start.assign(bg_atom.size() + 1, 0);
-    for (size_t k = 0; k < bg_atom.size(); ++k) bg_start[k + 1] = bg_start[k] + per_atom[bg_atom[k]];
-    // each term atom writes to the position of its atom's run, so that an
-    // atom's slots are contiguous for the gather
-    std::vector<int> fill(bg_atom.size(), 0);
-    std::vector<int> slot_map(slot_atom.size());
-    for (size_t sidx = 0; sidx < slot_atom.size(); ++sidx) {
-      const int k = pos[slot_atom[sidx]];
-      slot_map[sidx] = bg_start[k] + fill[k]++;
-    }
-    d.nbg = (int)bg_atom.size();
-    // gather blocks: consecutive atoms, at most kGatherAtoms of them and at
-    // most kGatherSlots slots unless a single atom has more
-    std::vector<int2> gwork;
-    for (int k0 = 0; k0 < d.nbg;) {
-      int k1 = k0 + 1;
-      while (k1 < d.nbg && k1 - k0 < kGatherAtoms && bg_start[k1 + 1] - bg_start[k0] <= kGatherSlots) ++k1;
-      gwork.push_back(make_int2(k0, k1));
-      k0 = k1;
-    }
-    d.ngw = (int)gwork.size();
-    int2* gwp;
-    UP(gwp, gwork); d.gather_work = gwp;
-    UP(ip, bg_atom); d.bg_atom = ip;
-    UP(ip, bg_start); d.bg_start = ip;
-    UP(ip, slot_map); d.slot_map = ip;
-    UP(ip, slot_atom); d.slot_atom = ip;
     // bonded tiles: terms ordered by their first (lowest) atom, cut into
-    // tiles of at most kBondTileTerms terms spanning at most kBondSpan atoms,
-    // each tile's terms grouped by kind
+    // tiles of at most kBondTileTerms terms of one window spanning at most
+    // kBondSpan atoms, each tile's terms grouped by kind
     {
       const int nat_kind[8] = {2, 3, 4, 4, 2, 3, 4, 4};
       const int nk[8] = {(int)b_ij.size(), (int)a_ijk.size(), (int)t_ijkl.size(), (int)i_ijkl.size(),
@@ -1089,7 +1049,8 @@ static int build_device(qmi_engine* e) {
         size_t k1 = k0 + 1;
         const int lo = terms[k0].lo;
         int hi = terms[k0].hi;
-        while (k1 < terms.size() && (int)(k1 - k0) < kBondTileTerms && std::max(hi, terms[k1].hi) - lo < kBondSpan) {
+        while (k1 < terms.size() && (int)(k1 - k0) < kBondTileTerms && std::max(hi, terms[k1].hi) - lo < kBondSpan &&
+               wid[terms[k1].lo] == wid[lo]) {
           hi = std::max(hi, terms[k1].hi);
           ++k1;
         }
@@ -1104,30 +1065,37 @@ static int build_device(qmi_engine* e) {
       UP(bt, btile); d.btile = bt;
       UP(ip, bterms); d.btile_terms = ip;
     }
-    // the q-q pair slots alone, grouped by atom, for bonded mode 2
-    {
-      const int nqs = (int)slot_atom.size() - d.qq_slot0;
-      std::vector<int> qcount(ao, 0);
-      for (int k = 0; k < nqs; ++k) qcount[slot_atom[d.qq_slot0 + k]]++;
-      std::vector<int> qqg_atom, qqg_start(1, 0), qpos(ao, -1);
-      for (int a = 0; a < ao; ++a)
-        if (qcount[a]) {
-          qpos[a] = (int)qqg_atom.size();
-          qqg_atom.push_back(a);
-          qqg_start.push_back(qqg_start.back() + qcount[a]);
-        }
-      std::vector<int> qfill(qqg_atom.size(), 0), qq_map(std::max(1, nqs), 0);
-      for (int k = 0; k < nqs; ++k) {
-        const int p = qpos[slot_atom[d.qq_slot0 + k]];
-        qq_map[k] = qqg_start[p] + qfill[p]++;
-      }
-      d.nqqg = (int)qqg_atom.size();
-      UP(ip, qqg_atom); d.qqg_atom = ip;
-      UP(ip, qqg_start); d.qqg_start = ip;
-      UP(ip, qq_map); d.qq_map = ip;
-      if ((rc = dev_alloc(e, &d.qqslot, 3 * (size_t)std::max(1, nqs))) != 0) return rc;
+  }
+  // q-q pairs by atom, both sides of every pair
+  {
+    std::vector<std::vector<std::pair<int, int>>> by(ao);   // (pair, partner)
+    for (int k = 0; k < d.nqq; ++k) {
+      const int i = q_atom[wd[qq_win[k]].q_off + qq_ij[k].x], j = qq_ij[k].y;
+      by[i].push_back({k, j});
+      by[j].push_back({k, i});
     }
-    if ((rc = dev_alloc(e, &d.bslot, 3 * std::max<size_t>(1, slot_atom.size()))) != 0) return rc;
+    std::vector<int> qqg_atom, qqg_start(1, 0);
+    std::vector<float4> qqg_ent;
+    for (int a = 0; a < ao; ++a) {
+      if (by[a].empty()) continue;
+      for (auto& e2 : by[a]) {
+        const int k = e2.first, st = qq_st[k];
+        const int4 p = qq_ij[k];
+        const bool expo = wd[qq_win[k]].qvdw && p.z && p.w == 2;
+        const int fl = st | (p.w == 3 ? 8 : 0) | (expo ? 16 : 0);
+        auto bits = [](int v) { float f; std::memcpy(&f, &v, 4); return f; };
+        qqg_ent.push_back(make_float4((float)((double)qq_q[k].x * (double)qq_q[k].y), qq_es[k], (float)qq_ab[k].x,
+                                      (float)qq_ab[k].y));
+        qqg_ent.push_back(make_float4(qq_sc[k], bits(e2.second), bits(fl), 0.f));
+      }
+      qqg_atom.push_back(a);
+      qqg_start.push_back((int)(qqg_ent.size() / 2));
+    }
+    d.nqqg = (int)qqg_atom.size();
+    UP(ip, qqg_atom); d.qqg_atom = ip;
+    UP(ip, qqg_start); d.qqg_start = ip;
+    float4* qe;
+    UP(qe, qqg_ent); d.qqg_ent = qe;
   }
   d.nrst = (int)rs_kwij.size();
   UP(i4, rs_kwij); d.rs_kwij = i4; UP(i2, rs_kf); d.rs_kf = i2; UP(dp, rs_par); d.rs_par = dp;
@@ -1499,7 +1467,7 @@ static int autotune(qmi_engine* e) {
     return best;
   };
   // a forces-only state with fresh lists and LRF expansions
-  launch_begin(d, e->stream, 0, 2, 1);
+  launch_begin(d, e->stream, 2, 1);
   launch_lists(d, e->stream, e->ngrp, e->nwc, e->nsc);
   HIP_OK(hipStreamSynchronize(e->stream));
   const int bs[3] = {256, 128, 64};
@@ -1511,21 +1479,22 @@ static int autotune(qmi_engine* e) {
   // 0: the q kernels (fixed work items)
   e->tuned[0] = kQItem;
   e->tune_us[0] = time_us([&] { launch_q(d, e->stream, false); });
-  // 1, 3: threads per block of the row kernels and of the bonded terms
-  int* field[3] = {&d.bs_rows, nullptr, &d.bs_bonded};
-  for (int g : {0, 2}) {
+  // 1: threads per block of the row kernels
+  {
     int bb = 256;
     double bt = 1e30;
     for (int b : bs) {
-      *field[g] = b;
-      const double t = g == 0 ? time_us([&] { launch_nonbonded(d, e->stream, true, false); })
-                              : time_us([&] { launch_bonded(d, e->stream); });
+      d.bs_rows = b;
+      const double t = time_us([&] { launch_nonbonded(d, e->stream, true, false); });
       if (faster(t, bt)) { bt = t; bb = b; }
     }
-    *field[g] = bb;
-    e->tuned[1 + g] = bb;
-    e->tune_us[1 + g] = bt;
+    d.bs_rows = bb;
+    e->tuned[1] = bb;
+    e->tune_us[1] = bt;
   }
+  // 3, 5: the bonded terms (fixed tiles)
+  e->tune_us[3] = time_us([&] { launch_bonded(d, e->stream); });
+  e->tune_us[5] = e->tune_us[3];
   // 2, 6: the LRF build (fixed shapes: they set the order of its sums)
   e->tuned[2] = 64 * kLrfWaves;
   e->tune_us[2] = time_us([&] { launch_lrf_build(d, e->stream); });
@@ -1550,23 +1519,9 @@ static int autotune(qmi_engine* e) {
     e->tuned[4] = d.xcd;
     e->tune_us[4] = tx[d.xcd];
   }
-  // 5: bonded and q-q gradients: LDS tiles (2), slots and a per-atom gather
-  // (0) or atomics (1)
-  {
-    int bm = 2;
-    double bt = 1e30;
-    for (int a : {2, 0, 1}) {
-      d.bond_atomic = a;
-      const double t = time_us([&] {
-        launch_nonbonded(d, e->stream, false, false);
-        launch_other_forces(d, e->stream);
-      });
-      if (faster(t, bt)) { bt = t; bm = a; }
-    }
-    d.bond_atomic = bm;
-    e->tuned[5] = bm;
-    e->tune_us[5] = bt;
-  }
+  // the timing runs added to the shared gradient, which steps expect at zero
+  HIP_OK(hipMemsetAsync(d.f, 0, (size_t)3 * d.ntot * sizeof(long long), e->stream));
+  HIP_OK(hipStreamSynchronize(e->stream));
   HIP_OK(hipGetLastError());
   (void)hipEventDestroy(t0);
   (void)hipEventDestroy(t1);
@@ -1855,33 +1810,28 @@ int qmi_run(qmi_engine* e, long long nsteps, int finalize) {
   double fam[5] = {0, 0, 0, 0, 0};
   auto t0 = std::chrono::steady_clock::now();
   long long done = 0;
+  // the first step's start; each step's last kernel begins the next one
+  launch_begin(e->d, e->stream, 0, 0);
   // one step = the same kernels with the same arguments every time (the
   // kernels read per-window step state from device memory), so outside the
   // timing pass it runs as one captured graph
   auto launch_step = [&](int variant) {
     const bool lists = variant & 1, qen = variant & 2;
-    launch_begin(e->d, e->stream, 0, 0, variant);
     // lists and forces on three streams; a failure here fails the capture
     if (launch_step_forces(e->d, e->stream, e->side_stream[0], e->side_stream[1], e->step_ev, lists, e->ngrp, e->nwc,
                            e->nsc, qen) != hipSuccess)
       return;
-    launch_integrate(e->d, e->stream, e->shake_any);
+    launch_integrate(e->d, e->stream, e->shake_any, variant);
   };
   if (!e->timing_on && !e->step_exec[0] && !e->graph_failed) {
     bool ok = true;
     for (int k = 0; k < 4 && ok; ++k) {
       hipGraph_t g = nullptr;
-      // energy steps keep the bonded slots and their gather even where the
-      // tuner picked the LDS tiles: beside the FP64 energy passes the tile
-      // kernel (164 VGPRs) finds few wave slots, and the result is the same
-      const int bond_mode = e->d.bond_atomic;
-      if ((k & 2) && bond_mode == 2) e->d.bond_atomic = 0;
       ok = hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal) == hipSuccess;
       if (ok) {
         launch_step(k);
         ok = hipStreamEndCapture(e->stream, &g) == hipSuccess && g != nullptr;
       }
-      e->d.bond_atomic = bond_mode;
       if (ok) ok = hipGraphInstantiate(&e->step_exec[k], g, nullptr, nullptr, 0) == hipSuccess;
       if (ok) {
         e->step_graph[k] = g;
@@ -1995,7 +1945,7 @@ int qmi_run(qmi_engine* e, long long nsteps, int finalize) {
       // the same kernel instances as the step graph of this step: those
       // with energy terms only where some window computes energies
       const bool qen = energy_at(done + k);
-      launch_begin(e->d, e->stream, 0, 0, 1 | (qen ? 2 : 0));
+      launch_offdiag(e->d, e->stream);
       if (e->timing_on) HIP_OK(hipEventRecord(e->ev[0], e->stream));
       launch_lists(e->d, e->stream, e->ngrp, e->nwc, e->nsc);
       if (e->timing_on) HIP_OK(hipEventRecord(e->ev[1], e->stream));
@@ -2006,7 +1956,7 @@ int qmi_run(qmi_engine* e, long long nsteps, int finalize) {
       launch_other_forces(e->d, e->stream, false);
       if (e->timing_on) HIP_OK(hipEventRecord(e->ev[4], e->stream));
       launch_atom_terms(e->d, e->stream);
-      launch_integrate(e->d, e->stream, e->shake_any);
+      launch_integrate(e->d, e->stream, e->shake_any, 1 | (qen ? 2 : 0));
       if (e->timing_on) {
         HIP_OK(hipEventRecord(e->ev[5], e->stream));
         HIP_OK(hipEventSynchronize(e->ev[5]));
@@ -2163,7 +2113,7 @@ int qmi_evaluate(qmi_engine* e, int rebuild_lists) {
 // windows stopped by a failure left out.
 static int evaluate(qmi_engine* e, int rebuild_lists, int mode) {
   HIP_OK(hipSetDevice(e->device));
-  launch_begin(e->d, e->stream, 1, mode, rebuild_lists ? 1 : 0);
+  launch_begin(e->d, e->stream, mode, rebuild_lists ? 1 : 0);
   launch_lists(e->d, e->stream, e->ngrp, e->nwc, e->nsc);
   launch_nonbonded(e->d, e->stream);
   launch_other_forces(e->d, e->stream);
@@ -2229,7 +2179,7 @@ static int get_atom_vec(qmi_engine* e, int w, double* out, long long cap, int wh
   if (cap < n3) return set_err(-3, "buffer too small");
   if (which == 2) {
     std::vector<long long> f(n3);
-    HIP_OK(hipMemcpy(f.data(), e->d.f + 3 * ao, n3 * 8, hipMemcpyDeviceToHost));
+    HIP_OK(hipMemcpy(f.data(), e->d.fterm + 3 * ao, n3 * 8, hipMemcpyDeviceToHost));
     for (long long k = 0; k < n3; ++k) out[k] = (double)f[k] / kFScale;
   } else {
     HIP_OK(hipMemcpy(out, (which == 0 ? e->d.x : e->d.v) + 3 * ao, n3 * 8, hipMemcpyDeviceToHost));
@@ -2253,8 +2203,9 @@ int qmi_set_state(qmi_engine* e, int w, const double* xyz, const double* v, long
     if (xyz) HIP_OK(hipMemcpy(e->d.x + 3 * ao, xyz, n3 * 8, hipMemcpyHostToDevice));
     if (v) HIP_OK(hipMemcpy(e->d.v + 3 * ao, v, n3 * 8, hipMemcpyHostToDevice));
     // refresh the FP32 copy of the coordinates
-    launch_begin(e->d, e->stream, 0, 1, 0);
     launch_refresh32(e->d, e->stream);
+    // no gradient at the new coordinates until the next step or evaluation
+    HIP_OK(hipMemsetAsync(e->d.fterm, 0, (size_t)3 * e->ntot * sizeof(long long), e->stream));
     HIP_OK(hipStreamSynchronize(e->stream));
   }
   return 0;

@@ -5,7 +5,10 @@
 #include "qmi_device.h"
 
 namespace qmi {
-void launch_begin(const Dev& d, hipStream_t s, int force_energy, int eval_only, int rebuild);
+// the start of a run's first step (eval 0) or of an evaluation (k_begin)
+void launch_begin(const Dev& d, hipStream_t s, int eval, int rebuild);
+// EVB off-diagonal elements at an MD step's starting coordinates
+void launch_offdiag(const Dev& d, hipStream_t s);
 void launch_lists(const Dev& d, hipStream_t s, int ngrp, int nwc, int nsc);
 // water-water rows alone, and all nonbonded kernels (with or without
 // them); `energy` / `q_energy`: the kernel instances that also evaluate the
@@ -26,7 +29,8 @@ hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, hipSt
                               bool lists, int ngrp, int nwc, int nsc, bool q_energy);
 // the end of an MD step; the gradient is completed with the per-atom terms
 // of launch_atom_terms, which must have run in the same step
-void launch_integrate(const Dev& d, hipStream_t s, int shake_any);
+// variant: bit 0 the step's list kernels were launched, bit 1 its energy terms
+void launch_integrate(const Dev& d, hipStream_t s, int shake_any, int variant);
 void launch_temperature(const Dev& d, hipStream_t s);
 void launch_refresh32(const Dev& d, hipStream_t s);
 }  // namespace qmi

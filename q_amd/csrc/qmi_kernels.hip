@@ -76,39 +76,6 @@ __device__ __forceinline__ void atom_grad(long long acc[3], double gx, double gy
   acc[2] += fix(gz, kFScale);
 }
 
-// gradient of term atom k (in term order): into its own slot (fixed point, no
-// atomic), or added to the atom's gradient with atomics (bonded mode 1); the
-// int64 values are the same either way
-__device__ __forceinline__ void put_slot(const Dev& d, int k, double gx, double gy, double gz) {
-  const long long fx = fix(gx, kFScale), fy = fix(gy, kFScale), fz = fix(gz, kFScale);
-  if (d.bond_atomic == 2) {
-    // bonded mode 2: only the q-q pairs come here, into slots of their own
-    // that k_qq_gather sums per atom (atomics would collide on the q-atoms)
-    const int m = d.qq_map[k - d.qq_slot0];
-    d.qqslot[3 * m + 0] = fx;
-    d.qqslot[3 * m + 1] = fy;
-    d.qqslot[3 * m + 2] = fz;
-    return;
-  }
-  if (d.bond_atomic) {
-    const int a = d.slot_atom[k];
-    atomicAdd((unsigned long long*)&d.f[3 * a + 0], (unsigned long long)fx);
-    atomicAdd((unsigned long long*)&d.f[3 * a + 1], (unsigned long long)fy);
-    atomicAdd((unsigned long long*)&d.f[3 * a + 2], (unsigned long long)fz);
-    return;
-  }
-  const int m = d.slot_map[k];
-  d.bslot[3 * m + 0] = fx;
-  d.bslot[3 * m + 1] = fy;
-  d.bslot[3 * m + 2] = fz;
-}
-
-// the gradient of a term atom into its slot, or with atomics (put_slot)
-struct SlotSink {
-  const Dev* d;
-  __device__ void operator()(int k, int, double gx, double gy, double gz) const { put_slot(*d, k, gx, gy, gz); }
-};
-
 __device__ __forceinline__ void add_energy(WinState* ws, int w, int slot, double e) {
   if (e != 0.0) atomicAdd((unsigned long long*)&ws[w].E[slot], (unsigned long long)fix(e, kEScale));
 }
@@ -238,74 +205,77 @@ __device__ __forceinline__ double r2_exact(const double* x, int i, int j) {
 }
 
 // ------------------------------------------------------ step control --
-// Step start, one thread per window (flags, energy accumulators) and per
-// atom (gradient accumulators of running windows start at zero).  The two
-// parts touch different fields of the window state.
+// The gradient array is zero between steps and evaluations: the kernel that
+// completes a gradient (k_integrate, k_atom_terms<false>) takes it and clears
+// it.
 __device__ __forceinline__ bool window_runs(const WinState& s) {
   return s.istep < s.stop_at && !s.shake_fail && !s.list_overflow;
 }
+// flags and energy accumulators at the start of the MD step s.istep
+__device__ __forceinline__ void begin_step(WinState& s, const WinDev& W) {
+  s.active = window_runs(s) ? 1 : 0;
+  s.wpol_acc = s.active;
+  s.list_now = (s.istep % W.nbcycle) == 0;
+  s.energy_now = (W.iene > 0 && s.istep % W.iene == 0 && s.istep > 0) || (W.iout > 0 && s.istep % W.iout == 0) ? 1 : 0;
+  if (s.energy_now)
+    for (int k = 0; k < E_NSLOT; ++k) s.E[k] = 0;
+}
 
-__global__ void k_begin(Dev d, int force_energy, int eval_only, int rebuild) {
+// start of a run's first step (eval 0; later steps are begun by k_temperature)
+// or of an evaluation, one thread per window.  eval 1: energy evaluation; 2:
+// forces only (the autotuner's timing runs); 3: the energy evaluation after
+// the last step of a run (md.f90:4207-4208), which is a pot_energy call of
+// the run for windows that completed; a window stopped by a failure is left
+// as it is.
+__global__ void k_begin(Dev d, int eval, int rebuild) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < d.nwin) {
-    WinState& s = d.ws[i];
-    const WinDev& W = d.win[i];
-    if (eval_only) {
-      // 1: energy evaluation; 2: forces only (the autotuner's timing runs);
-      // 3: the energy evaluation after the last step of a run (md.f90:4207-4208),
-      // which is a pot_energy call of the run for windows that completed;
-      // a window stopped by a failure is left as it is
-      s.active = eval_only != 3 || !(s.shake_fail || s.list_overflow);
-      s.list_now = rebuild;
-      s.energy_now = eval_only != 2 ? 1 : 0;
-      s.wpol_acc = eval_only == 3 && s.istep >= W.nsteps ? 1 : 0;
-    } else {
-      // MD step; rebuild bit 0: the list kernels were launched, bit 1: the
-      // q-side energy passes were
-      s.active = window_runs(s) ? 1 : 0;
-      s.wpol_acc = s.active;
-      s.list_now = (s.istep % W.nbcycle) == 0;
-      if (s.active && s.list_now && !(rebuild & 1)) s.list_missed = 1;
-      bool e = (W.iene > 0 && s.istep % W.iene == 0 && s.istep > 0) || (W.iout > 0 && s.istep % W.iout == 0) ||
-               force_energy;
-      s.energy_now = e ? 1 : 0;
-      if (s.active && e && !(rebuild & 2)) s.list_missed = 2;
-    }
-    if (s.energy_now)
-      for (int k = 0; k < E_NSLOT; ++k) s.E[k] = 0;
+  if (i >= d.nwin) return;
+  WinState& s = d.ws[i];
+  const WinDev& W = d.win[i];
+  if (!eval) {
+    begin_step(s, W);
+    return;
   }
-  if (i < d.ntot && (eval_only || window_runs(d.ws[d.wid[i]]))) {
-    d.f[3 * i] = 0; d.f[3 * i + 1] = 0; d.f[3 * i + 2] = 0;
-  }
-  // dynamic Q-atom lists (nbqplist / nbqwlist, md.f90:7875-7964, 8066-8118):
-  // at a list update, an atom is in the lists while the switching atom of
-  // its group (the oxygen of its water) lies within the q_atom cut-off of
-  // the Q centre; the Q tiles cover every candidate and test this flag
-  if (i < d.ntot && d.qref[i] >= 0) {
-    const WinState& s = d.ws[d.wid[i]];
-    const WinDev& W = d.win[d.wid[i]];
-    const bool upd = eval_only ? (rebuild & 1) != 0 : window_runs(s) && (s.istep % W.nbcycle) == 0;
-    if (upd) {
-      const int r = d.qref[i];
-      const double dx = __dsub_rn(d.x[3 * r], W.xpcent[0]), dy = __dsub_rn(d.x[3 * r + 1], W.xpcent[1]),
-                   dz = __dsub_rn(d.x[3 * r + 2], W.xpcent[2]);
-      d.qin[i] = __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz)) <= W.rcq2 ? 1 : 0;
-    }
-  }
-  // EVB off-diagonal elements at the step's starting coordinates (offdiag,
-  // md.f90:12911-12937), into the step's ring slot; the ring is read for
-  // steps the window ran, so a stopped window's slot goes unread
-  if (!eval_only && i < d.noffd_all) {
-    const WinState& s = d.ws[d.offd_win[i]];
-    const int2 kl = d.offd_kl[i];
-    const double dx = d.x[3 * kl.y] - d.x[3 * kl.x], dy = d.x[3 * kl.y + 1] - d.x[3 * kl.x + 1],
-                 dz = d.x[3 * kl.y + 2] - d.x[3 * kl.x + 2];
-    const double r = sqrt(dx * dx + dy * dy + dz * dz);
-    const double2 p = d.offd_par[i];
-    double* o = &d.o_ring[((size_t)((s.istep - s.ring_base) % d.ring_n) * d.noffd_all + i) * 2];
-    o[0] = p.x * exp(-p.y * r);
-    o[1] = r;
-  }
+  s.active = eval != 3 || !(s.shake_fail || s.list_overflow);
+  s.list_now = rebuild;
+  s.energy_now = eval != 2 ? 1 : 0;
+  s.wpol_acc = eval == 3 && s.istep >= W.nsteps ? 1 : 0;
+  if (s.energy_now)
+    for (int k = 0; k < E_NSLOT; ++k) s.E[k] = 0;
+}
+
+// dynamic Q-atom lists (nbqplist / nbqwlist, md.f90:7875-7964, 8066-8118): at
+// a list update, an atom is in the lists while the switching atom of its
+// group (the oxygen of its water) lies within the q_atom cut-off of the Q
+// centre; the static lists cover every candidate, and the q kernels test
+// this flag
+__global__ void k_qin(Dev d) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= d.ntot || d.qref[i] < 0) return;
+  const WinState& s = d.ws[d.wid[i]];
+  if (!s.active || !s.list_now) return;
+  const WinDev& W = d.win[d.wid[i]];
+  const int r = d.qref[i];
+  const double dx = __dsub_rn(d.x[3 * r], W.xpcent[0]), dy = __dsub_rn(d.x[3 * r + 1], W.xpcent[1]),
+               dz = __dsub_rn(d.x[3 * r + 2], W.xpcent[2]);
+  d.qin[i] = __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz)) <= W.rcq2 ? 1 : 0;
+}
+
+// EVB off-diagonal elements at the step's starting coordinates (offdiag,
+// md.f90:12911-12937), into the step's ring slot; the ring is read for steps
+// the window ran, so a stopped window's slot goes unread
+__global__ void k_offdiag(Dev d) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= d.noffd_all) return;
+  const WinState& s = d.ws[d.offd_win[i]];
+  const int2 kl = d.offd_kl[i];
+  const double dx = d.x[3 * kl.y] - d.x[3 * kl.x], dy = d.x[3 * kl.y + 1] - d.x[3 * kl.x + 1],
+               dz = d.x[3 * kl.y + 2] - d.x[3 * kl.x + 2];
+  const double r = sqrt(dx * dx + dy * dy + dz * dz);
+  const double2 p = d.offd_par[i];
+  double* o = &d.o_ring[((size_t)((s.istep - s.ring_base) % d.ring_n) * d.noffd_all + i) * 2];
+  o[0] = p.x * exp(-p.y * r);
+  o[1] = r;
 }
 
 // charge-group centres (cgp_centers, md.f90:1000-1019) and cluster bounding
@@ -1279,114 +1249,105 @@ __global__ void __launch_bounds__(64 * kQWaves) k_qp(Dev d) {
   q_store<3>(acc, wk.z, d.gq + 9 * (size_t)d.nwslot + 3 * (size_t)wk.y);
 }
 
-// q-q and q-(bonded neighbour) pairs (nonbond_qq, md.f90:10763-10868), one
-// thread per (pair, state)
-// q-q pair k, its gradients handed to `put` (slots qq_slot0 + 2k, + 1); k
-// past the last pair does nothing.  Every lane of the wave must call it.
-template <class Sink>
-__device__ __forceinline__ void qq_term(const Dev& d, int k, const Sink& put) {
-  bool valid = false, en = false;
+// q-q and q-(bonded neighbour) pairs (nonbond_qq, md.f90:10763-10868).
+// Forces: one wave per atom over the atom's pairs of every state (each pair
+// from both sides), FP32 from the packed record of the pair, summed in fixed
+// point over the wave, with one atomic per component.  As per-pair slots and
+// a gather it was two kernels in a row, 14 us for the 64-window ladder and 11
+// us (of an 86 us step) for one window.
+__device__ __forceinline__ void qq_atom(const Dev& d, int k) {
+  const int atom = d.qqg_atom[k], lane = threadIdx.x & 63;
+  const int w = d.wid[atom];
+  if (!d.ws[w].active) return;   // uniform over the wave
+  const WinDev& W = d.win[w];
+  const float4 pi = d.x32[atom];
+  long long gx = 0, gy = 0, gz = 0;
+  const int m1 = d.qqg_start[k + 1];
+  for (int m = d.qqg_start[k] + lane; m < m1; m += 64) {
+#pragma clang fp contract(off)
+    const float4 p = d.qqg_ent[2 * (size_t)m], r = d.qqg_ent[2 * (size_t)m + 1];
+    const float q = p.x, es = p.y, aLJ = p.z, bLJ = p.w, sc = r.x;
+    const int j = __float_as_int(r.y), fl = __float_as_int(r.z);   // partner; state, LJ code 3, exponential
+    const float4 pj = d.x32[j];
+    const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
+    const float r2 = r2_f(dx, dy, dz);
+    const float r4 = r2 * r2, r6hc = r2 * r4;
+    const float r2inv = 1.f / r2, ri = sqrtf(r2inv);
+    float vel = q * ri * es;
+    if (fl & 8) vel *= W.el14;
+    float t;
+    if (fl & 16) {
+      const float va = aLJ * expf(-bLJ / ri);
+      t = -vel - bLJ * va / ri;
+    } else {
+      const float r6 = 1.f / __builtin_fmaf(r2, r4, sc);
+      t = __builtin_fmaf(-r6, r6hc * __builtin_fmaf(aLJ * (r6 * r6), 12.f, -6.f * (bLJ * r6)), -vel);
+    }
+    const float dv = r2inv * t * (float)W.lambda[fl & 7];
+    gx += fix(-(double)(dv * dx), kFScale);
+    gy += fix(-(double)(dv * dy), kFScale);
+    gz += fix(-(double)(dv * dz), kFScale);
+  }
+  gx = wave_sum_i(gx);
+  gy = wave_sum_i(gy);
+  gz = wave_sum_i(gz);
+  if (lane < 3)
+    atomicAdd((unsigned long long*)&d.f[3 * (size_t)atom + lane], (unsigned long long)(lane == 0 ? gx : lane == 1 ? gy : gz));
+}
+
+// energies of q-q pair k and its state, FP64 (energy steps); k past the last
+// pair does nothing.  Every lane of the wave must call it.
+__device__ __forceinline__ void qq_energy(const Dev& d, int k) {
+  bool valid = false;
   int w = 0, s = 0, base = 6;
   double e_el = 0.0, e_vdw = 0.0;
   if (k < d.nqq) {
     w = d.qq_win[k];
     const WinState& st = d.ws[w];
-    if (st.active) {
+    if (st.active && st.energy_now) {
       valid = true;
-      en = st.energy_now;
       const WinDev& W = d.win[w];
       const int4 e = d.qq_ij[k];
       s = d.qq_st[k];
       const int i = d.q_atom[W.q_off + e.x], j = e.y, jq = e.z, iLJ = e.w;
-      const float es = d.qq_es[k];
-      // parameters (double, as the reference)
       const float2 qq = d.qq_q[k];
+      // qi qj is exact in FP64, as the reference's real(8) product
       const double qi = (double)qq.x, qj = (double)qq.y;
       const double2 ab = d.qq_ab[k];
-      const double aLJ = ab.x, bLJ = ab.y;
-      const double sc = d.qq_sc[k];
-      const bool expo = W.qvdw && jq && iLJ == 2;
-      // gradient in FP32 from the FP32 coordinates
-      const float4 pi = d.x32[i], pj = d.x32[j];
-      const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
-      const float r2 = dx * dx + dy * dy + dz * dz;
-      const float r6hc = r2 * r2 * r2;
-      const float r6 = 1.f / (r6hc + (float)sc);
-      const float r12 = r6 * r6;
-      const float r2inv = 1.f / r2, r = sqrtf(r2inv);
-      float vel = (float)(qi * qj) * r * es;
-      if (iLJ == 3) vel *= W.el14;
-      float dv;
-      if (expo) {
-        const float va = (float)aLJ * expf(-(float)bLJ / r);
-        dv = r2inv * (-vel - (float)bLJ * va / r) * (float)W.lambda[s];
+      const double ddx = d.x[3 * j] - d.x[3 * i], ddy = d.x[3 * j + 1] - d.x[3 * i + 1],
+                   ddz = d.x[3 * j + 2] - d.x[3 * i + 2];
+      const double rr2 = ddx * ddx + ddy * ddy + ddz * ddz;
+      e_el = qi * qj * rsqrt_e(rr2) * (double)d.qq_es[k];
+      if (iLJ == 3) e_el *= W.el14d;
+      if (W.qvdw && jq && iLJ == 2) {
+        e_vdw = ab.x * exp(-ab.y * sqrt(rr2));
       } else {
-        const float va = (float)aLJ * r12, vb = (float)bLJ * r6;
-        dv = r2inv * (-vel - (12.f * va - 6.f * vb) * r6hc * r6) * (float)W.lambda[s];
+        const double inv = rcp_e(rr2 * rr2 * rr2 + (double)d.qq_sc[k]);
+        e_vdw = ab.x * inv * inv - ab.y * inv;
       }
-      const int sl = d.qq_slot0 + 2 * k;
-      put(sl, 0, -(double)(dv * dx), -(double)(dv * dy), -(double)(dv * dz));
-      put(sl + 1, 1, (double)(dv * dx), (double)(dv * dy), (double)(dv * dz));
-      if (en) {
-        // FP64 energies; qi qj is exact in FP64, as the reference's real(8) product
-        const double ddx = d.x[3 * j] - d.x[3 * i], ddy = d.x[3 * j + 1] - d.x[3 * i + 1],
-                     ddz = d.x[3 * j + 2] - d.x[3 * i + 2];
-        const double rr2 = ddx * ddx + ddy * ddy + ddz * ddz;
-        double v = qi * qj * rsqrt_e(rr2) * (double)es;
-        if (iLJ == 3) v *= W.el14d;
-        e_el = v;
-        if (expo) {
-          e_vdw = aLJ * exp(-bLJ * sqrt(rr2));
-        } else {
-          const double inv = rcp_e(rr2 * rr2 * rr2 + sc);
-          e_vdw = aLJ * inv * inv - bLJ * inv;
-        }
-        base = jq ? 4 : 6;  // qq or qp slot
-      }
+      base = jq ? 4 : 6;  // qq or qp slot
     }
   }
-  wave_energy(d.ws, w, E_Q0 + 8 * s + base, e_el, valid && en);
-  wave_energy(d.ws, w, E_Q0 + 8 * s + base + 1, e_vdw, valid && en);
+  wave_energy(d.ws, w, E_Q0 + 8 * s + base, e_el, valid);
+  wave_energy(d.ws, w, E_Q0 + 8 * s + base + 1, e_vdw, valid);
 }
 
-__global__ void __launch_bounds__(128) k_qq(Dev d) {
-  qq_term(d, blockIdx.x * blockDim.x + threadIdx.x, SlotSink{&d});
+// waves of the q-q work: one per atom, then on energy steps one per 64 pairs
+template <bool EK>
+__device__ __forceinline__ void qq_wave(const Dev& d, int wave) {
+  if (wave < d.nqqg) qq_atom(d, wave);
+  else if (EK) qq_energy(d, (wave - d.nqqg) * 64 + (int)(threadIdx.x & 63));
 }
-
-// bonded mode 2: the q-q pair slots of each atom (contiguous), summed by
-// eight lanes per atom (a q-atom has a slot per partner and state, so one
-// lane alone would walk a long dependent run) and added to the gradient.
-// Every lane stays to the row sum.
-constexpr int kQqGatherLanes = 8;
-__global__ void __launch_bounds__(256) k_qq_gather(Dev d) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int k = t / kQqGatherLanes, l = t % kQqGatherLanes;
-  int atom = -1;
-  long long gx = 0, gy = 0, gz = 0;
-  if (k < d.nqqg) {
-    atom = d.qqg_atom[k];
-    if (d.ws[d.wid[atom]].active) {
-      const int m1 = d.qqg_start[k + 1];
-      for (int m = d.qqg_start[k] + l; m < m1; m += kQqGatherLanes) {
-        gx += d.qqslot[3 * (size_t)m];
-        gy += d.qqslot[3 * (size_t)m + 1];
-        gz += d.qqslot[3 * (size_t)m + 2];
-      }
-    } else {
-      atom = -1;
-    }
-  }
-  gx = row8_sum_i(gx);
-  gy = row8_sum_i(gy);
-  gz = row8_sum_i(gz);
-  if (l == 0 && atom >= 0) add_grad_fix(d.f, atom, gx, gy, gz);
+template <bool EK>
+__global__ void __launch_bounds__(256) k_qq(Dev d) {
+  qq_wave<EK>(d, __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6)));
 }
-
-static void launch_qq(const Dev& d, hipStream_t s) {
+static int qq_waves(const Dev& d, bool energy) { return d.nqqg + (energy ? (d.nqq + 63) / 64 : 0); }
+static void launch_qq(const Dev& d, hipStream_t s, bool energy) {
   if (!d.nqq) return;
-  k_qq<<<(d.nqq + 127) / 128, 128, 0, s>>>(d);
-  if (d.bond_atomic == 2 && d.nqqg)
-    k_qq_gather<<<((size_t)d.nqqg * kQqGatherLanes + 255) / 256, 256, 0, s>>>(d);
+  const int nb = (qq_waves(d, energy) * 64 + 255) / 256;
+  if (energy) k_qq<true><<<nb, 256, 0, s>>>(d);
+  else k_qq<false><<<nb, 256, 0, s>>>(d);
 }
 
 // ------------------------------------------------------------- LRF --
@@ -1661,17 +1622,12 @@ __device__ __forceinline__ void torsion_geom(const double* x, int i, int j, int 
   *scp_out = scp;
 }
 
-// Bonded terms write the fixed-point gradient of each of their atoms into a
-// slot of their own (no atomics); k_bonded_gather then sums every atom's
-// slots in a fixed order.  Integer sums make the result independent of the
-// order, so it equals the atomic form bit for bit.
-
 template <class Sink>
-__device__ __forceinline__ void put4(const Sink& put, int k, double dv, const double dp[12]) {
-  put(k + 0, 0, dv * dp[0], dv * dp[1], dv * dp[2]);
-  put(k + 1, 1, dv * dp[3], dv * dp[4], dv * dp[5]);
-  put(k + 2, 2, dv * dp[6], dv * dp[7], dv * dp[8]);
-  put(k + 3, 3, dv * dp[9], dv * dp[10], dv * dp[11]);
+__device__ __forceinline__ void put4(const Sink& put, const int4& a, double dv, const double dp[12]) {
+  put(a.x, 0, dv * dp[0], dv * dp[1], dv * dp[2]);
+  put(a.y, 1, dv * dp[3], dv * dp[4], dv * dp[5]);
+  put(a.z, 2, dv * dp[6], dv * dp[7], dv * dp[8]);
+  put(a.w, 3, dv * dp[9], dv * dp[10], dv * dp[11]);
 }
 
 // angle (md.f90:814-901): energy and the gradient factors di, dk of the end
@@ -1702,16 +1658,13 @@ __device__ __forceinline__ void angle_geom(const double* x, int i, int j, int k,
 
 // One bonded term t of the flat term index (bonds, angles, torsions,
 // impropers, then the q-bonds, q-angles, q-torsions and q-impropers), its
-// gradient handed to `put` per term atom (slot index in term order, and the
-// atom's place in the term); t past the last term does nothing.  Every lane of the wave must call it (the
-// energy goes through a wave sum).
+// gradient handed to `put` per term atom (the atom and its place in the term)
+// and its energy to put.energy; t past the last term does nothing.  Every lane
+// of the wave must call it (the energy goes through a wave sum).
 template <class Sink>
 __device__ __forceinline__ void bonded_term(const Dev& d, int t, const Sink& put) {
   const int n1 = d.nbond, n2 = n1 + d.nang, n3 = n2 + d.ntor, n4 = n3 + d.nimp;
   const int n5 = n4 + d.nqb, n6 = n5 + d.nqa, n7 = n6 + d.nqt, n8 = n7 + d.nqi;
-  // first slot of each kind (2, 3, 4, 4, 2, 3, 4, 4 atoms per term)
-  const int b1 = 0, b2 = b1 + 2 * d.nbond, b3 = b2 + 3 * d.nang, b4 = b3 + 4 * d.ntor;
-  const int b5 = b4 + 4 * d.nimp, b6 = b5 + 2 * d.nqb, b7 = b6 + 3 * d.nqa, b8 = b7 + 4 * d.nqt;
   const double* x = d.x;
   bool valid = false;
   int w = 0, eslot = 0;
@@ -1726,8 +1679,8 @@ __device__ __forceinline__ void bonded_term(const Dev& d, int t, const Sink& put
       const double bl = sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2]);
       const double db = bl - p.y;
       const double dv = p.x * db / bl;
-      put(b1 + 2 * t, 0, -r[0] * dv, -r[1] * dv, -r[2] * dv);
-      put(b1 + 2 * t + 1, 1, r[0] * dv, r[1] * dv, r[2] * dv);
+      put(ij.x, 0, -r[0] * dv, -r[1] * dv, -r[2] * dv);
+      put(ij.y, 1, r[0] * dv, r[1] * dv, r[2] * dv);
       valid = true;
       e = 0.5 * p.x * db * db;
       eslot = d.b_solv[t] ? E_W_BOND : E_P_BOND;
@@ -1752,9 +1705,9 @@ __device__ __forceinline__ void bonded_term(const Dev& d, int t, const Sink& put
         const double du = 2 * p.z * ru / dik;
         for (int c = 0; c < 3; ++c) { gk[c] += du * r[c]; gi[c] -= du * r[c]; }
       }
-      put(b2 + 3 * a, 0, gi[0], gi[1], gi[2]);
-      put(b2 + 3 * a + 1, 1, gj[0], gj[1], gj[2]);
-      put(b2 + 3 * a + 2, 2, gk[0], gk[1], gk[2]);
+      put(ijk.x, 0, gi[0], gi[1], gi[2]);
+      put(ijk.y, 1, gj[0], gj[1], gj[2]);
+      put(ijk.z, 2, gk[0], gk[1], gk[2]);
       valid = true;
       eslot = d.a_solv[a] ? E_W_ANG : E_P_ANG;
     }
@@ -1769,7 +1722,7 @@ __device__ __forceinline__ void bonded_term(const Dev& d, int t, const Sink& put
       const double arg = (double)p.y * phi - (double)p.z;
       e = (double)p.x * (1.0 + cos(arg)) * (double)p.w;
       const double dv = -(double)p.y * (double)p.x * sin(arg) * (double)p.w;
-      put4(put, b3 + 4 * a, dv, dp);
+      put4(put, q, dv, dp);
       valid = true;
       eslot = d.t_solv[a] ? E_W_TOR : E_P_TOR;
     }
@@ -1793,7 +1746,7 @@ __device__ __forceinline__ void bonded_term(const Dev& d, int t, const Sink& put
         dv = (double)p.x * arg;
         e = 0.5 * dv * arg;
       }
-      put4(put, b4 + 4 * a, dv, dp);
+      put4(put, q, dv, dp);
       valid = true;
       eslot = d.i_solv[a] ? E_W_IMP : E_P_IMP;
     }
@@ -1813,8 +1766,8 @@ __device__ __forceinline__ void bonded_term(const Dev& d, int t, const Sink& put
       const double fexp = exp(-p.y * db);
       e = p.x * (fexp * fexp - 2. * fexp) + 0.5 * p.w * db * db;
       const double dv = (2. * p.x * p.y * (fexp - fexp * fexp) + p.w * db) * lam / bl;
-      put(b5 + 2 * a, 0, -dv * r[0], -dv * r[1], -dv * r[2]);
-      put(b5 + 2 * a + 1, 1, dv * r[0], dv * r[1], dv * r[2]);
+      put(ij.x, 0, -dv * r[0], -dv * r[1], -dv * r[2]);
+      put(ij.y, 1, dv * r[0], dv * r[1], dv * r[2]);
       valid = true;
       eslot = E_Q0 + 8 * s + 0;
     }
@@ -1846,9 +1799,9 @@ __device__ __forceinline__ void bonded_term(const Dev& d, int t, const Sink& put
         di[c] = f1 * (rjk[c] / (bji * bjk) - scp * rji[c] / (bji * bji));
         dk[c] = f1 * (rji[c] / (bji * bjk) - scp * rjk[c] / (bjk * bjk));
       }
-      put(b6 + 3 * a, 0, dv * di[0], dv * di[1], dv * di[2]);
-      put(b6 + 3 * a + 1, 1, -dv * (di[0] + dk[0]), -dv * (di[1] + dk[1]), -dv * (di[2] + dk[2]));
-      put(b6 + 3 * a + 2, 2, dv * dk[0], dv * dk[1], dv * dk[2]);
+      put(i, 0, dv * di[0], dv * di[1], dv * di[2]);
+      put(j, 1, -dv * (di[0] + dk[0]), -dv * (di[1] + dk[1]), -dv * (di[2] + dk[2]));
+      put(k, 2, dv * dk[0], dv * dk[1], dv * dk[2]);
       valid = true;
       eslot = E_Q0 + 8 * s + 1;
     }
@@ -1878,108 +1831,91 @@ __device__ __forceinline__ void bonded_term(const Dev& d, int t, const Sink& put
         e = 0.5 * dv * arg;
         dv = dv * lam;
       }
-      put4(put, tors ? b7 + 4 * a : b8 + 4 * a, dv, dp);
+      put4(put, q, dv, dp);
       valid = true;
       eslot = E_Q0 + 8 * s + (tors ? 2 : 3);
     }
   }
-  const bool en = valid && d.ws[w].energy_now;
-  wave_energy(d.ws, w, eslot, e, en);
+  put.energy(eslot, e, valid);
 }
 
-__global__ void __launch_bounds__(256) k_bonded(Dev d) {
-  bonded_term(d, blockIdx.x * blockDim.x + threadIdx.x, SlotSink{&d});
-}
-
-// Bonded terms in tiles: a block takes the terms of one tile (consecutive
-// by their first atom, at most kBondTileTerms of them, grouped by kind so
-// that waves run one kind) and sums their gradients in LDS, per atom of the
-// tile's span, with integer atomics; then one atomic add per atom and
-// component goes to the gradient.  An atom outside the span (a term that
-// reaches further than kBondSpan atoms) goes to the gradient directly.  The
-// integer sums are the same as those of the slots and their gather.
+// Bonded terms in tiles: a block takes the terms of one tile (of one window,
+// consecutive by their first atom, at most kBondTileTerms of them, grouped by
+// kind so that waves run one kind) and sums their gradients in LDS, per atom
+// of the tile's span, and on energy steps their energies, with integer
+// atomics; then one atomic add per atom and component goes to the gradient
+// and one per energy.  An atom outside the span (a term that reaches further
+// than kBondSpan atoms) goes to the gradient directly.
 // The term's gradients are recorded per term atom (pos 0..3, a constant at
 // each call site, so the record stays in registers) and added to the tile's
 // LDS sums after the term, in one loop for every kind.
+// Bound by the latency of the terms' FP64 functions and gathers: 64-window
+// ladder 33 us alone, force-only or with energies.  On energy steps the terms
+// used to write a slot per term atom for a gather kernel (300 MB of traffic, 70
+// us alone), because tiles added every term's energy with a global atomic.
 struct TermRec {
   int k[4];
   long long g[4][3];
 };
 struct TileSink {
   TermRec* rec;
-  __device__ void operator()(int k, int pos, double gx, double gy, double gz) const {
-    rec->k[pos] = k;
+  unsigned long long* e;   // LDS energies by slot, or null
+  __device__ void operator()(int atom, int pos, double gx, double gy, double gz) const {
+    rec->k[pos] = atom;
     rec->g[pos][0] = fix(gx, kFScale);
     rec->g[pos][1] = fix(gy, kFScale);
     rec->g[pos][2] = fix(gz, kFScale);
   }
+  // as wave_energy, into LDS
+  __device__ void energy(int slot, double v, bool valid) const {
+    if (!e) return;   // uniform over the block
+    const unsigned long long vm = __ballot(valid);
+    if (vm == 0ull) return;
+    const int first = __ffsll((long long)vm) - 1;
+    const int slot0 = __builtin_amdgcn_readlane(valid ? slot : -1, first);
+    const long long ef = valid ? fix(v, kEScale) : 0ll;
+    if (__ballot(valid && slot != slot0) == 0ull) {
+      const long long sum = wave_sum_i(ef);
+      if ((int)(threadIdx.x & 63) == first) atomicAdd(&e[slot0], (unsigned long long)sum);
+    } else if (valid) {
+      atomicAdd(&e[slot], (unsigned long long)ef);
+    }
+  }
 };
 
-__global__ void __launch_bounds__(256) k_bonded_tiles(Dev d) {
-  __shared__ unsigned long long s_acc[3 * kBondSpan];
-  const int4 tl = d.btile[blockIdx.x];   // first entry, terms, first atom, atoms spanned
+__device__ __forceinline__ void bonded_tile(const Dev& d, int tile, unsigned long long* s_acc, unsigned long long* s_e) {
+  const int4 tl = d.btile[tile];   // first entry, terms, first atom, atoms spanned
+  const int w = d.wid[tl.z];
+  if (!d.ws[w].active) return;     // uniform over the block
+  const bool en = d.ws[w].energy_now;
   for (int m = threadIdx.x; m < 3 * tl.w; m += blockDim.x) s_acc[m] = 0ull;
+  if ((int)threadIdx.x < E_NSLOT) s_e[threadIdx.x] = 0ull;
   __syncthreads();
   for (int k0 = 0; k0 < tl.y; k0 += blockDim.x) {
     const int k = k0 + (int)threadIdx.x;
     TermRec rec;
 #pragma unroll
     for (int p = 0; p < 4; ++p) rec.k[p] = -1;
-    bonded_term(d, k < tl.y ? d.btile_terms[tl.x + k] : 0x7fffffff, TileSink{&rec});
+    bonded_term(d, k < tl.y ? d.btile_terms[tl.x + k] : 0x7fffffff, TileSink{&rec, en ? s_e : nullptr});
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
       if (rec.k[p] < 0) continue;
-      const int a = d.slot_atom[rec.k[p]];
-      const int l = a - tl.z;
+      const int l = rec.k[p] - tl.z;
       if (l >= 0 && l < kBondSpan) {
         for (int c = 0; c < 3; ++c) atomicAdd(&s_acc[3 * l + c], (unsigned long long)rec.g[p][c]);
       } else {
-        for (int c = 0; c < 3; ++c) atomicAdd((unsigned long long*)&d.f[3 * a + c], (unsigned long long)rec.g[p][c]);
+        add_grad_fix(d.f, rec.k[p], rec.g[p][0], rec.g[p][1], rec.g[p][2]);
       }
     }
   }
   __syncthreads();
-  for (int l = threadIdx.x; l < tl.w; l += blockDim.x) {
-    const long long gx = (long long)s_acc[3 * l], gy = (long long)s_acc[3 * l + 1], gz = (long long)s_acc[3 * l + 2];
-    if (gx | gy | gz) add_grad_fix(d.f, tl.z + l, gx, gy, gz);
-  }
+  for (int m = threadIdx.x; m < 3 * tl.w; m += blockDim.x)
+    if (s_acc[m]) atomicAdd((unsigned long long*)&d.f[3 * (size_t)tl.z + m], s_acc[m]);
+  if (en && (int)threadIdx.x < E_NSLOT) add_energy_fix(d.ws, w, threadIdx.x, (long long)s_e[threadIdx.x]);
 }
-
-// sum of each bonded atom's slots (CSR in slot order) into the gradient.  A
-// block takes consecutive atoms whose slots form one contiguous run: the run
-// is read into LDS with coalesced loads, then one thread per atom adds its
-// own slots, so the add to the gradient needs no atomic.  A block of one
-// atom with more slots than fit reads them from global memory.
-__global__ void __launch_bounds__(256) k_bonded_gather(Dev d) {
-  __shared__ long long s_slot[3 * kGatherSlots];
-  const int2 gw = d.gather_work[block_id(d.xcd)];
-  const int s0 = d.bg_start[gw.x], s1 = d.bg_start[gw.y];
-  const bool staged = s1 - s0 <= kGatherSlots;
-  if (staged) {
-    for (int m = threadIdx.x; m < 3 * (s1 - s0); m += blockDim.x) s_slot[m] = d.bslot[3 * (size_t)s0 + m];
-    __syncthreads();
-  }
-  for (int k = gw.x + (int)threadIdx.x; k < gw.y; k += blockDim.x) {
-    const int atom = d.bg_atom[k];
-    if (!d.ws[d.wid[atom]].active) continue;
-    long long gx = 0, gy = 0, gz = 0;
-    const int m0 = d.bg_start[k], m1 = d.bg_start[k + 1];
-    if (staged) {
-      for (int m = m0 - s0; m < m1 - s0; ++m) {
-        gx += s_slot[3 * m];
-        gy += s_slot[3 * m + 1];
-        gz += s_slot[3 * m + 2];
-      }
-    } else {
-      for (int m = m0; m < m1; ++m) {
-        gx += d.bslot[3 * (size_t)m];
-        gy += d.bslot[3 * (size_t)m + 1];
-        gz += d.bslot[3 * (size_t)m + 2];
-      }
-    }
-    // atomic: the nonbonded kernels may add to the same atoms concurrently
-    add_grad_fix(d.f, atom, gx, gy, gz);
-  }
+__global__ void __launch_bounds__(256) k_bonded(Dev d) {
+  __shared__ unsigned long long s_acc[3 * kBondSpan], s_e[E_NSLOT];
+  bonded_tile(d, blockIdx.x, s_acc, s_e);
 }
 
 // fixed/shell restraints (fix_shell, md.f90:1414-1450) and the radial
@@ -2036,8 +1972,8 @@ __device__ __forceinline__ void restr_atom(const Dev& d, int i, long long* acc) 
 // fixed, shell and solvent restraints (one thread per atom; every lane
 // reaches the wave energy sums of both).  STORE: the atom's sum of them is
 // stored in fterm, which k_integrate adds to the gradient (an MD step, where
-// it runs beside the pair kernels); else it is added to the gradient with the
-// row kernels' and q kernels' sums, after every other kernel of an evaluation
+// it runs beside the pair kernels); else it completes the gradient of an
+// evaluation as the integrator does, after every other kernel
 template <bool STORE>
 __global__ void __launch_bounds__(256) k_atom_terms(Dev d) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2051,7 +1987,8 @@ __global__ void __launch_bounds__(256) k_atom_terms(Dev d) {
     const int r = d.rslot[i];
     for (int c = 0; c < 3; ++c) {
       if (r >= 0) g[c] += d.grow[3 * (size_t)r + c] + d.gq[3 * (size_t)r + c];
-      d.f[3 * i + c] += g[c];
+      d.fterm[3 * i + c] = g[c] + d.f[3 * i + c];
+      d.f[3 * i + c] = 0;
     }
   }
 }
@@ -2450,13 +2387,15 @@ __device__ __forceinline__ void leapfrog_vals(const Dev& d, const WinState& st, 
 // gradient of atom i for the integrator: the step's per-atom terms (LRF
 // evaluation, fixed/shell and radial solvent restraints, stored by
 // k_atom_terms<true>), the row kernels' and q kernels' sums, and the gradient
-// the other kernels added up, stored back, so the gradient array ends complete
+// the other kernels added up, which is cleared for the next step; the complete
+// gradient takes the place of the per-atom terms
 __device__ __forceinline__ void step_gradient(const Dev& d, int i, long long g[3]) {
   const int r = d.rslot[i];
   for (int c = 0; c < 3; ++c) {
     g[c] = d.fterm[3 * i + c] + d.f[3 * i + c];
     if (r >= 0) g[c] += d.grow[3 * (size_t)r + c] + d.gq[3 * (size_t)r + c];
-    d.f[3 * i + c] = g[c];
+    d.fterm[3 * i + c] = g[c];
+    d.f[3 * i + c] = 0;
   }
 }
 
@@ -2686,10 +2625,12 @@ __global__ void __launch_bounds__(256) k_ekin_part(Dev d) {
 // temperatures and Berendsen factors (one wave per window) from the
 // kinetic-energy partials of k_ekin_part, or with `advance` (the end of a
 // step) from the fixed-point sums of k_integrate, which it clears for the
-// next step; with `advance` also the ring records of the step and the step
-// count.  The lanes copy the energy accumulators into the step's ring slot,
-// lane 0 does the rest.
-__global__ void __launch_bounds__(64) k_temperature(Dev d, int advance) {
+// next step; with `advance` also the ring records of the step, the step
+// count, and the start of the next step (begin_step).  The lanes copy the
+// energy accumulators into the step's ring slot, lane 0 does the rest.
+// `variant`: what the step launched, bit 0 the list kernels, bit 1 the kernel
+// instances with energy terms; a window that needed more is flagged.
+__global__ void __launch_bounds__(64) k_temperature(Dev d, int advance, int variant) {
   const int w = blockIdx.x;
   if (w >= d.nwin) return;
   WinState& st = d.ws[w];
@@ -2737,7 +2678,10 @@ __global__ void __launch_bounds__(64) k_temperature(Dev d, int advance) {
       tr[0] = st.temp; tr[1] = st.tfree; tr[2] = st.ekin;
       tr[3] = (double)st.istep + 4294967296.0 * (double)st.run_epoch;
       tr[4] = st.tfree_solute; tr[5] = st.tfree_solvent;
+      if (st.list_now && !(variant & 1)) st.list_missed = 1;
+      if (st.energy_now && !(variant & 2)) st.list_missed = 2;
       st.istep += 1;
+      begin_step(st, W);
     }
   }
 }
@@ -2745,9 +2689,11 @@ __global__ void __launch_bounds__(64) k_temperature(Dev d, int advance) {
 // ------------------------------------------------------ launchers --
 static inline int blocks(long long n, int bs) { return (int)((n + bs - 1) / bs); }
 
-void launch_begin(const Dev& d, hipStream_t s, int force_energy, int eval_only, int rebuild) {
-  k_begin<<<blocks(std::max(std::max(d.nwin, d.ntot), d.noffd_all), 256), 256, 0, s>>>(d, force_energy, eval_only,
-                                                                                         rebuild);
+void launch_begin(const Dev& d, hipStream_t s, int eval, int rebuild) {
+  k_begin<<<blocks(d.nwin, 64), 64, 0, s>>>(d, eval, rebuild);
+}
+void launch_offdiag(const Dev& d, hipStream_t s) {
+  if (d.noffd_all) k_offdiag<<<blocks(d.noffd_all, 64), 64, 0, s>>>(d);
 }
 
 void launch_lrf_build(const Dev& d, hipStream_t s) {
@@ -2758,17 +2704,14 @@ void launch_lrf_build(const Dev& d, hipStream_t s) {
 }
 
 void launch_bonded(const Dev& d, hipStream_t s) {
-  int nb = d.nbond + d.nang + d.ntor + d.nimp + d.nqb + d.nqa + d.nqt + d.nqi;
-  if (d.bond_atomic == 2) {
-    if (d.nbtile) k_bonded_tiles<<<d.nbtile, 256, 0, s>>>(d);
-  } else if (nb) {
-    k_bonded<<<blocks(nb, d.bs_bonded), d.bs_bonded, 0, s>>>(d);
-  }
+  if (d.nbtile) k_bonded<<<d.nbtile, 256, 0, s>>>(d);
+  if (d.nrst) k_prestr<<<d.nrst, 64, 0, s>>>(d);
 }
 
 // list update: group centres and cluster spheres, then the neighbour rows
 // and the LRF expansions (independent of each other)
 static void launch_list_prep(const Dev& d, hipStream_t s, int ngrp, int nwc, int nsc) {
+  if (d.any_qdyn) k_qin<<<blocks(d.ntot, 256), 256, 0, s>>>(d);
   k_centres<<<blocks(ngrp, 128), 128, 0, s>>>(d, ngrp);
   k_bounds<<<blocks(nwc + nsc, 128), 128, 0, s>>>(d, nwc, nsc);
 }
@@ -2844,7 +2787,7 @@ void launch_nonbonded(const Dev& d, hipStream_t s, bool with_ww, bool q_energy) 
   else launch_wrow_k<false, 2>(d, s);   // added to what launch_ww stored
   launch_srow(d, s, q_energy);
   launch_q(d, s, q_energy);
-  launch_qq(d, s);
+  launch_qq(d, s, q_energy);
 }
 
 static void launch_watpol(const Dev& d, hipStream_t s) {
@@ -2852,17 +2795,9 @@ static void launch_watpol(const Dev& d, hipStream_t s) {
   if (d.nwin <= kWpolWide) k_watpol<1024><<<d.nwin * kWpolMaxShell, 1024, 0, s>>>(d);
   else k_watpol<256><<<d.nwin * kWpolMaxShell, 256, 0, s>>>(d);
 }
-// bonded terms with their gather, which also collects the q-q pair slots
-// written by k_qq, and sequence restraints
-static void launch_bonded_gather(const Dev& d, hipStream_t s) {
-  const int nb = d.nbond + d.nang + d.ntor + d.nimp + d.nqb + d.nqa + d.nqt + d.nqi;
-  launch_bonded(d, s);
-  if ((nb || d.nqq) && !d.bond_atomic && d.ngw) k_bonded_gather<<<d.ngw, 256, 0, s>>>(d);
-  if (d.nrst) k_prestr<<<d.nrst, 64, 0, s>>>(d);
-}
 void launch_other_forces(const Dev& d, hipStream_t s, bool atom_terms) {
   launch_watpol(d, s);
-  launch_bonded_gather(d, s);
+  launch_bonded(d, s);
   if (atom_terms && d.ntot) k_atom_terms<false><<<blocks(d.ntot, 256), 256, 0, s>>>(d);   // last: completes the gradient
 }
 
@@ -2893,6 +2828,7 @@ hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, hipSt
   if (err == hipSuccess) err = hipStreamWaitEvent(s2, ev[0], 0);
   if (err == hipSuccess && !lists) err = hipStreamWaitEvent(s3, ev[0], 0);
   if (err != hipSuccess) return err;
+  launch_offdiag(d, s2);
   if (lists) {
     launch_list_prep(d, s, ngrp, nwc, nsc);
     err = hipEventRecord(ev[2], s);
@@ -2902,8 +2838,8 @@ hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, hipSt
     launch_rows_water(d, s);
   }
   launch_watpol(d, s2);
-  launch_qq(d, s2);
-  launch_bonded_gather(d, s2);
+  launch_qq(d, s2, q_energy);
+  launch_bonded(d, s2);
   launch_wrow(d, s, q_energy);
   launch_qw(d, s3, q_energy);
   launch_srow(d, s3, q_energy);
@@ -2929,14 +2865,14 @@ void launch_atom_terms(const Dev& d, hipStream_t s) {
   if (d.ntot) k_atom_terms<true><<<blocks(d.ntot, 256), 256, 0, s>>>(d);
 }
 
-void launch_integrate(const Dev& d, hipStream_t s, int shake_any) {
+void launch_integrate(const Dev& d, hipStream_t s, int shake_any, int variant) {
   if (d.nib) k_integrate<<<d.nib, kIntBlock, 0, s>>>(d, shake_any ? 1 : 0);
-  k_temperature<<<d.nwin, 64, 0, s>>>(d, 1);
+  k_temperature<<<d.nwin, 64, 0, s>>>(d, 1, variant);
 }
 
 void launch_temperature(const Dev& d, hipStream_t s) {
   k_ekin_part<<<d.nwin * kTempParts, 256, 0, s>>>(d);
-  k_temperature<<<d.nwin, 64, 0, s>>>(d, 0);
+  k_temperature<<<d.nwin, 64, 0, s>>>(d, 0, 0);
 }
 
 void launch_refresh32(const Dev& d, hipStream_t s) { k_refresh32<<<blocks(d.ntot, 256), 256, 0, s>>>(d); }
