@@ -214,6 +214,7 @@ struct Dev {
   // A, B, charge product and soft-core term ([(m * kMaxS + s) * 2 + k - 1])
   const float4* qcw_h;
   int any_wat3;          // some window has a 3-atom solvent
+  int small;             // a step's force kernels run as one launch
   // the same in FP64 for the energy terms: A, B, soft-core term, charge
   // product of member, state and water atom ([(m * kMaxS + s) * 3 + k])
   const double4* qcw_e;

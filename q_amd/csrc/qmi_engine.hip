@@ -1262,6 +1262,9 @@ static int build_device(qmi_engine* e) {
   if ((rc = make_rows(T_WP, wc_win)) != 0) return rc;
   if ((rc = make_rows(T_PW, sc_win)) != 0) return rc;
   if ((rc = make_rows(T_PP, sc_win)) != 0) return rc;
+  bool all3 = true;
+  for (int wi = 0; wi < NW; ++wi) all3 = all3 && wd[wi].wat3;
+  d.small = small_engine(d, d.any_wat3 && !all3) ? 1 : 0;
   return 0;
 }
 

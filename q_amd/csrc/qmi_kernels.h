@@ -24,6 +24,8 @@ void launch_nonbonded(const Dev& d, hipStream_t s, bool with_ww = true, bool q_e
 void launch_other_forces(const Dev& d, hipStream_t s, bool atom_terms = true);
 // the per-atom terms of an MD step into their own array (Dev::fterm)
 void launch_atom_terms(const Dev& d, hipStream_t s);
+// whether a step's force kernels run as one launch (Dev::small)
+bool small_engine(const Dev& d, bool mixed_solvent);
 // the lists and forces of an MD step on three streams (see the definition)
 hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, hipStream_t s3, const hipEvent_t ev[5],
                               bool lists, int ngrp, int nwc, int nsc, bool q_energy);

@@ -352,8 +352,7 @@ __device__ __forceinline__ int special_type(const Dev& d, int i, int j) {
 // member a of the i-cluster and member b of the j-cluster, and the passing
 // members are appended, in j order, to row a.
 template <int TT>
-__global__ void __launch_bounds__(256) k_build_rows(Dev d) {
-  const int wave = wave_id(d);
+__device__ __forceinline__ void build_row(const Dev& d, int wave) {
   const int lane = threadIdx.x & 63;
   const RowList L = d.rl[TT];
   if (wave >= L.nicl) return;
@@ -427,6 +426,19 @@ __global__ void __launch_bounds__(256) k_build_rows(Dev d) {
   }
 }
 
+// all four kinds of rows in one launch, the longest-running first
+__global__ void __launch_bounds__(256) k_build_rows(Dev d) {
+  int wave = wave_id(d);
+  const int np = (d.rl[T_PP].nicl + 3) & ~3, nw = (d.rl[T_WW].nicl + 3) & ~3;   // whole blocks of each kind
+  if (wave < np) return build_row<T_PP>(d, wave);
+  wave -= np;
+  if (wave < nw) return build_row<T_WW>(d, wave);
+  wave -= nw;
+  if (wave < nw) return build_row<T_WP>(d, wave);
+  wave -= nw;
+  if (wave < np) return build_row<T_PW>(d, wave);
+}
+
 // the number of chunks of 8 entries the wave must walk: the longest row
 constexpr int kUnroll = 4;   // row entries per pass of the pair kernels
 
@@ -483,8 +495,7 @@ struct RowGrad {
 // The energy sums run only on energy steps: EN selects the form of the
 // loop for the wave's window (uniform over the wave).
 template <bool EN, bool W3>
-__device__ __forceinline__ void ww_impl(const Dev& d, RowGrad& rg) {
-  const int wave = wave_id(d);
+__device__ __forceinline__ void ww_impl(const Dev& d, int wave, RowGrad& rg) {
   const int lane = threadIdx.x & 63;
   const RowList L = d.rl[T_WW];
   if (wave >= L.nicl) return;
@@ -594,8 +605,7 @@ __device__ __forceinline__ void ww_impl(const Dev& d, RowGrad& rg) {
 // (W<-P); otherwise rows are solute atoms and entries water slots (P<-W),
 // which also counts the energies.
 template <bool WATER_SIDE, bool EN, bool W3>
-__device__ __forceinline__ void pw_impl(const Dev& d, RowGrad& rg) {
-  const int wave = wave_id(d);
+__device__ __forceinline__ void pw_impl(const Dev& d, int wave, RowGrad& rg) {
   const int lane = threadIdx.x & 63;
   const RowList L = d.rl[WATER_SIDE ? T_WP : T_PW];
   if (wave >= L.nicl) return;
@@ -713,8 +723,7 @@ __device__ __forceinline__ void pw_impl(const Dev& d, RowGrad& rg) {
 // solute-solute (nonbond_pp, md.f90:10387-10491): 1-4 pairs use the third
 // LJ column and the el14 scale
 template <bool EN>
-__device__ __forceinline__ void pp_impl(const Dev& d, RowGrad& rg) {
-  const int wave = wave_id(d);
+__device__ __forceinline__ void pp_impl(const Dev& d, int wave, RowGrad& rg) {
   const int lane = threadIdx.x & 63;
   const RowList L = d.rl[T_PP];
   if (wave >= L.nicl) return;
@@ -824,17 +833,16 @@ __device__ __forceinline__ void pp_impl(const Dev& d, RowGrad& rg) {
 // PART (k_wrow): 1 water-water rows alone, 2 water<-solute rows alone, added
 // to what part 1 stored (for timing them), 3 both.
 template <bool W3, bool EK, int PART>
-__global__ void __launch_bounds__(256) k_wrow(Dev d) {
-  const int wave = wave_id(d);
+__device__ __forceinline__ void wrow_wave(const Dev& d, int wave) {
   if (wave >= d.rl[T_WW].nicl) return;
   const int w = d.wc_win[wave];
   if ((d.win[w].wat3 != 0) != W3 || !d.ws[w].active) return;
   RowGrad rg;
   if (PART & 1) {
-    if (EK && d.ws[w].energy_now) ww_impl<EK, W3>(d, rg);
-    else ww_impl<false, W3>(d, rg);
+    if (EK && d.ws[w].energy_now) ww_impl<EK, W3>(d, wave, rg);
+    else ww_impl<false, W3>(d, wave, rg);
   }
-  if (PART & 2) pw_impl<true, false, W3>(d, rg);
+  if (PART & 2) pw_impl<true, false, W3>(d, wave, rg);
   const int lane = threadIdx.x & 63, b = lane & 7, row = wave * kCl + (lane >> 3);
   if (d.wc_o[row] < 0) return;
   long long* o = d.grow + 9 * (size_t)row;
@@ -842,23 +850,30 @@ __global__ void __launch_bounds__(256) k_wrow(Dev d) {
   o[b] = rg.lo;
   if (b == 0) o[8] = PART == 2 ? o[8] + rg.hi : rg.hi;
 }
+template <bool W3, bool EK, int PART>
+__global__ void __launch_bounds__(256) k_wrow(Dev d) {
+  wrow_wave<W3, EK, PART>(d, wave_id(d));
+}
 
 template <bool W3, bool EK>
-__global__ void __launch_bounds__(256) k_srow(Dev d) {
-  const int wave = wave_id(d);
+__device__ __forceinline__ void srow_wave(const Dev& d, int wave) {
   if (wave >= d.rl[T_PP].nicl) return;
   const int w = d.sc_win[wave];
   if ((d.win[w].wat3 != 0) != W3 || !d.ws[w].active) return;
   RowGrad rg;
   if (EK && d.ws[w].energy_now) {
-    pw_impl<false, EK, W3>(d, rg);
-    pp_impl<EK>(d, rg);
+    pw_impl<false, EK, W3>(d, wave, rg);
+    pp_impl<EK>(d, wave, rg);
   } else {
-    pw_impl<false, false, W3>(d, rg);
-    pp_impl<false>(d, rg);
+    pw_impl<false, false, W3>(d, wave, rg);
+    pp_impl<false>(d, wave, rg);
   }
   const int lane = threadIdx.x & 63, b = lane & 7, row = wave * kCl + (lane >> 3);
   if (b < 3 && d.sc_a[row] >= 0) d.grow[9 * (size_t)d.nwslot + 3 * row + b] = rg.lo;
+}
+template <bool W3, bool EK>
+__global__ void __launch_bounds__(256) k_srow(Dev d) {
+  srow_wave<W3, EK>(d, wave_id(d));
 }
 
 // ---- q-atoms against water (nonbond_qw_spc, md.f90:11302-11411; 3-atom
@@ -907,18 +922,19 @@ __device__ __forceinline__ int4 q_item(const int4* work, int block) {
   const ConstI k = (ConstI)(const int*)work + 4 * (size_t)block;
   return make_int4(k[0], k[1], k[2], k[3]);
 }
-// the waves' sums of the N components of 64 slots (s[k][lane] of a wave) into
-// out[N * slot + k], for the item's slots
+// the sums of an item's waves of the N components of its slots into out[N *
+// slot + k]; s: LDS of N * 64 * kQWaves doubles for the group of kQWaves waves.
+// Every thread of the block calls it; a group without an item has 0 slots.
 template <int N>
-__device__ __forceinline__ void q_store(const double* acc, int slots, long long* out) {
-  __shared__ double s_acc[kQWaves][N][64];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+__device__ __forceinline__ void q_store(const double* acc, int slots, long long* out, double* s) {
+  constexpr int kStride = N * 64;
+  const int lane = threadIdx.x & 63, wv = (threadIdx.x >> 6) % kQWaves, t = threadIdx.x % (64 * kQWaves);
 #pragma unroll
-  for (int k = 0; k < N; ++k) s_acc[wv][k][lane] = acc[k];
+  for (int k = 0; k < N; ++k) s[wv * kStride + k * 64 + lane] = acc[k];
   __syncthreads();
-  for (int i = threadIdx.x; i < N * slots; i += 64 * kQWaves) {
-    const int m = i / N, k = i % N;
-    out[i] = fix((s_acc[0][k][m] + s_acc[1][k][m]) + (s_acc[2][k][m] + s_acc[3][k][m]), kFScale);
+  for (int i = t; i < N * slots; i += 64 * kQWaves) {
+    const double* p = s + (i % N) * 64 + i / N;
+    out[i] = fix((p[0] + p[kStride]) + (p[2 * kStride] + p[3 * kStride]), kFScale);
   }
 }
 
@@ -972,7 +988,7 @@ __device__ __forceinline__ void qw_impl(const Dev& d, const WinDev& W, const int
   const ConstI qat = (ConstI)d.qc_atom;
   constexpr int NLJ = W3 ? 3 : 1;
   double eel[kMaxS] = {}, evdw[kMaxS] = {};
-  for (int ch = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); ch < W.nqch; ch += kQWaves) {
+  for (int ch = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) % kQWaves); ch < W.nqch; ch += kQWaves) {
     const int q0 = (ch >> 1) * 4 * kCl + (ch & 1) * 4;   // the chunk's first q-atom
     const int slot0 = W.qc_off * kCl + q0;
     QReaction react;
@@ -1098,23 +1114,35 @@ __device__ __forceinline__ void qw_impl(const Dev& d, const WinDev& W, const int
     }
 }
 
-// W3: the instance for 3-atom solvent windows; EK: the instance of steps
-// where some window computes energies
+// the work item of a group of kQWaves waves (past the last item: nothing but
+// the barrier).  W3: the instance for 3-atom solvent windows; EK: the instance
+// of steps where some window computes energies
+template <bool W3, bool EK>
+__device__ __forceinline__ void qw_group(const Dev& d, int item, double* s) {
+  double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  int4 wk = make_int4(0, 0, 0, 0);
+  if (item < d.nqw_work) {
+    wk = q_item(d.qw_work, item);
+    const WinDev& W = d.win[wk.x];
+    if (!d.ws[wk.x].active || (W.wat3 != 0) != W3) {
+      wk.z = 0;
+    } else {
+      const bool en = EK && d.ws[wk.x].energy_now;
+      if (W.S == 2) {
+        if (en) qw_impl<W3, EK, 2>(d, W, wk, acc);
+        else qw_impl<W3, false, 2>(d, W, wk, acc);
+      } else {
+        if (en) qw_impl<W3, EK, 0>(d, W, wk, acc);
+        else qw_impl<W3, false, 0>(d, W, wk, acc);
+      }
+    }
+  }
+  q_store<9>(acc, wk.z, d.gq + 9 * (size_t)wk.y, s);
+}
 template <bool W3, bool EK>
 __global__ void __launch_bounds__(64 * kQWaves) k_qw(Dev d) {
-  const int4 wk = q_item(d.qw_work, block_id(d.xcd));
-  const WinDev& W = d.win[wk.x];
-  if (!d.ws[wk.x].active || (W.wat3 != 0) != W3) return;   // uniform over the block
-  const bool en = EK && d.ws[wk.x].energy_now;
-  double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-  if (W.S == 2) {
-    if (en) qw_impl<W3, EK, 2>(d, W, wk, acc);
-    else qw_impl<W3, false, 2>(d, W, wk, acc);
-  } else {
-    if (en) qw_impl<W3, EK, 0>(d, W, wk, acc);
-    else qw_impl<W3, false, 0>(d, W, wk, acc);
-  }
-  q_store<9>(acc, wk.z, d.gq + 9 * (size_t)wk.y);
+  __shared__ double s[9 * 64 * kQWaves];
+  qw_group<W3, EK>(d, block_id(d.xcd), s);
 }
 
 template <bool EN, int NS>
@@ -1144,7 +1172,7 @@ __device__ __forceinline__ void qp_impl(const Dev& d, const WinDev& W, const int
   const float* sct = d.q_sc + W.qsc_off + (size_t)iacj * S;
   const double* scd = d.q_scd + W.qsc_off + (size_t)iacj * S;
   double eel[kMaxS] = {}, evdw[kMaxS] = {};
-  for (int ch = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); ch < W.nqch; ch += kQWaves) {
+  for (int ch = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) % kQWaves); ch < W.nqch; ch += kQWaves) {
     const int q0 = (ch >> 1) * 4 * kCl + (ch & 1) * 4;   // the chunk's first q-atom
     const int slot0 = W.qc_off * kCl + q0;
     // 1-4 pairs with the chunk's q-atoms, bit j for q-atom j
@@ -1233,20 +1261,31 @@ __device__ __forceinline__ void qp_impl(const Dev& d, const WinDev& W, const int
 }
 
 template <bool EK>
-__global__ void __launch_bounds__(64 * kQWaves) k_qp(Dev d) {
-  const int4 wk = q_item(d.qp_work, block_id(d.xcd));
-  const WinDev& W = d.win[wk.x];
-  if (!d.ws[wk.x].active) return;   // uniform over the block
-  const bool en = EK && d.ws[wk.x].energy_now;
+__device__ __forceinline__ void qp_group(const Dev& d, int item, double* s) {
   double acc[3] = {0, 0, 0};
-  if (W.S == 2) {
-    if (en) qp_impl<EK, 2>(d, W, wk, acc);
-    else qp_impl<false, 2>(d, W, wk, acc);
-  } else {
-    if (en) qp_impl<EK, 0>(d, W, wk, acc);
-    else qp_impl<false, 0>(d, W, wk, acc);
+  int4 wk = make_int4(0, 0, 0, 0);
+  if (item < d.nqp_work) {
+    wk = q_item(d.qp_work, item);
+    const WinDev& W = d.win[wk.x];
+    if (!d.ws[wk.x].active) {
+      wk.z = 0;
+    } else {
+      const bool en = EK && d.ws[wk.x].energy_now;
+      if (W.S == 2) {
+        if (en) qp_impl<EK, 2>(d, W, wk, acc);
+        else qp_impl<false, 2>(d, W, wk, acc);
+      } else {
+        if (en) qp_impl<EK, 0>(d, W, wk, acc);
+        else qp_impl<false, 0>(d, W, wk, acc);
+      }
+    }
   }
-  q_store<3>(acc, wk.z, d.gq + 9 * (size_t)d.nwslot + 3 * (size_t)wk.y);
+  q_store<3>(acc, wk.z, d.gq + 9 * (size_t)d.nwslot + 3 * (size_t)wk.y, s);
+}
+template <bool EK>
+__global__ void __launch_bounds__(64 * kQWaves) k_qp(Dev d) {
+  __shared__ double s[3 * 64 * kQWaves];
+  qp_group<EK>(d, block_id(d.xcd), s);
 }
 
 // q-q and q-(bonded neighbour) pairs (nonbond_qq, md.f90:10763-10868).
@@ -1975,8 +2014,7 @@ __device__ __forceinline__ void restr_atom(const Dev& d, int i, long long* acc) 
 // it runs beside the pair kernels); else it completes the gradient of an
 // evaluation as the integrator does, after every other kernel
 template <bool STORE>
-__global__ void __launch_bounds__(256) k_atom_terms(Dev d) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void atom_terms(const Dev& d, int i) {
   long long g[3] = {0, 0, 0};
   lrf_taylor_atom(d, i, g);
   restr_atom(d, i, g);
@@ -1992,13 +2030,17 @@ __global__ void __launch_bounds__(256) k_atom_terms(Dev d) {
     }
   }
 }
+template <bool STORE>
+__global__ void __launch_bounds__(256) k_atom_terms(Dev d) {
+  atom_terms<STORE>(d, blockIdx.x * blockDim.x + threadIdx.x);
+}
 
-// p_restrain (md.f90:12940-13274): one 64-lane block per restraint record.
+// p_restrain (md.f90:12940-13274): one wave per restraint record.
 // Sequence and wall records walk their atom range across the lanes; the
 // centre forms first reduce the mean displacement over the block.
 // State-dependent records (position, distance, angle) add their energy to
 // every state (ipsi 0) or to state ipsi, whose lambda weights the force.
-__device__ __forceinline__ void state_restraint_energy(Dev& d, int w, const WinDev& W, int ipsi, double e) {
+__device__ __forceinline__ void state_restraint_energy(const Dev& d, int w, const WinDev& W, int ipsi, double e) {
   if (ipsi == 0) {
     for (int s = 0; s < W.S; ++s) add_energy(d.ws, w, E_QR0 + s, e);
     if (W.S == 0) add_energy(d.ws, w, E_PROT, e);
@@ -2007,8 +2049,7 @@ __device__ __forceinline__ void state_restraint_energy(Dev& d, int w, const WinD
   }
 }
 
-__global__ void __launch_bounds__(64) k_prestr(Dev d) {
-  const int r = blockIdx.x;
+__device__ __forceinline__ void prestr_wave(const Dev& d, int r) {
   if (r >= d.nrst) return;
   const int4 kwij = d.rs_kwij[r];
   const int kind = kwij.x, w = kwij.y, i0 = kwij.z, j0 = kwij.w;
@@ -2017,7 +2058,7 @@ __global__ void __launch_bounds__(64) k_prestr(Dev d) {
   const WinDev& W = d.win[w];
   const int2 kf = d.rs_kf[r];
   const double* P = &d.rs_par[8 * r];
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
   if (kind == R_SEQ_ATOMS || kind == R_WALL) {
     double e = 0.0;
     for (int a = i0 + lane; a <= j0; a += 64) {
@@ -2130,6 +2171,8 @@ __global__ void __launch_bounds__(64) k_prestr(Dev d) {
   }
 }
 
+__global__ void __launch_bounds__(64) k_prestr(Dev d) { prestr_wave(d, blockIdx.x); }
+
 // water polarisation restraint (watpol, md.f90:15122-15288), one block per
 // (window, shell): the waters whose oxygen lies in the shell are collected in
 // LDS with the angle theta between their dipole and the radial vector, each
@@ -2200,9 +2243,17 @@ __device__ __forceinline__ double watpol_force(const Dev& d, const WinDev& W, fl
 constexpr int kWpolWide = 24;
 constexpr int kWpolSum = 256;        // threads of the theta sum (its order is part of the result)
 template <int kWpolBlock>            // threads per (window, shell) block
-__global__ void __launch_bounds__(kWpolBlock) k_watpol(Dev d) {
+struct WpolLds {
+  double th[kWpolLds];
+  int iw[kWpolLds], rank[kWpolBlock];
+  int n;
+  float corr;
+  double red[kWpolSum / 64];
+};
+template <int kWpolBlock>
+__device__ __forceinline__ void watpol_block(const Dev& d, int block, WpolLds<kWpolBlock>& L) {
   constexpr int kWpolHeld = kWpolLds / kWpolBlock;   // members per thread of a shell held in LDS
-  const int w = blockIdx.x / kWpolMaxShell, is = blockIdx.x % kWpolMaxShell;
+  const int w = block / kWpolMaxShell, is = block % kWpolMaxShell;
   if (w >= d.nwin) return;
   const WinState& st = d.ws[w];
   const WinDev& W = d.win[w];
@@ -2210,11 +2261,10 @@ __global__ void __launch_bounds__(kWpolBlock) k_watpol(Dev d) {
   if (!st.active || !W.wpol || W.nwat == 0 || is >= nsh) return;
   const ShellDev* shells = d.shells + W.sh_off;
   ShellDev& sh = d.shells[W.sh_off + is];
-  __shared__ double s_th[kWpolLds];
-  __shared__ int s_iw[kWpolLds], s_rank[kWpolBlock];
-  __shared__ int s_n;
-  __shared__ float s_corr;
-  __shared__ double s_red[kWpolSum / 64];
+  double *s_th = L.th, *s_red = L.red;
+  int *s_iw = L.iw, *s_rank = L.rank;
+  int& s_n = L.n;
+  float& s_corr = L.corr;
   const int t = threadIdx.x;
   // theta_corr follows the shell's mean theta every 100 steps; only the
   // pot_energy calls of the run (MD steps and the final evaluation) advance
@@ -2341,6 +2391,71 @@ __global__ void __launch_bounds__(kWpolBlock) k_watpol(Dev d) {
     }
     wave_energy(d.ws, w, E_WPOL, e, on && en);
   }
+}
+template <int kWpolBlock>
+__global__ void __launch_bounds__(kWpolBlock) k_watpol(Dev d) {
+  __shared__ WpolLds<kWpolBlock> L;
+  watpol_block<kWpolBlock>(d, blockIdx.x, L);
+}
+
+// ------------------------------------------------ all forces at once --
+// Engines whose step is too small to fill the GPU run every force kernel of a
+// step as one launch, each block taking one kind of work (by block index, the
+// longest kinds first): a step then takes as long as its slowest kind, where
+// separate launches, on three streams, add up with the gaps between them.
+// us a step, separate and one launch: one ligand-in-water window 75 and 53, one
+// protein window 107 and 74, 11 small windows 97 and 68, 8 protein windows 161
+// and 133.  128 registers (the bonded terms spill 42) keep two blocks on a CU;
+// with twice as many the 8 windows take 162.
+constexpr int kAllBlock = 512;       // 8 waves: two q items, 8 row clusters
+// an engine of more blocks fills the GPU with separate launches, whose pair
+// kernels have more waves in flight: 16 + 16 windows (3400 blocks) 274 and
+// 270, 64 small windows (3200) 221 and 206, 32 protein windows (5300) 406 and
+// 440.  The results do not depend on it
+constexpr int kAllMost = 3500;
+struct AllPlan {
+  int wpol, bonded, qp, qw, srow, wrow, qq, rst, terms;   // first block of each kind
+  int total;
+};
+static AllPlan all_plan(const Dev& d, bool energy, bool terms) {
+  AllPlan p;
+  int n = 0;
+  auto take = [&](int& first, long long work, int per_block) {
+    first = n;
+    n += (int)((work + per_block - 1) / per_block);
+  };
+  const int waves = kAllBlock / 64;
+  take(p.wpol, d.nwat_total ? (long long)d.nwin * kWpolMaxShell : 0, 1);
+  take(p.bonded, d.nbtile, 1);
+  take(p.qp, d.nqp_work, waves / kQWaves);
+  take(p.qw, d.nqw_work, waves / kQWaves);
+  take(p.srow, d.rl[T_PP].nicl, waves);
+  take(p.wrow, d.rl[T_WW].nicl, waves);
+  take(p.qq, qq_waves(d, energy), waves);
+  take(p.rst, d.nrst, waves);
+  take(p.terms, terms ? d.ntot : 0, kAllBlock);
+  p.total = n;
+  return p;
+}
+template <bool W3, bool EK>
+__global__ void __launch_bounds__(kAllBlock, 4) k_all(Dev d, AllPlan p) {
+  __shared__ union {
+    WpolLds<kAllBlock> wpol;
+    struct { unsigned long long acc[3 * kBondSpan], e[E_NSLOT]; } bonded;
+    double q[kAllBlock / (64 * kQWaves)][9 * 64 * kQWaves];
+  } L;
+  const int b = blockIdx.x, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  constexpr int kWaves = kAllBlock / 64, kItems = kWaves / kQWaves;
+  const int group = wv / kQWaves;
+  if (b >= p.terms) return atom_terms<true>(d, (b - p.terms) * kAllBlock + (int)threadIdx.x);
+  if (b >= p.rst) return prestr_wave(d, (b - p.rst) * kWaves + wv);
+  if (b >= p.qq) return qq_wave<EK>(d, (b - p.qq) * kWaves + wv);
+  if (b >= p.wrow) return wrow_wave<W3, EK, 3>(d, (b - p.wrow) * kWaves + wv);
+  if (b >= p.srow) return srow_wave<W3, EK>(d, (b - p.srow) * kWaves + wv);
+  if (b >= p.qw) return qw_group<W3, EK>(d, (b - p.qw) * kItems + group, L.q[group]);
+  if (b >= p.qp) return qp_group<EK>(d, (b - p.qp) * kItems + group, L.q[group]);
+  if (b >= p.bonded) return bonded_tile(d, b - p.bonded, L.bonded.acc, L.bonded.e);
+  watpol_block<kAllBlock>(d, b, L.wpol);
 }
 
 // the FP32 coordinates of atom i from its FP64 ones, into x32 and, for a
@@ -2715,19 +2830,9 @@ static void launch_list_prep(const Dev& d, hipStream_t s, int ngrp, int nwc, int
   k_centres<<<blocks(ngrp, 128), 128, 0, s>>>(d, ngrp);
   k_bounds<<<blocks(nwc + nsc, 128), 128, 0, s>>>(d, nwc, nsc);
 }
-// the rows whose i-clusters are waters (water-water, water<-solute), and
-// those whose i-clusters are solute (solute<-water, solute-solute)
-static void launch_rows_water(const Dev& d, hipStream_t s) {
-  if (d.rl[T_WW].nicl) k_build_rows<T_WW><<<blocks((long long)d.rl[T_WW].nicl * 64, 256), 256, 0, s>>>(d);
-  if (d.rl[T_WP].nicl) k_build_rows<T_WP><<<blocks((long long)d.rl[T_WP].nicl * 64, 256), 256, 0, s>>>(d);
-}
-static void launch_rows_solute(const Dev& d, hipStream_t s) {
-  if (d.rl[T_PW].nicl) k_build_rows<T_PW><<<blocks((long long)d.rl[T_PW].nicl * 64, 256), 256, 0, s>>>(d);
-  if (d.rl[T_PP].nicl) k_build_rows<T_PP><<<blocks((long long)d.rl[T_PP].nicl * 64, 256), 256, 0, s>>>(d);
-}
 static void launch_list_rows(const Dev& d, hipStream_t s) {
-  launch_rows_water(d, s);
-  launch_rows_solute(d, s);
+  const int nb = 2 * (blocks(d.rl[T_PP].nicl, 4) + blocks(d.rl[T_WW].nicl, 4));
+  if (nb) k_build_rows<<<nb, 256, 0, s>>>(d);
 }
 void launch_lists(const Dev& d, hipStream_t s, int ngrp, int nwc, int nsc) {
   launch_list_prep(d, s, ngrp, nwc, nsc);
@@ -2822,8 +2927,45 @@ void launch_other_forces(const Dev& d, hipStream_t s, bool atom_terms) {
 // The kernels write the energies and the shared gradient only through integer
 // atomic adds, and everything else to buffers of their own, which the
 // integrator adds, so the result does not depend on how they overlap.
+static bool launch_all(const Dev& d, hipStream_t s, bool energy, bool terms) {
+  const AllPlan p = all_plan(d, energy, terms);
+  if (!p.total) return true;
+  if (d.any_wat3) {
+    if (energy) k_all<true, true><<<p.total, kAllBlock, 0, s>>>(d, p);
+    else k_all<true, false><<<p.total, kAllBlock, 0, s>>>(d, p);
+  } else {
+    if (energy) k_all<false, true><<<p.total, kAllBlock, 0, s>>>(d, p);
+    else k_all<false, false><<<p.total, kAllBlock, 0, s>>>(d, p);
+  }
+  return true;
+}
+bool small_engine(const Dev& d, bool mixed_solvent) { return !mixed_solvent && all_plan(d, true, true).total <= kAllMost; }
+
+// the lists and forces of a small engine: one launch for the forces, and on
+// list steps the LRF expansions beside the rows and the forces
+static hipError_t launch_small_forces(const Dev& d, hipStream_t s, hipStream_t s2, const hipEvent_t ev[5], bool lists,
+                                      int ngrp, int nwc, int nsc, bool energy) {
+  launch_offdiag(d, s);
+  if (!lists) {
+    launch_all(d, s, energy, true);
+    return hipSuccess;
+  }
+  launch_list_prep(d, s, ngrp, nwc, nsc);
+  hipError_t err = hipEventRecord(ev[0], s);
+  if (err == hipSuccess) err = hipStreamWaitEvent(s2, ev[0], 0);
+  if (err != hipSuccess) return err;
+  launch_lrf_build(d, s2);
+  launch_atom_terms(d, s2);
+  err = hipEventRecord(ev[1], s2);
+  if (err != hipSuccess) return err;
+  launch_list_rows(d, s);
+  launch_all(d, s, energy, false);
+  return hipStreamWaitEvent(s, ev[1], 0);
+}
+
 hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, hipStream_t s3, const hipEvent_t ev[5],
                               bool lists, int ngrp, int nwc, int nsc, bool q_energy) {
+  if (d.small) return launch_small_forces(d, s, s2, ev, lists, ngrp, nwc, nsc, q_energy);
   hipError_t err = hipEventRecord(ev[0], s);
   if (err == hipSuccess) err = hipStreamWaitEvent(s2, ev[0], 0);
   if (err == hipSuccess && !lists) err = hipStreamWaitEvent(s3, ev[0], 0);
@@ -2831,11 +2973,10 @@ hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, hipSt
   launch_offdiag(d, s2);
   if (lists) {
     launch_list_prep(d, s, ngrp, nwc, nsc);
+    launch_list_rows(d, s);
     err = hipEventRecord(ev[2], s);
     if (err == hipSuccess) err = hipStreamWaitEvent(s3, ev[2], 0);
     if (err != hipSuccess) return err;
-    launch_rows_solute(d, s3);
-    launch_rows_water(d, s);
   }
   launch_watpol(d, s2);
   launch_qq(d, s2, q_energy);
