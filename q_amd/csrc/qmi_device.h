@@ -215,6 +215,7 @@ struct Dev {
   const float4* qcw_h;
   int any_wat3;          // some window has a 3-atom solvent
   int small;             // a step's force kernels run as one launch
+  int any_lrf;           // some window uses LRF
   // the same in FP64 for the energy terms: A, B, soft-core term, charge
   // product of member, state and water atom ([(m * kMaxS + s) * 3 + k])
   const double4* qcw_e;

@@ -1263,7 +1263,10 @@ static int build_device(qmi_engine* e) {
   if ((rc = make_rows(T_PW, sc_win)) != 0) return rc;
   if ((rc = make_rows(T_PP, sc_win)) != 0) return rc;
   bool all3 = true;
-  for (int wi = 0; wi < NW; ++wi) all3 = all3 && wd[wi].wat3;
+  for (int wi = 0; wi < NW; ++wi) {
+    all3 = all3 && wd[wi].wat3;
+    d.any_lrf |= wd[wi].use_lrf;
+  }
   d.small = small_engine(d, d.any_wat3 && !all3) ? 1 : 0;
   return 0;
 }
@@ -1452,6 +1455,7 @@ int qmi_window_add(qmi_engine* e, const char* inp_path, long long seed_override,
 // pair or term, so the choice does not change results.
 static int autotune(qmi_engine* e) {
   Dev& d = e->d;
+  if (d.small) return 0;   // the step's one launch has no shapes to choose
   hipEvent_t t0, t1;
   HIP_OK(hipEventCreate(&t0));
   HIP_OK(hipEventCreate(&t1));
@@ -1822,7 +1826,7 @@ int qmi_run(qmi_engine* e, long long nsteps, int finalize) {
     const bool lists = variant & 1, qen = variant & 2;
     // lists and forces on three streams; a failure here fails the capture
     if (launch_step_forces(e->d, e->stream, e->side_stream[0], e->side_stream[1], e->step_ev, lists, e->ngrp, e->nwc,
-                           e->nsc, qen) != hipSuccess)
+                           e->nsc, qen, false) != hipSuccess)
       return;
     launch_integrate(e->d, e->stream, e->shake_any, variant);
   };
@@ -1956,7 +1960,7 @@ int qmi_run(qmi_engine* e, long long nsteps, int finalize) {
       if (e->timing_on) HIP_OK(hipEventRecord(e->ev[2], e->stream));
       launch_nonbonded(e->d, e->stream, false, qen);
       if (e->timing_on) HIP_OK(hipEventRecord(e->ev[3], e->stream));
-      launch_other_forces(e->d, e->stream, false);
+      launch_other_forces(e->d, e->stream);
       if (e->timing_on) HIP_OK(hipEventRecord(e->ev[4], e->stream));
       launch_atom_terms(e->d, e->stream);
       launch_integrate(e->d, e->stream, e->shake_any, 1 | (qen ? 2 : 0));
@@ -2117,9 +2121,8 @@ int qmi_evaluate(qmi_engine* e, int rebuild_lists) {
 static int evaluate(qmi_engine* e, int rebuild_lists, int mode) {
   HIP_OK(hipSetDevice(e->device));
   launch_begin(e->d, e->stream, mode, rebuild_lists ? 1 : 0);
-  launch_lists(e->d, e->stream, e->ngrp, e->nwc, e->nsc);
-  launch_nonbonded(e->d, e->stream);
-  launch_other_forces(e->d, e->stream);
+  HIP_OK(launch_step_forces(e->d, e->stream, e->side_stream[0], e->side_stream[1], e->step_ev, rebuild_lists != 0,
+                            e->ngrp, e->nwc, e->nsc, true, true));
   HIP_OK(hipGetLastError());
   const int NW = (int)e->wins.size();
   std::vector<WinState> ws(NW);

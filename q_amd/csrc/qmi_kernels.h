@@ -19,16 +19,16 @@ void launch_q(const Dev& d, hipStream_t s, bool energy = true);
 void launch_lrf_build(const Dev& d, hipStream_t s);
 void launch_bonded(const Dev& d, hipStream_t s);
 void launch_nonbonded(const Dev& d, hipStream_t s, bool with_ww = true, bool q_energy = true);
-// atom_terms false: the per-atom terms (LRF evaluation, fixed/shell and
-// radial solvent restraints) are left to launch_atom_terms
-void launch_other_forces(const Dev& d, hipStream_t s, bool atom_terms = true);
+// water polarisation, bonded terms and restraint records
+void launch_other_forces(const Dev& d, hipStream_t s);
 // the per-atom terms of an MD step into their own array (Dev::fterm)
 void launch_atom_terms(const Dev& d, hipStream_t s);
 // whether a step's force kernels run as one launch (Dev::small)
 bool small_engine(const Dev& d, bool mixed_solvent);
-// the lists and forces of an MD step on three streams (see the definition)
+// the lists and forces of an MD step or (eval) of an evaluation on three
+// streams (see the definition)
 hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, hipStream_t s3, const hipEvent_t ev[5],
-                              bool lists, int ngrp, int nwc, int nsc, bool q_energy);
+                              bool lists, int ngrp, int nwc, int nsc, bool q_energy, bool eval);
 // the end of an MD step; the gradient is completed with the per-atom terms
 // of launch_atom_terms, which must have run in the same step
 // variant: bit 0 the step's list kernels were launched, bit 1 its energy terms

@@ -2900,13 +2900,18 @@ static void launch_watpol(const Dev& d, hipStream_t s) {
   if (d.nwin <= kWpolWide) k_watpol<1024><<<d.nwin * kWpolMaxShell, 1024, 0, s>>>(d);
   else k_watpol<256><<<d.nwin * kWpolMaxShell, 256, 0, s>>>(d);
 }
-void launch_other_forces(const Dev& d, hipStream_t s, bool atom_terms) {
+void launch_other_forces(const Dev& d, hipStream_t s) {
   launch_watpol(d, s);
   launch_bonded(d, s);
-  if (atom_terms && d.ntot) k_atom_terms<false><<<blocks(d.ntot, 256), 256, 0, s>>>(d);   // last: completes the gradient
+}
+// the per-atom terms of an evaluation, after all its other kernels: completes
+// the gradient
+static void launch_complete(const Dev& d, hipStream_t s) {
+  if (d.ntot) k_atom_terms<false><<<blocks(d.ntot, 256), 256, 0, s>>>(d);
 }
 
-// The lists and forces of an MD step on three streams (after k_begin on s):
+// The lists and forces of an MD step, or of an evaluation (eval: the per-atom
+// terms come last and complete the gradient), on three streams:
 //   s:  on list steps the group centres and the water rows; then the water
 //       rows' forces, the per-atom terms, and the q-atoms against solute;
 //   s2: water polarisation (few latency-bound blocks, which start beside the
@@ -2927,9 +2932,9 @@ void launch_other_forces(const Dev& d, hipStream_t s, bool atom_terms) {
 // The kernels write the energies and the shared gradient only through integer
 // atomic adds, and everything else to buffers of their own, which the
 // integrator adds, so the result does not depend on how they overlap.
-static bool launch_all(const Dev& d, hipStream_t s, bool energy, bool terms) {
+static void launch_all(const Dev& d, hipStream_t s, bool energy, bool terms) {
   const AllPlan p = all_plan(d, energy, terms);
-  if (!p.total) return true;
+  if (!p.total) return;
   if (d.any_wat3) {
     if (energy) k_all<true, true><<<p.total, kAllBlock, 0, s>>>(d, p);
     else k_all<true, false><<<p.total, kAllBlock, 0, s>>>(d, p);
@@ -2937,40 +2942,46 @@ static bool launch_all(const Dev& d, hipStream_t s, bool energy, bool terms) {
     if (energy) k_all<false, true><<<p.total, kAllBlock, 0, s>>>(d, p);
     else k_all<false, false><<<p.total, kAllBlock, 0, s>>>(d, p);
   }
-  return true;
 }
 bool small_engine(const Dev& d, bool mixed_solvent) { return !mixed_solvent && all_plan(d, true, true).total <= kAllMost; }
 
 // the lists and forces of a small engine: one launch for the forces, and on
 // list steps the LRF expansions beside the rows and the forces
 static hipError_t launch_small_forces(const Dev& d, hipStream_t s, hipStream_t s2, const hipEvent_t ev[5], bool lists,
-                                      int ngrp, int nwc, int nsc, bool energy) {
-  launch_offdiag(d, s);
-  if (!lists) {
-    launch_all(d, s, energy, true);
-    return hipSuccess;
+                                      int ngrp, int nwc, int nsc, bool energy, bool eval) {
+  if (!eval) launch_offdiag(d, s);
+  if (lists) {
+    launch_list_prep(d, s, ngrp, nwc, nsc);
+    if (d.any_lrf) {
+      hipError_t err = hipEventRecord(ev[0], s);
+      if (err == hipSuccess) err = hipStreamWaitEvent(s2, ev[0], 0);
+      if (err != hipSuccess) return err;
+      launch_lrf_build(d, s2);
+      if (!eval) launch_atom_terms(d, s2);
+      err = hipEventRecord(ev[1], s2);
+      if (err != hipSuccess) return err;
+    }
+    launch_list_rows(d, s);
+    launch_all(d, s, energy, !eval && !d.any_lrf);
+    if (d.any_lrf) {
+      hipError_t err = hipStreamWaitEvent(s, ev[1], 0);
+      if (err != hipSuccess) return err;
+    }
+  } else {
+    launch_all(d, s, energy, !eval);
   }
-  launch_list_prep(d, s, ngrp, nwc, nsc);
-  hipError_t err = hipEventRecord(ev[0], s);
-  if (err == hipSuccess) err = hipStreamWaitEvent(s2, ev[0], 0);
-  if (err != hipSuccess) return err;
-  launch_lrf_build(d, s2);
-  launch_atom_terms(d, s2);
-  err = hipEventRecord(ev[1], s2);
-  if (err != hipSuccess) return err;
-  launch_list_rows(d, s);
-  launch_all(d, s, energy, false);
-  return hipStreamWaitEvent(s, ev[1], 0);
+  if (eval) launch_complete(d, s);
+  return hipSuccess;
 }
 
 hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, hipStream_t s3, const hipEvent_t ev[5],
-                              bool lists, int ngrp, int nwc, int nsc, bool q_energy) {
-  if (d.small) return launch_small_forces(d, s, s2, ev, lists, ngrp, nwc, nsc, q_energy);
+                              bool lists, int ngrp, int nwc, int nsc, bool q_energy, bool eval) {
+  if (d.small) return launch_small_forces(d, s, s2, ev, lists, ngrp, nwc, nsc, q_energy, eval);
   hipError_t err = hipEventRecord(ev[0], s);
   if (err == hipSuccess) err = hipStreamWaitEvent(s2, ev[0], 0);
   if (err == hipSuccess && !lists) err = hipStreamWaitEvent(s3, ev[0], 0);
   if (err != hipSuccess) return err;
-  launch_offdiag(d, s2);
+  if (!eval) launch_offdiag(d, s2);
   if (lists) {
     launch_list_prep(d, s, ngrp, nwc, nsc);
     launch_list_rows(d, s);
@@ -2986,7 +2997,7 @@ hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, hipSt
   launch_srow(d, s3, q_energy);
   err = hipEventRecord(ev[1], s3);
   if (err != hipSuccess) return err;
-  if (!lists) launch_atom_terms(d, s);
+  if (!lists && !eval) launch_atom_terms(d, s);
   launch_qp(d, s, q_energy);
   if (lists) {
     err = hipEventRecord(ev[4], s);
@@ -2994,11 +3005,12 @@ hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, hipSt
     if (err == hipSuccess) err = hipStreamWaitEvent(s2, ev[1], 0);
     if (err != hipSuccess) return err;
     launch_lrf_build(d, s2);
-    launch_atom_terms(d, s2);
+    if (!eval) launch_atom_terms(d, s2);
   }
   err = hipEventRecord(ev[3], s2);
   if (err == hipSuccess) err = hipStreamWaitEvent(s, ev[1], 0);
   if (err == hipSuccess) err = hipStreamWaitEvent(s, ev[3], 0);
+  if (err == hipSuccess && eval) launch_complete(d, s);
   return err;
 }
 
