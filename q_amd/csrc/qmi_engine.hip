@@ -1251,10 +1251,12 @@ static int build_device(qmi_engine* e) {
     for (int wi = 0; wi < NW; ++wi) maxj = std::max(maxj, kCl * (jw ? wd[wi].nwc : wd[wi].nsc));
     const int need = max_rows(tt);
     int cap = std::min(maxj, ((int)(1.3 * need) + 24 + 7) / 8 * 8);
-    L.cap = std::max(cap, 8);
+    // whole passes of the row kernels (4 entries a lane), which load a pass
+    // without looking at the row's length
+    L.cap = (std::max(cap, 8) + 31) / 32 * 32;
     int r;
     if ((r = dev_alloc(e, &L.cnt, (size_t)kCl * std::max(1, L.nicl))) != 0) return r;
-    if ((r = dev_alloc(e, &L.ent, (size_t)kCl * std::max(1, L.nicl) * L.cap)) != 0) return r;
+    if ((r = dev_alloc(e, &L.ent, (size_t)kCl * std::max(1, L.nicl) * L.cap + kCl)) != 0) return r;
     HIP_OK(hipMemset(L.cnt, 0, sizeof(int) * kCl * std::max(1, L.nicl)));
     return 0;
   };

@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "qmi_device.h"
 #include "qmi_kernels.h"
@@ -474,14 +475,24 @@ struct RowGrad {
   long long lo = 0, hi = 0;
   template <int N>
   __device__ __forceinline__ void add(const float* g, int b) {
-    double s[N];
+    if constexpr (N == 3) {
+      const double x = row8_sum((double)g[0]), y = row8_sum((double)g[1]), z = row8_sum((double)g[2]);
+      lo += fix(b == 0 ? x : b == 1 ? y : z, kFScale);
+    } else {
+      // each step halves the components a lane sums: after the step with
+      // lane l ^ m a lane holds those whose index agrees with its own in the
+      // bit m (the step of 4 by the mirrored lane, which differs in that bit)
+      const bool b4 = b & 4, b1 = b & 1, b2 = b & 2;
+      double s4[4], s2[2];
 #pragma unroll
-    for (int k = 0; k < N; ++k) s[k] = row8_sum((double)g[k]);
-    double v = s[0];
+      for (int k = 0; k < 4; ++k)
+        s4[k] = (double)(b4 ? g[k + 4] : g[k]) + (double)mv<kDppHalfMirror>(b4 ? g[k] : g[k + 4]);
 #pragma unroll
-    for (int k = 1; k < (N < 8 ? N : 8); ++k) v = b == k ? s[k] : v;
-    lo += fix(v, kFScale);
-    if constexpr (N == 9) hi += fix(s[8], kFScale);
+      for (int k = 0; k < 2; ++k)
+        s2[k] = (b1 ? s4[2 * k + 1] : s4[2 * k]) + mv<kDppXor1>(b1 ? s4[2 * k] : s4[2 * k + 1]);
+      lo += fix((b2 ? s2[1] : s2[0]) + mv<kDppXor2>(b2 ? s2[0] : s2[1]), kFScale);
+      hi += fix(row8_sum((double)g[8]), kFScale);
+    }
   }
 };
 
@@ -526,36 +537,36 @@ __device__ __forceinline__ void ww_impl(const Dev& d, int wave, RowGrad& rg) {
   double xi[9];
   if (en)
     for (int k = 0; k < 9; ++k) xi[k] = oa >= 0 ? d.x[3 * oa + k] : 0.0;
-  const int* ent = L.ent + (size_t)row * L.cap;
+  const int* ent = L.ent + (size_t)row * L.cap + b;
   // entries are water slots: the members of a neighbouring cluster are
   // contiguous in xw, so the 8 lanes of a row mostly read the same lines.
   // The next entry's slot and coordinates are loaded while the current one
-  // is evaluated (entries past the row end read slot 0 and are skipped)
-  int ob_next = ent[min(b, L.cap - 1)];
-  ob_next = b < n ? ob_next : 0;
+  // is evaluated (entries past the row end read slot 0 and are skipped; the
+  // table has kCl entries beyond its last row)
+  const int e0 = ent[0];
+  unsigned ob_next = b < n ? e0 : 0;
   float4 nx[3];
-  for (int s = 0; s < 3; ++s) nx[s] = d.xw[3 * ob_next + s];
+  for (int s = 0; s < 3; ++s) nx[s] = d.xw[3ull * ob_next + s];
   for (int t = 0; t < nch; ++t) {
     const int k = t * kCl + b;
-    const int ob = ob_next;
+    const unsigned ob = ob_next;
     float3 pj[3];
     for (int s = 0; s < 3; ++s) pj[s] = make_float3(nx[s].x, nx[s].y, nx[s].z);
     {
-      const int kn = k + kCl;
-      const int e = ent[min(kn, L.cap - 1)];   // in the row, so the load needs no branch
-      ob_next = kn < n ? e : 0;
-      for (int s = 0; s < 3; ++s) nx[s] = d.xw[3 * ob_next + s];
+      const int e = ent[(t + 1) * kCl];
+      ob_next = k + kCl < n ? e : 0;
+      for (int s = 0; s < 3; ++s) nx[s] = d.xw[3ull * ob_next + s];
     }
     if (k >= n) continue;
     // each unordered pair counted once, from the row with the lower slot: a
     // row's entries ascend in slot order, so the counted ones are a suffix
     // of the row and the 8 rows of the wave (consecutive slots) switch at
     // nearly the same place, which keeps the FP64 block from diverging
-    const bool cnt = en && row < ob;
+    const bool cnt = en && row < (int)ob;
     if (cnt) {
       double xj[9];
       for (int m = 0; m < 3; ++m) {
-        const double4 q = d.xwd[3 * ob + m];
+        const double4 q = d.xwd[3ull * ob + m];
         xj[3 * m] = q.x; xj[3 * m + 1] = q.y; xj[3 * m + 2] = q.z;
       }
       for (int p = 0; p < 3; ++p)
@@ -628,7 +639,6 @@ __device__ __forceinline__ void pw_impl(const Dev& d, int wave, RowGrad& rg) {
     if (ea >= 0) ljs = d.ljp[ea];
   }
   constexpr bool en = EN && !WATER_SIDE;
-  const bool arith = W.arith;
   constexpr bool wat3 = W3;
   float g[9];
   for (int k = 0; k < 9; ++k) g[k] = 0.f;
@@ -640,78 +650,76 @@ __device__ __forceinline__ void pw_impl(const Dev& d, int wave, RowGrad& rg) {
     for (int c = 0; c < 3; ++c) xs[c] = d.x[3 * ea + c];
     const double* tl = &d.t_lj[(size_t)(W.t_off + d.iac[ea]) * 4];
     for (int k = 0; k < (wat3 ? 3 : 1); ++k)
-      lj_ab(tl[0], tl[1], k == 0 ? W.aO1d : W.awd[k], k == 0 ? W.bO1d : W.bwd[k], arith, &Ad[k], &Bd[k]);
+      lj_ab(tl[0], tl[1], k == 0 ? W.aO1d : W.awd[k], k == 0 ? W.bO1d : W.bwd[k], W.arith, &Ad[k], &Bd[k]);
   }
-  const int* ent = L.ent + (size_t)row * L.cap;
-  // kUnroll entries per pass, loads first (as in k_pp)
-  for (int t0 = 0; t0 < nch; t0 += kUnroll) {
-    int e[kUnroll];
-    bool v[kUnroll];
+  const int* ent = L.ent + (size_t)row * L.cap + b;
+  // kUnroll entries per pass, loads first (as in pp_impl)
+  auto rows = [&](auto AR) {
+    constexpr bool arith = AR;
+    for (int t0 = 0; t0 < nch; t0 += kUnroll) {
+      unsigned e[kUnroll];
+      bool v[kUnroll];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const int kk = (t0 + u) * kCl + b;
-      v[u] = kk < n;
-      const int le = ent[min(kk, L.cap - 1)];   // in the row, so the load needs no branch
-      e[u] = v[u] ? le : 0;
-    }
-    float4 ld[kUnroll][3];
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      if (WATER_SIDE) {
-        ld[u][0] = d.x32[e[u]];
-        ld[u][1] = d.ljp[e[u]];
-      } else {
-        // water slots (contiguous per cluster)
-        ld[u][0] = d.xw[3 * e[u]]; ld[u][1] = d.xw[3 * e[u] + 1]; ld[u][2] = d.xw[3 * e[u] + 2];
+      for (int u = 0; u < kUnroll; ++u) {
+        v[u] = (t0 + u) * kCl + b < n;
+        const int le = ent[(t0 + u) * kCl];
+        e[u] = v[u] ? le : 0;
       }
-    }
+      float4 ld[kUnroll][3];
+      float2 lt[kUnroll];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      float4 ps, pw[3];
-      float4 lj;
-      if (WATER_SIDE) {
-        ps = ld[u][0]; lj = ld[u][1];
-        pw[0] = pi[0]; pw[1] = pi[1]; pw[2] = pi[2];
-      } else {
-        ps = pi[0]; lj = ljs;
-        pw[0] = ld[u][0]; pw[1] = ld[u][1]; pw[2] = ld[u][2];
-      }
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        // dx = x(water atom) - x(solute atom), as nonbond_pw with i solute, j water
-        float dx = pw[k].x - ps.x, dy = pw[k].y - ps.y, dz = pw[k].z - ps.z;
-        const float r2 = r2_f(dx, dy, dz);
-        float rinv = rsq_r2(r2);
-        float r2inv = rinv * rinv;
-        const float qq = ps.w * pw[k].w;
-        float dv;
-        if (k == 0 || wat3) {
-          float r6 = r2inv * r2inv * r2inv;
-          float A, B;
-          lj_ab(lj.x, lj.y, k == 0 ? W.aO1 : W.aw[k], k == 0 ? W.bO1 : W.bw[k], arith, &A, &B);
-          dv = pair_dv<!W3 && !en>(r2inv, rinv, qq, A * r6 * r6, B * r6);
+      for (int u = 0; u < kUnroll; ++u) {
+        if (WATER_SIDE) {
+          ld[u][0] = d.x32[e[u]];
+          lt[u] = *(const float2*)&d.ljp[e[u]];
         } else {
-          dv = r2inv * (-(qq * rinv));
+          // water slots (contiguous per cluster)
+          const float4* xe = d.xw + 3ull * e[u];
+          ld[u][0] = xe[0]; ld[u][1] = xe[1]; ld[u][2] = xe[2];
         }
+      }
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) {
+        const float4 ps = WATER_SIDE ? ld[u][0] : pi[0];
+        const float2 lj = WATER_SIDE ? lt[u] : make_float2(ljs.x, ljs.y);
         if (!v[u]) continue;
-        if (en) {
-          const double4 xa = d.xwd[3 * e[u] + k];   // the water atom of the slot, FP64
-          const double ddx = xa.x - xs[0], ddy = xa.y - xs[1], ddz = xa.z - xs[2];
-          const double rinv_d = rsqrt_e(ddx * ddx + ddy * ddy + ddz * ddz);
-          eel += (double)(ps.w * pw[k].w) * rinv_d;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const float4 pw = WATER_SIDE ? pi[k] : ld[u][k];
+          // dx = x(water atom) - x(solute atom), as nonbond_pw with i solute, j water
+          const float dx = pw.x - ps.x, dy = pw.y - ps.y, dz = pw.z - ps.z;
+          const float rinv = rsq_r2(r2_f(dx, dy, dz)), r2inv = rinv * rinv;
+          const float qq = ps.w * pw.w;
+          float dv;
           if (k == 0 || wat3) {
-            const double r2i = rinv_d * rinv_d, r6d = r2i * r2i * r2i;
-            evdw += Ad[k] * r6d * r6d - Bd[k] * r6d;
+            const float r6 = r2inv * r2inv * r2inv;
+            float A, B;
+            lj_ab(lj.x, lj.y, k == 0 ? W.aO1 : W.aw[k], k == 0 ? W.bO1 : W.bw[k], arith, &A, &B);
+            dv = pair_dv<!W3 && !en>(r2inv, rinv, qq, A * r6 * r6, B * r6);
+          } else {
+            dv = r2inv * (-(qq * rinv));
           }
+          if (en) {
+            const double4 xa = d.xwd[3ull * e[u] + k];   // the water atom of the slot, FP64
+            const double ddx = xa.x - xs[0], ddy = xa.y - xs[1], ddz = xa.z - xs[2];
+            const double rinv_d = rsqrt_e(ddx * ddx + ddy * ddy + ddz * ddz);
+            eel += (double)qq * rinv_d;
+            if (k == 0 || wat3) {
+              const double r2i = rinv_d * rinv_d, r6d = r2i * r2i * r2i;
+              evdw += Ad[k] * r6d * r6d - Bd[k] * r6d;
+            }
+          }
+          const float sd = WATER_SIDE ? dv : -dv;
+          const int o = WATER_SIDE ? 3 * k : 0;
+          g[o] = __builtin_fmaf(sd, dx, g[o]);
+          g[o + 1] = __builtin_fmaf(sd, dy, g[o + 1]);
+          g[o + 2] = __builtin_fmaf(sd, dz, g[o + 2]);
         }
-        const float sd = WATER_SIDE ? dv : -dv;
-        const int o = WATER_SIDE ? 3 * k : 0;
-        g[o] = __builtin_fmaf(sd, dx, g[o]);
-        g[o + 1] = __builtin_fmaf(sd, dy, g[o + 1]);
-        g[o + 2] = __builtin_fmaf(sd, dz, g[o + 2]);
       }
     }
-  }
+  };
+  if (W.arith) rows(std::true_type{});
+  else rows(std::false_type{});
   rg.add<WATER_SIDE ? 9 : 3>(g, b);
   if (en) {
     eel = wave_sum(eel);
@@ -739,7 +747,6 @@ __device__ __forceinline__ void pp_impl(const Dev& d, int wave, RowGrad& rg) {
   const int nch = row_chunks(n);
   const float4 pi = ea >= 0 ? d.x32[ea] : make_float4(0, 0, 0, 0);
   const float4 li = ea >= 0 ? d.ljp[ea] : make_float4(0, 0, 0, 0);
-  const bool arith = W.arith;
   constexpr bool en = EN;
   float g0 = 0.f, g1 = 0.f, g2 = 0.f;
   double eel = 0.0, evdw = 0.0;
@@ -751,43 +758,46 @@ __device__ __forceinline__ void pp_impl(const Dev& d, int wave, RowGrad& rg) {
     for (int c = 0; c < 3; ++c) xs[c] = d.x[3 * ea + c];
     tli = &d.t_lj[(size_t)(W.t_off + d.iac[ea]) * 4];
   }
-  const int* ent = L.ent + (size_t)row * L.cap;
+  const int* ent = L.ent + (size_t)row * L.cap + b;
   // kUnroll entries per pass: all their loads are issued before the
-  // arithmetic; entries past the row end read atom 0 and are masked, and
-  // the sums run in entry order as in a plain loop
-  for (int t = 0; t < nch; t += kUnroll) {
-    int e[kUnroll];
-    bool v[kUnroll];
+  // arithmetic (a row's capacity is a multiple of the entries of a pass, so
+  // they need no branch); entries past the row end read atom 0 and are
+  // masked, and the sums run in entry order as in a plain loop.  The LJ
+  // columns of a 1-4 pair are the second half of the atom's record.
+  auto rows = [&](auto AR) {
+    constexpr bool arith = AR;
+    const float lx = li.x, ly = li.y, l14x = li.z, l14y = li.w;
+    for (int t = 0; t < nch; t += kUnroll) {
+      unsigned e[kUnroll];
+      bool v[kUnroll], is14[kUnroll];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const int kk = (t + u) * kCl + b;
-      v[u] = kk < n;
-      const int ld = ent[min(kk, L.cap - 1)];   // in the row, so the load needs no branch
-      e[u] = v[u] ? ld : 0;
-    }
-    float4 pj[kUnroll], lj[kUnroll];
+      for (int u = 0; u < kUnroll; ++u) {
+        v[u] = (t + u) * kCl + b < n;
+        const int ld = ent[(t + u) * kCl];
+        const int eu = v[u] ? ld : 0;
+        is14[u] = (eu & kRow14) != 0;
+        e[u] = eu & ~kRow14;
+      }
+      float4 pj[kUnroll];
+      float2 lj[kUnroll];
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      pj[u] = d.x32[e[u] & ~kRow14];
-      lj[u] = d.ljp[e[u] & ~kRow14];
-    }
+      for (int u = 0; u < kUnroll; ++u) {
+        pj[u] = d.x32[e[u]];
+        lj[u] = ((const float2*)d.ljp)[2ull * e[u] + is14[u]];
+      }
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const bool is14 = (e[u] & kRow14) != 0;
-      const int eb = e[u] & ~kRow14;
-      float dx = pj[u].x - pi.x, dy = pj[u].y - pi.y, dz = pj[u].z - pi.z;
-      const float r2 = r2_f(dx, dy, dz);
-      float rinv = rsq_r2(r2);
-      float r2inv = rinv * rinv;
-      float r6 = r2inv * r2inv * r2inv;
-      float vel = (pi.w * pj[u].w) * rinv;
-      float aa, bb;
-      if (is14) { vel *= W.el14; lj_ab(li.z, li.w, lj[u].z, lj[u].w, arith, &aa, &bb); }
-      else lj_ab(li.x, li.y, lj[u].x, lj[u].y, arith, &aa, &bb);
-      const float va = r6 * r6 * aa, vb = r6 * bb;
-      const float dv = r2inv * __builtin_fmaf(6.f, vb, __builtin_fmaf(va, -12.f, -vel));
-      if (v[u]) {
+      for (int u = 0; u < kUnroll; ++u) {
+        const float dx = pj[u].x - pi.x, dy = pj[u].y - pi.y, dz = pj[u].z - pi.z;
+        const float rinv = rsq_r2(r2_f(dx, dy, dz)), r2inv = rinv * rinv;
+        const float r6 = r2inv * r2inv * r2inv;
+        const float vel = (pi.w * pj[u].w) * rinv * (is14[u] ? W.el14 : 1.f);
+        float aa, bb;
+        lj_ab(is14[u] ? l14x : lx, is14[u] ? l14y : ly, lj[u].x, lj[u].y, arith, &aa, &bb);
+        const float va = r6 * r6 * aa, vb = r6 * bb;
+        const float dv = r2inv * __builtin_fmaf(6.f, vb, __builtin_fmaf(va, -12.f, -vel));
+        if (!v[u]) continue;
         g0 = __builtin_fmaf(-dx, dv, g0); g1 = __builtin_fmaf(-dy, dv, g1); g2 = __builtin_fmaf(-dz, dv, g2);
+        const int eb = (int)e[u];
         if (en && ea < eb) {
           const double ddx = d.x[3 * eb] - xs[0], ddy = d.x[3 * eb + 1] - xs[1], ddz = d.x[3 * eb + 2] - xs[2];
           const double4 tlj = d.ljd[eb];   // the j atom's type row, without the type lookup
@@ -795,7 +805,7 @@ __device__ __forceinline__ void pp_impl(const Dev& d, int wave, RowGrad& rg) {
           const double r2i = rinv_d * rinv_d, r6d = r2i * r2i * r2i;
           double ad, bd;
           double vd = (double)(pi.w * pj[u].w) * rinv_d;
-          if (is14) {
+          if (is14[u]) {
             vd *= W.el14d;
             lj_ab(tli[2], tli[3], tlj.z, tlj.w, arith, &ad, &bd);
           } else {
@@ -806,7 +816,9 @@ __device__ __forceinline__ void pp_impl(const Dev& d, int wave, RowGrad& rg) {
         }
       }
     }
-  }
+  };
+  if (W.arith) rows(std::true_type{});
+  else rows(std::false_type{});
   const float g[3] = {g0, g1, g2};
   rg.add<3>(g, b);
   if (en) {
