@@ -121,18 +121,19 @@ int qmi_window_info(qmi_engine* e, int w, int32_t* info, int cap);
 /* Write window w's restart file (write_xfin, md.f90:15452-15470). */
 int qmi_write_restart(qmi_engine* e, int w, const char* path);
 
-/* The autotuner (on by default) times candidate launch shapes of the
- * pair-row and bonded kernels on the engine's own windows during
- * qmi_prepare and keeps the fastest; the candidates do not change results.
- * Call before qmi_prepare.  No reference counterpart. */
+/* Whether qmi_prepare times the kernel families of an engine that is large
+ * enough for separate pair and bonded launches (on by default).  The launch
+ * shapes are fixed, so this changes neither results nor speed.  Call before
+ * qmi_prepare.  No reference counterpart. */
 int qmi_set_autotune(qmi_engine* e, int on);
 
-/* Choices of the autotuner: q-atoms per chunk of the q kernels (fixed), threads per block of the row,
- * LRF-build and bonded kernels, whether blocks are grouped by XCD (0/1),
- * the bonded mode (0: per-term slots and a per-atom gather, 1: atomics, 2:
- * LDS sums per tile of terms), the number of source shares
- * of the LRF build (its shapes are fixed), then the measured microseconds of the first six chosen
- * configurations (13 values).  Returns the number written. */
+/* The launch shapes: q-atoms per chunk of the q kernels, threads per block of
+ * the row, LRF-build and bonded kernels, 0 (blocks are not grouped by XCD), 0
+ * (the bonded mode), the number of source shares of the LRF build; then
+ * microseconds measured by qmi_prepare, 0 when it measured none: q kernels, all
+ * pair kernels, LRF build, bonded terms with polarisation and restraints, all
+ * pair kernels and the bonded terms again (13 values).  Returns the number
+ * written. */
 int qmi_tuning(qmi_engine* e, double* out, int cap);
 
 /* Turn per-step HIP-event timing of the kernel families on or off for the

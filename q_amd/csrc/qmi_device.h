@@ -127,8 +127,9 @@ constexpr int kQItem = 16;          // q-atoms of a chunk of the q kernels: half
 
 // Neighbour rows of the dynamic pair lists (WW, W<-P, P<-W, P<-P): row
 // ic*8 + a belongs to member a of i-cluster ic and holds the j entries of
-// that member (water: its slot in xw; solute: atom; P<-P entries carry the
-// 1-4 flag in bit 30), in a fixed capacity `cap` per row.
+// that member: the index in xw of a water's oxygen, or a solute slot (P<-P
+// entries carry the 1-4 flag in bit 30), in a fixed capacity `cap` per row, a
+// multiple of the entries the row kernels take in a pass.
 struct RowList {
   int* cnt;        // entries per row
   int* ent;        // [row * cap + k]
@@ -137,6 +138,9 @@ struct RowList {
 };
 constexpr int kRow14 = 1 << 30;
 
+// index in Dev::xw of site k (O, H1, H2) of member m of water cluster c
+__host__ __device__ __forceinline__ int xw_at(int c, int m, int k) { return 3 * kCl * c + kCl * k + m; }
+
 struct Dev {
   int nwin, ntot;
   const WinDev* win;
@@ -144,19 +148,20 @@ struct Dev {
   // atoms
   double *x, *v, *xtop;
   float4* x32;          // x, y, z, scaled charge
-  // the water atoms' x32 again, in water-cluster slot order: slot
-  // c*8 + m (cluster c, member m) holds O, H1, H2 at 3*slot + 0..2, so the
-  // members of a cluster are contiguous; water-water and solute-water row
-  // entries name slots.  wslot: per atom, its index in xw (3*slot + site),
-  // or -1 for solute atoms
+  // x32 again in cluster-slot order, the order in which rows name their
+  // entries: per water cluster its 8 members' O, H1 and H2 (xw_at), so that a
+  // row's 8 lanes, which mostly hold the members of one cluster, read one
+  // 128-byte line a load; then one per solute slot (cluster * 8 + member).
+  // Zero for empty members.  wslot: per atom, its index, or -1 (q-atoms)
   float4* xw;
   const int* wslot;
-  double4* xwd;         // the same slots in FP64 (x, y, z, unused), for the energy terms
+  double4* xwd;         // the same in FP64 (x, y, z, unused), for the energy terms
+  float4* sljp;         // avdw1, bvdw1, avdw3, bvdw3 of the solute slots
+  const double4* sljd;  // their rows of t_lj
   // the q-atoms' x32 again, per q-cluster member slot (cluster * 8 + member;
   // zero for empty members); qmslot: per atom, its slot or -1
   float4* xq;
   const int* qmslot;
-  float4* ljp;          // avdw1, bvdw1, avdw3, bvdw3
   long long* f;         // shared gradient, 3 per atom, fixed point 2^-32; zero between steps
   // the row kernels' and the q kernels' sums, 3 per entry: entry 3 * slot +
   // site for the waters' cluster slots (nwslot of them), then one per solute
@@ -243,13 +248,7 @@ struct Dev {
   const double* q_scd;
   // topology LJ params in double per window type (energy path)
   const double* t_lj;    // [(t_off + t)*4]
-  const double4* ljd;    // per atom: its type's row of t_lj
   RowList rl[T_NTYPES];  // neighbour rows
-  // launch shapes chosen by the autotuner (threads per block); none of
-  // them changes the arithmetic of a wave or thread
-  int bs_rows;
-  // 1: blocks on one XCD take consecutive work (block_id in the kernels)
-  int xcd;
   // bonded tiles, each of one window: (first entry of btile_terms, terms, first
   // atom, atoms spanned); btile_terms: term indices, grouped by kind within a tile
   int nbtile;

@@ -91,12 +91,9 @@ struct qmi_engine {
   std::vector<double> timings;
   bool timing_on = false;
   hipEvent_t ev[8] = {};
-  // the autotuner's choices
+  // whether qmi_prepare times the kernel families of a large engine
   bool autotune = true;
-  // q-atoms per work item, row / LRF / bonded block sizes, XCD map, atomic bonded
-  // gradients, LRF source parts
-  int tuned[7] = {kQItem, 256, 64 * kLrfWaves, 256, 0, 0, kLrfParts * kLrfWaves};
-  double tune_us[6] = {0, 0, 0, 0, 0, 0};   // time of the chosen configuration per group
+  double tune_us[6] = {0, 0, 0, 0, 0, 0};
   // the launch sequence of one MD step, captured once and replayed: index
   // bit 0 with the pair-list and LRF kernels (some window updates its lists),
   // bit 1 with the q-side energy passes (some window computes energies)
@@ -109,10 +106,10 @@ struct qmi_engine {
   hipStream_t copy_stream = nullptr;
   hipEvent_t chunk_ev[2] = {nullptr, nullptr};
   hipEvent_t copy_ev = nullptr;               // the last drain's ring copies done
-  // the captured step's other streams (LRF, bonded, restraints and water
-  // polarisation; the Q tiles) and its fork/join events
-  hipStream_t side_stream[2] = {nullptr, nullptr};
-  hipEvent_t step_ev[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  // the step's other stream (bonded terms, restraints and water polarisation;
+  // a small engine's LRF expansions) and its fork/join events
+  hipStream_t side_stream = nullptr;
+  hipEvent_t step_ev[2] = {nullptr, nullptr};
   int run_epoch = 0;                          // qmi_run calls so far (tags the ring records)
   long long* h_er = nullptr;
   double* h_or = nullptr;                     // EVB off-diagonal ring, pinned
@@ -151,7 +148,7 @@ qmi_engine::~qmi_engine() {
   for (auto& x : chunk_ev) if (x) (void)hipEventDestroy(x);
   if (copy_ev) (void)hipEventDestroy(copy_ev);
   for (auto& x : step_ev) if (x) (void)hipEventDestroy(x);
-  for (auto& x : side_stream) if (x) (void)hipStreamDestroy(x);
+  if (side_stream) (void)hipStreamDestroy(side_stream);
   if (h_er) (void)hipHostFree(h_er);
   if (h_or) (void)hipHostFree(h_or);
   if (h_tr) (void)hipHostFree(h_tr);
@@ -750,15 +747,13 @@ static int build_device(qmi_engine* e) {
 
   Dev& d = e->d;
   d.nwin = NW;
-  d.bs_rows = 256;
-  d.xcd = 0;
   d.ntot = ao;
   int rc = 0;
 #define UP(dst, src) if ((rc = dev_upload(e, &dst, src)) != 0) return rc
   WinDev* wdp; UP(wdp, wd); d.win = wdp;
   UP(d.ws, wst);
   UP(d.x, x); UP(d.v, v); UP(d.xtop, xtop);
-  UP(d.x32, x32); UP(d.ljp, ljp);
+  UP(d.x32, x32);
   if ((rc = dev_alloc(e, &d.f, x.size())) != 0) return rc;
   if ((rc = dev_alloc(e, &d.fterm, x.size())) != 0) return rc;
   float* fwinv; UP(fwinv, winv); d.winv = fwinv;
@@ -821,24 +816,36 @@ static int build_device(qmi_engine* e) {
     UP(rp, sp_rng); d.sp_rng = rp;
   }
   UP(ip, wc_o); d.wc_o = ip;
-  // water coordinates in cluster-slot order (the row kernels' gathers of
-  // neighbouring waters then read contiguous memory)
+  // coordinates and LJ columns in cluster-slot order (the row kernels' gathers
+  // of neighbours then read contiguous memory)
   {
+    const size_t nw3 = 3 * wc_o.size(), ns = sc_a.size();
     std::vector<int> wslot(x32.size(), -1);
-    std::vector<float4> xw(std::max<size_t>(3, 3 * wc_o.size()), make_float4(0.f, 0.f, 0.f, 0.f));
+    std::vector<float4> xw(std::max<size_t>(1, nw3 + ns), make_float4(0.f, 0.f, 0.f, 0.f));
     std::vector<double4> xwd(xw.size(), make_double4(0.0, 0.0, 0.0, 0.0));
-    for (size_t m = 0; m < wc_o.size(); ++m) {
-      const int o = wc_o[m];
-      if (o < 0) continue;
-      for (int k = 0; k < 3; ++k) {
-        wslot[o + k] = 3 * (int)m + k;
-        xw[3 * m + k] = x32[o + k];
-        xwd[3 * m + k] = make_double4(x[3 * (o + k)], x[3 * (o + k) + 1], x[3 * (o + k) + 2], 0.0);
-      }
+    std::vector<float4> sljp(std::max<size_t>(1, ns), make_float4(0.f, 0.f, 0.f, 0.f));
+    std::vector<double4> sljd(sljp.size(), make_double4(0.0, 0.0, 0.0, 0.0));
+    auto place = [&](int at, size_t k) {
+      wslot[at] = (int)k;
+      xw[k] = x32[at];
+      xwd[k] = make_double4(x[3 * at], x[3 * at + 1], x[3 * at + 2], 0.0);
+    };
+    for (size_t m = 0; m < wc_o.size(); ++m)
+      for (int k = 0; k < 3 && wc_o[m] >= 0; ++k) place(wc_o[m] + k, xw_at((int)m / kCl, (int)m % kCl, k));
+    for (size_t m = 0; m < ns; ++m) {
+      const int at = sc_a[m];
+      if (at < 0) continue;
+      place(at, nw3 + m);
+      sljp[m] = ljp[at];
+      const double* r = &t_lj[(size_t)(wd[sc_win[m / kCl]].t_off + iac[at]) * 4];
+      sljd[m] = make_double4(r[0], r[1], r[2], r[3]);
     }
     UP(d.xw, xw);
     UP(d.xwd, xwd);
     UP(ip, wslot); d.wslot = ip;
+    UP(d.sljp, sljp);
+    double4* l4;
+    UP(l4, sljd); d.sljd = l4;
   }
   UP(ip, sc_a); d.sc_a = ip;
   {
@@ -979,17 +986,6 @@ static int build_device(qmi_engine* e) {
   UP(fp_, q_sc); d.q_sc = fp_;
   UP(dp, q_scd); d.q_scd = dp;
   UP(dp, t_lj); d.t_lj = dp;
-  {
-    // per atom: its type's FP64 LJ columns, for the energy passes' gathers
-    std::vector<double4> ljd(std::max<size_t>(iac.size(), 1), make_double4(0, 0, 0, 0));
-    for (int wi = 0; wi < NW; ++wi)
-      for (int a = wd[wi].ao; a < wd[wi].ao + wd[wi].natom; ++a) {
-        const double* r = &t_lj[(size_t)(wd[wi].t_off + iac[a]) * 4];
-        ljd[a] = make_double4(r[0], r[1], r[2], r[3]);
-      }
-    double4* l4;
-    UP(l4, ljd); d.ljd = l4;
-  }
   d.nqq = (int)qq_ij.size();
   int4* i4;
   UP(i4, qq_ij); d.qq_ij = i4;
@@ -1450,14 +1446,13 @@ int qmi_window_add(qmi_engine* e, const char* inp_path, long long seed_override,
   return 0;
 }
 
-// Autotuner: on the engine's own windows, time every candidate launch shape
-// of a kernel family (a forces-only evaluation, a few repeats, HIP events on
-// the engine's stream) and keep the fastest.  The candidates differ only in
-// how work is grouped into blocks and waves, never in the arithmetic of a
-// pair or term, so the choice does not change results.
-static int autotune(qmi_engine* e) {
+// The times of a large engine's kernel families on its own windows (a
+// forces-only evaluation, a few repeats, HIP events on the engine's stream).
+// The launch shapes are fixed: the step's kernels share the GPU, and the times
+// of one alone do not tell which shape is the better among the others.
+static int time_families(qmi_engine* e) {
   Dev& d = e->d;
-  if (d.small) return 0;   // the step's one launch has no shapes to choose
+  if (d.small) return 0;   // the step's forces are one launch
   hipEvent_t t0, t1;
   HIP_OK(hipEventCreate(&t0));
   HIP_OK(hipEventCreate(&t1));
@@ -1479,55 +1474,11 @@ static int autotune(qmi_engine* e) {
   launch_begin(d, e->stream, 2, 1);
   launch_lists(d, e->stream, e->ngrp, e->nwc, e->nsc);
   HIP_OK(hipStreamSynchronize(e->stream));
-  const int bs[3] = {256, 128, 64};
-  // Candidates are tried from the coarsest work grouping down, and a later
-  // one replaces the best so far only when it is more than 2 % faster:
-  // timed alone, close candidates differ by noise, and in the step graph,
-  // where the kernels share the GPU, the coarser groupings fare better.
-  auto faster = [](double t, double best) { return t < 0.98 * best; };
-  // 0: the q kernels (fixed work items)
-  e->tuned[0] = kQItem;
   e->tune_us[0] = time_us([&] { launch_q(d, e->stream, false); });
-  // 1: threads per block of the row kernels
-  {
-    int bb = 256;
-    double bt = 1e30;
-    for (int b : bs) {
-      d.bs_rows = b;
-      const double t = time_us([&] { launch_nonbonded(d, e->stream, true, false); });
-      if (faster(t, bt)) { bt = t; bb = b; }
-    }
-    d.bs_rows = bb;
-    e->tuned[1] = bb;
-    e->tune_us[1] = bt;
-  }
-  // 3, 5: the bonded terms (fixed tiles)
-  e->tune_us[3] = time_us([&] { launch_bonded(d, e->stream); });
-  e->tune_us[5] = e->tune_us[3];
-  // 2, 6: the LRF build (fixed shapes: they set the order of its sums)
-  e->tuned[2] = 64 * kLrfWaves;
+  e->tune_us[1] = time_us([&] { launch_nonbonded(d, e->stream, true, false); });
   e->tune_us[2] = time_us([&] { launch_lrf_build(d, e->stream); });
-  e->tuned[6] = kLrfParts * kLrfWaves;
-  // 4: XCD-grouped block order of the pair, Q-tile, LRF-build and gather kernels
-  {
-    double tx[2];
-    for (int x = 0; x < 2; ++x) {
-      d.xcd = x;
-      // the pair and Q-tile kernels, whose gathers the grouping keeps in
-      // one XCD's L2 (the LRF build, timed with them, would drown the
-      // difference in its own run-to-run spread)
-      tx[x] = time_us([&] {
-        launch_nonbonded(d, e->stream, true, false);
-        launch_q(d, e->stream, false);
-      });
-    }
-    // ungrouped unless grouped is clearly faster (grouping keeps each XCD's
-    // share of the water slots in its own L2, but in the step graph it was
-    // measured slower for the water-water and LRF kernels)
-    d.xcd = faster(tx[1], tx[0]) ? 1 : 0;
-    e->tuned[4] = d.xcd;
-    e->tune_us[4] = tx[d.xcd];
-  }
+  e->tune_us[3] = e->tune_us[5] = time_us([&] { launch_other_forces(d, e->stream); });
+  e->tune_us[4] = e->tune_us[1];
   // the timing runs added to the shared gradient, which steps expect at zero
   HIP_OK(hipMemsetAsync(d.f, 0, (size_t)3 * d.ntot * sizeof(long long), e->stream));
   HIP_OK(hipStreamSynchronize(e->stream));
@@ -1549,8 +1500,7 @@ int qmi_prepare(qmi_engine* e) {
   HIP_OK(hipSetDevice(e->device));
   if (!e->stream) HIP_OK(hipStreamCreate(&e->stream));
   if (!e->copy_stream) HIP_OK(hipStreamCreateWithFlags(&e->copy_stream, hipStreamNonBlocking));
-  for (auto& x : e->side_stream)
-    if (!x) HIP_OK(hipStreamCreateWithFlags(&x, hipStreamNonBlocking));
+  if (!e->side_stream) HIP_OK(hipStreamCreateWithFlags(&e->side_stream, hipStreamNonBlocking));
   for (auto& x : e->step_ev)
     if (!x) HIP_OK(hipEventCreateWithFlags(&x, hipEventDisableTiming));
   for (auto& x : e->chunk_ev)
@@ -1558,7 +1508,7 @@ int qmi_prepare(qmi_engine* e) {
   if (!e->copy_ev) HIP_OK(hipEventCreateWithFlags(&e->copy_ev, hipEventDisableTiming));
   int rc = build_device(e);
   if (rc) return rc;
-  if (e->autotune && (rc = autotune(e)) != 0) return rc;
+  if (e->autotune && (rc = time_families(e)) != 0) return rc;
   for (auto& h : e->wins) {
     Window& W = *h.w;
     if (W.inp.iene_cycle > 0 && !W.inp.ene_file.empty()) {
@@ -1826,8 +1776,8 @@ int qmi_run(qmi_engine* e, long long nsteps, int finalize) {
   // timing pass it runs as one captured graph
   auto launch_step = [&](int variant) {
     const bool lists = variant & 1, qen = variant & 2;
-    // lists and forces on three streams; a failure here fails the capture
-    if (launch_step_forces(e->d, e->stream, e->side_stream[0], e->side_stream[1], e->step_ev, lists, e->ngrp, e->nwc,
+    // lists and forces on two streams; a failure here fails the capture
+    if (launch_step_forces(e->d, e->stream, e->side_stream, e->step_ev, lists, e->ngrp, e->nwc,
                            e->nsc, qen, false) != hipSuccess)
       return;
     launch_integrate(e->d, e->stream, e->shake_any, variant);
@@ -2123,7 +2073,7 @@ int qmi_evaluate(qmi_engine* e, int rebuild_lists) {
 static int evaluate(qmi_engine* e, int rebuild_lists, int mode) {
   HIP_OK(hipSetDevice(e->device));
   launch_begin(e->d, e->stream, mode, rebuild_lists ? 1 : 0);
-  HIP_OK(launch_step_forces(e->d, e->stream, e->side_stream[0], e->side_stream[1], e->step_ev, rebuild_lists != 0,
+  HIP_OK(launch_step_forces(e->d, e->stream, e->side_stream, e->step_ev, rebuild_lists != 0,
                             e->ngrp, e->nwc, e->nsc, true, true));
   HIP_OK(hipGetLastError());
   const int NW = (int)e->wins.size();
@@ -2276,8 +2226,8 @@ int qmi_get_pairlist(qmi_engine* e, int w, int kind, int32_t* pi, int32_t* pj, i
       for (int k = 0; k < cnt[row]; ++k) {
         const int v = ent[row * L.cap + k];
         const bool is14 = (tt == T_PP) && (v & kRow14);
-        // water-water and solute-water entries name water slots
-        const int eb = (tt == T_PP ? (v & ~kRow14) : e->h_wc_o[v]) - (int)ao;
+        // the member's place in the slot coordinates (xw_at for a water)
+        const int eb = (tt == T_PP ? e->h_sc_a[v & ~kRow14] : e->h_wc_o[v / (3 * kCl) * kCl + v % (3 * kCl)]) - (int)ao;
         if (tt == T_WW) {
           if (ea < eb) out.push_back({ea + 1, eb + 1, 1});
         } else if (tt == T_PP) {
@@ -2327,8 +2277,7 @@ int qmi_set_autotune(qmi_engine* e, int on) {
 int qmi_tuning(qmi_engine* e, double* out, int cap) {
   if (!e || !out) return set_err(-1, "null argument");
   if (!e->prepared) return set_err(-2, "engine not prepared");
-  const double v[13] = {(double)e->tuned[0], (double)e->tuned[1], (double)e->tuned[2],
-                        (double)e->tuned[3], (double)e->tuned[4], (double)e->tuned[5], (double)e->tuned[6],
+  const double v[13] = {kQItem, 256, 64 * kLrfWaves, 256, 0, 0, kLrfParts * kLrfWaves,
                         e->tune_us[0], e->tune_us[1], e->tune_us[2], e->tune_us[3], e->tune_us[4], e->tune_us[5]};
   const int n = std::min(cap, 13);
   for (int k = 0; k < n; ++k) out[k] = v[k];

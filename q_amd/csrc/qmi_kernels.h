@@ -14,10 +14,9 @@ void launch_lists(const Dev& d, hipStream_t s, int ngrp, int nwc, int nsc);
 // them); `energy` / `q_energy`: the kernel instances that also evaluate the
 // energy terms of windows at an energy step (false: forces only)
 void launch_ww(const Dev& d, hipStream_t s, bool energy = true);
-// single families, for the autotuner's timing runs
+// single families, for timing
 void launch_q(const Dev& d, hipStream_t s, bool energy = true);
 void launch_lrf_build(const Dev& d, hipStream_t s);
-void launch_bonded(const Dev& d, hipStream_t s);
 void launch_nonbonded(const Dev& d, hipStream_t s, bool with_ww = true, bool q_energy = true);
 // water polarisation, bonded terms and restraint records
 void launch_other_forces(const Dev& d, hipStream_t s);
@@ -25,10 +24,10 @@ void launch_other_forces(const Dev& d, hipStream_t s);
 void launch_atom_terms(const Dev& d, hipStream_t s);
 // whether a step's force kernels run as one launch (Dev::small)
 bool small_engine(const Dev& d, bool mixed_solvent);
-// the lists and forces of an MD step or (eval) of an evaluation on three
+// the lists and forces of an MD step or (eval) of an evaluation on two
 // streams (see the definition)
-hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, hipStream_t s3, const hipEvent_t ev[5],
-                              bool lists, int ngrp, int nwc, int nsc, bool q_energy, bool eval);
+hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, const hipEvent_t ev[2], bool lists, int ngrp,
+                              int nwc, int nsc, bool energy, bool eval);
 // the end of an MD step; the gradient is completed with the per-atom terms
 // of launch_atom_terms, which must have run in the same step
 // variant: bit 0 the step's list kernels were launched, bit 1 its energy terms

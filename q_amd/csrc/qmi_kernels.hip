@@ -22,23 +22,11 @@
 namespace qmi {
 
 // ------------------------------------------------------------ helpers --
-// Workgroups go to the 8 XCDs in turn (block b to XCD b mod 8), each with its
-// own L2.  With xcd set, the blocks that land on one XCD take one contiguous
-// range of the work (the clusters or terms of a few windows), so a window's
-// coordinates are cached in one L2 instead of all eight.  The map is a
-// permutation of 0..gridDim.x-1.
-__device__ __forceinline__ int block_id(int xcd) {
-  const int b = blockIdx.x;
-  if (!xcd) return b;
-  const int nb = gridDim.x, x = b & 7, i = b >> 3, q = nb >> 3, r = nb & 7;
-  return x < r ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
-}
-
 // index of the calling wave in the grid (blocks are whole waves), read from
 // the first lane so the compiler keeps it, and the list loads it indexes, in
 // scalar registers
-__device__ __forceinline__ int wave_id(const Dev& d) {
-  return __builtin_amdgcn_readfirstlane((int)((block_id(d.xcd) * blockDim.x + threadIdx.x) >> 6));
+__device__ __forceinline__ int wave_id() {
+  return __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
 }
 
 __device__ __forceinline__ long long fix(double v, double scale) { return __double2ll_rn(v * scale); }
@@ -224,7 +212,7 @@ __device__ __forceinline__ void begin_step(WinState& s, const WinDev& W) {
 
 // start of a run's first step (eval 0; later steps are begun by k_temperature)
 // or of an evaluation, one thread per window.  eval 1: energy evaluation; 2:
-// forces only (the autotuner's timing runs); 3: the energy evaluation after
+// forces only (timing runs); 3: the energy evaluation after
 // the last step of a run (md.f90:4207-4208), which is a pot_energy call of
 // the run for windows that completed; a window stopped by a failure is left
 // as it is.
@@ -411,8 +399,9 @@ __device__ __forceinline__ void build_row(const Dev& d, int wave) {
       const unsigned rowbits = (unsigned)((kb >> (8 * a)) & 0xffull);
       if (keep) {
         const int idx = cnt + __popc(rowbits & ((1u << b) - 1u));
-        // water entries name the member's cluster slot
-        const int ev = jw ? (j0 + base + k) * kCl + b : (TT == T_PP && sp == 2) ? (eb | kRow14) : eb;
+        // entries name the member's place in the slot coordinates
+        const int jc = j0 + base + k;
+        const int ev = jw ? xw_at(jc, b, 0) : (jc * kCl + b) | (TT == T_PP && sp == 2 ? kRow14 : 0);
         if (idx < L.cap) L.ent[(size_t)row * L.cap + idx] = ev;
       }
       cnt += __popc(rowbits);
@@ -429,7 +418,7 @@ __device__ __forceinline__ void build_row(const Dev& d, int wave) {
 
 // all four kinds of rows in one launch, the longest-running first
 __global__ void __launch_bounds__(256) k_build_rows(Dev d) {
-  int wave = wave_id(d);
+  int wave = wave_id();
   const int np = (d.rl[T_PP].nicl + 3) & ~3, nw = (d.rl[T_WW].nicl + 3) & ~3;   // whole blocks of each kind
   if (wave < np) return build_row<T_PP>(d, wave);
   wave -= np;
@@ -517,12 +506,12 @@ __device__ __forceinline__ void ww_impl(const Dev& d, int wave, RowGrad& rg) {
   const WinDev& W = d.win[w];
   const int a = lane >> 3, b = lane & 7;
   const int row = ic * kCl + a;
-  const int oa = d.wc_o[ic * kCl + a];
-  const int n = oa >= 0 ? L.cnt[row] : 0;
+  const int n = L.cnt[row];   // none for an empty member
   const int nch = row_chunks(n);
+  const int xa = xw_at(ic, a, 0);
   float3 pi[3];
   for (int k = 0; k < 3; ++k) {
-    float4 q = oa >= 0 ? d.x32[oa + k] : make_float4(0, 0, 0, 0);
+    const float4 q = d.xw[xa + kCl * k];
     pi[k] = make_float3(q.x, q.y, q.z);
   }
   const float q0 = W.crg_w[0], q1 = W.crg_w[1], q2 = W.crg_w[2];
@@ -536,17 +525,20 @@ __device__ __forceinline__ void ww_impl(const Dev& d, int wave, RowGrad& rg) {
   // nonbond_ww_spc / nonbond_3atomsolvent evaluate them
   double xi[9];
   if (en)
-    for (int k = 0; k < 9; ++k) xi[k] = oa >= 0 ? d.x[3 * oa + k] : 0.0;
+    for (int k = 0; k < 3; ++k) {
+      const double4 q = d.xwd[xa + kCl * k];
+      xi[3 * k] = q.x; xi[3 * k + 1] = q.y; xi[3 * k + 2] = q.z;
+    }
   const int* ent = L.ent + (size_t)row * L.cap + b;
-  // entries are water slots: the members of a neighbouring cluster are
-  // contiguous in xw, so the 8 lanes of a row mostly read the same lines.
-  // The next entry's slot and coordinates are loaded while the current one
-  // is evaluated (entries past the row end read slot 0 and are skipped; the
-  // table has kCl entries beyond its last row)
+  // one site of a neighbouring cluster's members is one line of xw, so the 8
+  // lanes of a row mostly read one line a load.  The next entry and its
+  // coordinates are loaded while the current one is evaluated (entries past
+  // the row end read place 0 and are skipped; the table has kCl entries
+  // beyond its last row)
   const int e0 = ent[0];
   unsigned ob_next = b < n ? e0 : 0;
   float4 nx[3];
-  for (int s = 0; s < 3; ++s) nx[s] = d.xw[3ull * ob_next + s];
+  for (int s = 0; s < 3; ++s) nx[s] = (d.xw + ob_next)[kCl * s];
   for (int t = 0; t < nch; ++t) {
     const int k = t * kCl + b;
     const unsigned ob = ob_next;
@@ -555,18 +547,18 @@ __device__ __forceinline__ void ww_impl(const Dev& d, int wave, RowGrad& rg) {
     {
       const int e = ent[(t + 1) * kCl];
       ob_next = k + kCl < n ? e : 0;
-      for (int s = 0; s < 3; ++s) nx[s] = d.xw[3ull * ob_next + s];
+      for (int s = 0; s < 3; ++s) nx[s] = (d.xw + ob_next)[kCl * s];
     }
     if (k >= n) continue;
     // each unordered pair counted once, from the row with the lower slot: a
     // row's entries ascend in slot order, so the counted ones are a suffix
     // of the row and the 8 rows of the wave (consecutive slots) switch at
     // nearly the same place, which keeps the FP64 block from diverging
-    const bool cnt = en && row < (int)ob;
+    const bool cnt = en && xa < (int)ob;
     if (cnt) {
       double xj[9];
       for (int m = 0; m < 3; ++m) {
-        const double4 q = d.xwd[3ull * ob + m];
+        const double4 q = (d.xwd + ob)[kCl * m];
         xj[3 * m] = q.x; xj[3 * m + 1] = q.y; xj[3 * m + 2] = q.z;
       }
       for (int p = 0; p < 3; ++p)
@@ -627,16 +619,16 @@ __device__ __forceinline__ void pw_impl(const Dev& d, int wave, RowGrad& rg) {
   const WinDev& W = d.win[w];
   const int a = lane >> 3, b = lane & 7;
   const int row = ic * kCl + a;
-  const int ea = WATER_SIDE ? d.wc_o[ic * kCl + a] : d.sc_a[ic * kCl + a];
-  const int n = ea >= 0 ? L.cnt[row] : 0;
+  const int n = L.cnt[row];   // none for an empty member
   const int nch = row_chunks(n);
+  const float4* xs = d.xw + 3 * (size_t)d.nwslot;   // the solute slots
   float4 pi[3];
-  float4 ljs = make_float4(0, 0, 0, 0);
+  float2 ljs = make_float2(0, 0);
   if (WATER_SIDE) {
-    for (int k = 0; k < 3; ++k) pi[k] = ea >= 0 ? d.x32[ea + k] : make_float4(0, 0, 0, 0);
+    for (int k = 0; k < 3; ++k) pi[k] = d.xw[xw_at(ic, a, k)];
   } else {
-    pi[0] = ea >= 0 ? d.x32[ea] : make_float4(0, 0, 0, 0);
-    if (ea >= 0) ljs = d.ljp[ea];
+    pi[0] = xs[row];
+    ljs = *(const float2*)&d.sljp[row];
   }
   constexpr bool en = EN && !WATER_SIDE;
   constexpr bool wat3 = W3;
@@ -645,12 +637,13 @@ __device__ __forceinline__ void pw_impl(const Dev& d, int wave, RowGrad& rg) {
   double eel = 0.0, evdw = 0.0;
   // energy steps: the energy terms in FP64 from the FP64 coordinates and
   // LJ columns, as nonbond_pw / nonbond_3atomsolvent evaluate them
-  double xs[3] = {0, 0, 0}, Ad[3] = {0, 0, 0}, Bd[3] = {0, 0, 0};
-  if (en && ea >= 0) {
-    for (int c = 0; c < 3; ++c) xs[c] = d.x[3 * ea + c];
-    const double* tl = &d.t_lj[(size_t)(W.t_off + d.iac[ea]) * 4];
+  double4 xd = make_double4(0, 0, 0, 0);
+  double Ad[3] = {0, 0, 0}, Bd[3] = {0, 0, 0};
+  if (en) {
+    xd = d.xwd[3 * (size_t)d.nwslot + row];
+    const double4 tl = d.sljd[row];
     for (int k = 0; k < (wat3 ? 3 : 1); ++k)
-      lj_ab(tl[0], tl[1], k == 0 ? W.aO1d : W.awd[k], k == 0 ? W.bO1d : W.bwd[k], W.arith, &Ad[k], &Bd[k]);
+      lj_ab(tl.x, tl.y, k == 0 ? W.aO1d : W.awd[k], k == 0 ? W.bO1d : W.bwd[k], W.arith, &Ad[k], &Bd[k]);
   }
   const int* ent = L.ent + (size_t)row * L.cap + b;
   // kUnroll entries per pass, loads first (as in pp_impl)
@@ -670,18 +663,17 @@ __device__ __forceinline__ void pw_impl(const Dev& d, int wave, RowGrad& rg) {
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
         if (WATER_SIDE) {
-          ld[u][0] = d.x32[e[u]];
-          lt[u] = *(const float2*)&d.ljp[e[u]];
+          ld[u][0] = xs[e[u]];
+          lt[u] = *(const float2*)&d.sljp[e[u]];
         } else {
-          // water slots (contiguous per cluster)
-          const float4* xe = d.xw + 3ull * e[u];
-          ld[u][0] = xe[0]; ld[u][1] = xe[1]; ld[u][2] = xe[2];
+          const float4* xe = d.xw + e[u];
+          ld[u][0] = xe[0]; ld[u][1] = xe[kCl]; ld[u][2] = xe[2 * kCl];
         }
       }
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
         const float4 ps = WATER_SIDE ? ld[u][0] : pi[0];
-        const float2 lj = WATER_SIDE ? lt[u] : make_float2(ljs.x, ljs.y);
+        const float2 lj = WATER_SIDE ? lt[u] : ljs;
         if (!v[u]) continue;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
@@ -700,8 +692,8 @@ __device__ __forceinline__ void pw_impl(const Dev& d, int wave, RowGrad& rg) {
             dv = r2inv * (-(qq * rinv));
           }
           if (en) {
-            const double4 xa = d.xwd[3ull * e[u] + k];   // the water atom of the slot, FP64
-            const double ddx = xa.x - xs[0], ddy = xa.y - xs[1], ddz = xa.z - xs[2];
+            const double4 xa = (d.xwd + e[u])[kCl * k];   // the water atom, FP64
+            const double ddx = xa.x - xd.x, ddy = xa.y - xd.y, ddz = xa.z - xd.z;
             const double rinv_d = rsqrt_e(ddx * ddx + ddy * ddy + ddz * ddz);
             eel += (double)qq * rinv_d;
             if (k == 0 || wat3) {
@@ -742,21 +734,20 @@ __device__ __forceinline__ void pp_impl(const Dev& d, int wave, RowGrad& rg) {
   const WinDev& W = d.win[w];
   const int a = lane >> 3, b = lane & 7;
   const int row = ic * kCl + a;
-  const int ea = d.sc_a[ic * kCl + a];
-  const int n = ea >= 0 ? L.cnt[row] : 0;
+  const int n = L.cnt[row];   // none for an empty member
   const int nch = row_chunks(n);
-  const float4 pi = ea >= 0 ? d.x32[ea] : make_float4(0, 0, 0, 0);
-  const float4 li = ea >= 0 ? d.ljp[ea] : make_float4(0, 0, 0, 0);
+  const float4* xs = d.xw + 3 * (size_t)d.nwslot;      // the solute slots
+  const double4* xsd = d.xwd + 3 * (size_t)d.nwslot;
+  const float4 pi = xs[row], li = d.sljp[row];
   constexpr bool en = EN;
   float g0 = 0.f, g1 = 0.f, g2 = 0.f;
   double eel = 0.0, evdw = 0.0;
   // energy steps: the energy terms in FP64 from the FP64 coordinates and LJ
   // columns, as nonbond_pp evaluates them
-  double xs[3] = {0, 0, 0};
-  const double* tli = nullptr;
-  if (en && ea >= 0) {
-    for (int c = 0; c < 3; ++c) xs[c] = d.x[3 * ea + c];
-    tli = &d.t_lj[(size_t)(W.t_off + d.iac[ea]) * 4];
+  double4 xd = make_double4(0, 0, 0, 0), tli = make_double4(0, 0, 0, 0);
+  if (en) {
+    xd = xsd[row];
+    tli = d.sljd[row];
   }
   const int* ent = L.ent + (size_t)row * L.cap + b;
   // kUnroll entries per pass: all their loads are issued before the
@@ -782,8 +773,8 @@ __device__ __forceinline__ void pp_impl(const Dev& d, int wave, RowGrad& rg) {
       float2 lj[kUnroll];
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
-        pj[u] = d.x32[e[u]];
-        lj[u] = ((const float2*)d.ljp)[2ull * e[u] + is14[u]];
+        pj[u] = xs[e[u]];
+        lj[u] = ((const float2*)d.sljp)[2ull * e[u] + is14[u]];
       }
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
@@ -797,19 +788,20 @@ __device__ __forceinline__ void pp_impl(const Dev& d, int wave, RowGrad& rg) {
         const float dv = r2inv * __builtin_fmaf(6.f, vb, __builtin_fmaf(va, -12.f, -vel));
         if (!v[u]) continue;
         g0 = __builtin_fmaf(-dx, dv, g0); g1 = __builtin_fmaf(-dy, dv, g1); g2 = __builtin_fmaf(-dz, dv, g2);
-        const int eb = (int)e[u];
-        if (en && ea < eb) {
-          const double ddx = d.x[3 * eb] - xs[0], ddy = d.x[3 * eb + 1] - xs[1], ddz = d.x[3 * eb + 2] - xs[2];
-          const double4 tlj = d.ljd[eb];   // the j atom's type row, without the type lookup
+        // each pair counted once, from the row with the lower slot (a suffix
+        // of the row, as for the waters)
+        if (en && row < (int)e[u]) {
+          const double4 xj = xsd[e[u]], tlj = d.sljd[e[u]];
+          const double ddx = xj.x - xd.x, ddy = xj.y - xd.y, ddz = xj.z - xd.z;
           const double rinv_d = rsqrt_e(ddx * ddx + ddy * ddy + ddz * ddz);
           const double r2i = rinv_d * rinv_d, r6d = r2i * r2i * r2i;
           double ad, bd;
           double vd = (double)(pi.w * pj[u].w) * rinv_d;
           if (is14[u]) {
             vd *= W.el14d;
-            lj_ab(tli[2], tli[3], tlj.z, tlj.w, arith, &ad, &bd);
+            lj_ab(tli.z, tli.w, tlj.z, tlj.w, arith, &ad, &bd);
           } else {
-            lj_ab(tli[0], tli[1], tlj.x, tlj.y, arith, &ad, &bd);
+            lj_ab(tli.x, tli.y, tlj.x, tlj.y, arith, &ad, &bd);
           }
           eel += vd;
           evdw += ad * r6d * r6d - bd * r6d;
@@ -834,9 +826,12 @@ __device__ __forceinline__ void pp_impl(const Dev& d, int wave, RowGrad& rg) {
 // members is stored in the row buffer (Dev::grow), which the integrator adds:
 // atomics on the shared gradient array go past the XCDs' L2s to memory, at
 // about 22 per ns for the whole GPU, and were most of what these kernels
-// spent.  64-window ladder, force-only: water rows 58 + 67 us as two kernels
-// with atomics, 89 as one with stores; solute rows 34 + 55, now 68.  What
-// bounds them now is VALU issue.
+// spent.  64-window ladder, force-only, alone: water rows 58 + 67 us as two
+// kernels with atomics, 89 as one with stores, 85 with 82 -> 57 instructions a
+// water<-solute entry; solute rows 34 + 55, 74, then 70 with 70 -> 41 a solute
+// pair.  They are bound by VALU issue (about 75 %) and the gathers' return path
+// (76 %): with four floats loaded a water atom where three are used, the water
+// rows take 10 us more.
 // W3: the instance for windows with a 3-atom solvent (launched only when
 // there are any); each instance skips the other windows' rows.
 // EK: the instance launched on steps where some window computes energies
@@ -856,7 +851,6 @@ __device__ __forceinline__ void wrow_wave(const Dev& d, int wave) {
   }
   if (PART & 2) pw_impl<true, false, W3>(d, wave, rg);
   const int lane = threadIdx.x & 63, b = lane & 7, row = wave * kCl + (lane >> 3);
-  if (d.wc_o[row] < 0) return;
   long long* o = d.grow + 9 * (size_t)row;
   if (PART == 2) rg.lo += o[b];
   o[b] = rg.lo;
@@ -864,7 +858,7 @@ __device__ __forceinline__ void wrow_wave(const Dev& d, int wave) {
 }
 template <bool W3, bool EK, int PART>
 __global__ void __launch_bounds__(256) k_wrow(Dev d) {
-  wrow_wave<W3, EK, PART>(d, wave_id(d));
+  wrow_wave<W3, EK, PART>(d, wave_id());
 }
 
 template <bool W3, bool EK>
@@ -881,11 +875,11 @@ __device__ __forceinline__ void srow_wave(const Dev& d, int wave) {
     pp_impl<false>(d, wave, rg);
   }
   const int lane = threadIdx.x & 63, b = lane & 7, row = wave * kCl + (lane >> 3);
-  if (b < 3 && d.sc_a[row] >= 0) d.grow[9 * (size_t)d.nwslot + 3 * row + b] = rg.lo;
+  if (b < 3) d.grow[9 * (size_t)d.nwslot + 3 * row + b] = rg.lo;
 }
 template <bool W3, bool EK>
 __global__ void __launch_bounds__(256) k_srow(Dev d) {
-  srow_wave<W3, EK>(d, wave_id(d));
+  srow_wave<W3, EK>(d, wave_id());
 }
 
 // ---- q-atoms against water (nonbond_qw_spc, md.f90:11302-11411; 3-atom
@@ -985,11 +979,12 @@ __device__ __forceinline__ void qw_impl(const Dev& d, const WinDev& W, const int
   const int ow = lane < wk.z ? d.wc_o[slot] : -1;
   const bool on = ow >= 0 && d.qw_on[slot] && d.qin[ow];   // the lane's water is in the Q lists
   float4 pw[3];
-  for (int k = 0; k < 3; ++k) pw[k] = d.xw[3 * (size_t)slot + k];
+  const int xa = xw_at(slot / kCl, slot % kCl, 0);
+  for (int k = 0; k < 3; ++k) pw[k] = d.xw[xa + kCl * k];
   double pd[9];
   if (EN)
     for (int k = 0; k < 3; ++k) {
-      const double4 t = d.xwd[3 * (size_t)slot + k];
+      const double4 t = d.xwd[xa + kCl * k];
       pd[3 * k] = t.x; pd[3 * k + 1] = t.y; pd[3 * k + 2] = t.z;
     }
   float lam[kMaxS];
@@ -1154,7 +1149,7 @@ __device__ __forceinline__ void qw_group(const Dev& d, int item, double* s) {
 template <bool W3, bool EK>
 __global__ void __launch_bounds__(64 * kQWaves) k_qw(Dev d) {
   __shared__ double s[9 * 64 * kQWaves];
-  qw_group<W3, EK>(d, block_id(d.xcd), s);
+  qw_group<W3, EK>(d, blockIdx.x, s);
 }
 
 template <bool EN, int NS>
@@ -1167,13 +1162,13 @@ __device__ __forceinline__ void qp_impl(const Dev& d, const WinDev& W, const int
   const int pa = lane < wk.z ? d.sc_a[slot] : -1;
   const bool on = pa >= 0 && d.qp_on[slot] && d.qin[pa];   // the lane's solute atom is in the Q lists
   const int ia = pa >= 0 ? pa : W.ao;
-  const float4 pj = d.x32[ia], lj = d.ljp[ia];
+  const float4 pj = d.x32[ia], lj = d.sljp[slot];
   const int iacj = d.iac[ia];
   double xj[3];
   double4 tlj = make_double4(0, 0, 0, 0);
   if (EN) {
     for (int c = 0; c < 3; ++c) xj[c] = d.x[3 * (size_t)ia + c];
-    tlj = d.ljd[ia];
+    tlj = d.sljd[slot];
   }
   float lam[kMaxS];
   for (int s = 0; s < kMaxS; ++s) lam[s] = s < S ? (float)W.lambda[s] : 0.f;
@@ -1297,7 +1292,7 @@ __device__ __forceinline__ void qp_group(const Dev& d, int item, double* s) {
 template <bool EK>
 __global__ void __launch_bounds__(64 * kQWaves) k_qp(Dev d) {
   __shared__ double s[3 * 64 * kQWaves];
-  qp_group<EK>(d, block_id(d.xcd), s);
+  qp_group<EK>(d, blockIdx.x, s);
 }
 
 // q-q and q-(bonded neighbour) pairs (nonbond_qq, md.f90:10763-10868).
@@ -1391,7 +1386,7 @@ __device__ __forceinline__ void qq_wave(const Dev& d, int wave) {
 }
 template <bool EK>
 __global__ void __launch_bounds__(256) k_qq(Dev d) {
-  qq_wave<EK>(d, __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6)));
+  qq_wave<EK>(d, wave_id());
 }
 static int qq_waves(const Dev& d, bool energy) { return d.nqqg + (energy ? (d.nqq + 63) / 64 : 0); }
 static void launch_qq(const Dev& d, hipStream_t s, bool energy) {
@@ -1478,7 +1473,7 @@ __device__ __forceinline__ void lrf_add(double s[kLrfSums], double q, double dx,
 // through LDS and vector loads, all terms formed and 8 parts it was 2.07 ms,
 // and 131 us for the one window, now 40.
 __global__ void __launch_bounds__(64 * kLrfWaves, 4) k_lrf_build(Dev d) {
-  const int4 lw = d.lrf_work[block_id(d.xcd)];   // window, first target group, count, source part
+  const int4 lw = d.lrf_work[blockIdx.x];   // window, first target group, count, source part
   const WinState& st = d.ws[lw.x];
   const WinDev& W = d.win[lw.x];
   if (!st.active || !st.list_now || !W.use_lrf) return;   // uniform over the block
@@ -2246,13 +2241,14 @@ __device__ __forceinline__ double watpol_force(const Dev& d, const WinDev& W, fl
   return 0.5 * W.fkwpol * dth * dth;
 }
 
-// up to this many windows per engine a block has 1024 threads, beyond it 256:
-// a wide block shortens the chain (a step of one 1693-water window 153 -> 124
-// us, of 4 177 -> 147, of 16 259 -> 254), but its 16 waves start only on a CU
-// with that many free slots, and among many windows the ranking is not what
-// the step waits for (32 small windows 185 -> 187 us, 64 mixed 583 -> 598).
-// The results do not depend on the block size
-constexpr int kWpolWide = 24;
+// up to this many windows a large engine (kAllMost) has blocks of 1024 threads
+// for the polarisation, in a kernel of their own, beyond it 256, in one kernel
+// with the bonded terms: a wide block shortens the chain, but its 16 waves start
+// only on a CU with that many free slots, and the more windows there are the
+// less the step waits for the ranking.  us a step with 1024 and 256 threads: 8
+// protein windows 124 and 128, 4 + 4 windows 101 and 113, 16 protein windows
+// 197 and 189, 12 + 12 windows 188 and 181.  The results do not depend on it
+constexpr int kWpolWide = 12;
 constexpr int kWpolSum = 256;        // threads of the theta sum (its order is part of the result)
 template <int kWpolBlock>            // threads per (window, shell) block
 struct WpolLds {
@@ -2404,27 +2400,28 @@ __device__ __forceinline__ void watpol_block(const Dev& d, int block, WpolLds<kW
     wave_energy(d.ws, w, E_WPOL, e, on && en);
   }
 }
-template <int kWpolBlock>
-__global__ void __launch_bounds__(kWpolBlock) k_watpol(Dev d) {
-  __shared__ WpolLds<kWpolBlock> L;
-  watpol_block<kWpolBlock>(d, blockIdx.x, L);
+__global__ void __launch_bounds__(1024) k_watpol(Dev d) {
+  __shared__ WpolLds<1024> L;
+  watpol_block<1024>(d, blockIdx.x, L);
 }
 
 // ------------------------------------------------ all forces at once --
 // Engines whose step is too small to fill the GPU run every force kernel of a
 // step as one launch, each block taking one kind of work (by block index, the
 // longest kinds first): a step then takes as long as its slowest kind, where
-// separate launches, on three streams, add up with the gaps between them.
-// us a step, separate and one launch: one ligand-in-water window 75 and 53, one
-// protein window 107 and 74, 11 small windows 97 and 68, 8 protein windows 161
-// and 133.  128 registers (the bonded terms spill 42) keep two blocks on a CU;
-// with twice as many the 8 windows take 162.
+// separate launches add up with the gaps between them.
+// us a step, nine launches and one: one ligand-in-water window 75 and 53, one
+// protein window 107 and 74, 11 small windows 97 and 68.  128 registers (the
+// bonded terms spill 42) keep two blocks on a CU.
 constexpr int kAllBlock = 512;       // 8 waves: two q items, 8 row clusters
-// an engine of more blocks fills the GPU with separate launches, whose pair
-// kernels have more waves in flight: 16 + 16 windows (3400 blocks) 274 and
-// 270, 64 small windows (3200) 221 and 206, 32 protein windows (5300) 406 and
-// 440.  The results do not depend on it
-constexpr int kAllMost = 3500;
+// an engine of more blocks fills the GPU with the launches of a large engine
+// (k_pairs), whose pair waves need fewer registers, so that more of them are in
+// flight.  us a step, one launch and those: 11 small windows (550 blocks) 65 and
+// 82, 4 protein windows (660) 91 and 96, 20 small windows (1000) 93 and 100, 8
+// protein windows (1330) 129 and 124, 32 small windows (1600) 123 and 124, 16
+// protein windows 223 and 189, 64 small windows 210 and 200.  The results do not
+// depend on it
+constexpr int kAllMost = 1200;
 struct AllPlan {
   int wpol, bonded, qp, qw, srow, wrow, qq, rst, terms;   // first block of each kind
   int total;
@@ -2470,9 +2467,69 @@ __global__ void __launch_bounds__(kAllBlock, 4) k_all(Dev d, AllPlan p) {
   watpol_block<kAllBlock>(d, b, L.wpol);
 }
 
+// -------------------------------------------- forces of a large engine --
+// A step of an engine that fills the GPU takes two launches, side by side: the
+// pair forces with the per-atom terms, whose waves need few registers and
+// issue most of the step's instructions, and the few latency-bound blocks of
+// the water polarisation with the bonded terms.  The rows come first, which
+// run longest, then the q items, then the short waves that fill the end.
+// As nine launches on three streams the kernels queued behind each other on
+// each stream and the last ones ran with the GPU half empty: 16 + 16 windows
+// 264 us a step, now 233, 32 protein windows 393 and 378, the 64-window ladder
+// 485 and 473.  The q items first: 244, 384, 475.  The bonded terms as a
+// kernel of their own behind the polarisation: 245, 396, 479; on a third
+// stream 258, 407, 496.
+struct PairPlan {
+  int srow, qw, qp, qq, terms;   // first block of each kind; the water rows come first
+  int total;
+};
+constexpr int kPairBlock = 64 * kQWaves;   // a q item, 4 row clusters
+static PairPlan pair_plan(const Dev& d, bool energy, bool terms) {
+  PairPlan p;
+  int n = 0;
+  auto take = [&](int& first, long long work, int per_block) {
+    first = n;
+    n += (int)((work + per_block - 1) / per_block);
+  };
+  const int waves = kPairBlock / 64;
+  int wrow;
+  take(wrow, d.rl[T_WW].nicl, waves);
+  take(p.srow, d.rl[T_PP].nicl, waves);
+  take(p.qw, d.nqw_work, 1);
+  take(p.qp, d.nqp_work, 1);
+  take(p.qq, qq_waves(d, energy), waves);
+  take(p.terms, terms ? d.ntot : 0, kPairBlock);
+  p.total = n;
+  return p;
+}
+// (windows with a 3-atom solvent have instances of the row and q kernels of
+// their own, launched after this one)
+template <bool EK>
+__global__ void __launch_bounds__(kPairBlock, EK ? 4 : 6) k_pairs(Dev d, PairPlan p) {
+  __shared__ double s_q[9 * 64 * kQWaves];
+  const int b = blockIdx.x, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  constexpr int kWaves = kPairBlock / 64;
+  if (b >= p.terms) return atom_terms<true>(d, (b - p.terms) * kPairBlock + (int)threadIdx.x);
+  if (b >= p.qq) return qq_wave<EK>(d, (b - p.qq) * kWaves + wv);
+  if (b >= p.qp) return qp_group<EK>(d, b - p.qp, s_q);
+  if (b >= p.qw) return qw_group<false, EK>(d, b - p.qw, s_q);
+  if (b >= p.srow) return srow_wave<false, EK>(d, (b - p.srow) * kWaves + wv);
+  wrow_wave<false, EK, 3>(d, b * kWaves + wv);
+}
+// polarisation blocks first: they take longest
+__global__ void __launch_bounds__(256) k_other(Dev d, int nwp) {
+  __shared__ union {
+    WpolLds<256> wpol;
+    struct { unsigned long long acc[3 * kBondSpan], e[E_NSLOT]; } bonded;
+  } L;
+  const int b = blockIdx.x;
+  if (b >= nwp) return bonded_tile(d, b - nwp, L.bonded.acc, L.bonded.e);
+  watpol_block<256>(d, b, L.wpol);
+}
+
 // the FP32 coordinates of atom i from its FP64 ones, into x32 and, for a
-// water atom, into its cluster slot (with the FP64 ones), for a q-atom into
-// its q-cluster slot
+// water or solute atom, into its cluster slot (with the FP64 ones), for a q-atom
+// into its q-cluster slot
 __device__ __forceinline__ void store_x32_xyz(const Dev& d, int i, double x, double y, double z) {
   const float4 q = d.x32[i];
   const float4 n = make_float4((float)x, (float)y, (float)z, q.w);
@@ -2830,11 +2887,6 @@ void launch_lrf_build(const Dev& d, hipStream_t s) {
   k_lrf_reduce<<<blocks(d.ngrp_all, kLrfReduceGroups), kLrfReduceGroups * kLrfSums, 0, s>>>(d);
 }
 
-void launch_bonded(const Dev& d, hipStream_t s) {
-  if (d.nbtile) k_bonded<<<d.nbtile, 256, 0, s>>>(d);
-  if (d.nrst) k_prestr<<<d.nrst, 64, 0, s>>>(d);
-}
-
 // list update: group centres and cluster spheres, then the neighbour rows
 // and the LRF expansions (independent of each other)
 static void launch_list_prep(const Dev& d, hipStream_t s, int ngrp, int nwc, int nsc) {
@@ -2853,14 +2905,18 @@ void launch_lists(const Dev& d, hipStream_t s, int ngrp, int nwc, int nsc) {
 }
 
 // the q-atoms against water and solute; `energy`: the instances that also
-// evaluate the energy terms of windows at an energy step
+// evaluate the energy terms of windows at an energy step.  launch_*3: the
+// instances for windows with a 3-atom solvent
+static void launch_qw3(const Dev& d, hipStream_t s, bool energy) {
+  if (!d.nqw_work) return;
+  if (energy) k_qw<true, true><<<d.nqw_work, 64 * kQWaves, 0, s>>>(d);
+  else k_qw<true, false><<<d.nqw_work, 64 * kQWaves, 0, s>>>(d);
+}
 static void launch_qw(const Dev& d, hipStream_t s, bool energy) {
   if (!d.nqw_work) return;
   if (energy) k_qw<false, true><<<d.nqw_work, 64 * kQWaves, 0, s>>>(d);
   else k_qw<false, false><<<d.nqw_work, 64 * kQWaves, 0, s>>>(d);
-  if (!d.any_wat3) return;
-  if (energy) k_qw<true, true><<<d.nqw_work, 64 * kQWaves, 0, s>>>(d);
-  else k_qw<true, false><<<d.nqw_work, 64 * kQWaves, 0, s>>>(d);
+  if (d.any_wat3) launch_qw3(d, s, energy);
 }
 static void launch_qp(const Dev& d, hipStream_t s, bool energy) {
   if (!d.nqp_work) return;
@@ -2873,11 +2929,18 @@ void launch_q(const Dev& d, hipStream_t s, bool energy) {
 }
 
 // water rows; part: k_wrow's PART
+constexpr int kRowBlock = 256;   // 4 clusters
 template <bool EK, int PART>
 static void launch_wrow_k(const Dev& d, hipStream_t s) {
-  const int nb = blocks((long long)d.rl[T_WW].nicl * 64, d.bs_rows);
-  if (d.rl[T_WW].nicl) k_wrow<false, EK, PART><<<nb, d.bs_rows, 0, s>>>(d);
-  if (d.rl[T_WW].nicl && d.any_wat3) k_wrow<true, EK, PART><<<nb, d.bs_rows, 0, s>>>(d);
+  const int nb = blocks((long long)d.rl[T_WW].nicl * 64, kRowBlock);
+  if (d.rl[T_WW].nicl) k_wrow<false, EK, PART><<<nb, kRowBlock, 0, s>>>(d);
+  if (d.rl[T_WW].nicl && d.any_wat3) k_wrow<true, EK, PART><<<nb, kRowBlock, 0, s>>>(d);
+}
+static void launch_wrow3(const Dev& d, hipStream_t s, bool energy) {
+  const int nb = blocks((long long)d.rl[T_WW].nicl * 64, kRowBlock);
+  if (!d.rl[T_WW].nicl) return;
+  if (energy) k_wrow<true, true, 3><<<nb, kRowBlock, 0, s>>>(d);
+  else k_wrow<true, false, 3><<<nb, kRowBlock, 0, s>>>(d);
 }
 static void launch_wrow(const Dev& d, hipStream_t s, bool energy) {
   if (energy) launch_wrow_k<true, 3>(d, s);
@@ -2890,9 +2953,15 @@ void launch_ww(const Dev& d, hipStream_t s, bool energy) {
 // solute rows
 template <bool EK>
 static void launch_srow_k(const Dev& d, hipStream_t s) {
-  const int nb = blocks((long long)d.rl[T_PP].nicl * 64, d.bs_rows);
-  if (d.rl[T_PP].nicl) k_srow<false, EK><<<nb, d.bs_rows, 0, s>>>(d);
-  if (d.rl[T_PP].nicl && d.any_wat3) k_srow<true, EK><<<nb, d.bs_rows, 0, s>>>(d);
+  const int nb = blocks((long long)d.rl[T_PP].nicl * 64, kRowBlock);
+  if (d.rl[T_PP].nicl) k_srow<false, EK><<<nb, kRowBlock, 0, s>>>(d);
+  if (d.rl[T_PP].nicl && d.any_wat3) k_srow<true, EK><<<nb, kRowBlock, 0, s>>>(d);
+}
+static void launch_srow3(const Dev& d, hipStream_t s, bool energy) {
+  const int nb = blocks((long long)d.rl[T_PP].nicl * 64, kRowBlock);
+  if (!d.rl[T_PP].nicl) return;
+  if (energy) k_srow<true, true><<<nb, kRowBlock, 0, s>>>(d);
+  else k_srow<true, false><<<nb, kRowBlock, 0, s>>>(d);
 }
 static void launch_srow(const Dev& d, hipStream_t s, bool energy) {
   if (energy) launch_srow_k<true>(d, s);
@@ -2907,14 +2976,15 @@ void launch_nonbonded(const Dev& d, hipStream_t s, bool with_ww, bool q_energy) 
   launch_qq(d, s, q_energy);
 }
 
-static void launch_watpol(const Dev& d, hipStream_t s) {
-  if (!d.nwat_total) return;
-  if (d.nwin <= kWpolWide) k_watpol<1024><<<d.nwin * kWpolMaxShell, 1024, 0, s>>>(d);
-  else k_watpol<256><<<d.nwin * kWpolMaxShell, 256, 0, s>>>(d);
-}
 void launch_other_forces(const Dev& d, hipStream_t s) {
-  launch_watpol(d, s);
-  launch_bonded(d, s);
+  const int nwp = d.nwat_total ? d.nwin * kWpolMaxShell : 0;
+  if (d.nwin <= kWpolWide) {
+    if (nwp) k_watpol<<<nwp, 1024, 0, s>>>(d);
+    if (d.nbtile) k_bonded<<<d.nbtile, 256, 0, s>>>(d);
+  } else if (nwp + d.nbtile) {
+    k_other<<<nwp + d.nbtile, 256, 0, s>>>(d, nwp);
+  }
+  if (d.nrst) k_prestr<<<d.nrst, 64, 0, s>>>(d);
 }
 // the per-atom terms of an evaluation, after all its other kernels: completes
 // the gradient
@@ -2922,28 +2992,6 @@ static void launch_complete(const Dev& d, hipStream_t s) {
   if (d.ntot) k_atom_terms<false><<<blocks(d.ntot, 256), 256, 0, s>>>(d);
 }
 
-// The lists and forces of an MD step, or of an evaluation (eval: the per-atom
-// terms come last and complete the gradient), on three streams:
-//   s:  on list steps the group centres and the water rows; then the water
-//       rows' forces, the per-atom terms, and the q-atoms against solute;
-//   s2: water polarisation (few latency-bound blocks, which start beside the
-//       large kernels of the other streams), q-q pairs, bonded terms and
-//       restraints; on list steps, once every other kernel of the step is
-//       done, the LRF expansions and then the per-atom terms;
-//   s3: on list steps the solute rows, after the group centres; then the
-//       q-atoms against water and the solute rows' forces.
-// s then waits for s2 and s3.  The kernels' times alone add up to about the
-// same on each stream, so none is left to run by itself at the end (64-window
-// ladder, us a step: 512; bonded terms behind the water rows on s 533; water
-// polarisation last on s2 549; q-atoms against water behind the bonded terms
-// 527).
-// The LRF build comes last because it fills every CU for more than a
-// millisecond of FP64 work: beside the row builds and pair kernels it starves
-// them (they wait for its long-running blocks), and cutting its occupancy so
-// that they fit slows it more than it frees them.
-// The kernels write the energies and the shared gradient only through integer
-// atomic adds, and everything else to buffers of their own, which the
-// integrator adds, so the result does not depend on how they overlap.
 static void launch_all(const Dev& d, hipStream_t s, bool energy, bool terms) {
   const AllPlan p = all_plan(d, energy, terms);
   if (!p.total) return;
@@ -2959,7 +3007,7 @@ bool small_engine(const Dev& d, bool mixed_solvent) { return !mixed_solvent && a
 
 // the lists and forces of a small engine: one launch for the forces, and on
 // list steps the LRF expansions beside the rows and the forces
-static hipError_t launch_small_forces(const Dev& d, hipStream_t s, hipStream_t s2, const hipEvent_t ev[5], bool lists,
+static hipError_t launch_small_forces(const Dev& d, hipStream_t s, hipStream_t s2, const hipEvent_t ev[2], bool lists,
                                       int ngrp, int nwc, int nsc, bool energy, bool eval) {
   if (!eval) launch_offdiag(d, s);
   if (lists) {
@@ -2986,42 +3034,53 @@ static hipError_t launch_small_forces(const Dev& d, hipStream_t s, hipStream_t s
   return hipSuccess;
 }
 
-hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, hipStream_t s3, const hipEvent_t ev[5],
-                              bool lists, int ngrp, int nwc, int nsc, bool q_energy, bool eval) {
-  if (d.small) return launch_small_forces(d, s, s2, ev, lists, ngrp, nwc, nsc, q_energy, eval);
+// the pair forces (terms: with the per-atom terms)
+static void launch_pairs(const Dev& d, hipStream_t s, bool energy, bool terms) {
+  const PairPlan p = pair_plan(d, energy, terms);
+  if (p.total) {
+    if (energy) k_pairs<true><<<p.total, kPairBlock, 0, s>>>(d, p);
+    else k_pairs<false><<<p.total, kPairBlock, 0, s>>>(d, p);
+  }
+  if (d.any_wat3) {
+    launch_qw3(d, s, energy);
+    launch_wrow3(d, s, energy);
+    launch_srow3(d, s, energy);
+  }
+}
+
+// The lists and forces of an MD step, or of an evaluation (eval: the per-atom
+// terms come last and complete the gradient), on two streams:
+//   s:  on list steps the group centres and the rows; the pair forces; on list
+//       steps the LRF expansions and then the per-atom terms;
+//   s2: water polarisation, bonded terms and restraints.
+// s then waits for s2.  The LRF build comes last because it fills every CU for
+// more than a millisecond of FP64 work: beside the row builds and pair kernels
+// it starves them (they wait for its long-running blocks), and cutting its
+// occupancy so that they fit slows it more than it frees them.
+// The kernels write the energies and the shared gradient only through integer
+// atomic adds, and everything else to buffers of their own, which the
+// integrator adds, so the result does not depend on how they overlap.
+hipError_t launch_step_forces(const Dev& d, hipStream_t s, hipStream_t s2, const hipEvent_t ev[2], bool lists, int ngrp,
+                              int nwc, int nsc, bool energy, bool eval) {
+  if (d.small) return launch_small_forces(d, s, s2, ev, lists, ngrp, nwc, nsc, energy, eval);
   hipError_t err = hipEventRecord(ev[0], s);
   if (err == hipSuccess) err = hipStreamWaitEvent(s2, ev[0], 0);
-  if (err == hipSuccess && !lists) err = hipStreamWaitEvent(s3, ev[0], 0);
   if (err != hipSuccess) return err;
   if (!eval) launch_offdiag(d, s2);
+  launch_other_forces(d, s2);
+  err = hipEventRecord(ev[1], s2);
+  if (err != hipSuccess) return err;
   if (lists) {
     launch_list_prep(d, s, ngrp, nwc, nsc);
     launch_list_rows(d, s);
-    err = hipEventRecord(ev[2], s);
-    if (err == hipSuccess) err = hipStreamWaitEvent(s3, ev[2], 0);
-    if (err != hipSuccess) return err;
   }
-  launch_watpol(d, s2);
-  launch_qq(d, s2, q_energy);
-  launch_bonded(d, s2);
-  launch_wrow(d, s, q_energy);
-  launch_qw(d, s3, q_energy);
-  launch_srow(d, s3, q_energy);
-  err = hipEventRecord(ev[1], s3);
-  if (err != hipSuccess) return err;
-  if (!lists && !eval) launch_atom_terms(d, s);
-  launch_qp(d, s, q_energy);
-  if (lists) {
-    err = hipEventRecord(ev[4], s);
-    if (err == hipSuccess) err = hipStreamWaitEvent(s2, ev[4], 0);
-    if (err == hipSuccess) err = hipStreamWaitEvent(s2, ev[1], 0);
-    if (err != hipSuccess) return err;
-    launch_lrf_build(d, s2);
-    if (!eval) launch_atom_terms(d, s2);
+  const bool lrf = lists && d.any_lrf;
+  launch_pairs(d, s, energy, !eval && !lrf);
+  if (lrf) {
+    launch_lrf_build(d, s);
+    if (!eval) launch_atom_terms(d, s);
   }
-  err = hipEventRecord(ev[3], s2);
-  if (err == hipSuccess) err = hipStreamWaitEvent(s, ev[1], 0);
-  if (err == hipSuccess) err = hipStreamWaitEvent(s, ev[3], 0);
+  err = hipStreamWaitEvent(s, ev[1], 0);
   if (err == hipSuccess && eval) launch_complete(d, s);
   return err;
 }
