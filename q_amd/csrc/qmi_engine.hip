@@ -48,6 +48,12 @@ namespace {
 
 // steps per drain of the energy / temperature ring
 constexpr int kChunk = 64;
+// steps without energies and list updates that are launched with the step
+// before them: the GPU idles 4 us between two graphs.  Energy, output and list
+// intervals are mostly multiples of 5.  us a step of one ligand-in-water window
+// with 0, 1, 3, 4 and 7 such steps, energies every 5: 51.8,
+// 50.5, 49.6, 48.7, 52.5
+constexpr int kPlainSteps = 4;
 
 struct HostWin {
   std::unique_ptr<Window> w;
@@ -94,11 +100,12 @@ struct qmi_engine {
   // whether qmi_prepare times the kernel families of a large engine
   bool autotune = true;
   double tune_us[6] = {0, 0, 0, 0, 0, 0};
-  // the launch sequence of one MD step, captured once and replayed: index
-  // bit 0 with the pair-list and LRF kernels (some window updates its lists),
-  // bit 1 with the q-side energy passes (some window computes energies)
-  hipGraph_t step_graph[4] = {nullptr, nullptr, nullptr, nullptr};
-  hipGraphExec_t step_exec[4] = {nullptr, nullptr, nullptr, nullptr};
+  // the launch sequence of one MD step, captured when first needed and
+  // replayed: index bit 0 with the pair-list and LRF kernels (some window
+  // updates its lists), bit 1 with the energy terms (some window computes
+  // energies); bit 2: that step and kPlainSteps without either
+  hipGraph_t step_graph[8] = {};
+  hipGraphExec_t step_exec[8] = {};
   bool graph_failed = false;
   std::vector<int> nbcycle;   // per window, as on the device
   // ring drain: a chunk's records are copied on copy_stream into pinned
@@ -139,7 +146,7 @@ static int dev_alloc(qmi_engine* e, T** dst, size_t n) {
 }
 
 qmi_engine::~qmi_engine() {
-  for (int k = 0; k < 4; ++k) {
+  for (int k = 0; k < 8; ++k) {
     if (step_exec[k]) (void)hipGraphExecDestroy(step_exec[k]);
     if (step_graph[k]) (void)hipGraphDestroy(step_graph[k]);
   }
@@ -1773,7 +1780,7 @@ int qmi_run(qmi_engine* e, long long nsteps, int finalize) {
   launch_begin(e->d, e->stream, 0, 0);
   // one step = the same kernels with the same arguments every time (the
   // kernels read per-window step state from device memory), so outside the
-  // timing pass it runs as one captured graph
+  // timing pass steps run as captured graphs
   auto launch_step = [&](int variant) {
     const bool lists = variant & 1, qen = variant & 2;
     // lists and forces on two streams; a failure here fails the capture
@@ -1782,34 +1789,27 @@ int qmi_run(qmi_engine* e, long long nsteps, int finalize) {
       return;
     launch_integrate(e->d, e->stream, e->shake_any, variant);
   };
-  if (!e->timing_on && !e->step_exec[0] && !e->graph_failed) {
-    bool ok = true;
-    for (int k = 0; k < 4 && ok; ++k) {
-      hipGraph_t g = nullptr;
-      ok = hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal) == hipSuccess;
-      if (ok) {
-        launch_step(k);
-        ok = hipStreamEndCapture(e->stream, &g) == hipSuccess && g != nullptr;
-      }
-      if (ok) ok = hipGraphInstantiate(&e->step_exec[k], g, nullptr, nullptr, 0) == hipSuccess;
-      if (ok) {
-        e->step_graph[k] = g;
-      } else if (g) {
-        (void)hipGraphDestroy(g);
-      }
+  auto have_graph = [&](int k) -> bool {
+    if (e->step_exec[k]) return true;
+    if (e->graph_failed) return false;
+    hipGraph_t g = nullptr;
+    bool ok = hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal) == hipSuccess;
+    if (ok) {
+      launch_step(k & 3);
+      for (int r = 0; r < (k & 4 ? kPlainSteps : 0); ++r) launch_step(0);
+      ok = hipStreamEndCapture(e->stream, &g) == hipSuccess && g != nullptr;
     }
-    if (!ok) {
-      // run with direct launches instead
-      for (int k = 0; k < 4; ++k) {
-        if (e->step_exec[k]) (void)hipGraphExecDestroy(e->step_exec[k]);
-        if (e->step_graph[k]) (void)hipGraphDestroy(e->step_graph[k]);
-        e->step_exec[k] = nullptr;
-        e->step_graph[k] = nullptr;
-      }
-      e->graph_failed = true;
+    if (ok) ok = hipGraphInstantiate(&e->step_exec[k], g, nullptr, nullptr, 0) == hipSuccess;
+    if (ok) {
+      e->step_graph[k] = g;
+    } else {
+      if (g) (void)hipGraphDestroy(g);
+      e->step_exec[k] = nullptr;
+      e->graph_failed = true;   // the steps are then launched one by one
       (void)hipGetLastError();
     }
-  }
+    return ok;
+  };
   // whether any window updates its pair lists at step `k` of this run (the
   // condition k_begin evaluates per window; k_begin flags a window whose
   // update would be skipped)
@@ -1896,11 +1896,23 @@ int qmi_run(qmi_engine* e, long long nsteps, int finalize) {
     int chunk = (int)std::min<long long>(kChunk, nsteps - done);
     for (int k = 0; k < chunk; ++k)
       if ((any_trj && any_frame(done + k)) || any_backup(done + k)) { chunk = k + 1; break; }
-    if (!e->timing_on && e->step_exec[0]) {
-      for (int k = 0; k < chunk; ++k)
-        HIP_OK(hipGraphLaunch(e->step_exec[(lists_at(done + k) ? 1 : 0) | (energy_at(done + k) ? 2 : 0)], e->stream));
+    if (!e->timing_on) {
+      int kind[kChunk];
+      for (int k = 0; k < chunk; ++k) kind[k] = (lists_at(done + k) ? 1 : 0) | (energy_at(done + k) ? 2 : 0);
+      for (int k = 0; k < chunk; ++k) {
+        int plain = 0;
+        while (plain < kPlainSteps && k + plain + 1 < chunk && kind[k + plain + 1] == 0) ++plain;
+        if (plain == kPlainSteps && have_graph(kind[k] | 4)) {
+          HIP_OK(hipGraphLaunch(e->step_exec[kind[k] | 4], e->stream));
+          k += kPlainSteps;
+        } else if (have_graph(kind[k])) {
+          HIP_OK(hipGraphLaunch(e->step_exec[kind[k]], e->stream));
+        } else {
+          launch_step(kind[k]);
+        }
+      }
     }
-    for (int k = 0; k < chunk && (e->timing_on || !e->step_exec[0]); ++k) {
+    for (int k = 0; k < chunk && e->timing_on; ++k) {
       // the same kernel instances as the step graph of this step: those
       // with energy terms only where some window computes energies
       const bool qen = energy_at(done + k);
