@@ -119,6 +119,9 @@ constexpr int kTempParts = 8;      // blocks per window of the kinetic-energy su
 constexpr int kLrfParts = 4;
 constexpr int kLrfWaves = 8;
 constexpr int kIntBlock = 256;     // atoms per block of the integrator
+// bits of a three-constraint unit: its first entry within the block, the places
+// of a, b and c among its atoms, and that it is one
+constexpr int kTriFirst = 0xff, kTriA = 8, kTriB = 10, kTriC = 12, kTri = 1 << 14;
 constexpr int kWpolMaxShell = 8;
 constexpr int kWpolLds = 4096;     // waters of one polarisation shell held (and ordered) in LDS
 constexpr int kBondTileTerms = 512; // bonded terms per tile
@@ -296,12 +299,19 @@ struct Dev {
   const float2* sc_w;      // per constraint: inverse masses of i and j
   const uint8_t* sc_loc;   // per constraint: local atom numbers of i and j within the unit
   // integration units of k_integrate, each a SHAKE component or one
-  // unconstrained atom: (window, first entry in iu_atom, number of atoms,
-  // SHAKE unit or -1); a component's atoms are listed in the order its
-  // sc_loc numbers them.  Blocks of k_integrate: runs of whole units of at
-  // most kIntBlock atoms, (first iu_atom entry, atoms, first unit, units)
+  // unconstrained atom: (window, first entry, number of atoms, SHAKE unit or
+  // -1); a component's atoms are listed in the order its sc_loc numbers them.
+  // Blocks of k_integrate: runs of whole units of at most kIntBlock atoms,
+  // (first entry, atoms, first unit, units)
   int niu, nib;
-  const int4* iu; const int* iu_atom; const int4* ib;
+  const int4* iu; const int4* ib;
+  // per entry, what the integrator needs of the atom: (atom, window, rslot,
+  // wslot), (charge, inverse mass, qmslot, 1 solute | 2 excluded), mass
+  const int4* ie_i; const float4* ie_f; const double* ie_m;
+  // per unit: for three constraints among three atoms, the squared distances
+  // and (inverse masses of a, b and c, kTri bits), the constraints being a-b,
+  // a-c and b-c in their order; kTri 0 for other units
+  const double* tri_d2; const float4* tri;
   // water shells
   ShellDev* shells;
   double* wtheta;        // windows of more than kWpolLds waters: theta per shell and water, at WinDev::wp_off

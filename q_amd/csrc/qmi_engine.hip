@@ -823,11 +823,12 @@ static int build_device(qmi_engine* e) {
     UP(rp, sp_rng); d.sp_rng = rp;
   }
   UP(ip, wc_o); d.wc_o = ip;
+  std::vector<int> wslot, rslot, qmslot;   // per atom (Dev)
   // coordinates and LJ columns in cluster-slot order (the row kernels' gathers
   // of neighbours then read contiguous memory)
   {
     const size_t nw3 = 3 * wc_o.size(), ns = sc_a.size();
-    std::vector<int> wslot(x32.size(), -1);
+    wslot.assign(x32.size(), -1);
     std::vector<float4> xw(std::max<size_t>(1, nw3 + ns), make_float4(0.f, 0.f, 0.f, 0.f));
     std::vector<double4> xwd(xw.size(), make_double4(0.0, 0.0, 0.0, 0.0));
     std::vector<float4> sljp(std::max<size_t>(1, ns), make_float4(0.f, 0.f, 0.f, 0.f));
@@ -857,7 +858,7 @@ static int build_device(qmi_engine* e) {
   UP(ip, sc_a); d.sc_a = ip;
   {
     // entries of the row buffers
-    std::vector<int> rslot(x32.size(), -1);
+    rslot.assign(x32.size(), -1);
     d.nwslot = (int)wc_o.size();
     for (size_t m = 0; m < wc_o.size(); ++m)
       for (int k = 0; k < 3 && wc_o[m] >= 0; ++k) rslot[wc_o[m] + k] = 3 * (int)m + k;
@@ -909,7 +910,7 @@ static int build_device(qmi_engine* e) {
     UP(ip, qc_atom); d.qc_atom = ip;
     // q-atom coordinates per q-cluster member slot, kept with x32
     {
-      std::vector<int> qmslot(x32.size(), -1);
+      qmslot.assign(x32.size(), -1);
       std::vector<float4> xq(std::max<size_t>(1, qc_atom.size()), make_float4(0.f, 0.f, 0.f, 0.f));
       for (size_t m = 0; m < qc_atom.size(); ++m)
         if (qc_atom[m] >= 0) {
@@ -1141,10 +1142,42 @@ static int build_device(qmi_engine* e) {
       ib.back().y += iu[u].z;
       ib.back().w += 1;
     }
+    // the entries' records, and the units of three constraints among three
+    // atoms: a is the atom that the first two share
+    auto bits = [](int v) { float f; std::memcpy(&f, &v, 4); return f; };
+    std::vector<int4> ie_i(iu_atom.size());
+    std::vector<float4> ie_f(iu_atom.size());
+    std::vector<double> ie_m(iu_atom.size());
+    for (size_t k = 0; k < iu_atom.size(); ++k) {
+      const int at = iu_atom[k], w = wid[at];
+      ie_i[k] = make_int4(at, w, rslot[at], wslot[at]);
+      ie_f[k] = make_float4(x32[at].w, winv[at], bits(qmslot[at]),
+                            bits((at - wd[w].ao < wd[w].nat_solute ? 1 : 0) | (aflag[at] & 1 ? 2 : 0)));
+      ie_m[k] = mass[at];
+    }
+    std::vector<double> tri_d2(3 * iu.size(), 0.0);
+    std::vector<float4> tri(iu.size(), make_float4(0.f, 0.f, 0.f, bits(0)));
+    size_t blk = 0;
+    for (int u = 0; u < (int)iu.size(); ++u) {
+      while (u >= ib[blk].z + ib[blk].w) ++blk;
+      const int su = iu[u].w;
+      if (su < 0 || su_n[su] != 3 || iu[u].z != 3) continue;
+      const uint8_t* l = &sc_loc[2 * (size_t)su_start[su]];
+      const bool first = l[2] == l[0] || l[3] == l[0];        // the first atom is in the second constraint
+      const int a = first ? l[0] : l[1], b2 = first ? l[1] : l[0], c = 3 - a - b2;
+      auto pair = [&](int k, int p, int q) { return (l[2 * k] == p && l[2 * k + 1] == q) || (l[2 * k] == q && l[2 * k + 1] == p); };
+      if (l[0] > 2 || l[1] > 2 || l[0] == l[1] || !pair(1, a, c) || !pair(2, b2, c)) continue;
+      auto inv = [&](int p) { return winv[iu_atom[iu[u].y + p]]; };
+      for (int k = 0; k < 3; ++k) tri_d2[3 * u + k] = sc_d2[su_start[su] + k];
+      tri[u] = make_float4(inv(a), inv(b2), inv(c),
+                           bits((iu[u].y - ib[blk].x) | a << kTriA | b2 << kTriB | c << kTriC | kTri));
+    }
+    float4* fp4;
+    UP(i4, ie_i); d.ie_i = i4; UP(fp4, ie_f); d.ie_f = fp4; UP(dp, ie_m); d.ie_m = dp;
+    UP(dp, tri_d2); d.tri_d2 = dp; UP(fp4, tri); d.tri = fp4;
     d.niu = (int)iu.size();
     d.nib = (int)ib.size();
     UP(i4, iu); d.iu = i4;
-    UP(ip, iu_atom); d.iu_atom = ip;
     UP(i4, ib); d.ib = i4;
   }
   UP(dp, sc_d2); d.sc_d2 = dp;
