@@ -257,11 +257,11 @@ def main():
         "autotune": tuning,
         "roofline": {
             "bound": "valu_fp32",
-            "kernel": "k_ww<false, false> (SPC water-water rows, force-only instance; FP32 vector ALU; compute roof = FP32 vector peak)",
+            "kernel": "k_wrow<false, false, 1> (SPC water-water rows alone, force-only instance; FP32 vector ALU; compute roof = FP32 vector peak)",
             "achieved": round(achieved, 4) if achieved else None, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": round(achieved / FP32_PEAK_TFLOPS, 5) if achieved else None,
             "frac_nonpacked": round(achieved / FP32_NONPACKED_TFLOPS, 5) if achieved else None,
-            "traffic": traffic_per_launch("k_ww<false, false>"),
+            "traffic": traffic_per_launch("k_wrow<false, false, 1>"),
             "work": {"ww_molecule_pairs_per_step": n_ww_total, "flop_per_pair": 200,
                      "kernel_us_per_launch": round(us_ww, 2),
                      "timing": "50 back-to-back launches at the timed run's lists, HIP events"},

@@ -1188,6 +1188,7 @@ static int build_device(qmi_engine* e) {
   ShellDev* sd;
   UP(sd, shells); d.shells = sd;
   if ((rc = dev_alloc(e, &d.wtheta, (size_t)wp_rows)) != 0) return rc;
+  d.wpol_wide = wp_rows > 0;
   d.nwat_total = e->nwat_total;
   // two chunks of kChunk steps: one drains while the next runs
   d.ring_n = 2 * kChunk;

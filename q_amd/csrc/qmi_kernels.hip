@@ -2184,19 +2184,17 @@ __global__ void __launch_bounds__(64) k_prestr(Dev d) { prestr_wave(d, blockIdx.
 // (window, shell): the waters whose oxygen lies in the shell are collected in
 // LDS with the angle theta between their dipole and the radial vector, each
 // one's place in the order of the reference's first-minimum selection sort
-// (theta ascending, ties by water index) is found by counting the members
-// before it, and the place gives its target angle theta0, energy and forces.
-// The block also advances the shell's theta averages.
+// (theta ascending, ties by water index) gives its target angle theta0, energy
+// and forces.  The block also advances the shell's theta averages.
 //
-// Bound by latency: a shell has a few hundred waters, so counting is
-// n^2 LDS reads over one block.  A member's count is split over as many
-// threads as the block has for it (2 at 400 members), and compares one FP64
-// value per step; ties, which need the indices, are recounted.  As three
-// kernels (angles per water, ranking with a quarter of the threads, forces
-// per water) with the places passed through memory the chain took 30 us alone
-// for one 1109-water window and 65 us for a 1693-water one and was the step's
-// critical path there: a step of one window took 116 and 166 us, now 96 and
-// 124 us.
+// Bound by latency and by the one CU a shell has.  The members are ordered
+// through buckets of theta: a count, a scan of the buckets' first places, and
+// for each member a count of the smaller ones in its own bucket, usually none
+// or one.  Counting the smaller ones among all members took n^2 LDS reads: 25 us
+// alone for a 1693-water window with 1024 threads and most of the 41 us of a
+// step's forces there (512 threads); a step of that window 65.9 -> 53.5 us, of a
+// 1109-water one 43.6 -> 41.1, of 16 of the first 187 -> 181, of the 64-window
+// ladder 445 -> 441.
 __device__ __forceinline__ void water_dipole(const double* x, int i, const double cent[3], double rmu[3], double rcu[3],
                                              double* rm, double* rc) {
   for (int c = 0; c < 3; ++c) rmu[c] = x[3 * (i + 1) + c] + x[3 * (i + 2) + c] - 2. * x[3 * i + c];
@@ -2241,19 +2239,16 @@ __device__ __forceinline__ double watpol_force(const Dev& d, const WinDev& W, fl
   return 0.5 * W.fkwpol * dth * dth;
 }
 
-// up to this many windows a large engine (kAllMost) has blocks of 1024 threads
-// for the polarisation, in a kernel of their own, beyond it 256, in one kernel
-// with the bonded terms: a wide block shortens the chain, but its 16 waves start
-// only on a CU with that many free slots, and the more windows there are the
-// less the step waits for the ranking.  us a step with 1024 and 256 threads: 8
-// protein windows 124 and 128, 4 + 4 windows 101 and 113, 16 protein windows
-// 197 and 189, 12 + 12 windows 188 and 181.  The results do not depend on it
-constexpr int kWpolWide = 12;
 constexpr int kWpolSum = 256;        // threads of the theta sum (its order is part of the result)
+constexpr int kWpolBuckets = 1024;   // of the ordering by theta
+// (any monotone function of theta orders correctly)
+__device__ __forceinline__ int wpol_bucket(double th) {
+  return min(max((int)(th * (kWpolBuckets / 3.1415926535897932)), 0), kWpolBuckets - 1);
+}
 template <int kWpolBlock>            // threads per (window, shell) block
 struct WpolLds {
   double th[kWpolLds];
-  int iw[kWpolLds], rank[kWpolBlock];
+  int iw[kWpolLds], start[kWpolBuckets], wsum[kWpolBlock / 64];
   int n;
   float corr;
   double red[kWpolSum / 64];
@@ -2270,7 +2265,7 @@ __device__ __forceinline__ void watpol_block(const Dev& d, int block, WpolLds<kW
   const ShellDev* shells = d.shells + W.sh_off;
   ShellDev& sh = d.shells[W.sh_off + is];
   double *s_th = L.th, *s_red = L.red;
-  int *s_iw = L.iw, *s_rank = L.rank;
+  int *s_iw = L.iw, *s_start = L.start;
   int& s_n = L.n;
   float& s_corr = L.corr;
   const int t = threadIdx.x;
@@ -2288,7 +2283,7 @@ __device__ __forceinline__ void watpol_block(const Dev& d, int block, WpolLds<kW
     s_corr = sh.theta_corr;
     s_n = 0;
   }
-  s_rank[t] = 0;
+  for (int b = t; b < kWpolBuckets; b += kWpolBlock) s_start[b] = 0;
   __syncthreads();
   // the shell's bounds: waters beyond the innermost radius (a single-precision
   // difference, as the bounds are real(4)) lie in the innermost shell whose
@@ -2321,36 +2316,68 @@ __device__ __forceinline__ void watpol_block(const Dev& d, int block, WpolLds<kW
   double th[kWpolHeld];
   int iw[kWpolHeld], rank[kWpolHeld];
   if (in_lds) {
-    // threads per member: 8, 4, 2 or 1; a part's j are uniform over a wave
-    int span = 128;
-    while (span < n && span < kWpolBlock) span <<= 1;
-    const int parts = kWpolBlock / span, part = t / span, j0 = part * n / parts, j1 = (part + 1) * n / parts;
+    // members per bucket, and each member's place among its bucket's (in any
+    // order)
 #pragma unroll
     for (int m = 0; m < kWpolHeld; ++m) {
-      const int k = t % span + kWpolBlock * m;
+      const int k = t + kWpolBlock * m;
       rank[m] = -1;
       if (k >= n) continue;
       th[m] = s_th[k];
       iw[m] = s_iw[k];
-      int r = 0, eq = 0;
+      rank[m] = atomicAdd(&s_start[wpol_bucket(th[m])], 1);
+    }
+    __syncthreads();
+    // the buckets' first places
+    constexpr int kPer = kWpolBuckets / kWpolBlock;
+    int c[kPer], sum = 0;
+    for (int q = 0; q < kPer; ++q) {
+      c[q] = s_start[kPer * t + q];
+      sum += c[q];
+    }
+    int incl = sum;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o);
+      if ((t & 63) >= o) incl += v;
+    }
+    if ((t & 63) == 63) L.wsum[t >> 6] = incl;
+    __syncthreads();
+    int first = incl - sum;
+    for (int q = 0; q < (t >> 6); ++q) first += L.wsum[q];
+    for (int q = 0; q < kPer; ++q) {
+      s_start[kPer * t + q] = first;
+      first += c[q];
+    }
+    __syncthreads();
+    // the members by bucket
+#pragma unroll
+    for (int m = 0; m < kWpolHeld; ++m) {
+      if (rank[m] < 0) continue;
+      const int k = s_start[wpol_bucket(th[m])] + rank[m];
+      s_th[k] = th[m];
+      s_iw[k] = iw[m];
+    }
+    __syncthreads();
+    // a member's rank: its bucket's first place and the smaller ones of its
+    // bucket (at the same angle the lower water)
+#pragma unroll
+    for (int m = 0; m < kWpolHeld; ++m) {
+      if (rank[m] < 0) continue;
+      const int b = wpol_bucket(th[m]), j0 = s_start[b], j1 = b + 1 < kWpolBuckets ? s_start[b + 1] : n;
+      int r = j0;
       for (int j = j0; j < j1; ++j) {
         const double tj = s_th[j];
-        r += tj < th[m] ? 1 : 0;
-        eq += tj == th[m] ? 1 : 0;
+        r += tj < th[m] || (tj == th[m] && s_iw[j] < iw[m]) ? 1 : 0;
       }
-      if (eq > (k >= j0 && k < j1 ? 1 : 0))   // other members at the same angle
-        for (int j = j0; j < j1; ++j) r += (s_th[j] == th[m] && s_iw[j] < iw[m]) ? 1 : 0;
       rank[m] = r;
-      if (parts > 1) atomicAdd(&s_rank[k], r);
     }
     __syncthreads();
     // the members in order
 #pragma unroll
     for (int m = 0; m < kWpolHeld; ++m) {
-      if (rank[m] < 0 || part != 0) continue;
-      const int r = parts > 1 ? s_rank[t] : rank[m];
-      s_th[r] = th[m];
-      s_iw[r] = iw[m];
+      if (rank[m] < 0) continue;
+      s_th[rank[m]] = th[m];
+      s_iw[rank[m]] = iw[m];
     }
     __syncthreads();
   }
@@ -2416,11 +2443,10 @@ __global__ void __launch_bounds__(1024) k_watpol(Dev d) {
 constexpr int kAllBlock = 512;       // 8 waves: two q items, 8 row clusters
 // an engine of more blocks fills the GPU with the launches of a large engine
 // (k_pairs), whose pair waves need fewer registers, so that more of them are in
-// flight.  us a step, one launch and those: 11 small windows (550 blocks) 65 and
-// 82, 4 protein windows (660) 91 and 96, 20 small windows (1000) 93 and 100, 8
-// protein windows (1330) 129 and 124, 32 small windows (1600) 123 and 124, 16
-// protein windows 223 and 189, 64 small windows 210 and 200.  The results do not
-// depend on it
+// flight.  us a step, one launch and those: 11 small windows (550 blocks) 55 and
+// 72, 4 protein windows (660) 82 and 89, 20 small windows (1000) 78 and 87, 8
+// protein windows (1330) 120 and 115, 32 small windows (1600) 105 and 109, 16
+// protein windows 209 and 181.  The results do not depend on it
 constexpr int kAllMost = 1200;
 struct AllPlan {
   int wpol, bonded, qp, qw, srow, wrow, qq, rst, terms;   // first block of each kind
@@ -3033,9 +3059,12 @@ void launch_nonbonded(const Dev& d, hipStream_t s, bool with_ww, bool q_energy) 
   launch_qq(d, s, q_energy);
 }
 
+// Shells beyond LDS are ordered by counting in memory, for which the blocks are
+// wide; else 256 threads order as fast as 1024 (a step of 8 protein windows 116
+// and 116 us) and share a launch with the bonded terms
 void launch_other_forces(const Dev& d, hipStream_t s) {
   const int nwp = d.nwat_total ? d.nwin * kWpolMaxShell : 0;
-  if (d.nwin <= kWpolWide) {
+  if (d.wpol_wide) {
     if (nwp) k_watpol<<<nwp, 1024, 0, s>>>(d);
     if (d.nbtile) k_bonded<<<d.nbtile, 256, 0, s>>>(d);
   } else if (nwp + d.nbtile) {
