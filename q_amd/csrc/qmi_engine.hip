@@ -2348,6 +2348,9 @@ int qmi_time_kernel(qmi_engine* e, int which, int reps, double* us) {
   hipError_t err = hipEventCreate(&ev[0]);
   if (err == hipSuccess) err = hipEventCreate(&ev[1]);
   if (err == hipSuccess) {
+    // (after a run no window has a step left: the start of a forces-only
+    // evaluation at the current lists makes them all active)
+    launch_begin(e->d, e->stream, 2, 0);
     launch_ww(e->d, e->stream, false);   // first launch untimed
     err = hipEventRecord(ev[0], e->stream);
   }

@@ -2745,6 +2745,11 @@ __device__ __forceinline__ void wave_ekin(const Dev& d, int w, const long long e
   }
 }
 
+// (outside the integrator's contract(off): its sum is fused)
+__device__ __forceinline__ double kinetic(double mass, const double v[3]) {
+  return 0.5 * mass * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
+}
+
 // k_integrate: one block per run of whole integration units (Dev::ib), in
 // three phases.  1: one atom per thread, its gradient and leapfrog, the new
 // and old coordinates into LDS.  2: one unit per thread, the SHAKE sweeps,
@@ -2838,7 +2843,7 @@ __global__ void __launch_bounds__(kIntBlock) k_integrate(Dev d, int post) {
       d.v[3 * i + c] = v[c];
     }
     store_copies(d, i, A.w, __float_as_int(P.z), P.x, x[0], x[1], x[2]);
-    const long long e = fix(0.5 * mass * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]), kEScale);
+    const long long e = fix(kinetic(mass, v), kEScale);
     const bool solute = fl & 1, freeat = !(fl & 2);
     ek[0] += solute ? e : 0ll;
     ek[1] += solute && freeat ? e : 0ll;
