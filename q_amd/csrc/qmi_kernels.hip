@@ -892,12 +892,12 @@ __global__ void __launch_bounds__(256) k_srow(Dev d) {
 // coordinates and parameters are the same for every lane and come through
 // scalar loads.  The q-atoms of a chunk are members 4h .. 4h+3 (h its half) of
 // four consecutive q-clusters, taken member by member: FP32 sums run over the
-// four clusters, what is added up beyond that is FP64, in an order the window
-// alone sets, so the result does not depend on the batch.  The waves' sums
-// are added in LDS and stored in the q row buffer (Dev::gq), which the
-// integrator adds.  Reactions on a q-atom are summed over a cluster's 8 lanes
-// in FP32, over the clusters in FP64, and one atomic per chunk adds them.  On
-// energy steps the same pass adds the per-state energies in FP64.
+// four clusters and go to fixed point, as do the reactions on a q-atom, summed
+// in FP32 over a cluster's 8 lanes; what is added up beyond that are integers,
+// so the gradient depends on neither the batch nor the split into chunks.  The
+// waves' sums are added in LDS and stored in the q row buffer (Dev::gq), which
+// the integrator adds; the reactions take one atomic per chunk.  On energy steps
+// the same pass adds the per-state energies in FP64.
 //
 // Bound by VALU issue (about 150 instructions per 64 pairs with water and
 // two states).  As 8 x 8 tiles with both sides gathered per lane, the q-atom
@@ -906,7 +906,8 @@ __global__ void __launch_bounds__(256) k_srow(Dev d) {
 // more kernels.  Chunks of 16: four waves hold the 50 q-atoms of a ligand.
 // (With a wave per chunk and an atomic per component the kernel took 157 us
 // for the 64-window ladder, all of it atomics.)  64-window ladder, force-only:
-// water 86 + solute 39 + gather 9 us as tiles, now 29 + 26.
+// water 86 + solute 39 + gather 9 us as tiles, now 35 + 40 (31 + 39 when sums
+// beyond the four clusters are FP64, but then their last bits depend on the split).
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 // (12 va - 6 vb) ratio
 __device__ __forceinline__ float lj_f(float va, float vb, float ratio) {
@@ -929,18 +930,18 @@ __device__ __forceinline__ int4 q_item(const int4* work, int block) {
   return make_int4(k[0], k[1], k[2], k[3]);
 }
 // the sums of an item's waves of the N components of its slots into out[N *
-// slot + k]; s: LDS of N * 64 * kQWaves doubles for the group of kQWaves waves.
+// slot + k]; s: LDS of N * 64 * kQWaves integers for the group of kQWaves waves.
 // Every thread of the block calls it; a group without an item has 0 slots.
 template <int N>
-__device__ __forceinline__ void q_store(const double* acc, int slots, long long* out, double* s) {
+__device__ __forceinline__ void q_store(const long long* acc, int slots, long long* out, long long* s) {
   constexpr int kStride = N * 64;
   const int lane = threadIdx.x & 63, wv = (threadIdx.x >> 6) % kQWaves, t = threadIdx.x % (64 * kQWaves);
 #pragma unroll
   for (int k = 0; k < N; ++k) s[wv * kStride + k * 64 + lane] = acc[k];
   __syncthreads();
   for (int i = t; i < N * slots; i += 64 * kQWaves) {
-    const double* p = s + (i % N) * 64 + i / N;
-    out[i] = fix((p[0] + p[kStride]) + (p[2 * kStride] + p[3 * kStride]), kFScale);
+    const long long* p = s + (i % N) * 64 + i / N;
+    out[i] = (p[0] + p[kStride]) + (p[2 * kStride] + p[3 * kStride]);
   }
 }
 
@@ -948,13 +949,13 @@ __device__ __forceinline__ void q_store(const double* acc, int slots, long long*
 // chunk's q-atom j (-r is its gradient), flush() adds them.  Every lane calls
 // both.
 struct QReaction {
-  double v[2] = {0.0, 0.0};   // lane (k, c): component c of q-atoms k and k + 8
+  long long v[2] = {0, 0};   // lane (k, c): component c of q-atoms k and k + 8
   __device__ __forceinline__ void add(int j, float x, float y, float z) {
     x = row8_sum_t(x);
     y = row8_sum_t(y);
     z = row8_sum_t(z);
     const int c = threadIdx.x & 7;
-    const double t = col8_sum_t((double)(c == 0 ? x : c == 1 ? y : z));
+    const long long t = col8_sum_t(fix(-(double)(c == 0 ? x : c == 1 ? y : z), kFScale));
     if ((int)((threadIdx.x >> 3) & 7) == (j & 7)) v[j >> 3] = t;
   }
   // slot0: q-cluster slot of the chunk's first q-atom (j = 4 member + cluster)
@@ -964,14 +965,14 @@ struct QReaction {
     for (int h = 0; h < 2; ++h) {
       const int j = k + 8 * h, m = kCl * (j & 3) + (j >> 2);
       if (c < 3 && m < q_left)
-        atomicAdd((unsigned long long*)&d.f[3 * (size_t)d.qc_atom[slot0 + m] + c], (unsigned long long)fix(-v[h], kFScale));
+        atomicAdd((unsigned long long*)&d.f[3 * (size_t)d.qc_atom[slot0 + m] + c], (unsigned long long)v[h]);
     }
   }
 };
 
 // NS: number of states, or 0 to read it from the window
 template <bool W3, bool EN, int NS>
-__device__ __forceinline__ void qw_impl(const Dev& d, const WinDev& W, const int4 wk, double acc[9]) {
+__device__ __forceinline__ void qw_impl(const Dev& d, const WinDev& W, const int4 wk, long long acc[9]) {
   const int lane = threadIdx.x & 63, w = wk.x;
   const int S = NS ? NS : W.S;
   const bool qvdw = W.qvdw;
@@ -1105,7 +1106,7 @@ __device__ __forceinline__ void qw_impl(const Dev& d, const WinDev& W, const int
         }
         react.add(4 * mb + u, rx, ry, rz);
       }
-      for (int k = 0; k < 9; ++k) acc[k] += (double)g[k];
+      for (int k = 0; k < 9; ++k) acc[k] += fix((double)g[k], kFScale);
     }
     react.flush(d, slot0, W.nq - q0);
   }
@@ -1125,8 +1126,8 @@ __device__ __forceinline__ void qw_impl(const Dev& d, const WinDev& W, const int
 // the barrier).  W3: the instance for 3-atom solvent windows; EK: the instance
 // of steps where some window computes energies
 template <bool W3, bool EK>
-__device__ __forceinline__ void qw_group(const Dev& d, int item, double* s) {
-  double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+__device__ __forceinline__ void qw_group(const Dev& d, int item, long long* s) {
+  long long acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
   int4 wk = make_int4(0, 0, 0, 0);
   if (item < d.nqw_work) {
     wk = q_item(d.qw_work, item);
@@ -1148,12 +1149,12 @@ __device__ __forceinline__ void qw_group(const Dev& d, int item, double* s) {
 }
 template <bool W3, bool EK>
 __global__ void __launch_bounds__(64 * kQWaves) k_qw(Dev d) {
-  __shared__ double s[9 * 64 * kQWaves];
+  __shared__ long long s[9 * 64 * kQWaves];
   qw_group<W3, EK>(d, blockIdx.x, s);
 }
 
 template <bool EN, int NS>
-__device__ __forceinline__ void qp_impl(const Dev& d, const WinDev& W, const int4 wk, double acc[3]) {
+__device__ __forceinline__ void qp_impl(const Dev& d, const WinDev& W, const int4 wk, long long acc[3]) {
   const int lane = threadIdx.x & 63, w = wk.x;
   const int S = NS ? NS : W.S;
   const bool qvdw = W.qvdw, arith = W.arith;
@@ -1251,7 +1252,7 @@ __device__ __forceinline__ void qp_impl(const Dev& d, const WinDev& W, const int
         }
         react.add(j, rx, ry, rz);
       }
-      acc[0] += (double)g0; acc[1] += (double)g1; acc[2] += (double)g2;
+      atom_grad(acc, (double)g0, (double)g1, (double)g2);
     }
     react.flush(d, slot0, W.nq - q0);
   }
@@ -1268,8 +1269,8 @@ __device__ __forceinline__ void qp_impl(const Dev& d, const WinDev& W, const int
 }
 
 template <bool EK>
-__device__ __forceinline__ void qp_group(const Dev& d, int item, double* s) {
-  double acc[3] = {0, 0, 0};
+__device__ __forceinline__ void qp_group(const Dev& d, int item, long long* s) {
+  long long acc[3] = {0, 0, 0};
   int4 wk = make_int4(0, 0, 0, 0);
   if (item < d.nqp_work) {
     wk = q_item(d.qp_work, item);
@@ -1291,7 +1292,7 @@ __device__ __forceinline__ void qp_group(const Dev& d, int item, double* s) {
 }
 template <bool EK>
 __global__ void __launch_bounds__(64 * kQWaves) k_qp(Dev d) {
-  __shared__ double s[3 * 64 * kQWaves];
+  __shared__ long long s[3 * 64 * kQWaves];
   qp_group<EK>(d, blockIdx.x, s);
 }
 
@@ -2477,7 +2478,7 @@ __global__ void __launch_bounds__(kAllBlock, 4) k_all(Dev d, AllPlan p) {
   __shared__ union {
     WpolLds<kAllBlock> wpol;
     struct { unsigned long long acc[3 * kBondSpan], e[E_NSLOT]; } bonded;
-    double q[kAllBlock / (64 * kQWaves)][9 * 64 * kQWaves];
+    long long q[kAllBlock / (64 * kQWaves)][9 * 64 * kQWaves];
   } L;
   const int b = blockIdx.x, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   constexpr int kWaves = kAllBlock / 64, kItems = kWaves / kQWaves;
@@ -2532,7 +2533,7 @@ static PairPlan pair_plan(const Dev& d, bool energy, bool terms) {
 // their own, launched after this one)
 template <bool EK>
 __global__ void __launch_bounds__(kPairBlock, EK ? 4 : 6) k_pairs(Dev d, PairPlan p) {
-  __shared__ double s_q[9 * 64 * kQWaves];
+  __shared__ long long s_q[9 * 64 * kQWaves];
   const int b = blockIdx.x, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   constexpr int kWaves = kPairBlock / 64;
   if (b >= p.terms) return atom_terms<true>(d, (b - p.terms) * kPairBlock + (int)threadIdx.x);

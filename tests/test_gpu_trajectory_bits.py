@@ -1,0 +1,35 @@
+"""Gradient and trajectory to the last bit against committed values: the
+gradient is a sum of integers whose terms do not depend on how the work is
+split, so a change of the kernels' tiling or launches keeps it.  Last-bit
+differences are not harmless in a trajectory: a SHAKE sweep that ends one sweep
+earlier turns a quantum of 2^-32 into 1e-4 A, which grows.
+
+No tolerance: equal bits."""
+import os
+
+import numpy as np
+import pytest
+
+from tests.golden import trajectory_bits as T
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def golden():
+    return np.load(os.path.join(os.path.dirname(T.__file__), "trajectory_bits.npz"))
+
+
+def compare(golden, name, got):
+    for key, (digest, values) in got.items():
+        ref = golden[f"{name}.{key}"]
+        off = int((values != ref).sum())
+        assert off == 0, f"{name} {key}: {off} of {len(ref)} values differ, by up to {np.abs(values - ref).max()}"
+        assert digest == str(golden[f"{name}.{key}.digest"]), f"{name} {key}"
+
+
+@pytest.mark.parametrize("name", [n for n, c in T.CASES.items() if c[0] == T.Q])
+def test_q_sums(systems, golden, name):
+    from q_amd.engine import Engine
+    (got,) = T.record(Engine, [T.window(systems, name)])
+    compare(golden, name, got)
