@@ -113,11 +113,9 @@ enum RowType { T_WW = 0, T_WP, T_PW, T_PP, T_NTYPES };
 // T_free solute, T_free solvent
 constexpr int kTRing = 6;
 constexpr int kTempParts = 8;      // blocks per window of the kinetic-energy sum
-// the LRF build splits a window's source groups in kLrfParts parts (blocks) of
-// kLrfWaves shares (waves), summed in a fixed order; constants, so the
-// expansions do not depend on launch shapes
-constexpr int kLrfParts = 4;
-constexpr int kLrfWaves = 8;
+// the LRF build splits a window's source groups in this many parts, summed in
+// part order; a constant, so the expansions do not depend on launch shapes
+constexpr int kLrfParts = 8;
 constexpr int kIntBlock = 256;     // atoms per block of the integrator
 // bits of a three-constraint unit: its first entry within the block, the places
 // of a, b and c among its atoms, and that it is one
@@ -196,7 +194,7 @@ struct Dev {
   int ngrp_all;         // groups of all windows
   int nlrfw;            // LRF build blocks: (window, first target group, count <= 64, source part)
   const int4* lrf_work;
-  double* g_lrf_part;    // [part][group][20] sums over the kLrfParts source parts (lrf_add)
+  double* g_lrf_part;    // [part][group][20] sums over the kLrfParts source parts
   // LRF sources, packed at every build: switching atom of each group
   // (x, y, z, excluded) and the group's non-q atoms (x, y, z, charge)
   double4* ls_sw;

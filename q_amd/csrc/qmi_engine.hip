@@ -786,12 +786,12 @@ static int build_device(qmi_engine* e) {
   if ((rc = dev_alloc(e, &d.g_lrf, 20 * (size_t)goff)) != 0) return rc;
   d.ngrp_all = goff;
   {
-    // LRF build: one block per (window, 64 consecutive targets, part of the
-    // sources)
+    // LRF build: one block per (window, part of the sources, 64 consecutive
+    // targets)
     std::vector<int4> lw;
     for (int wi = 0; wi < NW; ++wi)
-      for (int g0 = 0; g0 < wd[wi].ngrp; g0 += 64)
-        for (int p = 0; p < kLrfParts; ++p)
+      for (int p = 0; p < kLrfParts; ++p)
+        for (int g0 = 0; g0 < wd[wi].ngrp; g0 += 64)
           lw.push_back(make_int4(wi, wd[wi].g_off + g0, std::min(64, wd[wi].ngrp - g0), p));
     int4* lwp;
     UP(lwp, lw);
@@ -816,7 +816,7 @@ static int build_device(qmi_engine* e) {
     UP(ip, ls_n); d.ls_n = ip;
     UP(ip, ls_atom); d.ls_atom = ip;
     if ((rc = dev_alloc(e, &d.ls_sw, std::max<size_t>(1, goff))) != 0) return rc;
-    if ((rc = dev_alloc(e, &d.ls_xq, std::max<size_t>(1, ls_atom.size()))) != 0) return rc;
+    if ((rc = dev_alloc(e, &d.ls_xq, ls_atom.size() + 3)) != 0) return rc;   // (the build loads three a group)
   }
   UP(ip, sp_start); d.sp_start = ip;
   UP(ip, sp_j); d.sp_j = ip;
@@ -2326,7 +2326,7 @@ int qmi_set_autotune(qmi_engine* e, int on) {
 int qmi_tuning(qmi_engine* e, double* out, int cap) {
   if (!e || !out) return set_err(-1, "null argument");
   if (!e->prepared) return set_err(-2, "engine not prepared");
-  const double v[13] = {kQItem, 256, 64 * kLrfWaves, 256, 0, 0, kLrfParts * kLrfWaves,
+  const double v[13] = {kQItem, 256, 64, 256, 0, 0, kLrfParts,
                         e->tune_us[0], e->tune_us[1], e->tune_us[2], e->tune_us[3], e->tune_us[4], e->tune_us[5]};
   const int n = std::min(cap, 13);
   for (int k = 0; k < n; ++k) out[k] = v[k];

@@ -1429,57 +1429,82 @@ __device__ __forceinline__ double r2_pos(double ax, double ay, double az, double
 
 // Taylor terms of one source charge q at d = x(source) - centre: potential,
 // field, field gradient and its derivative (the sums of nbpw/nbww lists with
-// LRF, md.f90:5589-5700).  The derivatives of 1/r are traceless, so of the 20
-// terms only 16 are independent; with u = q/r, the sums kept are
-//   0      u              1..3   u/r^2 d_a          9       u/r^2
-//   4..8   u/r^4 d_a d_b  (xx xy xz yy yz)          10..12  u/r^4 d_a
-//   13..19 u/r^6 d_a d_b d_c  (xxx xxy xxz xyy xyz yyy yyz)
-// and the sums with a further z factor follow from r^2 = x^2 + y^2 + z^2
-// (k_lrf_reduce): 45 FP64 instructions per source, where forming all terms
-// took 58.
-constexpr int kLrfSums = 20;
-__device__ __forceinline__ void lrf_add(double s[kLrfSums], double q, double dx, double dy, double dz) {
+// LRF, md.f90:5589-5700), with the shared factors hoisted.  The terms of the
+// form u - f0 (diagonal of the gradient) and u - g d (derivative) are split:
+// acc takes the u parts and aux the sums of f0 and of g d_x, g d_y, g d_z,
+// which lrf_finish subtracts once.  Which products are fused is spelled out, as
+// for the FP32 pairs.  SET: kLrfLow the potential, field and gradient (acc 0..9),
+// kLrfHigh the derivative (acc 10..19), or both.
+// (The derivatives of 1/r are traceless, so 16 of the 20 sums and r^2 would do,
+// with 45 FP64 instructions a source for 55.  But r^2 times the squared
+// reciprocal root is 1 only to the root's 1e-12, and with the sums' other last
+// bits the gradient moves by a quantum now and then, and with it a trajectory.)
+constexpr int kLrfLow = 1, kLrfHigh = 2, kLrfSums = 20;
+template <int SET>
+__device__ __forceinline__ void lrf_add(double acc[kLrfSums], double aux[4], double q, double dx, double dy, double dz) {
+#pragma clang fp contract(off)
   const double r2 = fma(dz, dz, fma(dy, dy, dx * dx));
   const double ir = rsqrt_e(r2);
   const double ir2 = ir * ir;
-  const double u = q * ir, u3 = u * ir2, u5 = u3 * ir2, u7 = u5 * ir2;
-  s[0] += u;
-  s[1] = fma(u3, dx, s[1]); s[2] = fma(u3, dy, s[2]); s[3] = fma(u3, dz, s[3]);
-  s[9] += u3;
-  const double ax = u5 * dx, ay = u5 * dy;
-  s[4] = fma(ax, dx, s[4]); s[5] = fma(ax, dy, s[5]); s[6] = fma(ax, dz, s[6]);
-  s[7] = fma(ay, dy, s[7]); s[8] = fma(ay, dz, s[8]);
-  s[10] += ax; s[11] += ay; s[12] = fma(u5, dz, s[12]);
-  const double px = u7 * dx, py = u7 * dy;
-  const double xx = px * dx, xy = px * dy, yy = py * dy;
-  s[13] = fma(xx, dx, s[13]); s[14] = fma(xx, dy, s[14]); s[15] = fma(xx, dz, s[15]);
-  s[16] = fma(yy, dx, s[16]); s[17] = fma(xy, dz, s[17]);
-  s[18] = fma(yy, dy, s[18]); s[19] = fma(yy, dz, s[19]);
+  const double qr = q * ir;            // q / r
+  const double f0 = qr * ir2;          // q / r^3
+  const double f1 = 3.0 * f0 * ir2;    // 3 q / r^5
+  if constexpr (SET & kLrfLow) {
+    acc[0] = fma(q, ir, acc[0]);
+    acc[1] = fma(-f0, dx, acc[1]); acc[2] = fma(-f0, dy, acc[2]); acc[3] = fma(-f0, dz, acc[3]);
+    const double ax = f1 * dx, ay = f1 * dy;
+    acc[4] = fma(ax, dx, acc[4]); acc[5] = fma(ax, dy, acc[5]); acc[6] = fma(ax, dz, acc[6]);
+    acc[7] = fma(ay, dy, acc[7]); acc[8] = fma(ay, dz, acc[8]); acc[9] = fma(f1 * dz, dz, acc[9]);
+    aux[0] = fma(qr, ir2, aux[0]);
+  }
+  if constexpr (SET & kLrfHigh) {
+    // f2 (5 d_a d_b d_c - r2 (delta_ab d_c + delta_ac d_b + delta_bc d_a))
+    const double f2 = -f1 * ir2;       // -3 q / r^7
+    const double c5 = 5.0 * f2, g = f2 * r2;
+    const double px = c5 * dx, py = c5 * dy;
+    const double xx = px * dx, yy = py * dy, zz = c5 * dz * dz;
+    acc[10] = fma(xx, dx, acc[10]); acc[11] = fma(xx, dy, acc[11]); acc[12] = fma(xx, dz, acc[12]);
+    acc[13] = fma(yy, dx, acc[13]); acc[14] = fma(px * dy, dz, acc[14]); acc[15] = fma(zz, dx, acc[15]);
+    acc[16] = fma(yy, dy, acc[16]); acc[17] = fma(yy, dz, acc[17]); acc[18] = fma(zz, dy, acc[18]);
+    acc[19] = fma(zz, dz, acc[19]);
+    aux[1] = fma(g, dx, aux[1]); aux[2] = fma(g, dy, aux[2]); aux[3] = fma(g, dz, aux[3]);
+  }
+}
+template <int SET>
+__device__ __forceinline__ void lrf_finish(double acc[kLrfSums], const double aux[4]) {
+#pragma clang fp contract(off)
+  if constexpr (SET & kLrfLow) {
+    acc[4] -= aux[0]; acc[7] -= aux[0]; acc[9] -= aux[0];
+  }
+  if constexpr (SET & kLrfHigh) {
+    acc[10] = fma(-3.0, aux[1], acc[10]); acc[11] -= aux[2]; acc[12] -= aux[3];
+    acc[13] -= aux[1]; acc[15] -= aux[1];
+    acc[16] = fma(-3.0, aux[2], acc[16]); acc[17] -= aux[3]; acc[18] -= aux[2];
+    acc[19] = fma(-3.0, aux[3], acc[19]);
+  }
 }
 
-// Build: one lane per target group; a block takes 64 consecutive targets and
-// one of kLrfParts parts of the window's source groups, each of its kLrfWaves
-// waves a contiguous share of the part.  The sources are the same for all
-// lanes, so they are read into scalar registers.  Every wave sums its sources
-// in index order, the waves are added pairwise in LDS in a fixed order and the
-// parts in k_lrf_reduce, so the sums depend on neither batch nor scheduling.
+// Build: one lane per target group; a block is a wave, which takes 64 consecutive
+// targets and one of kLrfParts parts of the window's source groups.  The sources
+// are the same for all lanes, so they are read into scalar registers.  Every wave
+// sums its sources in index order and k_lrf_reduce adds the parts in theirs, so
+// the sums depend on neither batch nor scheduling.
 //
-// Bound by the FP64 rate for many windows (46 instructions a term at one per
-// 4 cycles, of 1.04 ms for the 64-window ladder's 820 M terms) and by latency
-// for one, which is why the sources are cut 32 ways (one 1109-water window:
-// 576 waves on 1024 SIMDs); the split stays within the block, so 4 partial
-// sums a group go through memory and not 32.  Loading the next group's record
-// and sources ahead costs 34 registers and with them three of seven waves a
-// SIMD: 1.54 ms for the ladder against 1.38 without.  With sources broadcast
-// through LDS and vector loads, all terms formed and 8 parts it was 2.07 ms,
-// and 131 us for the one window, now 40.
-__global__ void __launch_bounds__(64 * kLrfWaves, 4) k_lrf_build(Dev d) {
-  const int4 lw = d.lrf_work[blockIdx.x];   // window, first target group, count, source part
-  const WinState& st = d.ws[lw.x];
+// Bound by the FP64 rate for many windows (55 instructions a source at one per 4
+// cycles, 1.2 of the 2.0 ms that the 64-window ladder's 820 M take; blocks of
+// 256 threads 2.3 ms) and by latency for few, whose waves are fewer than the
+// SIMDs.  Those take SPLIT: two waves for one, each with one of the sums' two
+// sets, the next group's record and first three sources loaded while the current
+// ones are summed, three sources at a time.  One ligand-in-water window 132 us
+// without, 68 with; one protein window 310 and 189; the ladder 2005 and 3035 (the
+// common factors are formed twice).
+constexpr int kLrfSplitMost = 1024;   // waves without SPLIT, one a SIMD: 5, 7, 9 small windows (720, 1008, 1296)
+                                      // 153, 172, 176 us without and 119, 160, 194 with
+template <int SET>
+__device__ __forceinline__ void lrf_wave(const Dev& d, int4 lw) {
+  constexpr bool kAhead = SET != (kLrfLow | kLrfHigh);
   const WinDev& W = d.win[lw.x];
-  if (!st.active || !st.list_now || !W.use_lrf) return;   // uniform over the block
-  __shared__ double s_sum[kLrfWaves / 2][kLrfSums][64];
-  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int lane = threadIdx.x & 63;
   const int g = lw.y + lane;
   bool g_ok = lane < lw.z;
   double4 sg = make_double4(0, 0, 0, 1);
@@ -1492,91 +1517,94 @@ __global__ void __launch_bounds__(64 * kLrfWaves, 4) k_lrf_build(Dev d) {
     cx = d.g_cent[3 * g]; cy = d.g_cent[3 * g + 1]; cz = d.g_cent[3 * g + 2];
   }
   const double rclrf2 = W.rclrf2;
-  double acc[kLrfSums];
+  double acc[kLrfSums], aux[4] = {0.0, 0.0, 0.0, 0.0};
   for (int k = 0; k < kLrfSums; ++k) acc[k] = 0.0;
-  constexpr int P = kLrfParts * kLrfWaves;
-  const int sub = lw.w * kLrfWaves + wv;
   // (wave-uniform: kept in scalar registers, with what they index)
-  const int h_beg = __builtin_amdgcn_readfirstlane(W.g_off + (int)(((long long)sub * W.ngrp) / P));
-  const int h_end = __builtin_amdgcn_readfirstlane(W.g_off + (int)(((long long)(sub + 1) * W.ngrp) / P));
+  const int h_beg = __builtin_amdgcn_readfirstlane(W.g_off + (int)(((long long)lw.w * W.ngrp) / kLrfParts));
+  const int h_end = __builtin_amdgcn_readfirstlane(W.g_off + (int)(((long long)(lw.w + 1) * W.ngrp) / kLrfParts));
   const int h_sol = __builtin_amdgcn_readfirstlane(min(max(W.g_off + W.ngrp_solute, h_beg), h_end));
   const ConstD sw = (ConstD)(const double*)d.ls_sw, xq = (ConstD)(const double*)d.ls_xq;
   const ConstI nn = (ConstI)d.ls_n;
   // the groups' sources are consecutive
   int f = __builtin_amdgcn_readfirstlane(h_beg < h_end ? d.ls_first[h_beg] : 0);
+  // in range of the group whose switching atom is at s (a target is within the
+  // cut-off of itself)
+  auto in_range = [&](double x, double y, double z, double excluded, double rc2) {
+    const double r2g = r2_pos(sg.x, sg.y, sg.z, x, y, z);
+    return excluded == 0.0 && g_ok && !(r2g <= rc2) && !(r2g > rclrf2);
+  };
+  double hs[4], a[12];
+  int n = 0;
+  if (kAhead && h_beg < h_end) {
+    n = nn[h_beg];
+    for (int k = 0; k < 4; ++k) hs[k] = sw[4 * (size_t)h_beg + k];
+    for (int k = 0; k < 12; ++k) a[k] = xq[4 * (size_t)f + k];
+  }
+#pragma unroll 1
   for (int seg = 0; seg < 2; ++seg) {
     // cut-off against a solute, then against a water source group
     const double rc2 = seg ? (gw ? W.rcww2 : W.rcpw2) : (gw ? W.rcpw2 : W.rcpp2);
     const int h1 = seg ? h_end : h_sol;
+#pragma unroll 1
     for (int h = seg ? h_sol : h_beg; h < h1; ++h) {
-      const int n = nn[h];
-      const ConstD hs = sw + 4 * (size_t)h;
-      // (a target is within the cut-off of itself)
-      const double r2g = r2_pos(sg.x, sg.y, sg.z, hs[0], hs[1], hs[2]);
-      if (hs[3] == 0.0 && g_ok && !(r2g <= rc2) && !(r2g > rclrf2)) {
-        for (int k = 0; k < n; ++k) {
-          const ConstD a = xq + 4 * (size_t)(f + k);
-          lrf_add(acc, a[3], a[0] - cx, a[1] - cy, a[2] - cz);
+      if constexpr (kAhead) {
+        // (the last group loads itself again)
+        const int hn = h + 1 < h_end ? h + 1 : h, fn = h + 1 < h_end ? f + n : f, n1 = nn[hn];
+        double hs1[4], a1[12];
+        for (int k = 0; k < 4; ++k) hs1[k] = sw[4 * (size_t)hn + k];
+        for (int k = 0; k < 12; ++k) a1[k] = xq[4 * (size_t)fn + k];
+        if (in_range(hs[0], hs[1], hs[2], hs[3], rc2)) {
+          if (n == 3) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) lrf_add<SET>(acc, aux, a[4 * k + 3], a[4 * k] - cx, a[4 * k + 1] - cy, a[4 * k + 2] - cz);
+          } else {
+            for (int k = 0; k < n; ++k) {
+              const ConstD b = xq + 4 * (size_t)(f + k);
+              lrf_add<SET>(acc, aux, b[3], b[0] - cx, b[1] - cy, b[2] - cz);
+            }
+          }
         }
+        f = fn;
+        n = n1;
+        for (int k = 0; k < 4; ++k) hs[k] = hs1[k];
+        for (int k = 0; k < 12; ++k) a[k] = a1[k];
+      } else {
+        const int m = nn[h];
+        const ConstD s = sw + 4 * (size_t)h;
+        if (in_range(s[0], s[1], s[2], s[3], rc2)) {
+#pragma unroll 1
+          for (int k = 0; k < m; ++k) {
+            const ConstD b = xq + 4 * (size_t)(f + k);
+            lrf_add<SET>(acc, aux, b[3], b[0] - cx, b[1] - cy, b[2] - cz);
+          }
+        }
+        f += m;
       }
-      f += n;
     }
   }
-  // waves s .. 2s-1 onto waves 0 .. s-1
-#pragma unroll
-  for (int s = kLrfWaves / 2; s > 0; s >>= 1) {
-    if (wv >= s && wv < 2 * s)
-      for (int k = 0; k < kLrfSums; ++k) s_sum[wv - s][k][lane] = acc[k];
-    __syncthreads();
-    if (wv < s)
-      for (int k = 0; k < kLrfSums; ++k) acc[k] += s_sum[wv][k][lane];
-    __syncthreads();
-  }
-  if (wv != 0 || !g_ok) return;
+  if (!g_ok) return;
+  lrf_finish<SET>(acc, aux);
   double* out = d.g_lrf_part + kLrfSums * ((size_t)lw.w * d.ngrp_all + g);
-  for (int k = 0; k < kLrfSums; ++k) out[k] = acc[k];
+  for (int k = SET & kLrfLow ? 0 : 10; k < (SET & kLrfHigh ? kLrfSums : 10); ++k) out[k] = acc[k];
+}
+template <bool SPLIT>
+__global__ void __launch_bounds__(64, 4) k_lrf_build(Dev d) {
+  const int4 lw = q_item(d.lrf_work, SPLIT ? blockIdx.x >> 1 : blockIdx.x);   // window, first target group, count, source part
+  if (!d.ws[lw.x].active || !d.ws[lw.x].list_now || !d.win[lw.x].use_lrf) return;
+  if (!SPLIT) lrf_wave<kLrfLow | kLrfHigh>(d, lw);
+  else if (blockIdx.x & 1) lrf_wave<kLrfHigh>(d, lw);
+  else lrf_wave<kLrfLow>(d, lw);
 }
 
-// sum of the source parts in part order, one thread per (group, sum), then
-// the 20 Taylor terms of each group from its sums
-constexpr int kLrfReduceGroups = 12;
-__global__ void __launch_bounds__(kLrfReduceGroups * kLrfSums) k_lrf_reduce(Dev d) {
-  __shared__ double s_v[kLrfReduceGroups][kLrfSums];
-  const int lg = threadIdx.x / kLrfSums, k = threadIdx.x % kLrfSums, g = blockIdx.x * kLrfReduceGroups + lg;
-  bool on = g < d.ngrp_all;
-  if (on) {
-    const int w = d.g_win[g];
-    on = d.ws[w].active && d.ws[w].list_now && d.win[w].use_lrf && d.ls_sw[g].w == 0.0;
-  }
+// sum of the source parts in part order, one thread per (group, term)
+__global__ void __launch_bounds__(256) k_lrf_reduce(Dev d) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= kLrfSums * d.ngrp_all) return;
+  const int g = i / kLrfSums, w = d.g_win[g];
+  if (!d.ws[w].active || !d.ws[w].list_now || !d.win[w].use_lrf || d.ls_sw[g].w != 0.0) return;
   double v = 0.0;
-  if (on)
-    for (int p = 0; p < kLrfParts; ++p) v += d.g_lrf_part[((size_t)p * d.ngrp_all + g) * kLrfSums + k];
-  s_v[lg][k] = v;
-  __syncthreads();
-  if (!on) return;
-  const double* s = s_v[lg];
-  double o;
-  switch (k) {
-    case 0: o = s[0]; break;
-    case 1: case 2: case 3: o = -s[k]; break;
-    case 4: o = 3.0 * s[4] - s[9]; break;                        // xx
-    case 5: o = 3.0 * s[5]; break;
-    case 6: o = 3.0 * s[6]; break;
-    case 7: o = 3.0 * s[7] - s[9]; break;                        // yy
-    case 8: o = 3.0 * s[8]; break;
-    case 9: o = 3.0 * (s[9] - s[4] - s[7]) - s[9]; break;        // zz
-    case 10: o = 9.0 * s[10] - 15.0 * s[13]; break;              // xxx
-    case 11: o = 3.0 * s[11] - 15.0 * s[14]; break;              // xxy
-    case 12: o = 3.0 * s[12] - 15.0 * s[15]; break;              // xxz
-    case 13: o = 3.0 * s[10] - 15.0 * s[16]; break;              // xyy
-    case 14: o = -15.0 * s[17]; break;                           // xyz
-    case 15: o = 3.0 * s[10] - 15.0 * (s[10] - s[13] - s[16]); break;   // xzz
-    case 16: o = 9.0 * s[11] - 15.0 * s[18]; break;              // yyy
-    case 17: o = 3.0 * s[12] - 15.0 * s[19]; break;              // yyz
-    case 18: o = 3.0 * s[11] - 15.0 * (s[11] - s[14] - s[18]); break;   // yzz
-    default: o = 9.0 * s[12] - 15.0 * (s[12] - s[15] - s[19]); break;   // zzz
-  }
-  d.g_lrf[20 * (size_t)g + k] = o;
+  for (int p = 0; p < kLrfParts; ++p) v += d.g_lrf_part[(size_t)p * kLrfSums * d.ngrp_all + i];
+  d.g_lrf[i] = v;
 }
 
 // Evaluation per atom (lrf_taylor, md.f90:3646-3712), FP64.
@@ -2972,8 +3000,9 @@ void launch_offdiag(const Dev& d, hipStream_t s) {
 void launch_lrf_build(const Dev& d, hipStream_t s) {
   if (!d.nlrfw) return;
   k_lrf_pack<<<blocks(std::max(d.ngrp_all, d.nls), 256), 256, 0, s>>>(d);
-  k_lrf_build<<<d.nlrfw, 64 * kLrfWaves, 0, s>>>(d);
-  k_lrf_reduce<<<blocks(d.ngrp_all, kLrfReduceGroups), kLrfReduceGroups * kLrfSums, 0, s>>>(d);
+  if (d.nlrfw <= kLrfSplitMost) k_lrf_build<true><<<2 * d.nlrfw, 64, 0, s>>>(d);
+  else k_lrf_build<false><<<d.nlrfw, 64, 0, s>>>(d);
+  k_lrf_reduce<<<blocks((long long)kLrfSums * d.ngrp_all, 256), 256, 0, s>>>(d);
 }
 
 // list update: group centres and cluster spheres, then the neighbour rows

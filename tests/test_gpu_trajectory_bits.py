@@ -33,3 +33,20 @@ def test_q_sums(systems, golden, name):
     from q_amd.engine import Engine
     (got,) = T.record(Engine, [T.window(systems, name)])
     compare(golden, name, got)
+
+
+@pytest.mark.parametrize("name", [n for n, c in T.CASES.items() if c[0] == T.LRF])
+def test_lrf_sums(systems, golden, name):
+    from q_amd.engine import Engine
+    (got,) = T.record(Engine, [T.window(systems, name)])
+    compare(golden, name, got)
+
+
+def test_many_windows(systems, golden):
+    """the launches of a large engine: two solvent models, enough groups for the
+    LRF build's other form"""
+    from q_amd.engine import Engine
+    names = ["ligand_lrf", "tip3", "protein_lrf", "dual_lrf", "arith", "qcut"] + ["ligand_lrf"] * 8
+    inputs = {n: T.window(systems, n) for n in set(names)}
+    for name, got in zip(names, T.record(Engine, [inputs[n] for n in names])):
+        compare(golden, name, got)
