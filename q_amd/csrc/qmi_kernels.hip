@@ -2054,10 +2054,10 @@ __device__ __forceinline__ void atom_terms(const Dev& d, int i) {
   long long g[3] = {0, 0, 0};
   lrf_taylor_atom(d, i, g);
   restr_atom(d, i, g);
-  if (i >= d.ntot) return;
+  if (i >= d.ntot || !d.ws[d.wid[i]].active) return;   // (a stopped window keeps its last gradient, which is in fterm)
   if (STORE) {
     for (int c = 0; c < 3; ++c) d.fterm[3 * i + c] = g[c];
-  } else if (d.ws[d.wid[i]].active) {
+  } else {
     const int r = d.rslot[i];
     for (int c = 0; c < 3; ++c) {
       if (r >= 0) g[c] += d.grow[3 * (size_t)r + c] + d.gq[3 * (size_t)r + c];
