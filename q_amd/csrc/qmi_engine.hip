@@ -1490,8 +1490,9 @@ int qmi_window_add(qmi_engine* e, const char* inp_path, long long seed_override,
   return 0;
 }
 
-// The times of a large engine's kernel families on its own windows (a
-// forces-only evaluation, a few repeats, HIP events on the engine's stream).
+// The times of a large engine's kernel families on its own windows, at the
+// state and lists of qmi_prepare (a few repeats, HIP events on the engine's
+// stream).
 // The launch shapes are fixed: the step's kernels share the GPU, and the times
 // of one alone do not tell which shape is the better among the others.
 static int time_families(qmi_engine* e) {
@@ -1514,10 +1515,6 @@ static int time_families(qmi_engine* e) {
     }
     return best;
   };
-  // a forces-only state with fresh lists and LRF expansions
-  launch_begin(d, e->stream, 2, 1);
-  launch_lists(d, e->stream, e->ngrp, e->nwc, e->nsc);
-  HIP_OK(hipStreamSynchronize(e->stream));
   e->tune_us[0] = time_us([&] { launch_q(d, e->stream, false); });
   e->tune_us[1] = time_us([&] { launch_nonbonded(d, e->stream, true, false); });
   e->tune_us[2] = time_us([&] { launch_lrf_build(d, e->stream); });
@@ -1552,6 +1549,11 @@ int qmi_prepare(qmi_engine* e) {
   if (!e->copy_ev) HIP_OK(hipEventCreateWithFlags(&e->copy_ev, hipEventDisableTiming));
   int rc = build_device(e);
   if (rc) return rc;
+  // lists and LRF expansions at the starting coordinates (of a forces-only
+  // evaluation), for pair-list queries and evaluations that keep the lists
+  launch_begin(e->d, e->stream, 2, 1);
+  launch_lists(e->d, e->stream, e->ngrp, e->nwc, e->nsc);
+  HIP_OK(hipGetLastError());
   if (e->autotune && (rc = time_families(e)) != 0) return rc;
   for (auto& h : e->wins) {
     Window& W = *h.w;
