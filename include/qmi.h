@@ -65,8 +65,9 @@ int qmi_window_add(qmi_engine* e, const char* inp_path, long long seed_override,
  * qmi_prepare. */
 int qmi_window_set_log(qmi_engine* e, int w, const char* path);
 
-/* Upload all windows to the GPU, build the static Q-atom lists, pick launch shapes
- * and capture the step graph.  Replaces distribute_nonbonds
+/* Upload all windows to the GPU and build the static Q-atom lists and the pair
+ * lists at the starting coordinates (the step graphs are captured by the first
+ * qmi_run).  Replaces distribute_nonbonds
  * (md.f90:1044-1361) and the set-up half of md_run (md.f90:3917-4000). */
 int qmi_prepare(qmi_engine* e);
 

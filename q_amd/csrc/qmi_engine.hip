@@ -103,7 +103,7 @@ struct qmi_engine {
   // whether qmi_prepare times the kernel families of a large engine
   bool autotune = true;
   double tune_us[6] = {0, 0, 0, 0, 0, 0};
-  // the launch sequence of one MD step, captured when first needed and
+  // the launch sequence of one MD step, captured at the first run and
   // replayed: index bit 0 with the pair-list and LRF kernels (some window
   // updates its lists), bit 1 with the energy terms (some window computes
   // energies); bit 2: that step and kPlainSteps without either
@@ -1849,6 +1849,14 @@ int qmi_run(qmi_engine* e, long long nsteps, int finalize) {
     }
     return ok;
   };
+  // every graph that the windows' intervals can ask for before the first step, so
+  // that no later step waits for a capture
+  if (!e->timing_on && nsteps > 0 && !e->step_exec[0]) {
+    bool any_energy = false;
+    for (auto& h : e->wins) any_energy = any_energy || h.w->inp.iene_cycle > 0 || h.w->inp.iout_cycle > 0;
+    for (int k = 0; k < 8; ++k)
+      if (any_energy || !(k & 2)) (void)have_graph(k);
+  }
   // whether any window updates its pair lists at step `k` of this run (the
   // condition k_begin evaluates per window; k_begin flags a window whose
   // update would be skipped)
