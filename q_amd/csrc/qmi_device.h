@@ -313,7 +313,7 @@ struct Dev {
   // water shells
   ShellDev* shells;
   double* wtheta;        // windows of more than kWpolLds waters: theta per shell and water, at WinDev::wp_off
-  int wpol_wide;         // some window has such rows
+  int wpol_wide;         // some shell starts with more waters than LDS holds
   int nwat_total;
   // energy snapshots for output: [ring slot][window][E_NSLOT] + temperature
   long long* e_ring;

@@ -234,6 +234,7 @@ static int build_device(qmi_engine* e) {
   // shells
   std::vector<ShellDev> shells;
   long long wp_rows = 0;
+  bool wpol_wide = false;
   // static Q lists (Dev::qw_on .. qp_work)
   std::vector<uint8_t> qw_on, qp_on;
   std::vector<uint16_t> qp14;
@@ -721,7 +722,21 @@ static int build_device(qmi_engine* e) {
     D.nshell = (int)W.wshell.size();
     if (D.nshell > kWpolMaxShell) return set_err(-10, "more than 8 water polarisation shells");
     D.wp_off = wp_rows;
-    if (W.nwat > kWpolLds) wp_rows += (long long)D.nshell * W.nwat;
+    if (W.nwat > kWpolLds) {
+      wp_rows += (long long)D.nshell * W.nwat;
+      // members of each shell at the start (as watpol_block finds them)
+      std::vector<int> members(D.nshell, 0);
+      for (int k = 0; k < W.nwat && D.nshell > 0 && D.wpol; ++k) {
+        const int o = NS + 3 * k;
+        double r2 = 0.0;
+        for (int c = 0; c < 3; ++c) r2 += (W.x[3 * o + c] - t.xwcent[c]) * (W.x[3 * o + c] - t.xwcent[c]);
+        const double r = std::sqrt(r2);
+        if (t.excl[o] || !(r > (double)(W.wshell.back().rout - W.wshell.back().dr))) continue;
+        int is = D.nshell - 1;
+        while (is > 0 && r > W.wshell[is].rout) --is;
+        if (++members[is] > kWpolLds) wpol_wide = true;
+      }
+    }
     for (auto& sh : W.wshell) {
       ShellDev s{};
       s.rout = sh.rout; s.dr = sh.dr; s.cstb = sh.cstb; s.theta_corr = sh.theta_corr;
@@ -1188,7 +1203,7 @@ static int build_device(qmi_engine* e) {
   ShellDev* sd;
   UP(sd, shells); d.shells = sd;
   if ((rc = dev_alloc(e, &d.wtheta, (size_t)wp_rows)) != 0) return rc;
-  d.wpol_wide = wp_rows > 0;
+  d.wpol_wide = wpol_wide;
   d.nwat_total = e->nwat_total;
   // two chunks of kChunk steps: one drains while the next runs
   d.ring_n = 2 * kChunk;

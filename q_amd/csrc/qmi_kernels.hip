@@ -3095,7 +3095,8 @@ void launch_nonbonded(const Dev& d, hipStream_t s, bool with_ww, bool q_energy) 
 }
 
 // Shells beyond LDS are ordered by counting in memory, for which the blocks are
-// wide; else 256 threads order as fast as 1024 (a step of 8 protein windows 116
+// wide (one window with a shell of more than 4096 of its 13056 waters: an
+// evaluation 20 ms, with the 512 threads of k_all 33); else 256 threads order as fast as 1024 (a step of 8 protein windows 116
 // and 116 us) and share a launch with the bonded terms
 void launch_other_forces(const Dev& d, hipStream_t s) {
   const int nwp = d.nwat_total ? d.nwin * kWpolMaxShell : 0;
@@ -3124,7 +3125,9 @@ static void launch_all(const Dev& d, hipStream_t s, bool energy, bool terms) {
     else k_all<false, false><<<p.total, kAllBlock, 0, s>>>(d, p);
   }
 }
-bool small_engine(const Dev& d, bool mixed_solvent) { return !mixed_solvent && all_plan(d, true, true).total <= kAllMost; }
+bool small_engine(const Dev& d, bool mixed_solvent) {
+  return !mixed_solvent && !d.wpol_wide && all_plan(d, true, true).total <= kAllMost;
+}
 
 // the lists and forces of a small engine: one launch for the forces, and on
 // list steps the LRF expansions beside the rows and the forces
