@@ -18,7 +18,8 @@ import numpy as np
 STEPS = (25, 120)   # one list update; four, and the polarisation's update at step 100
 EVERY = 37          # components kept as values beside the digest of all
 Q, LRF = "q-atoms, no LRF", "LRF"
-# name: (what it covers, configuration, input options)
+STATES = "numbers of states"
+# name: (what it covers, configuration, input options; states other than 2)
 CASES = {
     "ligand": (Q, "ligwat", dict(lrf=False)),
     "tip3": (Q, "ligtip3", dict(lrf=False)),
@@ -30,14 +31,57 @@ CASES = {
     "ligand_lrf": (LRF, "ligwat", {}),
     "dual_lrf": (LRF, "ligdual", {}),
     "protein_lrf": (LRF, "protein", {}),
+    "one": (STATES, "ligwat", dict(states=1)),
+    "three": (STATES, "ligwat", dict(states=3)),
+    "four": (STATES, "ligqcut", dict(states=4)),
+    "four_tip3": (STATES, "ligtip3", dict(states=4)),
+    "three_protein": (STATES, "protein", dict(states=3)),
 }
+LAMBDAS = {1: (1.0,), 3: (0.5, 0.2, 0.3), 4: (0.4, 0.3, 0.2, 0.1)}
+
+
+def with_states(inp, n):
+    """The window of `inp` (two states) with n: state 3 has the types and terms of
+    the first and state 4 those of the second, with charges of their own"""
+    folder = os.path.dirname(inp)
+    text = open(inp).read().split("\n")
+    k = next(i for i, l in enumerate(text) if l.startswith("fep "))
+    fep = text[k].split()[1]
+    text[k] = f"fep {n}_{fep}"
+    k = text.index("[lambdas]") + 1
+    text[k] = " ".join(f"{v:.6f}" for v in LAMBDAS[n])
+    out, section = [], ""
+    for line in open(os.path.join(folder, fep)):
+        t = line.split()
+        if line.startswith("["):
+            section = t[0]
+        elif t and t[0] == "states":
+            line = f"states {n}\n"
+        elif t and (section.startswith("[change_") or section == "[softcore]"):
+            two = t[-2:]
+            if section == "[change_charges]":
+                mean = 0.5 * (float(two[0]) + float(two[1]))
+                two += [f"{mean:.4f}", f"{0.9 * mean:.4f}"]
+            else:
+                two += two
+            line = " ".join(t[:-2] + two[:n]) + "\n"
+        out.append(line)
+    with open(os.path.join(folder, f"{n}_{fep}"), "w") as f:
+        f.writelines(out)
+    path = os.path.join(folder, f"states{n}_{os.path.basename(inp)}")
+    with open(path, "w") as f:
+        f.write("\n".join(text))
+    return path
 
 
 def window(make, name):
     """input file of a case; make(config, seed=, **options)"""
     _, config, options = CASES[name]
-    return make(config, seed=2 if config == "protein" else 0, md_seed=7, lam=0.3, steps=100000, energy=10,
-                output=100000, **options)
+    options = dict(options)
+    states = options.pop("states", 2)
+    inp = make(config, seed=2 if config == "protein" else 0, md_seed=7, lam=0.3, steps=100000, energy=10,
+               output=100000, **options)
+    return inp if states == 2 else with_states(inp, states)
 
 
 def record(Engine, inputs):

@@ -50,3 +50,19 @@ def test_many_windows(systems, golden):
     inputs = {n: T.window(systems, n) for n in set(names)}
     for name, got in zip(names, T.record(Engine, [inputs[n] for n in names])):
         compare(golden, name, got)
+
+
+@pytest.mark.parametrize("name", [n for n, c in T.CASES.items() if c[0] == T.STATES])
+def test_states(systems, golden, name):
+    from q_amd.engine import Engine
+    (got,) = T.record(Engine, [T.window(systems, name)])
+    compare(golden, name, got)
+
+
+def test_states_together(systems, golden):
+    """windows of one to four states in one launch, with one solvent model and
+    with two"""
+    from q_amd.engine import Engine
+    for names in (["one", "ligand_lrf", "three", "four"], ["four_tip3", "one", "three_protein", "ligand_lrf", "four"]):
+        for name, got in zip(names, T.record(Engine, [T.window(systems, n) for n in names])):
+            compare(golden, name, got)
