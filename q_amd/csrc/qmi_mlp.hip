@@ -435,7 +435,7 @@ struct qmi_mlp {
   hip_bfloat16* pb = nullptr;   // BF16 working copy
   float *g = nullptr, *m = nullptr, *v = nullptr;
   Packs pk{};                   // packed weights of a fused network (pk.ip != 0)
-  float* part = nullptr;        // fused: partial gradients of kPartBlocks blocks
+  float* part = nullptr;        // fused: partial gradients of kPartBlocks blocks, from the first gradient on
   long long step = 0;
   // activations for a batch of up to cap rows
   int cap = 0;
@@ -477,6 +477,13 @@ int ensure_batch(qmi_mlp* M, int B) {
   if ((rc = M->alloc(&M->loss, 1)) != 0) return rc;
   M->cap = B;
   return 0;
+}
+
+// the buffer of a fused network's partial gradients (21 MB for 34 inputs and 128
+// hidden units), which a network that only predicts has no use for
+int ensure_part(qmi_mlp* M) {
+  if (!M->pk.ip || M->part) return 0;
+  return M->alloc(&M->part, (size_t)kPartBlocks * (M->np + 1));
 }
 
 template <typename TA_, typename TB_, bool TA, bool TB>
@@ -619,7 +626,7 @@ int qmi_mlp_create(int hip_device, int n_in, int n_hidden, unsigned long long se
     M->pk = Packs{n_in, n_hidden, n_in <= 64 ? 64 : 128, nullptr, nullptr, nullptr};
     unsigned short* w = nullptr;
     const size_t n1 = (size_t)kHp * M->pk.ip, n2 = (size_t)kHp * kHp;
-    if ((rc = M->alloc(&w, n1 + 2 * n2)) || (rc = M->alloc(&M->part, (size_t)kPartBlocks * (M->np + 1)))) {
+    if ((rc = M->alloc(&w, n1 + 2 * n2)) != 0) {
       delete M;
       return rc;
     }
@@ -713,7 +720,7 @@ int qmi_mlp_grad(qmi_mlp* M, const float* x, const float* t, int batch, float* l
   if (!M || !x || !t || batch < 1) return mlp_err(-1, "invalid argument");
   MLP_OK(hipSetDevice(M->device));
   int rc;
-  if ((rc = ensure_batch(M, batch)) != 0) return rc;
+  if ((rc = ensure_batch(M, batch)) != 0 || (rc = ensure_part(M)) != 0) return rc;
   MLP_OK(hipMemcpyAsync(M->x, x, (size_t)batch * M->n_in * 4, hipMemcpyHostToDevice, M->s));
   MLP_OK(hipMemcpyAsync(M->t, t, (size_t)batch * 4, hipMemcpyHostToDevice, M->s));
   if (M->pk.ip) {
@@ -740,7 +747,7 @@ int qmi_mlp_train(qmi_mlp* M, const float* X, const float* T, int n, int epochs,
   MLP_OK(hipSetDevice(M->device));
   batch = std::min(batch, n);
   int rc;
-  if ((rc = ensure_batch(M, batch)) != 0) return rc;
+  if ((rc = ensure_batch(M, batch)) != 0 || (rc = ensure_part(M)) != 0) return rc;
   // the training set, the row order and the last pass's losses stay on the
   // device for the whole call
   const size_t nx = (size_t)n * M->n_in, per_pass = (size_t)(n / batch);
