@@ -299,11 +299,16 @@ __global__ void __launch_bounds__(kFusedBlock) k_mlp(int B, Net N, const float* 
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const float d1 = d1a[k] * silu_d(z1[k]);
-        s_d[4 * q + k][h] = d1;   // the wave's own columns, which it alone reads below
+        s_d[4 * q + k][h] = d1;   // the wave's own columns, which its other lanes read below
         t1 += d1;
       }
       gb1 += t1;
+      // (a wave's LDS accesses are in order; the fence keeps the compiler from
+      // moving the loads before the other lanes' stores, which a wave barrier
+      // alone does not promise)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
       for (int m = 0; m < 4; ++m) dr[m] = s_d[4 * m + q][h];
 #pragma unroll
