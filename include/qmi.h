@@ -130,7 +130,7 @@ int qmi_set_autotune(qmi_engine* e, int on);
 
 /* The launch shapes: q-atoms per chunk of the q kernels, threads per block of
  * the row, LRF-build and bonded kernels, 0 (blocks are not grouped by XCD), 0
- * (the bonded mode), the number of source shares of the LRF build; then
+ * (the bonded mode), the number of source parts of the LRF build; then
  * microseconds measured by qmi_prepare, 0 when it measured none: q kernels, all
  * pair kernels, LRF build, bonded terms with polarisation and restraints, all
  * pair kernels and the bonded terms again (13 values).  Returns the number
@@ -142,10 +142,13 @@ int qmi_tuning(qmi_engine* e, double* out, int cap);
 int qmi_set_timing(qmi_engine* e, int on);
 
 /* Device time per kernel family of the last qmi_run, in microseconds per
- * step (no reference counterpart).  Order: pair-list + LRF build,
- * nonbonded tiles, bonded + sequence restraints + water polarisation, LRF
+ * step (no reference counterpart).  Order: pair-list + LRF build, all pair
+ * kernels, bonded + sequence restraints + water polarisation, LRF
  * evaluation + atom restraints + leapfrog + SHAKE + thermostat, the
- * water-water tile kernel alone, wall-clock total.  All but
+ * water-water rows alone, wall-clock total.  With timing on a family's kernels
+ * are launched by themselves and one after the other, where other steps hold
+ * several families in one launch: the results are the same, the times do not
+ * add up to such a step's.  All but
  * the last are zero unless qmi_set_timing was on.  Returns the number of
  * values written. */
 int qmi_timings(qmi_engine* e, double* out, int cap);

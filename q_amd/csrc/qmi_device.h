@@ -158,7 +158,7 @@ struct Dev {
   const int* wslot;
   double4* xwd;         // the same in FP64 (x, y, z, unused), for the energy terms
   float4* sljp;         // avdw1, bvdw1, avdw3, bvdw3 of the solute slots
-  const double4* sljd;  // their rows of t_lj
+  const double4* sljd;  // the same in FP64
   // the q-atoms' x32 again, per q-cluster member slot (cluster * 8 + member;
   // zero for empty members); qmslot: per atom, its slot or -1
   float4* xq;
@@ -171,7 +171,6 @@ struct Dev {
   int nwslot;
   const int* rslot;
   long long* fterm;     // per-atom terms of the step (LRF evaluation, atom restraints), then the complete gradient
-  const float* winv;
   const double* mass;
   const int* wid;       // window of atom
   const int* iac;       // 0-based window-local atom type
@@ -247,8 +246,6 @@ struct Dev {
   const double* q_ljd;   // same in double, for the energy path
   const float* q_sc;     // [(q*natyps + t)*S + s]
   const double* q_scd;
-  // topology LJ params in double per window type (energy path)
-  const double* t_lj;    // [(t_off + t)*4]
   RowList rl[T_NTYPES];  // neighbour rows
   // bonded tiles, each of one window: (first entry of btile_terms, terms, first
   // atom, atoms spanned); btile_terms: term indices, grouped by kind within a tile
@@ -291,7 +288,6 @@ struct Dev {
   int nrst;
   const int4* rs_kwij; const int2* rs_kf; const double* rs_par;
   // shake units (independent constraint components): their constraints
-  int nsu;
   const int* su_start; const int* su_n;
   const double* sc_d2;     // per constraint: d0^2
   const float2* sc_w;      // per constraint: inverse masses of i and j
@@ -301,7 +297,7 @@ struct Dev {
   // -1); a component's atoms are listed in the order its sc_loc numbers them.
   // Blocks of k_integrate: runs of whole units of at most kIntBlock atoms,
   // (first entry, atoms, first unit, units)
-  int niu, nib;
+  int nib;
   const int4* iu; const int4* ib;
   // per entry, what the integrator needs of the atom: (atom, window, rslot,
   // wslot), (charge, inverse mass, qmslot, 1 solute | 2 excluded), mass

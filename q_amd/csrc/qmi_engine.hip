@@ -2,11 +2,11 @@
 //
 // An engine owns one HIP stream and all device memory of its windows.  At
 // qmi_prepare every window is flattened into the batched device layout of
-// qmi_device.h (per-window offsets), the static Q-atom tile lists are built
-// and the initial thermostat state is computed; qmi_run then launches, per
-// MD step and for all windows at once: list build (at list-update steps),
-// nonbonded tiles, LRF, bonded and restraint kernels, leapfrog, SHAKE and
-// the thermostat.  Energy snapshots go to a device ring that the host drains
+// qmi_device.h (per-window offsets), the static Q-atom lists and the pair
+// lists are built and the initial thermostat state is computed; qmi_run then
+// launches, per MD step and for all windows at once: list build and LRF
+// expansions (at list-update steps), pair, bonded and restraint forces,
+// leapfrog, SHAKE and the thermostat.  Energy snapshots go to a device ring that the host drains
 // after each chunk of steps to write .en records and the log.
 #include <hip/hip_runtime.h>
 
@@ -526,7 +526,7 @@ static int build_device(qmi_engine* e) {
         int col = t.natyps + pq.jq - 1;  // sc_lookup(iq, natyps+jq, s), jq = 0 gives column natyps
         qq_sc.push_back((float)fp.sc_lookup[((size_t)pq.iq * ncol + col) * S + s]);
       }
-    // --- static Q tiles: nbqplist (md.f90:7875-7964) and nbqwlist (8066-8118)
+    // --- static Q lists: nbqplist (md.f90:7875-7964) and nbqwlist (8066-8118)
     if (fp.nqat > 0) {
       const double rcq2 = p.rcq * p.rcq;
       auto r2c = [&](int a) {
@@ -538,7 +538,7 @@ static int build_device(qmi_engine* e) {
       hw.qp_pairs.clear();
       std::vector<char> wlisted(W.nwat, 0);
       // dynamic lists: every water and group that may come within the
-      // cut-off is tiled, and the device flags (qin) select them
+      // cut-off is listed, and the device flags (qin) select them
       const bool dyn = D.qlist_dynamic != 0;
       for (int k = 0; k < W.nwat; ++k) {
         int o = NS + 3 * k;
@@ -781,7 +781,6 @@ static int build_device(qmi_engine* e) {
   UP(d.x32, x32);
   if ((rc = dev_alloc(e, &d.f, x.size())) != 0) return rc;
   if ((rc = dev_alloc(e, &d.fterm, x.size())) != 0) return rc;
-  float* fwinv; UP(fwinv, winv); d.winv = fwinv;
   double* fmass; UP(fmass, mass); d.mass = fmass;
   int* ip;
   UP(ip, wid); d.wid = ip;
@@ -1011,7 +1010,6 @@ static int build_device(qmi_engine* e) {
   UP(dp, q_ljd); d.q_ljd = dp;
   UP(fp_, q_sc); d.q_sc = fp_;
   UP(dp, q_scd); d.q_scd = dp;
-  UP(dp, t_lj); d.t_lj = dp;
   d.nqq = (int)qq_ij.size();
   int4* i4;
   UP(i4, qq_ij); d.qq_ij = i4;
@@ -1121,7 +1119,6 @@ static int build_device(qmi_engine* e) {
   }
   d.nrst = (int)rs_kwij.size();
   UP(i4, rs_kwij); d.rs_kwij = i4; UP(i2, rs_kf); d.rs_kf = i2; UP(dp, rs_par); d.rs_par = dp;
-  d.nsu = (int)su_n.size();
   UP(ip, su_start); d.su_start = ip; UP(ip, su_n); d.su_n = ip;
   UP(up, sc_loc); d.sc_loc = up;
   {
@@ -1193,7 +1190,6 @@ static int build_device(qmi_engine* e) {
     float4* fp4;
     UP(i4, ie_i); d.ie_i = i4; UP(fp4, ie_f); d.ie_f = fp4; UP(dp, ie_m); d.ie_m = dp;
     UP(dp, tri_d2); d.tri_d2 = dp; UP(fp4, tri); d.tri = fp4;
-    d.niu = (int)iu.size();
     d.nib = (int)ib.size();
     UP(i4, iu); d.iu = i4;
     UP(i4, ib); d.ib = i4;
@@ -1531,7 +1527,7 @@ static int time_families(qmi_engine* e) {
     return best;
   };
   e->tune_us[0] = time_us([&] { launch_q(d, e->stream, false); });
-  e->tune_us[1] = time_us([&] { launch_nonbonded(d, e->stream, true, false); });
+  e->tune_us[1] = time_us([&] { launch_pair_forces(d, e->stream); });
   e->tune_us[2] = time_us([&] { launch_lrf_build(d, e->stream); });
   e->tune_us[3] = e->tune_us[5] = time_us([&] { launch_other_forces(d, e->stream); });
   e->tune_us[4] = e->tune_us[1];
@@ -1825,7 +1821,7 @@ int qmi_run(qmi_engine* e, long long nsteps, int finalize) {
   HIP_OK(hipMemcpy(e->d.ws, ws.data(), NW * sizeof(WinState), hipMemcpyHostToDevice));
   if (e->timing_on && !e->ev[0])
     for (auto& x : e->ev) HIP_OK(hipEventCreate(&x));
-  // per family: 0 lists+LRF build, 1 nonbonded tiles, 2 bonded/sequence restraints/polarisation,
+  // per family: 0 lists+LRF build, 1 all pair kernels, 2 bonded/sequence restraints/polarisation,
   // 3 per-atom terms + integrate
   double fam[5] = {0, 0, 0, 0, 0};
   auto t0 = std::chrono::steady_clock::now();
@@ -1984,7 +1980,7 @@ int qmi_run(qmi_engine* e, long long nsteps, int finalize) {
       if (e->timing_on) HIP_OK(hipEventRecord(e->ev[1], e->stream));
       launch_ww(e->d, e->stream, qen);
       if (e->timing_on) HIP_OK(hipEventRecord(e->ev[2], e->stream));
-      launch_nonbonded(e->d, e->stream, false, qen);
+      launch_nonbonded(e->d, e->stream, qen);
       if (e->timing_on) HIP_OK(hipEventRecord(e->ev[3], e->stream));
       launch_other_forces(e->d, e->stream);
       if (e->timing_on) HIP_OK(hipEventRecord(e->ev[4], e->stream));
@@ -1996,10 +1992,10 @@ int qmi_run(qmi_engine* e, long long nsteps, int finalize) {
         float ms[5];
         for (int f = 0; f < 5; ++f) HIP_OK(hipEventElapsedTime(&ms[f], e->ev[f], e->ev[f + 1]));
         fam[0] += ms[0] * 1000.0;                 // lists + LRF build
-        fam[1] += (ms[1] + ms[2]) * 1000.0;       // all nonbonded tiles
+        fam[1] += (ms[1] + ms[2]) * 1000.0;       // all pair kernels
         fam[2] += ms[3] * 1000.0;                 // bonded, sequence restraints, polarisation
         fam[3] += ms[4] * 1000.0;                 // LRF evaluation, atom restraints, leapfrog, SHAKE, thermostat
-        fam[4] += ms[1] * 1000.0;                 // water-water tiles alone
+        fam[4] += ms[1] * 1000.0;                 // water-water rows alone
       }
     }
     HIP_OK(hipGetLastError());
@@ -2273,7 +2269,7 @@ int qmi_get_pairlist(qmi_engine* e, int w, int kind, int32_t* pi, int32_t* pj, i
   };
   auto ljc = [&](int i, int j) { return W.ljcod[(t.iac[i] - 1) * t.natyps + (t.iac[j] - 1)]; };
   if (kind == QMI_LIST_QW || kind == QMI_LIST_QP) {
-    // the tiled superset, less what the last list update put out of range
+    // the static superset, less what the last list update put out of range
     std::vector<uint8_t> in(W.natom, 1);
     HIP_OK(hipMemcpy(in.data(), e->d.qin + ao, W.natom, hipMemcpyDeviceToHost));
     if (kind == QMI_LIST_QW) {

@@ -10,14 +10,15 @@ void launch_begin(const Dev& d, hipStream_t s, int eval, int rebuild);
 // EVB off-diagonal elements at an MD step's starting coordinates
 void launch_offdiag(const Dev& d, hipStream_t s);
 void launch_lists(const Dev& d, hipStream_t s, int ngrp, int nwc, int nsc);
-// water-water rows alone, and all nonbonded kernels (with or without
-// them); `energy` / `q_energy`: the kernel instances that also evaluate the
-// energy terms of windows at an energy step (false: forces only)
-void launch_ww(const Dev& d, hipStream_t s, bool energy = true);
-// single families, for timing
-void launch_q(const Dev& d, hipStream_t s, bool energy = true);
+// the timing pass: the water-water rows alone, then all other pair kernels;
+// `energy`: the instances that also evaluate the energy terms of windows at an
+// energy step (false: forces only)
+void launch_ww(const Dev& d, hipStream_t s, bool energy);
+void launch_nonbonded(const Dev& d, hipStream_t s, bool energy);
+// single families, for timing: the q kernels, the LRF build, the pair kernels
+void launch_q(const Dev& d, hipStream_t s, bool energy);
 void launch_lrf_build(const Dev& d, hipStream_t s);
-void launch_nonbonded(const Dev& d, hipStream_t s, bool with_ww = true, bool q_energy = true);
+void launch_pair_forces(const Dev& d, hipStream_t s);
 // water polarisation, bonded terms and restraint records
 void launch_other_forces(const Dev& d, hipStream_t s);
 // the per-atom terms of an MD step into their own array (Dev::fterm)

@@ -142,7 +142,6 @@ __device__ __forceinline__ T row8_sum_t(T v) {
   v += mv<kDppHalfMirror>(v);
   return v;
 }
-__device__ __forceinline__ long long row8_sum_i(long long v) { return row8_sum_t(v); }
 // sum over the 8 lanes that share lane&7: partners l^8, l^16, l^32
 template <class T>
 __device__ __forceinline__ T col8_sum_t(T v) {
@@ -181,17 +180,6 @@ __device__ __forceinline__ void wave_energy(WinState* ws, int w, int slot, doubl
 }
 
 __device__ __forceinline__ double row8_sum(double v) { return row8_sum_t(v); }
-__device__ __forceinline__ double col8_sum(double v) { return col8_sum_t(v); }
-
-// squared distance in FP64 evaluated as the reference does, left to right
-// and without fused multiply-add: (dx*dx + dy*dy) + dz*dz
-__device__ __forceinline__ double r2_exact(const double* x, int i, int j) {
-#pragma clang fp contract(off)
-  double dx = __dsub_rn(x[3 * i + 0], x[3 * j + 0]);
-  double dy = __dsub_rn(x[3 * i + 1], x[3 * j + 1]);
-  double dz = __dsub_rn(x[3 * i + 2], x[3 * j + 2]);
-  return __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz));
-}
 
 // ------------------------------------------------------ step control --
 // The gradient array is zero between steps and evaluations: the kernel that
@@ -316,12 +304,7 @@ __global__ void k_bounds(Dev d, int nwc_total, int nsc_total) {
   bs[0] = cx; bs[1] = cy; bs[2] = cz; bs[3] = n > 0 ? r : -1.0;
 }
 
-// ------------------------------------------------------- tile builder --
-// One wave per i-cluster scans the j-clusters of its window in order; each
-// lane tests one candidate j-cluster (bounding-sphere prune, then the exact
-// FP64 group tests of the reference for all 64 member pairs); surviving
-// tiles are compacted in j order (ballot + popcount), so lists are
-// deterministic.
+// ------------------------------------------------- neighbour rows --
 __device__ __forceinline__ int special_type(const Dev& d, int i, int j) {
   // 1 = excluded pair, 2 = 1-4 pair, 0 = normal (listex/list14 and the long
   // lists of topo.f90, as nbpplist checks them, md.f90:5256-5294)
@@ -333,7 +316,6 @@ __device__ __forceinline__ int special_type(const Dev& d, int i, int j) {
   return 0;
 }
 
-// ------------------------------------------------- neighbour rows --
 // Pair-list build (nbwwlist/nbpwlist/nbpplist without LRF bookkeeping,
 // md.f90:8370-8556, 6864-7068, 5448-5700): one wave per i-cluster.  Candidate
 // j-clusters come from the bounding spheres of the switching atoms; for each
@@ -429,9 +411,8 @@ __global__ void __launch_bounds__(256) k_build_rows(Dev d) {
   if (wave < np) return build_row<T_PW>(d, wave);
 }
 
-// the number of chunks of 8 entries the wave must walk: the longest row
 constexpr int kUnroll = 4;   // row entries per pass of the pair kernels
-
+// the number of chunks of 8 entries the wave must walk: the longest row
 __device__ __forceinline__ int row_chunks(int n) {
   int m = n;
   m = max(m, mv<kDppRor8>(m));
@@ -1647,7 +1628,7 @@ __device__ __forceinline__ void lrf_taylor_atom(const Dev& d, int i, long long* 
 
 // ---------------------------------------------------------- bonded --
 __device__ __forceinline__ void torsion_geom(const double* x, int i, int j, int k, int l, double* phi,
-                                             double* scp_out, double dp[12], bool inv_style) {
+                                             double* scp_out, double dp[12]) {
   double rji[3], rjk[3], rkl[3], rnj[3], rnk[3];
   for (int c = 0; c < 3; ++c) {
     rji[c] = x[3 * i + c] - x[3 * j + c];
@@ -1674,7 +1655,6 @@ __device__ __forceinline__ void torsion_geom(const double* x, int i, int j, int 
   if (fabs(f1) < 1.e-12) f1 = 1.e-12;
   f1 = -1.0 / f1;
   double di[3], dl[3];
-  (void)inv_style;
   for (int c = 0; c < 3; ++c) {
     di[c] = f1 * (rnk[c] * (bjinv * bkinv) - scp * rnj[c] * bj2inv);
     dl[c] = f1 * (rnj[c] * (bjinv * bkinv) - scp * rnk[c] * bk2inv);
@@ -1793,7 +1773,7 @@ __device__ __forceinline__ void bonded_term(const Dev& d, int t, const Sink& put
       const int4 q = d.t_ijkl[a];
       const float4 p = d.t_par[a];  // fk, rmult, deltor, paths (1/paths)
       double phi, scp, dp[12];
-      torsion_geom(x, q.x, q.y, q.z, q.w, &phi, &scp, dp, false);
+      torsion_geom(x, q.x, q.y, q.z, q.w, &phi, &scp, dp);
       const double arg = (double)p.y * phi - (double)p.z;
       e = (double)p.x * (1.0 + cos(arg)) * (double)p.w;
       const double dv = -(double)p.y * (double)p.x * sin(arg) * (double)p.w;
@@ -1808,7 +1788,7 @@ __device__ __forceinline__ void bonded_term(const Dev& d, int t, const Sink& put
       const int4 q = d.i_ijkl[a];
       const float2 p = d.i_par[a];
       double phi, scp, dp[12];
-      torsion_geom(x, q.x, q.y, q.z, q.w, &phi, &scp, dp, false);
+      torsion_geom(x, q.x, q.y, q.z, q.w, &phi, &scp, dp);
       double dv;
       if (d.i_kind[w] == 2) {
         const double arg = 2 * phi - (double)p.y;
@@ -1889,7 +1869,7 @@ __device__ __forceinline__ void bonded_term(const Dev& d, int t, const Sink& put
     if (d.ws[w].active) {
       const int4 q = tors ? d.qt_ijkl[a] : d.qi_ijkl[a];
       double phi, scp, dp[12];
-      torsion_geom(x, q.x, q.y, q.z, q.w, &phi, &scp, dp, true);
+      torsion_geom(x, q.x, q.y, q.z, q.w, &phi, &scp, dp);
       const double lam = d.win[w].lambda[s];
       double dv;
       if (tors) {
@@ -3060,10 +3040,6 @@ static void launch_wrow3(const Dev& d, hipStream_t s, bool energy) {
   if (energy) k_wrow<true, true, 3><<<nb, kRowBlock, 0, s>>>(d);
   else k_wrow<true, false, 3><<<nb, kRowBlock, 0, s>>>(d);
 }
-static void launch_wrow(const Dev& d, hipStream_t s, bool energy) {
-  if (energy) launch_wrow_k<true, 3>(d, s);
-  else launch_wrow_k<false, 3>(d, s);
-}
 void launch_ww(const Dev& d, hipStream_t s, bool energy) {
   if (energy) launch_wrow_k<true, 1>(d, s);
   else launch_wrow_k<false, 1>(d, s);
@@ -3086,12 +3062,17 @@ static void launch_srow(const Dev& d, hipStream_t s, bool energy) {
   else launch_srow_k<false>(d, s);
 }
 
-void launch_nonbonded(const Dev& d, hipStream_t s, bool with_ww, bool q_energy) {
-  if (with_ww) launch_wrow(d, s, q_energy);
-  else launch_wrow_k<false, 2>(d, s);   // added to what launch_ww stored
-  launch_srow(d, s, q_energy);
-  launch_q(d, s, q_energy);
-  launch_qq(d, s, q_energy);
+void launch_nonbonded(const Dev& d, hipStream_t s, bool energy) {
+  launch_wrow_k<false, 2>(d, s);   // added to what launch_ww stored
+  launch_srow(d, s, energy);
+  launch_q(d, s, energy);
+  launch_qq(d, s, energy);
+}
+void launch_pair_forces(const Dev& d, hipStream_t s) {
+  launch_wrow_k<false, 3>(d, s);
+  launch_srow(d, s, false);
+  launch_q(d, s, false);
+  launch_qq(d, s, false);
 }
 
 // Shells beyond LDS are ordered by counting in memory, for which the blocks are

@@ -202,7 +202,9 @@ class Engine:
         _check(self.lib.qmi_set_autotune(self._h, 1 if on else 0))
 
     def tuning(self) -> dict:
-        """launch shapes and the kernel families' times measured by prepare (us)"""
+        """launch shapes and the kernel families' times measured by prepare (us, 0
+        for a small engine): q_tiles_per_wave is q-atoms per chunk, xcd_grouped and
+        bonded_mode are 0, us.xcd repeats us.rows and us.bonded_mode us.bonded"""
         a = np.zeros(13)
         _check(self.lib.qmi_tuning(self._h, a.ctypes.data_as(C.POINTER(C.c_double)), 13))
         return dict(q_tiles_per_wave=int(a[0]), rows_block=int(a[1]), lrf_block=int(a[2]), bonded_block=int(a[3]),
